@@ -1850,6 +1850,25 @@ void pool_release(mgf_context ctx) {
     ctx->pool.streams.clear();
 }
 
+OpScratch::OpScratch(mgf_context ctx, size_t bytes) : buf(ctx->op) {
+    kept = bytes <= kOpScratchKeep && buf.mu.try_lock();
+    if (kept && buf.bytes < bytes) {
+        if (buf.p) (void)hipFree(buf.p);
+        buf.p = nullptr;
+        buf.bytes = 0;
+        if (hipMalloc(&buf.p, bytes) == hipSuccess) buf.bytes = bytes;
+        else buf.p = nullptr;
+    }
+    if (kept) p = buf.p;
+    else if (hipMalloc(&p, std::max<size_t>(bytes, 256)) != hipSuccess) p = nullptr;
+    if (!p) (void)hipGetLastError();
+}
+
+OpScratch::~OpScratch() {
+    if (kept) buf.mu.unlock();
+    else if (p) (void)hipFree(p);
+}
+
 bool lockstep_eligible(mgf_scene s) { return lock_eligible(s); }
 
 // The extrapolation layers of every scene from its offsets (in Q.offs_host):
@@ -2193,6 +2212,7 @@ mgf_status mgf_shutdown(mgf_context ctx) {
     (void)hipStreamSynchronize(ctx->stream);
     (void)hipStreamDestroy(ctx->stream);
     pool_release(ctx);
+    if (ctx->op.p) (void)hipFree(ctx->op.p);
     delete ctx;
     return MGF_OK;
 }
@@ -2852,9 +2872,14 @@ mgf_status mgf_op_particles_to_grid(mgf_context ctx, const mgf_grid* grid, int32
     if (!pg_alg_ok(alg) || alg == MGF_PG_G2PNEAREST)
         return fail(MGF_ERR_INVALID, "particle-to-grid algorithm must be P2GSUM, LINEAR, QUADRATIC or CUBIC");
     MGF_HIP(hipSetDevice(ctx->device));
-    MGF_HIP(launch_p2g(ctx->stream, make_grid(grid), field_kind, n, pos, values, span, offset, alg, field, weight,
-                       normalize));
-    MGF_HIP(hipStreamSynchronize(ctx->stream));
+    const GridDev g = make_grid(grid);
+    OpScratch work(ctx, sizeof(uint32_t) * p2g_work_words(g, n));
+    if (!work.p) return fail(MGF_ERR_NOMEM, "particle splat scratch");
+    const hipError_t e = launch_p2g(ctx->stream, g, field_kind, n, pos, values, span, offset, alg, field, weight,
+                                    normalize, static_cast<uint32_t*>(work.p));
+    const hipError_t w = hipStreamSynchronize(ctx->stream);   // also after a failed launch: the scratch is returned
+    MGF_HIP(e);
+    MGF_HIP(w);
     return MGF_OK;
 }
 

@@ -97,6 +97,19 @@ struct CtxPool {
     std::vector<Buf> bufs;
     std::vector<hipStream_t> streams;   // free streams (default priority)
 };
+// Scratch of the operator entry points, kept by the context from call to call
+// (an allocation and a free cost more than a small operator's kernels): one
+// buffer, grown to the largest call's needs up to kOpScratchKeep and freed by
+// mgf_shutdown.  OpScratch is one call's use of it; a call that needs more, or
+// finds the buffer in use by another thread's call, gets memory of its own.
+// The operators wait for their stream before they return, so the buffer is
+// idle whenever no call holds it.
+constexpr size_t kOpScratchKeep = size_t(256) << 20;
+struct OpBuf {
+    std::mutex mu;
+    void* p = nullptr;
+    size_t bytes = 0;
+};
 }  // namespace mgf
 
 struct mgf_context_s {
@@ -106,6 +119,7 @@ struct mgf_context_s {
     size_t lds_per_block = 65536;
     bool lockstep = true;   // mgf_batch_step runs eligible scenes in lockstep
     mgf::CtxPool pool;
+    mgf::OpBuf op;
 };
 
 struct mgf_scene_s {
@@ -210,6 +224,7 @@ struct mgf_psolver_s {
     // the particles binned by support corner for the splat (valid for bins_version)
     uint32_t *bin_counts = nullptr, *bin_tiles = nullptr, *bin_start = nullptr, *bin_cursor = nullptr;
     uint32_t* order = nullptr;
+    uint32_t* splat_work = nullptr;                  // scratch of the wide kernels' splat (QUADRATIC, CUBIC)
     float* acc = nullptr;                            // the splat's per-bin slots (LINEAR)
     float* pos_s = nullptr;                          // positions in bin order (3n)
     float* vel_s = nullptr;                          // velocities in bin order (3n)
@@ -219,6 +234,19 @@ struct mgf_psolver_s {
 };
 
 namespace mgf {
+
+// Device scratch for one operator call on ctx (null: the allocation failed).
+struct OpScratch {
+    OpScratch(mgf_context ctx, size_t bytes);
+    ~OpScratch();   // the context's stream must have finished with it
+    OpScratch(const OpScratch&) = delete;
+    OpScratch& operator=(const OpScratch&) = delete;
+    void* p = nullptr;
+
+private:
+    OpBuf& buf;
+    bool kept = false;
+};
 
 constexpr int kBlock = 256;
 constexpr int kMaxBlocks = 4096;   // fused reductions use at most this many blocks
@@ -557,8 +585,10 @@ hipError_t launch_fluid_sdf(hipStream_t s, const GridDev& g, const float* phi, i
                             float* out);
 // ---- particles (mgf_kernels_particles.hip); kind 0 cells, 1..3 face grids ----
 size_t pg_field_count(const GridDev& g, int kind);
+// work: p2g_work_words(g, np) words of scratch.
+size_t p2g_work_words(const GridDev& g, int64_t np);
 hipError_t launch_p2g(hipStream_t s, const GridDev& g, int kind, int64_t np, const float* pos, const float* val,
-                      int span, int off, int alg, float* field, float* weight, int normalize);
+                      int span, int off, int alg, float* field, float* weight, int normalize, uint32_t* work);
 hipError_t launch_g2p(hipStream_t s, const GridDev& g, int kind, int64_t np, const float* pos, const float* field,
                       int alg, float* val, int span, int off);
 hipError_t launch_particle_markers(hipStream_t s, const GridDev& g, const float* solid, int64_t np, const float* pos,

@@ -151,7 +151,7 @@ mgf_status particles_advect_run(hipStream_t st, const GridDev& g, Vel V, int64_t
 
 // One field splatted from the particles' values (span, off) onto grid `kind`,
 // normalised: LINEAR through the bins, the wider kernels through the
-// per-particle splat.
+// tile-sorted splat.
 mgf_status splat(mgf_psolver s, hipStream_t st, const GridDev& g, int kind, const float* val, int span, int off,
                  float* out, float* weight) {
     mgf_particles p = s->p;
@@ -161,7 +161,7 @@ mgf_status splat(mgf_psolver s, hipStream_t st, const GridDev& g, int kind, cons
         MGF_HIP(launch_p2g_binned(st, g, kind, s->bin_start, s->order, s->pos_s, sorted ? s->vel_s : val, span, off,
                                   sorted ? 1 : 0, s->acc, out, weight, 1));
     else
-        MGF_HIP(launch_p2g(st, g, kind, p->n, p->pos, val, span, off, s->alg, out, weight, 1));
+        MGF_HIP(launch_p2g(st, g, kind, p->n, p->pos, val, span, off, s->alg, out, weight, 1, s->splat_work));
     return MGF_OK;
 }
 
@@ -385,6 +385,8 @@ mgf_status mgf_psolver_create(mgf_context ctx, const mgf_grid* grid, int32_t kin
             TRY(owned_alloc(s->allocations, &s->acc, p2g_acc_floats(g)));
             TRY(owned_alloc(s->allocations, &s->pos_s, 3 * size_t(particles->n)));
             TRY(owned_alloc(s->allocations, &s->vel_s, 3 * size_t(particles->n)));
+        } else {
+            TRY(owned_alloc(s->allocations, &s->splat_work, p2g_work_words(g, particles->n)));
         }
         MGF_HIP(hipStreamSynchronize(ctx->stream));
         return MGF_OK;

@@ -126,6 +126,50 @@ def test_p2g_matches_oracle(ctx, orc, setup, alg):
             assert_close(f[keep], ef[keep], what)
 
 
+@pytest.mark.parametrize("alg", ALGS_P2G)
+@pytest.mark.parametrize("n, edge", [(1, 1), (65, 2), (2048, 1), (2049, 3), (6000, 3)])
+def test_p2g_tiles(ctx, orc, alg, n, edge):
+    """The tile-sorted splat at the edges of its tiles (8 nodes an axis) and
+    chunks (2048 particles): crowds around tile corners, particles outside
+    the grid, in sorted and in random order.  Bound: a node's sum of m terms
+    differs from the exact sum by at most (m + 4) 2^-24 sum |w v| in either
+    order (4: the product's own roundings), and m <= n."""
+    res, origin, spacing = (18, 9, 25), (0.5, -1.0, 0.0), (0.25, 0.25, 0.25)
+    rng = np.random.default_rng(n * 10 + edge)
+    corners = np.array([(x, y, z) for x in (0, 8, 16) for y in (0, 8) for z in (8, 24)], np.float64)[:edge]
+    pos = (corners[rng.integers(0, edge, n)] + rng.uniform(-2.5, 2.5, (n, 3))) * 0.25 + origin
+    pos = pos.astype(np.float32)
+    # far outside, within the int range of (p - o) / h: beyond 2^31 the
+    # oracle's truncation to int is undefined
+    pos[n // 2] = (-50.0, 60.0, 1e8)
+    val = rng.standard_normal(n).astype(np.float32)
+    for order in (np.arange(n), np.lexsort(pos.T)):
+        for kind in (0, 1 + edge % 3):
+            p, v = pos[order], val[order]
+            f, w = mgf.particles_to_grid(ctx, res, origin, spacing, kind, p, v, alg, normalize=False)
+            ef, ew = orc.p2g(res, origin, spacing, kind, p, v, alg, normalize=False)
+            sf, sw = orc.p2g(res, origin, spacing, kind, p, np.abs(v), alg, normalize=False)
+            bound = 2.0 * (n + 4) * 2.0 ** -24
+            assert np.all(np.abs(f - ef.ravel()) <= bound * sf.ravel() + 1e-37), (alg, kind)
+            assert np.all(np.abs(w - ew.ravel()) <= bound * sw.ravel() + 1e-37), (alg, kind)
+
+
+@pytest.mark.parametrize("alg", ALGS_P2G)
+def test_p2g_values_not_finite(ctx, orc, alg):
+    """Infinities and NaN reach the same nodes as in the oracle (a zero
+    corner weight times an infinity is a NaN), and no others."""
+    res, origin, spacing = (20, 11, 9), (0.0, 0.0, 0.0), (1.0, 1.0, 1.0)
+    pos = np.array([[3.2, 4.1, 5.0], [12.5, 8.0, 4.7], [19.9, 0.2, 8.8], [7.0, 7.0, 1.3]], np.float32)
+    val = np.array([np.inf, -np.inf, np.nan, 2.0], np.float32)
+    for kind in range(4):
+        f, _ = mgf.particles_to_grid(ctx, res, origin, spacing, kind, pos, val, alg, normalize=False)
+        ef, _ = orc.p2g(res, origin, spacing, kind, pos, val, alg, normalize=False)
+        ef = ef.ravel()
+        assert np.array_equal(np.isnan(f), np.isnan(ef)) and np.array_equal(np.isinf(f), np.isinf(ef))
+        fine = np.isfinite(ef)
+        assert_close(f[fine], ef[fine], alg)
+
+
 @pytest.mark.parametrize("setup", range(len(SETUPS)))
 @pytest.mark.parametrize("alg", ALGS_G2P)
 def test_g2p_bitexact(ctx, orc, setup, alg):
