@@ -78,10 +78,10 @@ void ProbeSink::release() {
 }  // namespace mgf
 
 // Scratch of mgf_op_extrapolate_fc_noalloc (layout and limits with the entry
-// point below): 35.1 MB held by every device the library runs on until the
+// point below): 8.9 MB held by every device the library runs on until the
 // process ends.  Host code never passes this name to a kernel: it uses the
 // device address looked up per device (na_setup).
-static constexpr size_t kNoAllocScratchBytes = 35143424;
+static constexpr size_t kNoAllocScratchBytes = 8912896;
 static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
 
 namespace {
@@ -824,26 +824,18 @@ mgf_status alloc_scene(mgf_scene s) {
 }
 
 // ---------------------------------------------------------------------------
-// Extrapolation: distances, counting sort by distance, one gather kernel per
-// layer; returns the largest non-empty layer (< layers).
+// Extrapolation: distances, then passes over the bricks the layers cross;
+// returns the largest non-empty layer (< layers).
 mgf_status alloc_extrapolation(mgf_scene s, size_t nface) {
-    const int32_t K = std::min<int32_t>(ext_max_distance(s->g), 65535);
-    TRY(dalloc(s, &s->layer, nface));
-    TRY(dalloc(s, &s->list, nface));
-    TRY(dalloc(s, &s->lmask, nface));
-    TRY(dalloc(s, &s->fmask, nface));
-    TRY(dalloc(s, &s->counts, ext_counts_size(K)));
-    if (s->dry) return MGF_OK;
-    if (hipHostMalloc(reinterpret_cast<void**>(&s->host_offs), sizeof(uint32_t) * (size_t(K) + 3)) != hipSuccess) {
-        (void)hipGetLastError();
-        s->host_offs = nullptr;
-        return fail(MGF_ERR_NOMEM, "hipHostMalloc failed");
-    }
+    // the faces' distances, and the fluid SDF's scratch (a word a cell; fewer
+    // than half as many cells as faces)
+    TRY(dalloc(s, &s->dist, nface));
+    TRY(dalloc(s, &s->ext_work, ext_work_words(s->g)));
     return MGF_OK;
 }
 
 mgf_status extrapolate(mgf_scene s, float* u, float* v, float* w, int layers, int* used) {
-    ExtBufs B{reinterpret_cast<uint16_t*>(s->layer), s->list, s->lmask, s->fmask, s->counts, s->host_offs};
+    ExtBufs B{s->dist, s->ext_work, reinterpret_cast<uint32_t*>(s->host_scratch)};
     return extrapolate_run(s->stream, s->g, u, v, w, layers, B, used);
 }
 
@@ -1058,10 +1050,11 @@ mgf_status lock_prepare(mgf_scene s) {
 // buffers are `c` (advection with forces, markers, right-hand side, stencil
 // codes, the hierarchy's markers and codes, x64 = 0 and ||b||^2: advect,
 // pressure() and cg_mixed's prologue), and after them (projection with the
-// FP64 pressure, the extrapolation's distance transform and sort, its layer
-// offsets and largest layer copied to `offs_out`), as keyed records; the
-// layers themselves are launched from those offsets.
-mgf_status phase_records(mgf_scene s, int c, std::vector<KRec>& pre, std::vector<KRec>& post, uint32_t* offs_out) {
+// FP64 pressure, the extrapolation's distance transform, which marks the
+// bricks of its first pass and leaves the largest distance in `far`), as
+// keyed records.
+mgf_status phase_records(mgf_scene s, int c, std::vector<KRec>& pre, std::vector<KRec>& post, uint16_t* mark,
+                         uint32_t* far) {
     const int n = 1 - c;
     const float dt = s->desc.dt;
     float sa[3], sg[3];
@@ -1141,13 +1134,8 @@ mgf_status phase_records(mgf_scene s, int c, std::vector<KRec>& pre, std::vector
             return fail(MGF_ERR_UNSUPPORTED, "extrapolation over more than one layer needs nx + ny + nz + 3 < 65535 "
                                              "(16-bit face distances)");
         r.clear();
-        const uint32_t* maxd = nullptr;
-        rec_ext_device(r, s->g, s->u[n], s->v[n], s->w[n], reinterpret_cast<uint16_t*>(s->layer), cap, K, s->counts,
-                       s->list, s->lmask, s->fmask, &maxd, false);
+        rec_ext_distance(r, s->g, s->u[n], s->v[n], s->w[n], s->dist, mark, far);
         keyed(post, r, 1, 0, 0);
-        r.clear();
-        rec_copy_offs(r, s->counts, K, cap, offs_out);
-        keyed(post, r, 2, 0, 0);
     }
     return MGF_OK;
 }
@@ -1268,19 +1256,21 @@ mgf_status run_seq(LockPlan& P, const LSeq& seq) { return run_seq_at(P.stream, P
 struct PhasePlan {
     mgf_context ctx = nullptr;
     LSeq pre, post;
-    unsigned char* dev = nullptr;   // the packed layer offsets, the layer table, then tables and maps
-    std::vector<size_t> offs_at;    // per scene: its offsets' first word in the packed area (cap + 3 words)
+    // the far words (kExtFarWords a scene) and the brick stamps, zeroed each
+    // step; the brick table and each brick's scene; then tables and maps
+    unsigned char* dev = nullptr;
     std::vector<int32_t> cap;       // per scene: the layer cap (0: no extrapolation)
-    size_t offs_words = 0;
-    size_t layer_tab = 0;           // byte offset of the per-scene k_multi_layer arguments
-    uint32_t* offs_host = nullptr;  // pinned copy of the packed offsets
+    std::vector<uint32_t> first;    // per scene: its first brick
+    uint32_t bricks = 0;            // of all scenes
+    size_t stamps_at = 0, tab_at = 0, scene_at = 0;   // byte offsets
+    uint32_t* far_host = nullptr;   // pinned copy of the far words
     PhasePlan() = default;
     PhasePlan(const PhasePlan&) = delete;
     PhasePlan& operator=(const PhasePlan&) = delete;
     ~PhasePlan() {
         if (ctx) {
             pool_put(ctx, dev);
-            pool_put(ctx, offs_host);
+            pool_put(ctx, far_host);
         }
     }
 };
@@ -1288,34 +1278,45 @@ struct PhasePlan {
 mgf_status build_phase(const std::vector<mgf_scene>& sc, const std::vector<uint8_t>& cur, hipStream_t st,
                        PhasePlan& Q) {
     const size_t n = sc.size();
-    Q.offs_at.assign(n, 0);
     Q.cap.assign(n, 0);
-    Q.offs_words = 0;
+    Q.first.assign(n, 0);
+    Q.bricks = 0;
     for (size_t i = 0; i < n; ++i) {
         const int32_t K = ext_max_distance(sc[i]->g);
         Q.cap[i] = int32_t(std::max<int64_t>(0, std::min<int64_t>(int64_t(sc[i]->desc.extrapolation_layers) - 1, K)));
-        Q.offs_at[i] = Q.offs_words;
-        if (Q.cap[i] > 0) Q.offs_words += size_t(Q.cap[i]) + 3;
+        Q.first[i] = Q.bricks;
+        if (Q.cap[i] > 0) Q.bricks += ext_bricks(sc[i]->g);
     }
-    Q.layer_tab = (Q.offs_words * sizeof(uint32_t) + 255) / 256 * 256;
-    const size_t head = Q.layer_tab + (n * layer_arg_bytes() + 255) / 256 * 256;
+    auto align = [](size_t b) { return (b + 255) / 256 * 256; };
+    Q.stamps_at = align(n * kExtFarWords * 4);
+    Q.tab_at = align(Q.stamps_at + size_t(Q.bricks) * 4);
+    Q.scene_at = align(Q.tab_at + n * brick_arg_bytes());
+    const size_t head = align(Q.scene_at + size_t(Q.bricks) * 2);
     std::vector<std::vector<KRec>> pre(n), post(n);
     // the layout first (records with null addresses), then allocate and fill
     size_t total = 0;
     for (int pass = 0; pass < 2; ++pass) {
-        uint32_t* packed = reinterpret_cast<uint32_t*>(pass == 0 ? nullptr : Q.dev);
+        unsigned char* dev = pass == 0 ? nullptr : Q.dev;
         for (size_t i = 0; i < n; ++i) {
             pre[i].clear();
             post[i].clear();
-            TRY(phase_records(sc[i], cur[i], pre[i], post[i], packed + Q.offs_at[i]));
+            // the first pass reads the second stamp buffer
+            uint16_t* mark = dev ? reinterpret_cast<uint16_t*>(dev + Q.stamps_at) + Q.bricks + Q.first[i] : nullptr;
+            uint32_t* far = dev ? reinterpret_cast<uint32_t*>(dev) + i * kExtFarWords : nullptr;
+            TRY(phase_records(sc[i], cur[i], pre[i], post[i], mark, far));
         }
         std::vector<unsigned char> blob(pass == 0 ? 0 : total, 0);
         unsigned char* bp = pass == 0 ? nullptr : blob.data();
         for (size_t i = 0; bp && i < n; ++i) {
             mgf_scene s = sc[i];
             const int c1 = 1 - cur[i];
-            layer_args(bp + Q.layer_tab + i * layer_arg_bytes(), s->g, s->u[c1], s->v[c1], s->w[c1], s->list,
-                       s->lmask, s->counts, ext_max_distance(s->g));
+            brick_args(bp + Q.tab_at + i * brick_arg_bytes(), s->g, s->u[c1], s->v[c1], s->w[c1], s->dist, Q.cap[i],
+                       Q.first[i]);
+            if (Q.cap[i] > 0) {
+                const uint16_t scene = uint16_t(i);
+                for (uint32_t b = 0; b < ext_bricks(s->g); ++b)
+                    std::memcpy(bp + Q.scene_at + 2 * (size_t(Q.first[i]) + b), &scene, 2);
+            }
         }
         size_t at = head;
         Q.pre = merge_seq(pre, bp, at);
@@ -1326,8 +1327,8 @@ mgf_status build_phase(const std::vector<mgf_scene>& sc, const std::vector<uint8
             Q.ctx = sc[0]->ctx;
             Q.dev = static_cast<unsigned char*>(pool_get(Q.ctx, total, false));
             if (!Q.dev) return fail(MGF_ERR_NOMEM, "lockstep phases: hipMalloc failed");
-            Q.offs_host = static_cast<uint32_t*>(pool_get(Q.ctx, std::max<size_t>(Q.offs_words, 1) * 4, true));
-            if (!Q.offs_host) return fail(MGF_ERR_NOMEM, "lockstep phases: hipHostMalloc failed");
+            Q.far_host = static_cast<uint32_t*>(pool_get(Q.ctx, n * kExtFarWords * 4, true));
+            if (!Q.far_host) return fail(MGF_ERR_NOMEM, "lockstep phases: hipHostMalloc failed");
             continue;
         }
         if (at != total) return fail(MGF_ERR_INVALID, "lockstep phases: the layout changed between its passes");
@@ -1669,19 +1670,17 @@ mgf_status div_end(mgf_scene s, mgf_step_stats* acc) {
 // that the entry point allocates nothing.  Every device the library runs on
 // holds its own copy until the process ends; its address is looked up once
 // per device at mgf_init (hipGetSymbolAddress with that device current).
-// Layout (each part 256-byte aligned): face distances uint16[kNaFaces],
-// sorted list uint32[kNaFaces], list masks uint8[kNaFaces], face masks
-// uint8[kNaFaces], sort counters uint32[kNaCountWords].
+// Layout (each part 256-byte aligned): face distances uint16[kNaFaces], the
+// largest distance and the brick stamps uint32[kNaWorkWords].
 constexpr size_t kNaFaces = size_t(1) << 22;   // faces of all three components
 constexpr int32_t kNaMaxK = 4093;              // nx + ny + nz + 3 with more than one layer
-constexpr size_t kNaCountWords = (3 * 32 + 1) * (size_t(kNaMaxK) + 2) + 1;
+// A brick of a grid within those limits holds at least 128 faces on average
+// (16 x 16 x 1 in a grid one cell thick, an axis rounded up at worst by half).
+constexpr size_t kNaWorkWords = size_t(1) << 17;
 constexpr size_t na_align(size_t b) { return (b + 255) / 256 * 256; }
 constexpr size_t kNaDistOff = 0;
-constexpr size_t kNaListOff = kNaDistOff + na_align(2 * kNaFaces);
-constexpr size_t kNaLmaskOff = kNaListOff + na_align(4 * kNaFaces);
-constexpr size_t kNaFmaskOff = kNaLmaskOff + na_align(kNaFaces);
-constexpr size_t kNaCountOff = kNaFmaskOff + na_align(kNaFaces);
-constexpr size_t kNaBytes = kNaCountOff + na_align(4 * kNaCountWords);
+constexpr size_t kNaWorkOff = kNaDistOff + na_align(2 * kNaFaces);
+constexpr size_t kNaBytes = kNaWorkOff + na_align(4 * kNaWorkWords);
 static_assert(kNaBytes <= kNoAllocScratchBytes, "the scratch array holds the layout");
 
 constexpr int kNaMaxDevices = 64;
@@ -1732,8 +1731,11 @@ mgf_status scene_bytes_for(mgf_context ctx, const mgf_scene_desc* desc, int64_t*
     return MGF_OK;
 }
 
+// The far words, then two stamps a brick.
+size_t ext_work_words(const GridDev& g) { return kExtFarWords + size_t(ext_bricks(g)); }
+
 mgf_status extrapolate_run(hipStream_t st, const GridDev& g, float* u, float* v, float* w, int layers,
-                           const ExtBufs& B, int* used, bool device_only) {
+                           const ExtBufs& B, int* used) {
     *used = 0;
     const int32_t K = ext_max_distance(g);
     const int32_t cap = int32_t(std::min<int64_t>(int64_t(layers) - 1, K));
@@ -1741,51 +1743,17 @@ mgf_status extrapolate_run(hipStream_t st, const GridDev& g, float* u, float* v,
     if (K >= 65535)
         return fail(MGF_ERR_UNSUPPORTED, "extrapolation over more than one layer needs nx + ny + nz + 3 < 65535 "
                                          "(16-bit face distances)");
-    uint16_t* dist = B.dist;
-    MGF_HIP(launch_ext_distance(st, g, u, v, w, dist));
-    const uint32_t* offs = nullptr;
-    const uint32_t* maxd = nullptr;
-    MGF_HIP(launch_ext_sort(st, g, dist, cap, K, B.counts, B.list, B.lmask, B.fmask, &offs, &maxd));
-    if (device_only) {
-        probe_next_bytes(0.0);
-        MGF_HIP(launch_ext_tail(st, g, u, v, w, B.list, B.lmask, offs, 1, 0, maxd));
-        MGF_HIP(hipMemcpyAsync(B.host_offs, maxd, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
-        *used = -1;
-        return MGF_OK;
-    }
-    // offsets of layers 0..cap+1, then the largest distance present
-    MGF_HIP(hipMemcpyAsync(B.host_offs, offs, sizeof(uint32_t) * (size_t(cap) + 2), hipMemcpyDeviceToHost, st));
-    MGF_HIP(hipMemcpyAsync(B.host_offs + cap + 2, maxd, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
+    uint16_t* stamps = reinterpret_cast<uint16_t*>(B.work + kExtFarWords);
+    MGF_HIP(launch_ext_zero(st, B.work, ext_work_words(g)));
+    MGF_HIP(launch_ext_distance(st, g, u, v, w, B.dist, stamps + ext_bricks(g), B.work));
+    // the largest distance bounds the passes
+    MGF_HIP(hipMemcpyAsync(B.host, B.work, sizeof(uint32_t) * kExtFarWords, hipMemcpyDeviceToHost, st));
     MGF_HIP(hipStreamSynchronize(st));
-    const int32_t top = int32_t(B.host_offs[cap + 2]);
-    // Small layers are launch-bound: two of them share a launch (the second
-    // recomputes its previous-layer neighbours, several loads per face).
-    // Large layers are bound by their gathers, which the pairing would
-    // multiply, so they run one per launch.
-    constexpr uint32_t kPairMax = 65536;   // faces of two layers launched together
-    // From the first layer after which no layer exceeds kTailMax entries on,
-    // the layers run in one work-group (k_ext_tail): a launch per layer
-    // costs ~8 us, a small layer ~2-4 us there.
-    constexpr uint32_t kTailMax = 1024;
-    int32_t tail = top + 1;
-    while (tail > 1 && B.host_offs[tail] - B.host_offs[tail - 1] <= kTailMax) --tail;
-    for (int32_t L = 1; L < tail;) {
-        const uint32_t b = B.host_offs[L], m = B.host_offs[L + 1];
-        const uint32_t e = L + 1 < tail ? B.host_offs[L + 2] : m;
-        const bool pair = L + 1 < tail && e - b <= kPairMax;
-        // per entry: list 4 + mask 1 + write 4 + the values of the previous-layer neighbours (one on average)
-        probe_next_bytes(13.0 * double((pair ? e : m) - b));
-        if (pair)
-            MGF_HIP(launch_ext_layer2(st, g, u, v, w, B.list, B.lmask, B.fmask, b, m - b, e - m));
-        else
-            MGF_HIP(launch_ext_layer(st, g, u, v, w, B.list, B.lmask, b, m - b));
-        L += pair ? 2 : 1;
-    }
-    if (tail <= top) {
-        probe_next_bytes(13.0 * double(B.host_offs[top + 1] - B.host_offs[tail]));
-        MGF_HIP(launch_ext_tail(st, g, u, v, w, B.list, B.lmask, offs, tail, top));
-    }
-    *used = top;
+    const uint32_t top = std::min(*std::max_element(B.host, B.host + kExtFarWords), uint32_t(cap));
+    const uint32_t passes = ext_passes(g, top);
+    for (uint32_t p = 1; p <= passes; ++p)
+        MGF_HIP(launch_ext_bricks(st, g, u, v, w, B.dist, cap, stamps, p));
+    *used = int(top);
     return MGF_OK;
 }
 
@@ -1871,70 +1839,6 @@ OpScratch::~OpScratch() {
 
 bool lockstep_eligible(mgf_scene s) { return lock_eligible(s); }
 
-// The extrapolation layers of every scene from its offsets (in Q.offs_host):
-// for each layer index, one k_multi_layer launch over the scenes whose layer
-// is larger than kBatchTailMax entries, then one launch of every scene's
-// remaining layers (from the first layer after which none is large) in one
-// work-group each.  A scene's layers run in order: its large layers are a
-// prefix, and launches on one stream run in order.
-mgf_status launch_layers(hipStream_t st, const std::vector<mgf_scene>& sc, const PhasePlan& Q,
-                         std::vector<unsigned char>& host, unsigned char*& dev, size_t& dev_cap) {
-    constexpr uint32_t kBatchTailMax = 4096;
-    const size_t n = sc.size();
-    const uint32_t epb = layer_entries_per_block();
-    const size_t tb = tail_arg_bytes();
-    std::vector<std::vector<uint32_t>> maps;
-    std::vector<uint32_t> tail_map;
-    host.assign((n * tb + 255) / 256 * 256, 0);
-    for (size_t i = 0; i < n; ++i) {
-        const int32_t cap = Q.cap[i];
-        if (cap <= 0) continue;
-        const uint32_t* o = Q.offs_host + Q.offs_at[i];
-        const int32_t top = int32_t(o[cap + 2]);
-        int32_t first = top + 1;
-        while (first > 1 && o[first] - o[first - 1] <= kBatchTailMax) --first;
-        if (maps.size() < size_t(first)) maps.resize(size_t(first));
-        for (int32_t L = 1; L < first; ++L) {
-            const uint32_t cnt = o[L + 1] - o[L];
-            for (uint32_t b = 0; b * epb < cnt; ++b) maps[size_t(L)].push_back((uint32_t(i) << kMapShift) | b);
-        }
-        if (first <= top) {
-            mgf_scene s = sc[i];
-            tail_args(host.data() + i * tb, s->g, s->u[s->cur], s->v[s->cur], s->w[s->cur], s->list, s->lmask,
-                      s->counts, ext_max_distance(s->g), first, top);
-            tail_map.push_back(uint32_t(i) << kMapShift);
-        }
-    }
-    std::vector<size_t> map_at(maps.size(), 0);
-    for (size_t L = 0; L < maps.size(); ++L) {
-        map_at[L] = host.size();
-        const unsigned char* p = reinterpret_cast<const unsigned char*>(maps[L].data());
-        host.insert(host.end(), p, p + 4 * maps[L].size());
-    }
-    const size_t tail_map_at = host.size();
-    const unsigned char* tp = reinterpret_cast<const unsigned char*>(tail_map.data());
-    host.insert(host.end(), tp, tp + 4 * tail_map.size());
-    if (host.size() > dev_cap) {
-        MGF_HIP(hipStreamSynchronize(st));
-        pool_put(sc[0]->ctx, dev);
-        dev = nullptr;
-        dev_cap = 0;
-        const size_t want = host.size() + host.size() / 2 + 4096;
-        dev = static_cast<unsigned char*>(pool_get(sc[0]->ctx, want, false));
-        if (!dev) {
-            return fail(MGF_ERR_NOMEM, "lockstep layers: hipMalloc failed");
-        }
-        dev_cap = want;
-    }
-    MGF_HIP(hipMemcpyAsync(dev, host.data(), host.size(), hipMemcpyHostToDevice, st));
-    for (size_t L = 1; L < maps.size(); ++L)
-        MGF_HIP(launch_multi_layer(st, Q.dev + Q.layer_tab, reinterpret_cast<const uint32_t*>(dev + map_at[L]),
-                                   uint32_t(maps[L].size()), int32_t(L)));
-    MGF_HIP(launch_multi(st, kMkExtTail, dev, reinterpret_cast<const uint32_t*>(dev + tail_map_at),
-                         uint32_t(tail_map.size()), 0, nullptr));
-    return MGF_OK;
-}
-
 mgf_status batch_lockstep(mgf_context ctx, const std::vector<mgf_scene>& sc, int32_t nsteps, int32_t workers,
                           std::vector<mgf_step_stats>& stats, std::vector<mgf_status>& status,
                           std::vector<std::string>& errs, double* step_ms) {
@@ -1952,13 +1856,9 @@ mgf_status batch_lockstep(mgf_context ctx, const std::vector<mgf_scene>& sc, int
     if (!P.stream) return fail(MGF_ERR_DEVICE, "hipStreamCreate failed");
     hipEvent_t ev = nullptr;
     std::vector<std::pair<std::vector<uint8_t>, std::unique_ptr<PhasePlan>>> phases;
-    std::vector<unsigned char> step_host;   // this step's layer maps and tail table
-    unsigned char* step_dev = nullptr;
-    size_t step_cap = 0;
     auto cleanup = [&]() {
         (void)hipStreamSynchronize(P.stream);
         if (ev) (void)hipEventDestroy(ev);
-        pool_put(ctx, step_dev);
         phases.clear();
         pool_stream_put(ctx, P.stream);
         P.stream = nullptr;
@@ -2087,6 +1987,8 @@ mgf_status batch_lockstep(mgf_context ctx, const std::vector<mgf_scene>& sc, int
         result = lock_solve(P, stats);
         if (result != MGF_OK) return fin(result);
         const double t2 = now_ms();
+        // far words and stamps (the stamps' pad up to the table is not read)
+        if (Q->bricks > 0) MGF_HIP(launch_ext_zero(P.stream, Q->dev, Q->stamps_at / 4 + size_t(Q->bricks)));
         result = run_seq_at(P.stream, Q->dev, Q->post, nullptr);
         if (result != MGF_OK) return fin(result);
         for (int i = 0; i < n; ++i) {
@@ -2095,21 +1997,29 @@ mgf_status batch_lockstep(mgf_context ctx, const std::vector<mgf_scene>& sc, int
                 MGF_HIP(launch_div_check(P.stream, s->g, s->markers, s->u[s->cur], s->v[s->cur], s->w[s->cur], s->b,
                                          s->red.partials, kDivBlocks, s->div_dev));
         }
-        // the layers: each scene's offsets to the host, then per layer index
-        // one launch over every scene whose layer is large, then each
-        // scene's tail of small layers in one work-group (all scenes in one
-        // launch)
-        if (Q->offs_words > 0) {
-            MGF_HIP(hipMemcpyAsync(Q->offs_host, Q->dev, sizeof(uint32_t) * Q->offs_words, hipMemcpyDeviceToHost,
-                                   P.stream));
+        // the layers: every scene's largest distance to the host, then the
+        // passes over all scenes' bricks
+        std::vector<uint32_t> top(size_t(n), 0);
+        if (Q->bricks > 0) {
+            MGF_HIP(hipMemcpyAsync(Q->far_host, Q->dev, sizeof(uint32_t) * kExtFarWords * size_t(n),
+                                   hipMemcpyDeviceToHost, P.stream));
             MGF_HIP(hipStreamSynchronize(P.stream));
-            result = launch_layers(P.stream, sc, *Q, step_host, step_dev, step_cap);
-            if (result != MGF_OK) return fin(result);
+            uint32_t passes = 0;
+            for (int i = 0; i < n; ++i) {
+                if (Q->cap[size_t(i)] <= 0) continue;
+                const uint32_t* w = Q->far_host + size_t(i) * kExtFarWords;
+                top[size_t(i)] = std::min(*std::max_element(w, w + kExtFarWords), uint32_t(Q->cap[size_t(i)]));
+                passes = std::max(passes, ext_passes(sc[size_t(i)]->g, top[size_t(i)]));
+            }
+            for (uint32_t p = 1; p <= passes; ++p)
+                MGF_HIP(launch_multi_bricks(P.stream, Q->dev + Q->tab_at,
+                                            reinterpret_cast<const uint16_t*>(Q->dev + Q->scene_at),
+                                            reinterpret_cast<uint16_t*>(Q->dev + Q->stamps_at), Q->bricks, p));
         }
         MGF_HIP(hipStreamSynchronize(P.stream));
         for (int i = 0; i < n; ++i) {
             mgf_step_stats& a = stats[size_t(i)];
-            a.extrapolation_layers = Q->cap[size_t(i)] > 0 ? int32_t(Q->offs_host[Q->offs_at[size_t(i)] + size_t(Q->cap[size_t(i)]) + 2]) : 0;
+            a.extrapolation_layers = int32_t(top[size_t(i)]);
             a.steps += 1;
             if (!std::isfinite(a.residual_rel) && status[size_t(i)] == MGF_OK) {
                 status[size_t(i)] = MGF_ERR_NONFINITE;
@@ -2298,7 +2208,6 @@ mgf_status mgf_scene_destroy(mgf_scene s) {
     for (void* p : s->allocations) (void)hipFree(p);
     for (auto& so : s->solids) (void)hipFree(so.sdf0);
     if (s->host_scratch) (void)hipHostFree(s->host_scratch);
-    if (s->host_offs) (void)hipHostFree(s->host_offs);
     s->sink.release();
     if (s->stream) (void)hipStreamDestroy(s->stream);
     delete s;
@@ -2461,7 +2370,8 @@ mgf_status download_field(mgf_scene s, int32_t field, float* out, int64_t count,
             break;
         case MGF_FIELD_FLUID_SDF:
             if (s->desc.extrapolation_layers > 0)
-                MGF_HIP(launch_fluid_sdf(st, s->g, s->phi[c], s->desc.extrapolation_layers, s->layer, s->ap));
+                MGF_HIP(launch_fluid_sdf(st, s->g, s->phi[c], s->desc.extrapolation_layers,
+                                         reinterpret_cast<int32_t*>(s->dist), s->ap));
             else   // no pass: the freshly resized field's zeros (ScalarGrid.cpp:33-37)
                 MGF_HIP(launch_fill(st, s->ap, s->ncell, 0.0f));
             src = s->ap;
@@ -2952,21 +2862,23 @@ mgf_status mgf_op_extrapolate_fc(mgf_context ctx, const mgf_grid* grid, float* u
     if (!ctx) return fail(MGF_ERR_INVALID, "null context");
     TRY(check_grid(grid));
     if (layers < 0) return fail(MGF_ERR_INVALID, "layers < 0");
-    // A transient scene-shaped holder of the extrapolation scratch.
     MGF_HIP(hipSetDevice(ctx->device));
-    mgf_scene_s tmp;
-    tmp.ctx = ctx;
-    tmp.stream = ctx->stream;
-    tmp.g = make_grid(grid);
+    const GridDev g = make_grid(grid);
     const size_t nface = size_t(grid->nx + 1) * grid->ny * grid->nz +
                          size_t(grid->nx) * (grid->ny + 1) * grid->nz +
                          size_t(grid->nx) * grid->ny * (grid->nz + 1);
-    mgf_status st = alloc_extrapolation(&tmp, nface);
+    const size_t dist_bytes = (2 * nface + 255) / 256 * 256;
     int used = 0;
-    if (st == MGF_OK) st = extrapolate(&tmp, u, v, w, layers, &used);
-    (void)hipStreamSynchronize(ctx->stream);
-    for (void* p : tmp.allocations) (void)hipFree(p);
-    if (tmp.host_offs) (void)hipHostFree(tmp.host_offs);
+    mgf_status st = MGF_OK;
+    {
+        OpScratch work(ctx, dist_bytes + 4 * ext_work_words(g));
+        if (!work.p) return fail(MGF_ERR_NOMEM, "extrapolation scratch");
+        uint32_t far[kExtFarWords];
+        ExtBufs B{static_cast<uint16_t*>(work.p),
+                  reinterpret_cast<uint32_t*>(static_cast<unsigned char*>(work.p) + dist_bytes), far};
+        st = extrapolate_run(ctx->stream, g, u, v, w, layers, B, &used);
+        (void)hipStreamSynchronize(ctx->stream);
+    }
     if (layers_used) *layers_used = used;
     return st;
 }
@@ -2984,17 +2896,16 @@ mgf_status mgf_op_extrapolate_fc_noalloc(mgf_context ctx, const mgf_grid* grid, 
                                          " faces exceed its scratch (" + std::to_string(kNaFaces) + " faces)");
     const GridDev g = make_grid(grid);
     const int32_t K = ext_max_distance(g);
-    if (layers > 1 && (K > kNaMaxK || ext_counts_size(K) > kNaCountWords))
+    if (layers > 1 && (K > kNaMaxK || ext_work_words(g) > kNaWorkWords))
         return fail(MGF_ERR_INVALID, "mgf_op_extrapolate_fc_noalloc: nx + ny + nz + 3 = " + std::to_string(K) +
                                          " exceeds its scratch (" + std::to_string(kNaMaxK) + ")");
     std::string err;
     MGF_HIP(hipSetDevice(ctx->device));
     unsigned char* base = static_cast<unsigned char*>(na_ptr(ctx->device, &err));
     if (!base) return fail(MGF_ERR_DEVICE, "mgf_op_extrapolate_fc_noalloc: " + err);
-    // the layer offsets come back into this stack buffer (no host allocation)
-    uint32_t offs[kNaMaxK + 3];
-    ExtBufs B{reinterpret_cast<uint16_t*>(base + kNaDistOff), reinterpret_cast<uint32_t*>(base + kNaListOff),
-              base + kNaLmaskOff, base + kNaFmaskOff, reinterpret_cast<uint32_t*>(base + kNaCountOff), offs};
+    // the largest distance comes back into this stack buffer (no host allocation)
+    uint32_t far[kExtFarWords];
+    ExtBufs B{reinterpret_cast<uint16_t*>(base + kNaDistOff), reinterpret_cast<uint32_t*>(base + kNaWorkOff), far};
     int used = 0;
     const mgf_status st = extrapolate_run(ctx->stream, g, u, v, w, layers, B, &used);
     MGF_HIP(hipStreamSynchronize(ctx->stream));

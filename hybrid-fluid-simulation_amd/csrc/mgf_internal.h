@@ -155,7 +155,7 @@ struct mgf_scene_s {
     float* ap = nullptr;           // plain: A p
     mgf::CgScalars* scal = nullptr;
     mgf::ReduceBuf red;
-    double* host_scratch = nullptr; // pinned host mirror of small reductions
+    double* host_scratch = nullptr; // pinned host mirror of small reductions (and of the largest distance)
     uint16_t* codes = nullptr;     // per-cell stencil codes of the pressure matrix
     // preconditioner (allocated on first use)
     float* z = nullptr;            // M^-1 r
@@ -173,12 +173,8 @@ struct mgf_scene_s {
     bool x64_valid = false;        // x64 holds a finished mixed solve (a warm start's guess)
 
     // extrapolation scratch
-    int32_t* layer = nullptr;      // nfx+nfy+nfz words: the faces' uint16 distances, or the SDF's scratch
-    uint32_t* list = nullptr;      // faces sorted by distance (nfx+nfy+nfz)
-    uint8_t* lmask = nullptr;      // previous-layer neighbour mask of each list entry
-    uint8_t* fmask = nullptr;      // the same mask per face (read for neighbours of the next layer)
-    uint32_t* counts = nullptr;    // counting-sort scratch [ext_counts_size(K)]
-    uint32_t* host_offs = nullptr; // pinned mirror of the offsets and the max distance
+    uint16_t* dist = nullptr;      // the faces' distances (nfx+nfy+nfz); the SDF's scratch too (ncell int32)
+    uint32_t* ext_work = nullptr;  // ext_work_words: the largest distance, the brick stamps
 
     std::vector<mgf::Solid> solids;
     bool boundary_dirty = false;   // solids changed since the last refresh
@@ -284,24 +280,19 @@ void pool_release(mgf_context ctx);
 mgf_status batch_lockstep(mgf_context ctx, const std::vector<mgf_scene>& sc, int32_t nsteps, int32_t workers,
                           std::vector<mgf_step_stats>& stats, std::vector<mgf_status>& status,
                           std::vector<std::string>& errs, double* step_ms);
-// Extrapolation buffers (face count F, K = ext_max_distance, below 65535):
-// dist F, list F, lmask F, fmask F, counts ext_counts_size(K); host_offs is
-// host memory of K + 3 words the layer offsets are read into.
+// Extrapolation buffers: dist one word per face, work ext_work_words(g)
+// words; host is host memory of kExtFarWords words.
+constexpr uint32_t kExtFarWords = 256;
 struct ExtBufs {
     uint16_t* dist;
-    uint32_t* list;
-    uint8_t* lmask;
-    uint8_t* fmask;
-    uint32_t* counts;
-    uint32_t* host_offs;
+    uint32_t* work;
+    uint32_t* host;
 };
+size_t ext_work_words(const GridDev& g);
 // extrapolatingDataInvoker(FCV) on (u, v, w) in place on stream st; *used
-// receives the largest non-empty layer (< layers).  device_only: no host
-// synchronisation (every layer in one work-group, the largest layer copied
-// to host_offs[0] when the stream gets there; *used = -1 when kernels were
-// enqueued).
+// receives the largest non-empty layer (< layers).
 mgf_status extrapolate_run(hipStream_t st, const GridDev& g, float* u, float* v, float* w, int layers,
-                           const ExtBufs& B, int* used, bool device_only = false);
+                           const ExtBufs& B, int* used);
 #define MGF_HIP(expr)                                                           \
     do {                                                                        \
         hipError_t e_ = (expr);                                                 \
@@ -453,8 +444,7 @@ enum MultiKind : int32_t {
     kMkRestrict, kMkRestrict2, kMkRestrictTile, kMkCoarse, kMkMarchDesc, kMkMarchAsc, kMkMarchAscRz, kMkGather,
     kMkRefine0, kMkCodes, kMkFlatWet, kMkCoarsen, kMkMarchWet, kMkMarchPlan,
     kMkAdvectFc, kMkAdvectCc, kMkAdvectCc4, kMkMarkers, kMkRhs, kMkProject, kMkCopyWord,
-    kMkExtRows, kMkExtRowsReg4, kMkExtRowsReg8, kMkExtRowsReg16, kMkExtLines1, kMkExtLines2, kMkExtZero, kMkExtCount,
-    kMkExtScan, kMkExtScatter, kMkExtTail, kMkCopyOffs, kMkExtRowsReg5,
+    kMkExtRows, kMkExtRowsReg4, kMkExtRowsReg8, kMkExtRowsReg16, kMkExtLines1, kMkExtLines2, kMkExtRowsReg5,
     kMkExtLinesSeg,                          // 8 kinds: (axis - 1) * 4 + segment size class
     kMkExtLinesSegLast = kMkExtLinesSeg + 7,
     kMkExtRowsShort1, kMkExtRowsShort2,
@@ -519,26 +509,18 @@ void rec_rhs(std::vector<MRec>& out, const GridDev& g, Vel U, Vel S, const uint8
 void rec_project(std::vector<MRec>& out, const GridDev& g, const float sg[3], const uint8_t* markers, const float* p32,
                  const double* p64, float* u, float* v, float* w, const float* us, const float* vs, const float* ws);
 void rec_copy_word(std::vector<MRec>& out, const uint32_t* src, uint32_t* dst);
-// The extrapolation with no host synchronisation (distance transform, sort,
-// every layer in one work-group; *maxd = the device address of the largest
-// layer); K = ext_max_distance(g) < 65535, 1 <= cap <= K.
-void rec_ext_device(std::vector<MRec>& out, const GridDev& g, float* u, float* v, float* w, uint16_t* dist,
-                    int32_t cap, int32_t K, uint32_t* counts, uint32_t* list, uint8_t* lmask, uint8_t* fmask,
-                    const uint32_t** maxd, bool with_layers = true);
-// The sort's offsets 0..cap+1 and largest layer packed into dst (cap + 3 words).
-void rec_copy_offs(std::vector<MRec>& out, uint32_t* counts, int32_t K, int32_t cap, uint32_t* dst);
-// Layer L of many scenes in one launch (k_multi_layer): a table of
-// layer_arg_bytes() per scene (layer_args), map entries (scene, block) with
-// layer_entries_per_block() entries a block.
-uint32_t layer_entries_per_block();
-size_t layer_arg_bytes();
-void layer_args(unsigned char* dst, const GridDev& g, float* u, float* v, float* w, const uint32_t* list,
-                const uint8_t* lmask, uint32_t* counts, int32_t K);
-hipError_t launch_multi_layer(hipStream_t s, const void* tab, const uint32_t* map, uint32_t nblocks, int32_t L);
-// The one-work-group layers first..last as a kMkExtTail record's arguments.
-size_t tail_arg_bytes();
-void tail_args(unsigned char* dst, const GridDev& g, float* u, float* v, float* w, const uint32_t* list,
-               const uint8_t* lmask, uint32_t* counts, int32_t K, int32_t first, int32_t last);
+// The extrapolation's distance transform; mark = the scene's bricks in the
+// stamp buffer of pass 1, far = its kExtFarWords words.
+void rec_ext_distance(std::vector<MRec>& out, const GridDev& g, float* u, float* v, float* w, uint16_t* dist,
+                      uint16_t* mark, uint32_t* far);
+// One pass over the bricks of many scenes: a table of brick_arg_bytes() per
+// scene (brick_args; first = its first brick), the scene of each of `total`
+// bricks (a multiple of 8), stamps of 2 * total words.
+size_t brick_arg_bytes();
+void brick_args(unsigned char* dst, const GridDev& g, float* u, float* v, float* w, const uint16_t* dist, int32_t cap,
+                uint32_t first);
+hipError_t launch_multi_bricks(hipStream_t s, const void* tab, const uint16_t* scene_of, uint16_t* stamps,
+                               uint32_t total, uint32_t pass);
 hipError_t launch_multi_k(hipStream_t s, int32_t kind, const void* tab, const uint32_t* map, uint32_t nblocks,
                           uint32_t shmem, const uint8_t* active);
 hipError_t launch_multi_ext(hipStream_t s, int32_t kind, const void* tab, const uint32_t* map, uint32_t nblocks,
@@ -552,32 +534,22 @@ hipError_t launch_multi(hipStream_t s, int32_t kind, const void* tab, const uint
 // ---- extrapolation (mgf_kernels_ext.hip) ------------------------------------
 // Largest L1 distance between two faces of one component grid (+ margin).
 int32_t ext_max_distance(const GridDev& g);
+// Bricks of the grid's three face components (rounded up to a multiple of 8)
+// and the passes that set every face within `far` layers.
+uint32_t ext_bricks(const GridDev& g);
+uint32_t ext_passes(const GridDev& g, uint32_t far);
 // dist = L1 distance of every face to the nearest known face (65535 where
 // a component has none; nx + ny + nz + 3 must be below 65535); faces indexed
-// u, then v, then w.
+// u, then v, then w.  mark (ext_bricks entries, zero): 1 for every brick
+// with a face at distance 1; far (kExtFarWords words, zero): their maximum
+// receives the largest distance.
+hipError_t launch_ext_zero(hipStream_t s, void* p, size_t words);
 hipError_t launch_ext_distance(hipStream_t s, const GridDev& g, const float* u, const float* v, const float* w,
-                               uint16_t* dist);
-// Counting sort of the faces with 1 <= dist <= cap (cap <= K) into list, by
-// distance; lmask[k] = the mask of list[k]'s neighbours one layer below.  counts: ext_counts_size(K) entries of scratch; *offs receives
-// the device address of offs[0..cap+1] (offs[L] = first slot of distance L,
-// offs[cap+1] = total) and *maxd that of the largest distance present.
-size_t ext_counts_size(int32_t K);
-hipError_t launch_ext_sort(hipStream_t s, const GridDev& g, const uint16_t* dist, int32_t cap, int32_t K,
-                           uint32_t* counts, uint32_t* list, uint8_t* lmask, uint8_t* fmask, const uint32_t** offs,
-                           const uint32_t** maxd);
-// One layer: list[begin, begin+count) take the mean of their neighbours in
-// the previous layer (lmask).
-hipError_t launch_ext_layer(hipStream_t s, const GridDev& g, float* u, float* v, float* w, const uint32_t* list,
-                            const uint8_t* lmask, uint32_t begin, uint32_t count);
-// Layers first..last in one work-group (offs: the device offsets of the
-// sort; with last_dev, last is read from there on the device).
-hipError_t launch_ext_tail(hipStream_t s, const GridDev& g, float* u, float* v, float* w, const uint32_t* list,
-                           const uint8_t* lmask, const uint32_t* offs, int32_t first, int32_t last,
-                           const uint32_t* last_dev = nullptr);
-// Layers L and L+1 (n0 then n1 list entries from `begin`) in one launch;
-// fmask = every face's lower-neighbour mask.
-hipError_t launch_ext_layer2(hipStream_t s, const GridDev& g, float* u, float* v, float* w, const uint32_t* list,
-                             const uint8_t* lmask, const uint8_t* fmask, uint32_t begin, uint32_t n0, uint32_t n1);
+                               uint16_t* dist, uint16_t* mark, uint32_t* far);
+// Pass `pass` (from 1) over the marked bricks: layers 1..cap.  stamps: two
+// buffers of ext_bricks entries, the second marked by the distance transform.
+hipError_t launch_ext_bricks(hipStream_t s, const GridDev& g, float* u, float* v, float* w, const uint16_t* dist,
+                             int32_t cap, uint16_t* stamps, uint32_t pass);
 // buildFluidDensity / buildFluidSDF (EulerSolverTool.cu:324-448) on the
 // cell-centred grid; scratch holds ncell int32.
 hipError_t launch_fluid_density(hipStream_t s, const GridDev& g, const float* phi, const float* solid, float* out);

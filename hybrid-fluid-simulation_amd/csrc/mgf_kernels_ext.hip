@@ -9,17 +9,14 @@
 // on the full face grid with no obstacles, so the marker of a face is its L1
 // distance to the nearest known face (unknown beyond N-1).  Here:
 //
-//   1. distance transform, exact and separable: along x a wave-wide
-//      min-plus scan per row, along y and z a forward and a backward sweep per
-//      line (d = min(d, neighbour + 1));
-//   2. counting sort of the faces with 1 <= d <= N-1 by d (LDS histogram per
-//      block, one global atomic per block and distance into one of 32
-//      private copies);
-//   3. one gather kernel per pair of layers, over those layers' faces only,
-//      in layer order: the neighbours in layers below L are final when layer
-//      L runs, and a layer-L+1 face recomputes its layer-L neighbours' values
-//      (the sort also stores each face's mask of previous-layer neighbours,
-//      per list entry and per face).
+//   1. distance transform, exact and separable: along x the nearest known
+//      faces of a row from ballots, along y and z a min-plus transform per
+//      line; the z pass also marks the bricks (32 x 16 x 16 faces of one
+//      component) that hold a face at distance 1, and the largest distance;
+//   2. passes over bricks: a work-group takes a marked brick and its
+//      one-face halo into LDS and sets, in layer order, every face whose
+//      neighbours one layer below are final; a brick that set a face on one
+//      of its sides marks the brick there for the next pass.
 //
 // The mean is summed in the reference's neighbour order (-x, +x, -y, +y, -z,
 // +z) in FP32 and divided once, so the values are bitwise the reference's.
@@ -46,6 +43,28 @@ struct Faces {
     uint32_t ylines[4];   // prefix counts of y-lines (ex * ez)
     uint32_t zlines[4];   // prefix counts of z-lines (ex * ey)
     double rex[3], rexy[3];   // 1/ex, 1/(ex*ey)
+};
+
+// Bricks of a component's faces (the unit of a pass, below).
+constexpr uint32_t kBrickX = 32, kBrickY = 16, kBrickZ = 16;
+__host__ __device__ __forceinline__ uint32_t brick_nx(uint32_t ex) { return (ex + kBrickX - 1) / kBrickX; }
+__host__ __device__ __forceinline__ uint32_t brick_ny(uint32_t ey) { return (ey + kBrickY - 1) / kBrickY; }
+__host__ __device__ __forceinline__ uint32_t brick_nz(uint32_t ez) { return (ez + kBrickZ - 1) / kBrickZ; }
+// First brick of component c (3: all bricks).
+__host__ __device__ __forceinline__ uint32_t brick_base(const Faces& F, int c) {
+    uint32_t n = 0;
+    for (int k = 0; k < 3; ++k)
+        if (k < c) n += brick_nx(F.ex[k]) * brick_ny(F.ey[k]) * brick_nz(F.ez[k]);
+    return n;
+}
+// What the z pass of the distance transform leaves for the brick passes:
+// mark[brick] = 1 where the brick holds a face at distance 1, and the largest
+// distance as the maximum of kFarWords words (spread, so that work-groups do
+// not queue at one).
+constexpr uint32_t kFarWords = kExtFarWords;
+struct ExtSeed {
+    uint16_t* mark;
+    uint32_t* far;
 };
 
 __device__ __forceinline__ int comp_of(const uint32_t (&pre)[4], uint32_t t) {
@@ -154,7 +173,8 @@ struct MExtRows {
 // loads in flight per chunk (a line is a chain of dependent minima, so the
 // loads of a chunk are issued before its first minimum).
 template <int AXIS>
-__device__ __forceinline__ void k_ext_lines_run(Faces F, uint16_t* __restrict__ dist, uint32_t blk, uint32_t slot) {
+__device__ __forceinline__ void k_ext_lines_run(Faces F, uint16_t* __restrict__ dist, ExtSeed seed, uint32_t blk,
+                                                uint32_t slot) {
     (void)blk;
     (void)slot;
     const uint32_t t = slot * kBlock + threadIdx.x;
@@ -184,6 +204,9 @@ __device__ __forceinline__ void k_ext_lines_run(Faces F, uint16_t* __restrict__ 
         }
     }
     prev = kFaceInf;
+    uint32_t far = 0;
+    const uint32_t nbx = brick_nx(ex), nbxy = nbx * brick_ny(ey);
+    uint16_t* mark = AXIS == 2 ? seed.mark + brick_base(F, c) + (w / kBrickY) * nbx + x / kBrickX : nullptr;
     for (uint32_t k1 = len; k1 > 0;) {
         const uint32_t k0 = k1 >= K ? k1 - K : 0;
         const uint32_t m = k1 - k0;
@@ -195,15 +218,20 @@ __device__ __forceinline__ void k_ext_lines_run(Faces F, uint16_t* __restrict__ 
             if (uint32_t(q) < m) {
                 prev = min(v[q], prev + 1);
                 d[size_t(k1 - 1 - q) * stride] = uint16_t(min(prev, kFaceInf));
+                if (AXIS == 2) {
+                    if (prev == 1) mark[((k1 - 1 - q) / kBrickZ) * nbxy] = 1;
+                    far = max(far, prev < kFaceInf ? uint32_t(prev) : 0u);
+                }
             }
         }
         k1 = k0;
     }
+    if (AXIS == 2 && far) atomicMax(&seed.far[t % kFarWords], far);
 }
 
 template <int AXIS>
-__global__ void __launch_bounds__(kBlock) k_ext_lines(Faces F, uint16_t* __restrict__ dist) {
-    k_ext_lines_run<AXIS>(F, dist, xcd_block(), blockIdx.x);
+__global__ void __launch_bounds__(kBlock) k_ext_lines(Faces F, uint16_t* __restrict__ dist, ExtSeed seed) {
+    k_ext_lines_run<AXIS>(F, dist, seed, xcd_block(), blockIdx.x);
 }
 
 template <int AXIS>
@@ -211,8 +239,9 @@ struct MExtLines {
     static constexpr int kThreads = kBlock;
     Faces F;
     uint16_t* dist;
+    ExtSeed seed;
     uint32_t G;
-    __device__ void run(uint32_t vb) const { k_ext_lines_run<AXIS>(F, dist, xcd_of(vb, G), vb); }
+    __device__ void run(uint32_t vb) const { k_ext_lines_run<AXIS>(F, dist, seed, xcd_of(vb, G), vb); }
 };
 
 // 1b'. The same line transform in one read and one write of the distances
@@ -238,7 +267,8 @@ __device__ __forceinline__ uint32_t seg_stripes(const Faces& F, int c) {
 }
 
 template <int AXIS, int SEG, int WAVES = kLineSegWaves>
-__device__ __forceinline__ void k_ext_lines_seg_run(Faces F, uint16_t* __restrict__ dist, uint32_t blk, uint32_t slot) {
+__device__ __forceinline__ void k_ext_lines_seg_run(Faces F, uint16_t* __restrict__ dist, ExtSeed seed, uint32_t blk,
+                                                    uint32_t slot) {
     (void)slot;
     __shared__ int32_t sp[WAVES][64], ss[WAVES][64];
     const uint32_t(&pre)[4] = AXIS == 1 ? F.ylines : F.zlines;
@@ -261,6 +291,8 @@ __device__ __forceinline__ void k_ext_lines_seg_run(Faces F, uint16_t* __restric
     const uint32_t seg = (len + WAVES - 1) / WAVES;
     const uint32_t a = wv * seg;
     const uint32_t n = a < len ? min(seg, len - a) : 0u;   // faces of this wave's segment
+    uint32_t* far_word = AXIS == 2 ? seed.far + (blk * WAVES + wv) % kFarWords : nullptr;
+    const uint32_t seen = AXIS == 2 ? *far_word : 0u;
     // Buffer accesses: the lane's line start in the VGPR offset, the row's
     // wave-uniform byte offset in the SGPR offset (no 64-bit address per row).
     const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(dist, int16_t(0), int32_t(2u * F.off[3]), kBufWord3);
@@ -296,6 +328,30 @@ __device__ __forceinline__ void k_ext_lines_seg_run(Faces F, uint16_t* __restric
         g = min(g, v[q] + int32_t(a + q));
         v[q] = g - int32_t(a + q);
     }
+    if (AXIS == 2) {
+        // the final distances: bricks with a face at distance 1, the largest
+        const uint32_t nbx = brick_nx(ex), nbxy = nbx * brick_ny(ey);
+        uint16_t* mark = seed.mark + brick_base(F, c) + (w / kBrickY) * nbx + x / kBrickX;
+        int32_t far = 0;
+        uint32_t hits = 0;   // bit k: a distance of 1 in the k-th brick along z from this segment's first
+        const uint32_t za = a / kBrickZ;
+#pragma unroll
+        for (int q = 0; q < SEG; ++q) {
+            if (uint32_t(q) < n) {   // wave-uniform
+                hits |= v[q] == 1 ? 1u << ((a + q) / kBrickZ - za) : 0u;
+                far = max(far, v[q]);
+            }
+        }
+        // a component is reached everywhere or nowhere
+        if (!ok || far >= kFaceInf) far = 0;
+        if (!ok) hits = 0;
+        far = __builtin_amdgcn_readlane(-wave_min_prefix(-far), 63);
+        // one word a wave, spread, and only where it grows (the word as read
+        // when the wave began, which may be old)
+        if (lane == 0 && uint32_t(far) > seen) atomicMax(far_word, uint32_t(far));
+        for (uint32_t k = 0; k <= (SEG + kBrickZ - 1) / kBrickZ; ++k)
+            if ((hits >> k) & 1u) mark[(za + k) * nbxy] = 1;
+    }
 #pragma unroll
     for (int q = 0; q < SEG; ++q) {
         if (ok && uint32_t(q) < n)
@@ -304,8 +360,9 @@ __device__ __forceinline__ void k_ext_lines_seg_run(Faces F, uint16_t* __restric
 }
 
 template <int AXIS, int SEG, int WAVES = kLineSegWaves>
-__global__ void __launch_bounds__(64 * WAVES) k_ext_lines_seg(Faces F, uint16_t* __restrict__ dist) {
-    k_ext_lines_seg_run<AXIS, SEG, WAVES>(F, dist, xcd_block(), blockIdx.x);
+__global__ void __launch_bounds__(64 * WAVES) k_ext_lines_seg(Faces F, uint16_t* __restrict__ dist,
+                                                             ExtSeed seed) {
+    k_ext_lines_seg_run<AXIS, SEG, WAVES>(F, dist, seed, xcd_block(), blockIdx.x);
 }
 
 template <int AXIS, int SEG, int WAVES = kLineSegWaves>
@@ -313,8 +370,9 @@ struct MExtLinesSeg {
     static constexpr int kThreads = 64 * WAVES;
     Faces F;
     uint16_t* dist;
+    ExtSeed seed;
     uint32_t G;
-    __device__ void run(uint32_t vb) const { k_ext_lines_seg_run<AXIS, SEG, WAVES>(F, dist, xcd_of(vb, G), vb); }
+    __device__ void run(uint32_t vb) const { k_ext_lines_seg_run<AXIS, SEG, WAVES>(F, dist, seed, xcd_of(vb, G), vb); }
 };
 
 // Short lines (at most kLineShortWaves * SEG faces) in work-groups of
@@ -497,482 +555,348 @@ struct MExtRowsReg {
 };
 
 // ---------------------------------------------------------------------------
-// 2. Counting sort by distance.  Bins 1..cap.  A block counts its faces in
-// LDS (kLdsBins bins; larger distances go straight to the global counters),
-// then adds its non-zero bins to one of kCopies private copies of the global
-// histogram (copy = block % kCopies): the atomics of different blocks on one
-// distance are spread over kCopies addresses instead of serialising on one.
-constexpr int kLdsBins = 2048;
-constexpr int kSortCpt = 8;   // faces per work-item
-constexpr int kCopies = 32;
+// 2. Passes over bricks.
+//
+// One launch per layer is bound by launches and latency: a layer is a thin
+// shell, 222 of them at 256^3, 8 us each for gathers that move 11x the bytes
+// they need, after a counting sort of the faces by distance (0.32 ms); 1.96 ms
+// in all.  A brick in LDS takes all the layers that cross it in one visit:
+// 18 passes of 74 us (1.34 ms; 512^3: 10.2 -> 4.7 ms).  What bounds a pass is
+// a visit's latency, about 20 us (load 5, masks 3, sort 4, a layer 0.3).
+//
+// Which faces a visit can set: a face at distance L needs its neighbours at
+// distance L - 1 (a path down to a known face is a shortest one, so it is
+// monotone along each axis), inside the brick or on the halo as the brick was
+// loaded.  A face is set (not UNKNOWN) or still UNKNOWN, never anything else: a
+// mean over values other than UNKNOWN (FLT_MAX) is FLT_MAX only if its sum
+// is, which needs one neighbour that is.  Reading a neighbouring brick's face
+// while that brick is being visited gives either, and either is fine: a brick
+// that sets a face for which one beyond its side waits marks the brick there
+// for the next pass.  By
+// induction along the paths, a face is set at the latest in pass
+// 1 + (brick sides its longest path crosses), whatever the order of visits, so
+// ext_passes() passes set every face, and each face once, from final values.
+//
+// Marks are stamps: pass p visits the bricks whose stamp in buffer p % 2 is p
+// and stamps p + 1 into the other one, so no pass reads what it writes.
+// Every work-group counts all stamps of its pass (two bytes a brick, from L2)
+// and takes the bricks whose rank is its own index, and every gridDim.x-th
+// after it: no list, no counter that all work-groups would queue at.
+constexpr int kBrickPer = int(kBrickX) / 4;   // faces a work-item: the 4 x 4 x 4 groups of a wave along x
+constexpr int kBrickThreads = int(kBrickX * kBrickY * kBrickZ) / kBrickPer;
+constexpr int kHx = int(kBrickX) + 2, kHy = int(kBrickY) + 2, kHz = int(kBrickZ) + 2, kHalo = kHx * kHy * kHz;
 
-// Layout of the counter buffer for bins 0..K+1 (K2 = K + 2 entries a row):
-// hist[kCopies][K2], cursor[kCopies][K2], poff[kCopies][K2], offs[K2], maxd.
-struct SortBufs {
-    uint32_t *hist, *cursor, *poff, *offs, *maxd;
+struct BrickArgs {
+    Faces F;
+    const uint16_t* dist;
+    int32_t cap;        // layers 1..cap are set
+    uint32_t first;     // this scene's first brick among the stamps
 };
-static SortBufs sort_bufs(uint32_t* counts, int32_t K) {
-    const size_t K2 = size_t(K) + 2;
-    SortBufs b;
-    b.hist = counts;
-    b.cursor = b.hist + kCopies * K2;
-    b.poff = b.cursor + kCopies * K2;
-    b.offs = b.poff + kCopies * K2;
-    b.maxd = b.offs + K2;
-    return b;
-}
 
-// Counts the active lanes of a wave by key into LDS counters and returns, per
-// active lane, a slot in [old counter, old counter + lanes with its key).
-// Where every active lane holds the same key (the common case: a row of faces
-// at one distance) one lane adds them all with one atomic; otherwise each lane
-// adds itself (distances along a row differ, so the addresses mostly differ).
-__device__ __forceinline__ uint32_t lds_count(uint32_t* ctr_of_key, int32_t key, bool active) {
-    const uint64_t act = __ballot(active);
-    if (act == 0) return 0;
-    const int lane = threadIdx.x & 63;
-    const int leader = __ffsll((unsigned long long)act) - 1;
-    const int32_t k0 = __builtin_amdgcn_readlane(key, leader);
-    const uint64_t same = __ballot(active && key == k0);
-    if (same == act) {
-        uint32_t base = 0;
-        if (lane == leader) base = atomicAdd(&ctr_of_key[k0], uint32_t(__popcll(act)));
-        base = __builtin_amdgcn_readlane(base, leader);
-        return base + uint32_t(__popcll(act & ((1ull << lane) - 1ull)));
+// LDS of a work-group, 80 KB: two fit a CU.
+constexpr int kBrickWaves = kBrickThreads / 64;
+constexpr int kBrickFaces = kBrickThreads * kBrickPer;
+struct BrickLds {
+    float v[kHalo];
+    union {
+        uint16_t d[kHalo];
+        uint32_t list[kBrickFaces];   // by layer: the face's place in v, its mask (m) from bit 14 on
+    };
+    uint32_t at[kBrickWaves][64];     // a wave's faces by layer
+    uint32_t wsum[kBrickWaves];
+    int32_t lo, hi;
+    uint32_t sides, brick;
+};
+
+// One visit; stamps: this scene's bricks in the buffer written.
+//
+// A layer holds a few of a wave's faces, so a wave that walked its own faces
+// layer by layer would run each mean for a few lanes (390 us a pass at 256^3
+// that way).  The faces still to be set are first sorted by layer in LDS, and
+// a layer's work-items then take list entries densely.  The sort uses no LDS
+// atomics (a layer's counter would take them one lane at a time): a wave
+// holds 4 x 4 x 4 faces a register, which cross at most 10 layers, finds the
+// lanes of one layer with a ballot, and keeps its count of each layer in the
+// lane of that number (a brick spans at most 31 + 15 + 15 + 1 layers).
+// Bricks of 32 x 8 x 16, 32 x 8 x 8 and 16 x 8 x 8 faces (more passes, more
+// stamps) measured slower at 256^3: 8.31, 8.78 and 9.56 ms a step against 8.22.
+__device__ __forceinline__ void brick_visit(const BrickArgs& A, uint32_t lb, uint16_t* __restrict__ stamps,
+                                            uint32_t pass, BrickLds& S) {
+    const Faces& F = A.F;
+    int t = threadIdx.x;
+    // what depends on the work-item alone is formed in the visit: hoisted out
+    // of the loop over bricks it takes the registers of a second work-group
+    asm volatile("" : "+v"(t));
+    const int lane = t & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
+    const uint32_t b1 = brick_base(F, 1), b2 = brick_base(F, 2);
+    const int c = lb < b1 ? 0 : (lb < b2 ? 1 : 2);
+    const uint32_t q = lb - (c == 0 ? 0u : (c == 1 ? b1 : b2));
+    const int ex = int(pick(F.ex, c)), ey = int(pick(F.ey, c)), ez = int(pick(F.ez, c));
+    const uint32_t nbx = brick_nx(ex), nby = brick_ny(ey), nbz = brick_nz(ez);
+    const uint32_t bx = q % nbx, by = (q / nbx) % nby, bz = q / (nbx * nby);
+    const int x0 = int(bx * kBrickX) - 1, y0 = int(by * kBrickY) - 1, z0 = int(bz * kBrickZ) - 1;
+    float* f = pick(F.f, c);
+    const uint16_t* dist = A.dist + pick4(F.off, c);
+    if (t == 0) {
+        S.lo = kFaceInf;
+        S.hi = 0;
+        S.sides = 0;
     }
-    return active ? atomicAdd(&ctr_of_key[key], 1u) : 0u;
+    // the brick and its halo; outside the grid: unreached
+    constexpr int kLoads = (kHalo + kBrickThreads - 1) / kBrickThreads, kBatch = 11;
+#pragma unroll
+    for (int k0 = 0; k0 < kLoads; k0 += kBatch) {
+        float lv[kBatch];
+        uint32_t ld[kBatch];
+#pragma unroll
+        for (int k = 0; k < kBatch; ++k) {
+            const int i = (k0 + k) * kBrickThreads + t;
+            const int x = x0 + i % kHx, y = y0 + (i / kHx) % kHy, z = z0 + i / (kHx * kHy);
+            const bool in = i < kHalo && x >= 0 && y >= 0 && z >= 0 && x < ex && y < ey && z < ez;
+            const uint32_t j = in ? (uint32_t(z) * uint32_t(ey) + uint32_t(y)) * uint32_t(ex) + uint32_t(x) : 0u;
+            lv[k] = f[j];
+            ld[k] = dist[j];
+            if (!in) ld[k] = uint32_t(kFaceInf);
+        }
+#pragma unroll
+        for (int k = 0; k < kBatch; ++k) {
+            const int i = (k0 + k) * kBrickThreads + t;
+            if (i < kHalo) {
+                S.v[i] = lv[k];
+                S.d[i] = uint16_t(ld[k]);
+            }
+        }
+        asm volatile("" ::: "memory");
+    }
+    __syncthreads();
+    // this work-item's faces: the wave's 4 x 4 x 4 groups are k = 0..7 along x
+    // in rows of groups along y, then z
+    constexpr int kRows = int(kBrickY) / 4;
+    const int gy = 4 * (wv % kRows) + ((lane >> 2) & 3), gz = 4 * (wv / kRows) + (lane >> 4);
+    const int at0 = ((gz + 1) * kHy + gy + 1) * kHx + (lane & 3) + 1;
+    const int nb[6] = {-1, 1, -kHx, kHx, -kHx * kHy, kHx * kHy};
+    int32_t d[kBrickPer];
+    // neighbours one layer below (0: nothing to set), and from bit 6 on the
+    // brick's sides across which a face waits for this one (a face one layer
+    // above one still to be set is)
+    uint32_t m[kBrickPer];
+    int32_t lo = kFaceInf, hi = 0;
+    const uint32_t side_yz = (gy == 0 ? 4u : 0u) | (gy == int(kBrickY) - 1 ? 8u : 0u) | (gz == 0 ? 16u : 0u) |
+                             (gz == int(kBrickZ) - 1 ? 32u : 0u);
+#pragma unroll
+    for (int k = 0; k < kBrickPer; ++k) {
+        const int o = at0 + 4 * k;
+        d[k] = S.d[o];
+        int32_t dn[6];
+#pragma unroll
+        for (int n = 0; n < 6; ++n) dn[n] = S.d[o + nb[n]];
+        const bool wait = d[k] >= 1 && d[k] <= A.cap && S.v[o] == MGF_UNKNOWN;
+        uint32_t below = 0, above = 0;
+#pragma unroll
+        for (int n = 0; n < 6; ++n) {
+            below |= dn[n] < d[k] ? 1u << n : 0u;
+            above |= dn[n] == d[k] + 1 ? 1u << n : 0u;
+        }
+        const uint32_t side = side_yz | (k == 0 && (lane & 3) == 0 ? 1u : 0u) |
+                              (k == kBrickPer - 1 && (lane & 3) == 3 ? 2u : 0u);
+        m[k] = wait ? below | ((above & side) << 6) : 0u;
+        lo = min(lo, wait ? d[k] : kFaceInf);
+        hi = max(hi, wait ? d[k] : 0);
+        // two work-groups a CU need 64 VGPRs: not every group's reads at once
+        if (k & 1) asm volatile("" ::: "memory");
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        lo = min(lo, __shfl_xor(lo, o, 64));
+        hi = max(hi, __shfl_xor(hi, o, 64));
+    }
+    if (lane == 0) {
+        atomicMin(&S.lo, lo);
+        atomicMax(&S.hi, hi);
+    }
+    __syncthreads();   // S.d is free from here on
+    const int32_t first = __builtin_amdgcn_readfirstlane(S.lo), last = __builtin_amdgcn_readfirstlane(S.hi);
+    if (first > last) return;   // nothing to set (the same for every work-item)
+    uint32_t rank[kBrickPer], mine = 0;   // mine: the wave's faces of layer first + lane
+#pragma unroll
+    for (int k = 0; k < kBrickPer; ++k) {
+        rank[k] = 0;
+        uint64_t todo = __ballot(m[k] != 0);
+        while (todo) {
+            const int32_t l = __builtin_amdgcn_readlane(d[k], __ffsll((unsigned long long)todo) - 1);
+            const uint64_t same = __ballot(m[k] != 0 && d[k] == l);
+            const uint32_t had = uint32_t(__builtin_amdgcn_readlane(int(mine), l - first));
+            if (d[k] == l) rank[k] = had + __builtin_amdgcn_mbcnt_hi(uint32_t(same >> 32),
+                                                                    __builtin_amdgcn_mbcnt_lo(uint32_t(same), 0u));
+            if (lane == l - first) mine += uint32_t(__popcll(same));
+            todo &= ~same;
+        }
+    }
+    // first list entry of each layer, and of this wave's faces of each: the
+    // layer in the lane of its number (every wave for itself)
+    S.at[wv][lane] = mine;
+    __syncthreads();
+    uint32_t all = 0, here = 0;
+#pragma unroll
+    for (int w = 0; w < kBrickWaves; ++w) {
+        const uint32_t x = S.at[w][lane];
+        here += w < wv ? x : 0u;
+        all += x;
+    }
+    uint32_t starts = all;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t u = uint32_t(__shfl_up(int(starts), o, 64));
+        if (lane >= o) starts += u;
+    }
+    const uint32_t faces = uint32_t(__builtin_amdgcn_readlane(int(starts), 63));
+    starts -= all;
+    here += starts;
+#pragma unroll
+    for (int k = 0; k < kBrickPer; ++k) {
+        const uint32_t to = uint32_t(__shfl(int(here), (m[k] ? d[k] - first : 0), 64)) + rank[k];
+        if (m[k]) S.list[to] = uint32_t(at0 + 4 * k) | (m[k] << 14);
+    }
+    __syncthreads();
+    // The layers, one barrier each.  A layer's step is a chain of latencies
+    // (list entry, neighbours, sum, quotient, store, barrier), so the next
+    // layer's entries are read beside this one's neighbours, waves without an
+    // entry skip it, and the sum selects with bit masks.
+    const int32_t layers = last - first + 1;
+    uint32_t b0 = 0, e0 = uint32_t(__builtin_amdgcn_readlane(int(starts), 1));
+    auto entry = [&](uint32_t e) { return S.list[min(e, faces - 1)]; };
+    uint32_t next = entry(t);
+    auto set = [&](uint32_t e, uint32_t w, uint32_t ahead) {
+        const int o = int(w & 0x3FFFu);
+        uint32_t fv[6];
+#pragma unroll
+        for (int n = 0; n < 6; ++n) fv[n] = __float_as_uint(S.v[o + nb[n]]);
+        next = entry(ahead);
+        // an unused neighbour adds +0: the sum starts at +0, so it is never
+        // -0 and stays as it is
+        float acc = 0.0f;
+        uint32_t known = ~0u;   // 0 once a neighbour used is UNKNOWN
+#pragma unroll
+        for (int n = 0; n < 6; ++n) {
+            const uint32_t u = fv[n] & uint32_t(__builtin_amdgcn_sbfe(int(w), 14 + n, 1));
+            known = min(known, u ^ 0x7F7FFFFFu);
+            acc += __uint_as_float(u);
+        }
+        // 1, 2 and 4: the reciprocal and the product are exact as the quotient is
+        const uint32_t cnt = uint32_t(__popc((w >> 14) & 63u));
+        float mean = acc * __builtin_amdgcn_rcpf(float(cnt));
+        if (cnt == 3u || cnt > 4u) mean = acc / float(cnt);
+        if (e < e0 && known != 0u) S.v[o] = mean;
+    };
+    for (int32_t l = 0; l < layers; ++l) {
+        const uint32_t b1 = e0, e1 = uint32_t(__builtin_amdgcn_readlane(int(starts), min(l + 2, 63)));
+        if (b0 + 64u * uint32_t(wv) < e0) {
+            set(b0 + t, next, b1 + t);
+            for (uint32_t q = b0 + kBrickThreads; q + 64u * uint32_t(wv) < e0; q += kBrickThreads) set(q + t, entry(q + t), b1 + t);
+        } else {
+            next = entry(b1 + t);
+        }
+        b0 = b1;
+        e0 = e1;
+        __syncthreads();
+    }
+    // the faces set in this visit, and the sides beyond which one waits for them
+    uint32_t sides = 0;
+    for (uint32_t e = t; e < faces; e += kBrickThreads) {
+        const uint32_t w = S.list[e];
+        const int o = int(w & 0x3FFFu);
+        const float v = S.v[o];
+        if (v != MGF_UNKNOWN) {
+            const int lx = o % kHx, ly = (o / kHx) % kHy, lz = o / (kHx * kHy);
+            f[(uint32_t(z0 + lz) * uint32_t(ey) + uint32_t(y0 + ly)) * uint32_t(ex) + uint32_t(x0 + lx)] = v;
+            sides |= w >> 20;
+        }
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) sides |= uint32_t(__shfl_xor(int(sides), o, 64));
+    if (lane == 0 && sides) atomicOr(&S.sides, sides);
+    __syncthreads();
+    if (t < 6 && ((S.sides >> t) & 1u)) {
+        const bool in = t == 0 ? bx > 0 : (t == 1 ? bx + 1 < nbx : (t == 2 ? by > 0 : (t == 3 ? by + 1 < nby
+                        : (t == 4 ? bz > 0 : bz + 1 < nbz))));
+        const int32_t step = t == 0 ? -1 : (t == 1 ? 1 : (t == 2 ? -int32_t(nbx) : (t == 3 ? int32_t(nbx)
+                             : (t == 4 ? -int32_t(nbx * nby) : int32_t(nbx * nby)))));
+        if (in) stamps[int64_t(lb) + step] = uint16_t(pass + 1);
+    }
+    __syncthreads();   // S is reused by the next visit
 }
 
-__device__ __forceinline__ void k_ext_zero_run(uint32_t* __restrict__ a, uint32_t n, uint32_t blk, uint32_t slot) {
-    (void)blk;
-    (void)slot;
-    const uint32_t i = slot * kBlock + threadIdx.x;
+// The bricks of one pass; total: bricks of all scenes, a multiple of 8 with
+// padding that is never stamped; scene_of: each brick's scene (null: one).
+template <bool MULTI>
+__device__ __forceinline__ void bricks_run(const BrickArgs* __restrict__ tab, const BrickArgs& one,
+                                           const uint16_t* __restrict__ scene_of, uint16_t* stamps, uint32_t total,
+                                           uint32_t pass) {
+    __shared__ BrickLds S;
+    const uint16_t* rd = stamps + size_t(pass & 1u) * total;
+    uint16_t* wr = stamps + size_t((pass + 1u) & 1u) * total;
+    const int t = threadIdx.x;
+    const uint32_t chunks = total / 8, per = (chunks + kBrickThreads - 1) / kBrickThreads;
+    const uint32_t c0 = min(chunks, uint32_t(t) * per), c1 = min(chunks, c0 + per);
+    const uint4* rv = reinterpret_cast<const uint4*>(rd);
+    auto count = [&](uint32_t w) { return uint32_t((w & 0xFFFFu) == pass) + uint32_t((w >> 16) == pass); };
+    uint32_t cnt = 0;
+    for (uint32_t i = c0; i < c1; ++i) {
+        const uint4 w = rv[i];
+        cnt += count(w.x) + count(w.y) + count(w.z) + count(w.w);
+    }
+    uint32_t incl = cnt;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t u = uint32_t(__shfl_up(int(incl), o, 64));
+        if ((t & 63) >= o) incl += u;
+    }
+    if ((t & 63) == 63) S.wsum[t >> 6] = incl;
+    __syncthreads();
+    uint32_t before = incl - cnt, all = 0;
+    for (int w = 0; w < kBrickWaves; ++w) {
+        if (w < (t >> 6)) before += S.wsum[w];
+        all += S.wsum[w];
+    }
+    for (uint32_t k = blockIdx.x; k < all; k += gridDim.x) {
+        if (k >= before && k < before + cnt) {
+            uint32_t left = k - before;
+            for (uint32_t i = c0 * 8; i < c1 * 8; ++i) {
+                if (rd[i] != pass) continue;
+                if (left == 0) {
+                    S.brick = i;
+                    break;
+                }
+                --left;
+            }
+        }
+        __syncthreads();
+        const uint32_t b = S.brick;
+        if constexpr (MULTI) {
+            const BrickArgs& A = tab[scene_of[b]];
+            brick_visit(A, b - A.first, wr + A.first, pass, S);
+        } else {
+            brick_visit(one, b, wr, pass, S);
+        }
+    }
+}
+
+__global__ void __launch_bounds__(kBrickThreads, 8) k_ext_bricks(BrickArgs A, uint16_t* stamps, uint32_t total,
+                                                              uint32_t pass) {
+    bricks_run<false>(nullptr, A, nullptr, stamps, total, pass);
+}
+__global__ void __launch_bounds__(kBrickThreads, 8) k_multi_bricks(const BrickArgs* __restrict__ tab,
+                                                                const uint16_t* __restrict__ scene_of,
+                                                                uint16_t* stamps, uint32_t total, uint32_t pass) {
+    bricks_run<true>(tab, BrickArgs{}, scene_of, stamps, total, pass);
+}
+
+// The stamps and the far words, before the distance transform.
+__global__ void __launch_bounds__(kBlock) k_ext_zero(uint32_t* __restrict__ a, uint32_t n) {
+    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
     if (i < n) a[i] = 0;
 }
-
-__global__ void __launch_bounds__(kBlock) k_ext_zero(uint32_t* __restrict__ a, uint32_t n) {
-    k_ext_zero_run(a, n, xcd_block(), blockIdx.x);
-}
-
-struct MExtZero {
-    static constexpr int kThreads = kBlock;
-    uint32_t* a;
-    uint32_t n;
-    uint32_t G;
-    __device__ void run(uint32_t vb) const { k_ext_zero_run(a, n, xcd_of(vb, G), vb); }
-};
-
-__device__ __forceinline__ void k_ext_count_run(const uint16_t* __restrict__ dist, uint32_t total, int32_t cap,
-                                                      uint32_t* __restrict__ hist, uint32_t K2, uint32_t blk, uint32_t slot) {
-    (void)blk;
-    (void)slot;
-    __shared__ uint32_t h[kLdsBins];
-    const int32_t nb = min(cap + 1, kLdsBins);
-    for (int b = threadIdx.x; b < nb; b += kBlock) h[b] = 0;
-    __syncthreads();
-    uint32_t* hp = hist + size_t(slot % kCopies) * K2;
-    const uint32_t base = blk * (kBlock * kSortCpt) + threadIdx.x;
-    // all loads first (clamped index, no branch), then the counting
-    int32_t dv[kSortCpt];
-#pragma unroll
-    for (int k = 0; k < kSortCpt; ++k) {
-        const uint32_t i = base + uint32_t(k) * kBlock;
-        dv[k] = dist[i < total ? i : total - 1];
-        if (i >= total) dv[k] = 0;
-    }
-#pragma unroll
-    for (int k = 0; k < kSortCpt; ++k) {
-        const bool in = dv[k] >= 1 && dv[k] <= cap;
-        (void)lds_count(h, dv[k] < kLdsBins ? dv[k] : 0, in && dv[k] < kLdsBins);
-        if (in && dv[k] >= kLdsBins) atomicAdd(&hp[dv[k]], 1u);
-    }
-    __syncthreads();
-    for (int b = 1 + threadIdx.x; b < nb; b += kBlock)
-        if (h[b]) atomicAdd(&hp[b], h[b]);
-}
-
-__global__ void __launch_bounds__(kBlock) k_ext_count(const uint16_t* __restrict__ dist, uint32_t total, int32_t cap,
-                                                      uint32_t* __restrict__ hist, uint32_t K2) {
-    k_ext_count_run(dist, total, cap, hist, K2, xcd_block(), blockIdx.x);
-}
-
-struct MExtCount {
-    static constexpr int kThreads = kBlock;
-    const uint16_t* dist;
-    uint32_t total;
-    int32_t cap;
-    uint32_t* hist;
-    uint32_t K2;
-    uint32_t G;
-    __device__ void run(uint32_t vb) const { k_ext_count_run(dist, total, cap, hist, K2, xcd_of(vb, G), vb); }
-};
-
-// Per distance b: T = sum over copies; offs[b] = exclusive scan of T over
-// b = 1..cap (offs[cap+1] = total); poff[p][b] = offs[b] + counts of the
-// copies before p; cursors cleared; *maxd = the largest non-empty distance.
-// One block.
-__device__ __forceinline__ void k_ext_scan_run(const uint32_t* __restrict__ hist, int32_t cap, uint32_t K2,
-                                                   uint32_t* __restrict__ offs, uint32_t* __restrict__ poff,
-                                                   uint32_t* __restrict__ cursor, uint32_t* __restrict__ maxd, uint32_t blk, uint32_t slot) {
-    (void)blk;
-    (void)slot;
-    __shared__ uint32_t wsum[16];
-    __shared__ uint32_t carry;
-    __shared__ int32_t top;
-    if (threadIdx.x == 0) { carry = 0; top = 0; }
-    __syncthreads();
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    for (int32_t b0 = 1; b0 <= cap; b0 += 1024) {
-        const int32_t b = b0 + int32_t(threadIdx.x);
-        uint32_t v = 0;
-        if (b <= cap) {
-#pragma unroll 8
-            for (int p = 0; p < kCopies; ++p) v += hist[size_t(p) * K2 + b];
-        }
-        uint32_t incl = v;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const uint32_t t = __shfl_up(incl, o, 64);
-            if (lane >= o) incl += t;
-        }
-        if (lane == 63) wsum[wv] = incl;
-        __syncthreads();
-        uint32_t before = carry;
-        for (int q = 0; q < wv; ++q) before += wsum[q];
-        if (b <= cap) {
-            const uint32_t o = before + incl - v;
-            offs[b] = o;
-            uint32_t run = o;
-            for (int p = 0; p < kCopies; ++p) {
-                poff[size_t(p) * K2 + b] = run;
-                cursor[size_t(p) * K2 + b] = 0;
-                run += hist[size_t(p) * K2 + b];
-            }
-            if (v) atomicMax(&top, b);
-        }
-        __syncthreads();
-        if (threadIdx.x == 1023) carry = before + incl;
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        offs[cap + 1] = carry;
-        *maxd = uint32_t(top);
-    }
-}
-
-__global__ void __launch_bounds__(1024) k_ext_scan(const uint32_t* __restrict__ hist, int32_t cap, uint32_t K2,
-                                                   uint32_t* __restrict__ offs, uint32_t* __restrict__ poff,
-                                                   uint32_t* __restrict__ cursor, uint32_t* __restrict__ maxd) {
-    k_ext_scan_run(hist, cap, K2, offs, poff, cursor, maxd, xcd_block(), blockIdx.x);
-}
-
-struct MExtScan {
-    static constexpr int kThreads = 1024;
-    const uint32_t* hist;
-    int32_t cap;
-    uint32_t K2;
-    uint32_t* offs;
-    uint32_t* poff;
-    uint32_t* cursor;
-    uint32_t* maxd;
-    uint32_t G;
-    __device__ void run(uint32_t vb) const { k_ext_scan_run(hist, cap, K2, offs, poff, cursor, maxd, xcd_of(vb, G), vb); }
-};
-
-// Bit q of the lower-neighbour mask of a face: its in-grid neighbour in
-// direction q (-x, +x, -y, +y, -z, +z) has a smaller distance, i.e. lies in
-// the previous layer.
-__device__ __forceinline__ uint32_t lower_mask(const Faces& F, const uint16_t* __restrict__ dist, uint32_t gi,
-                                               int32_t dv) {
-    const int c = comp_of(F.off, gi);
-    const uint32_t o = pick4(F.off, c);
-    const uint32_t i = gi - o;
-    const uint32_t ex = pick(F.ex, c), ey = pick(F.ey, c), ez = pick(F.ez, c), sz = ex * ey;
-    const uint32_t z = udiv_r(i, sz, pick(F.rexy, c));
-    const uint32_t rem = i - z * sz;
-    const uint32_t y = udiv_r(rem, ex, pick(F.rex, c));
-    const uint32_t x = rem - y * ex;
-    const bool in[6] = {x > 0, x + 1 < ex, y > 0, y + 1 < ey, z > 0, z + 1 < ez};
-    const uint32_t j[6] = {in[0] ? gi - 1 : gi, in[1] ? gi + 1 : gi, in[2] ? gi - ex : gi,
-                           in[3] ? gi + ex : gi, in[4] ? gi - sz : gi, in[5] ? gi + sz : gi};
-    int32_t dn[6];
-#pragma unroll
-    for (int q = 0; q < 6; ++q) dn[q] = dist[j[q]];
-    uint32_t m = 0;
-#pragma unroll
-    for (int q = 0; q < 6; ++q) m |= (in[q] && dn[q] < dv) ? (1u << q) : 0u;
-    return m;
-}
-
-__device__ __forceinline__ void k_ext_scatter_run(Faces F, const uint16_t* __restrict__ dist, uint32_t total,
-                                                        int32_t cap, uint32_t K2, const uint32_t* __restrict__ poff,
-                                                        uint32_t* cursor, uint32_t* __restrict__ list,
-                                                        uint8_t* __restrict__ lmask, uint8_t* __restrict__ fmask, uint32_t blk, uint32_t slot) {
-    (void)blk;
-    (void)slot;
-    __shared__ uint32_t h[kLdsBins];
-    const int32_t nb = min(cap + 1, kLdsBins);
-    for (int b = threadIdx.x; b < nb; b += kBlock) h[b] = 0;
-    __syncthreads();
-    const size_t copy = size_t(slot % kCopies) * K2;
-    const uint32_t* po = poff + copy;
-    uint32_t* cu = cursor + copy;
-    const uint32_t base = blk * (kBlock * kSortCpt) + threadIdx.x;
-    int32_t dv[kSortCpt];
-    uint32_t rank[kSortCpt];
-#pragma unroll
-    for (int k = 0; k < kSortCpt; ++k) {
-        const uint32_t i = base + uint32_t(k) * kBlock;
-        dv[k] = dist[i < total ? i : total - 1];
-        if (i >= total) dv[k] = 0;
-    }
-#pragma unroll
-    for (int k = 0; k < kSortCpt; ++k) {
-        const bool in = dv[k] >= 1 && dv[k] <= cap;
-        rank[k] = lds_count(h, dv[k] < kLdsBins ? dv[k] : 0, in && dv[k] < kLdsBins);
-        if (in && dv[k] >= kLdsBins) rank[k] = atomicAdd(&cu[dv[k]], 1u);
-    }
-    __syncthreads();
-    // reserve each bin's range in this block's copy: the bin's slot now holds its base
-    for (int b = 1 + threadIdx.x; b < nb; b += kBlock)
-        if (h[b]) h[b] = atomicAdd(&cu[b], h[b]);
-    __syncthreads();
-    // Only faces that enter the list need their mask: known faces (0) and
-    // those past the cap skip the six neighbour loads.
-    uint32_t msk[kSortCpt];
-#pragma unroll
-    for (int k = 0; k < kSortCpt; ++k) {
-        const uint32_t i = base + uint32_t(k) * kBlock;
-        msk[k] = (dv[k] >= 1 && dv[k] <= cap) ? lower_mask(F, dist, i < total ? i : total - 1, dv[k]) : 0u;
-    }
-#pragma unroll
-    for (int k = 0; k < kSortCpt; ++k) {
-        const uint32_t i = base + uint32_t(k) * kBlock;
-        if (dv[k] >= 1 && dv[k] <= cap) {
-            const uint32_t pos = po[dv[k]] + (dv[k] < kLdsBins ? h[dv[k]] : 0u) + rank[k];
-            list[pos] = i;
-            lmask[pos] = uint8_t(msk[k]);
-            fmask[i] = uint8_t(msk[k]);
-        }
-    }
-}
-
-__global__ void __launch_bounds__(kBlock) k_ext_scatter(Faces F, const uint16_t* __restrict__ dist, uint32_t total,
-                                                        int32_t cap, uint32_t K2, const uint32_t* __restrict__ poff,
-                                                        uint32_t* cursor, uint32_t* __restrict__ list,
-                                                        uint8_t* __restrict__ lmask, uint8_t* __restrict__ fmask) {
-    k_ext_scatter_run(F, dist, total, cap, K2, poff, cursor, list, lmask, fmask, xcd_block(), blockIdx.x);
-}
-
-struct MExtScatter {
-    static constexpr int kThreads = kBlock;
-    Faces F;
-    const uint16_t* dist;
-    uint32_t total;
-    int32_t cap;
-    uint32_t K2;
-    const uint32_t* poff;
-    uint32_t* cursor;
-    uint32_t* list;
-    uint8_t* lmask;
-    uint8_t* fmask;
-    uint32_t G;
-    __device__ void run(uint32_t vb) const { k_ext_scatter_run(F, dist, total, cap, K2, poff, cursor, list, lmask, fmask, xcd_of(vb, G), vb); }
-};
-
-// ---------------------------------------------------------------------------
-// 3. Layer L: each listed face takes the mean of its neighbours in the
-// previous layer (lower-neighbour mask from the sort); only those are loaded,
-// all at once, and no distance is read.
-//
-// The mean of face i (component-local) over the neighbours flagged in m, in
-// the reference's order (-x, +x, -y, +y, -z, +z) with one divide; the
-// conditional sums as selects (an unused neighbour leaves the sum untouched,
-// a -0.0 included).
-// The flagged neighbours' values (0 for the others, never summed): only the
-// flagged ones are loaded.
-__device__ __forceinline__ void layer_loads(const float* f, uint32_t i, uint32_t m, uint32_t ex, uint32_t sz,
-                                            float (&fv)[6]) {
-    const uint32_t j[6] = {(m & 1u) ? i - 1 : i, (m & 2u) ? i + 1 : i, (m & 4u) ? i - ex : i,
-                           (m & 8u) ? i + ex : i, (m & 16u) ? i - sz : i, (m & 32u) ? i + sz : i};
-#pragma unroll
-    for (int q = 0; q < 6; ++q) fv[q] = ((m >> q) & 1u) ? f[j[q]] : 0.0f;
-}
-
-// Every loaded value in a register here, before any is used: without this
-// the compiler moves the first sum (0 + the first value) into that load's
-// branch, whose wait then holds back the other loads by a memory round trip.
-template <int N>
-__device__ __forceinline__ void loads_done(float (&v)[N]) {
-#pragma unroll
-    for (int q = 0; q < N; ++q) asm volatile("" : "+v"(v[q]));
-}
-
-__device__ __forceinline__ float layer_sum(uint32_t m, const float (&fv)[6]) {
-    float acc = 0.0f, cnt = 0.0f;
-#pragma unroll
-    for (int q = 0; q < 6; ++q) {
-        const bool use = (m >> q) & 1u;
-        acc = use ? acc + fv[q] : acc;
-        cnt = use ? cnt + 1.0f : cnt;
-    }
-    if (cnt != 0.0f) acc /= cnt;
-    return acc;
-}
-
-__device__ __forceinline__ float layer_mean(const float* f, uint32_t i, uint32_t m, uint32_t ex, uint32_t sz) {
-    float fv[6];
-    layer_loads(f, i, m, ex, sz, fv);
-    loads_done(fv);
-    return layer_sum(m, fv);
-}
-
-__global__ void __launch_bounds__(kBlock) k_ext_layer(Faces F, const uint32_t* __restrict__ list,
-                                                      const uint8_t* __restrict__ lmask, uint32_t begin,
-                                                      uint32_t count) {
-    const uint32_t t = blockIdx.x * kBlock + threadIdx.x;
-    if (t >= count) return;
-    const uint32_t gi = list[begin + t];
-    const uint32_t m = lmask[begin + t];
-    const int c = comp_of(F.off, gi);
-    const uint32_t i = gi - pick4(F.off, c);
-    const uint32_t ex = pick(F.ex, c), sz = ex * pick(F.ey, c);
-    float* f = pick(F.f, c);
-    f[i] = layer_mean(f, i, m, ex, sz);
-}
-
-// Layers L and L+1 in one launch (their list segments are adjacent: n0 faces
-// of layer L from `begin`, then n1 of layer L+1).  A layer-L+1 face needs the
-// new values of its layer-L neighbours; it recomputes each of them with the
-// same operations from the final layer-(L-1) values (the neighbour's own
-// lower mask is in the per-face mask array fmask) instead of reading what the
-// layer-L work-items write in this launch, so no work-item reads a value
-// written in the launch and the results are bitwise those of two launches.
-__global__ void __launch_bounds__(kBlock) k_ext_layer2(Faces F, const uint32_t* __restrict__ list,
-                                                       const uint8_t* __restrict__ lmask,
-                                                       const uint8_t* __restrict__ fmask, uint32_t begin,
-                                                       uint32_t n0, uint32_t n1) {
-    const uint32_t t = blockIdx.x * kBlock + threadIdx.x;
-    if (t >= n0 + n1) return;
-    const uint32_t gi = list[begin + t];
-    const uint32_t m = lmask[begin + t];
-    const int c = comp_of(F.off, gi);
-    const uint32_t o = pick4(F.off, c);
-    const uint32_t i = gi - o;
-    const uint32_t ex = pick(F.ex, c), sz = ex * pick(F.ey, c);
-    float* f = pick(F.f, c);
-    if (t < n0) {
-        f[i] = layer_mean(f, i, m, ex, sz);
-        return;
-    }
-    const uint32_t j[6] = {(m & 1u) ? i - 1 : i, (m & 2u) ? i + 1 : i, (m & 4u) ? i - ex : i,
-                           (m & 8u) ? i + ex : i, (m & 16u) ? i - sz : i, (m & 32u) ? i + sz : i};
-    uint32_t mn[6];
-#pragma unroll
-    for (int q = 0; q < 6; ++q) mn[q] = ((m >> q) & 1u) ? uint32_t(fmask[o + j[q]]) : 0u;
-    // the layer-L neighbours' means: all their loads, then the sums
-    float nv[6][6];
-#pragma unroll
-    for (int q = 0; q < 6; ++q) layer_loads(f, j[q], mn[q], ex, sz, nv[q]);
-#pragma unroll
-    for (int q = 0; q < 6; ++q) loads_done(nv[q]);
-    float fv[6];
-#pragma unroll
-    for (int q = 0; q < 6; ++q) fv[q] = layer_sum(mn[q], nv[q]);
-    float acc = 0.0f, cnt = 0.0f;
-#pragma unroll
-    for (int q = 0; q < 6; ++q) {
-        const bool use = (m >> q) & 1u;
-        acc = use ? acc + fv[q] : acc;
-        cnt = use ? cnt + 1.0f : cnt;
-    }
-    if (cnt != 0.0f) acc /= cnt;
-    f[i] = acc;
-}
-
-// Layers first..last in one work-group: layer by layer, a barrier between
-// layers ordering each layer's stores before the next layer's loads (the
-// work-group's work-items share one CU), kTailCpt entries per work-item per
-// round.  A round is latency-bound (list entry, then the neighbours, then
-// the store), so every load of a round is issued before any is used: the
-// six neighbours are loaded unconditionally (an unflagged one at the face's
-// own index) and only the flagged ones are summed.  For the tail of small
-// layers, where a launch per layer costs more than the layer's work, and
-// for small scenes' whole extrapolation.
-constexpr int kTailThreads = 1024;
-constexpr int kTailCpt = 8;
-
-__device__ __forceinline__ void k_ext_tail_run(Faces F, const uint32_t* __restrict__ list,
-                                               const uint8_t* __restrict__ lmask, const uint32_t* __restrict__ offs,
-                                               int32_t first, int32_t last, const uint32_t* __restrict__ last_dev,
-                                               uint32_t blk, uint32_t slot) {
-    (void)blk;
-    (void)slot;
-    if (last_dev) last = int32_t(*last_dev);
-    for (int32_t L = first; L <= last; ++L) {
-        const uint32_t b = offs[L], e = offs[L + 1];
-        for (uint32_t r0 = b; r0 < e; r0 += uint32_t(kTailThreads * kTailCpt)) {
-            uint32_t gi[kTailCpt], m[kTailCpt];
-#pragma unroll
-            for (int k = 0; k < kTailCpt; ++k) {
-                const uint32_t t = r0 + uint32_t(k * kTailThreads) + threadIdx.x;
-                const uint32_t tc = t < e ? t : e - 1;
-                gi[k] = list[tc];
-                m[k] = t < e ? uint32_t(lmask[tc]) : 0u;
-            }
-            float fv[kTailCpt][6];
-#pragma unroll
-            for (int k = 0; k < kTailCpt; ++k) {
-                const int c = comp_of(F.off, gi[k]);
-                const uint32_t i = gi[k] - pick4(F.off, c);
-                const uint32_t ex = pick(F.ex, c), sz = ex * pick(F.ey, c);
-                const float* f = pick(F.f, c);
-                const uint32_t mk = m[k];
-                const uint32_t j[6] = {(mk & 1u) ? i - 1 : i, (mk & 2u) ? i + 1 : i, (mk & 4u) ? i - ex : i,
-                                       (mk & 8u) ? i + ex : i, (mk & 16u) ? i - sz : i, (mk & 32u) ? i + sz : i};
-#pragma unroll
-                for (int q = 0; q < 6; ++q) fv[k][q] = f[j[q]];
-            }
-#pragma unroll
-            for (int k = 0; k < kTailCpt; ++k) {
-                const uint32_t t = r0 + uint32_t(k * kTailThreads) + threadIdx.x;
-                float acc = 0.0f, cnt = 0.0f;
-#pragma unroll
-                for (int q = 0; q < 6; ++q) {
-                    const bool use = (m[k] >> q) & 1u;
-                    acc = use ? acc + fv[k][q] : acc;
-                    cnt = use ? cnt + 1.0f : cnt;
-                }
-                if (cnt != 0.0f) acc /= cnt;
-                if (t < e) {
-                    const int c = comp_of(F.off, gi[k]);
-                    pick(F.f, c)[gi[k] - pick4(F.off, c)] = acc;
-                }
-            }
-        }
-        __syncthreads();
-    }
-}
-
-__global__ void __launch_bounds__(kTailThreads) k_ext_tail(Faces F, const uint32_t* __restrict__ list,
-                                                           const uint8_t* __restrict__ lmask,
-                                                           const uint32_t* __restrict__ offs, int32_t first,
-                                                           int32_t last, const uint32_t* __restrict__ last_dev) {
-    k_ext_tail_run(F, list, lmask, offs, first, last, last_dev, xcd_block(), blockIdx.x);
-}
-
-struct MExtTail {
-    static constexpr int kThreads = kTailThreads;
-    Faces F;
-    const uint32_t* list;
-    const uint8_t* lmask;
-    const uint32_t* offs;
-    int32_t first;
-    int32_t last;
-    const uint32_t* last_dev;
-    uint32_t G;
-    __device__ void run(uint32_t vb) const { k_ext_tail_run(F, list, lmask, offs, first, last, last_dev, xcd_of(vb, G), vb); }
-};
 
 // ===========================================================================
 // Fields the hybrid coupling reads (GridFluidSolver.cpp:571-613) on the
@@ -1201,8 +1125,41 @@ static uint32_t line_seg_grid(const Faces& F, int axis) {
     return (n + kXcds - 1) / kXcds * kXcds;
 }
 
+uint32_t ext_bricks(const GridDev& g) {
+    const Faces F = faces_of(g, nullptr, nullptr, nullptr);
+    return (brick_base(F, 3) + 7) / 8 * 8;
+}
+
+// Passes that set every face within `far` layers: a path of `far` faces
+// crosses at most bricks - 1 sides along an axis, and at most one more than
+// the brick edges it spans.
+uint32_t ext_passes(const GridDev& g, uint32_t far) {
+    const Faces F = faces_of(g, nullptr, nullptr, nullptr);
+    uint32_t most = 0;
+    for (int c = 0; c < 3; ++c) {
+        const uint32_t nb[3] = {brick_nx(F.ex[c]), brick_ny(F.ey[c]), brick_nz(F.ez[c])};
+        const uint32_t edge[3] = {kBrickX, kBrickY, kBrickZ};
+        uint32_t sides = 0, axes = 0, shortest = kBrickX;
+        for (int a = 0; a < 3; ++a) {
+            sides += nb[a] - 1;
+            if (nb[a] > 1) {
+                ++axes;
+                shortest = std::min(shortest, edge[a]);
+            }
+        }
+        most = std::max(most, std::min(sides, far / shortest + axes));
+    }
+    return far ? 1 + most : 0;
+}
+
+hipError_t launch_ext_zero(hipStream_t s, void* p, size_t words) {
+    return launch_dims(k_ext_zero, "k_ext_zero", dim3(uint32_t((words + kBlock - 1) / kBlock)), dim3(kBlock), 0u, s,
+                       static_cast<uint32_t*>(p), uint32_t(words));
+}
+
 hipError_t launch_ext_distance(hipStream_t s, const GridDev& g, const float* u, const float* v, const float* w,
-                               uint16_t* dist) {
+                               uint16_t* dist, uint16_t* mark, uint32_t* far) {
+    const ExtSeed seed{mark, far};
     const Faces F = faces_of(g, const_cast<float*>(u), const_cast<float*>(v), const_cast<float*>(w));
     // rows: held in registers when they fit 16 chunks of 64 faces
     const uint32_t exm = F.ex[0];   // the x-faces have the longest rows
@@ -1224,10 +1181,10 @@ hipError_t launch_ext_distance(hipStream_t s, const GridDev& g, const float* u, 
         if (sc >= 0) {
             const dim3 gr(line_seg_grid(F, axis)), bl(64 * kLineShortWaves);
             switch ((axis - 1) * 2 + sc) {
-                case 0: (void)launch_dims(k_ext_lines_seg<1, kLineShortSizes[0], kLineShortWaves>, "k_ext_lines_seg", gr, bl, 0, s, F, dist); break;
-                case 1: (void)launch_dims(k_ext_lines_seg<1, kLineShortSizes[1], kLineShortWaves>, "k_ext_lines_seg", gr, bl, 0, s, F, dist); break;
-                case 2: (void)launch_dims(k_ext_lines_seg<2, kLineShortSizes[0], kLineShortWaves>, "k_ext_lines_seg", gr, bl, 0, s, F, dist); break;
-                default: (void)launch_dims(k_ext_lines_seg<2, kLineShortSizes[1], kLineShortWaves>, "k_ext_lines_seg", gr, bl, 0, s, F, dist); break;
+                case 0: (void)launch_dims(k_ext_lines_seg<1, kLineShortSizes[0], kLineShortWaves>, "k_ext_lines_seg", gr, bl, 0, s, F, dist, seed); break;
+                case 1: (void)launch_dims(k_ext_lines_seg<1, kLineShortSizes[1], kLineShortWaves>, "k_ext_lines_seg", gr, bl, 0, s, F, dist, seed); break;
+                case 2: (void)launch_dims(k_ext_lines_seg<2, kLineShortSizes[0], kLineShortWaves>, "k_ext_lines_seg", gr, bl, 0, s, F, dist, seed); break;
+                default: (void)launch_dims(k_ext_lines_seg<2, kLineShortSizes[1], kLineShortWaves>, "k_ext_lines_seg", gr, bl, 0, s, F, dist, seed); break;
             }
             const hipError_t e1 = hipGetLastError();
             if (e1 != hipSuccess) return e1;
@@ -1236,19 +1193,19 @@ hipError_t launch_ext_distance(hipStream_t s, const GridDev& g, const float* u, 
         const int cls = line_seg_class(F, axis);
         if (cls < 0) {
             const uint32_t n = axis == 1 ? F.ylines[3] : F.zlines[3];
-            if (axis == 1) (void)launch_dims(k_ext_lines<1>, "k_ext_lines", dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, s, F, dist);
-            else (void)launch_dims(k_ext_lines<2>, "k_ext_lines", dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, s, F, dist);
+            if (axis == 1) (void)launch_dims(k_ext_lines<1>, "k_ext_lines", dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, s, F, dist, seed);
+            else (void)launch_dims(k_ext_lines<2>, "k_ext_lines", dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, s, F, dist, seed);
         } else {
             const dim3 gr(line_seg_grid(F, axis)), bl(kLineSegThreads);
             switch ((axis - 1) * 4 + cls) {
-                case 0: (void)launch_dims(k_ext_lines_seg<1, kLineSegSizes[0]>, "k_ext_lines_seg", gr, bl, 0, s, F, dist); break;
-                case 1: (void)launch_dims(k_ext_lines_seg<1, kLineSegSizes[1]>, "k_ext_lines_seg", gr, bl, 0, s, F, dist); break;
-                case 2: (void)launch_dims(k_ext_lines_seg<1, kLineSegSizes[2]>, "k_ext_lines_seg", gr, bl, 0, s, F, dist); break;
-                case 3: (void)launch_dims(k_ext_lines_seg<1, kLineSegSizes[3]>, "k_ext_lines_seg", gr, bl, 0, s, F, dist); break;
-                case 4: (void)launch_dims(k_ext_lines_seg<2, kLineSegSizes[0]>, "k_ext_lines_seg", gr, bl, 0, s, F, dist); break;
-                case 5: (void)launch_dims(k_ext_lines_seg<2, kLineSegSizes[1]>, "k_ext_lines_seg", gr, bl, 0, s, F, dist); break;
-                case 6: (void)launch_dims(k_ext_lines_seg<2, kLineSegSizes[2]>, "k_ext_lines_seg", gr, bl, 0, s, F, dist); break;
-                default: (void)launch_dims(k_ext_lines_seg<2, kLineSegSizes[3]>, "k_ext_lines_seg", gr, bl, 0, s, F, dist); break;
+                case 0: (void)launch_dims(k_ext_lines_seg<1, kLineSegSizes[0]>, "k_ext_lines_seg", gr, bl, 0, s, F, dist, seed); break;
+                case 1: (void)launch_dims(k_ext_lines_seg<1, kLineSegSizes[1]>, "k_ext_lines_seg", gr, bl, 0, s, F, dist, seed); break;
+                case 2: (void)launch_dims(k_ext_lines_seg<1, kLineSegSizes[2]>, "k_ext_lines_seg", gr, bl, 0, s, F, dist, seed); break;
+                case 3: (void)launch_dims(k_ext_lines_seg<1, kLineSegSizes[3]>, "k_ext_lines_seg", gr, bl, 0, s, F, dist, seed); break;
+                case 4: (void)launch_dims(k_ext_lines_seg<2, kLineSegSizes[0]>, "k_ext_lines_seg", gr, bl, 0, s, F, dist, seed); break;
+                case 5: (void)launch_dims(k_ext_lines_seg<2, kLineSegSizes[1]>, "k_ext_lines_seg", gr, bl, 0, s, F, dist, seed); break;
+                case 6: (void)launch_dims(k_ext_lines_seg<2, kLineSegSizes[2]>, "k_ext_lines_seg", gr, bl, 0, s, F, dist, seed); break;
+                default: (void)launch_dims(k_ext_lines_seg<2, kLineSegSizes[3]>, "k_ext_lines_seg", gr, bl, 0, s, F, dist, seed); break;
             }
         }
         const hipError_t e2 = hipGetLastError();
@@ -1257,66 +1214,20 @@ hipError_t launch_ext_distance(hipStream_t s, const GridDev& g, const float* u, 
     return hipSuccess;
 }
 
-size_t ext_counts_size(int32_t K) { return (3 * size_t(kCopies) + 1) * (size_t(K) + 2) + 1; }
+// Work-groups of a pass: two fit each of 256 CUs; each takes every 512th brick.
+constexpr uint32_t kBrickGroups = 512;
 
-hipError_t launch_ext_sort(hipStream_t s, const GridDev& g, const uint16_t* dist, int32_t cap, int32_t K,
-                           uint32_t* counts, uint32_t* list, uint8_t* lmask, uint8_t* fmask, const uint32_t** offs,
-                           const uint32_t** maxd) {
-    const Faces F = faces_of(g, nullptr, nullptr, nullptr);
-    const uint32_t total = F.off[3];
-    const uint32_t K2 = uint32_t(K) + 2;
-    const SortBufs B = sort_bufs(counts, K);
-    *offs = B.offs;
-    *maxd = B.maxd;
-    const uint32_t nh = kCopies * K2;
-    (void)launch_dims(k_ext_zero, "k_ext_zero", dim3((nh + kBlock - 1) / kBlock), dim3(kBlock), 0, s, B.hist, nh);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    size_t G = (size_t(total) + size_t(kBlock) * kSortCpt - 1) / (size_t(kBlock) * kSortCpt);
-    G = (G + kXcds - 1) / kXcds * kXcds;
-    probe_next_bytes(2.0 * double(total));
-    (void)launch_dims(k_ext_count, "k_ext_count", dim3(uint32_t(G)), dim3(kBlock), 0, s, dist, total, cap, B.hist, K2);
-    e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    (void)launch_dims(k_ext_scan, "k_ext_scan", dim3(1), dim3(1024), 0, s, B.hist, cap, K2, B.offs, B.poff, B.cursor, B.maxd);
-    e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    probe_next_bytes(4.0 * double(total));   // distance 2 read, fmask 1 and (listed faces) list 4 + lmask 1 written
-    (void)launch_dims(k_ext_scatter, "k_ext_scatter", dim3(uint32_t(G)), dim3(kBlock), 0, s, F, dist, total, cap, K2, B.poff,
-                       B.cursor, list, lmask, fmask);
-    return hipGetLastError();
-}
-
-hipError_t launch_ext_layer(hipStream_t s, const GridDev& g, float* u, float* v, float* w, const uint32_t* list,
-                            const uint8_t* lmask, uint32_t begin, uint32_t count) {
-    if (count == 0) return hipSuccess;
-    const Faces F = faces_of(g, u, v, w);
-    return launch_dims(k_ext_layer, "k_ext_layer", dim3((count + kBlock - 1) / kBlock), dim3(kBlock), 0u, s, F, list, lmask, begin,
-                       count);
-}
-
-hipError_t launch_ext_tail(hipStream_t s, const GridDev& g, float* u, float* v, float* w, const uint32_t* list,
-                           const uint8_t* lmask, const uint32_t* offs, int32_t first, int32_t last,
-                           const uint32_t* last_dev) {
-    if (!last_dev && last < first) return hipSuccess;
-    const Faces F = faces_of(g, u, v, w);
-    return launch_dims(k_ext_tail, "k_ext_tail", dim3(1), dim3(kTailThreads), 0u, s, F, list, lmask, offs, first, last,
-                       last_dev);
-}
-
-hipError_t launch_ext_layer2(hipStream_t s, const GridDev& g, float* u, float* v, float* w, const uint32_t* list,
-                             const uint8_t* lmask, const uint8_t* fmask, uint32_t begin, uint32_t n0, uint32_t n1) {
-    if (n0 + n1 == 0) return hipSuccess;
-    const Faces F = faces_of(g, u, v, w);
-    return launch_dims(k_ext_layer2, "k_ext_layer2", dim3((n0 + n1 + kBlock - 1) / kBlock), dim3(kBlock), 0u, s, F, list, lmask,
-                       fmask, begin, n0, n1);
+hipError_t launch_ext_bricks(hipStream_t s, const GridDev& g, float* u, float* v, float* w, const uint16_t* dist,
+                             int32_t cap, uint16_t* stamps, uint32_t pass) {
+    const uint32_t total = ext_bricks(g);
+    const BrickArgs A{faces_of(g, u, v, w), dist, cap, 0u};
+    return launch_dims(k_ext_bricks, "k_ext_bricks", dim3(std::min(total, kBrickGroups)), dim3(kBrickThreads), 0u, s, A,
+                       stamps, total, pass);
 }
 
 // ===========================================================================
-// Multi-scene records of the distance transform, the counting sort and the
-// one-work-group layers (launch_ext_distance, launch_ext_sort and
-// launch_ext_tail with the last layer read on the device): the same
-// arguments and grids.
+// Multi-scene records of the distance transform (launch_ext_distance): the
+// same arguments and grids.
 template <class A>
 static void push_rec_e(std::vector<MRec>& out, int32_t kind, const A& a, uint32_t blocks) {
     static_assert(sizeof(A) <= kMRecBytes, "argument struct fits a record");
@@ -1328,9 +1239,9 @@ static void push_rec_e(std::vector<MRec>& out, int32_t kind, const A& a, uint32_
     out.push_back(r);
 }
 
-void rec_ext_device(std::vector<MRec>& out, const GridDev& g, float* u, float* v, float* w, uint16_t* dist,
-                    int32_t cap, int32_t K, uint32_t* counts, uint32_t* list, uint8_t* lmask, uint8_t* fmask,
-                    const uint32_t** maxd, bool with_layers) {
+void rec_ext_distance(std::vector<MRec>& out, const GridDev& g, float* u, float* v, float* w, uint16_t* dist,
+                      uint16_t* mark, uint32_t* far) {
+    const ExtSeed seed{mark, far};
     const Faces F = faces_of(g, u, v, w);
     const uint32_t exm = F.ex[0];
     const uint32_t rg = (F.rows[3] + 3) / 4;
@@ -1347,141 +1258,47 @@ void rec_ext_device(std::vector<MRec>& out, const GridDev& g, float* u, float* v
             const uint32_t gl = line_seg_grid(F, axis);
             const int32_t kind = kMkExtLinesShort + (axis - 1) * 2 + sc;
             switch ((axis - 1) * 2 + sc) {
-                case 0: push_rec_e(out, kind, MExtLinesSeg<1, kLineShortSizes[0], kLineShortWaves>{F, dist, gl}, gl); break;
-                case 1: push_rec_e(out, kind, MExtLinesSeg<1, kLineShortSizes[1], kLineShortWaves>{F, dist, gl}, gl); break;
-                case 2: push_rec_e(out, kind, MExtLinesSeg<2, kLineShortSizes[0], kLineShortWaves>{F, dist, gl}, gl); break;
-                default: push_rec_e(out, kind, MExtLinesSeg<2, kLineShortSizes[1], kLineShortWaves>{F, dist, gl}, gl); break;
+                case 0: push_rec_e(out, kind, MExtLinesSeg<1, kLineShortSizes[0], kLineShortWaves>{F, dist, seed, gl}, gl); break;
+                case 1: push_rec_e(out, kind, MExtLinesSeg<1, kLineShortSizes[1], kLineShortWaves>{F, dist, seed, gl}, gl); break;
+                case 2: push_rec_e(out, kind, MExtLinesSeg<2, kLineShortSizes[0], kLineShortWaves>{F, dist, seed, gl}, gl); break;
+                default: push_rec_e(out, kind, MExtLinesSeg<2, kLineShortSizes[1], kLineShortWaves>{F, dist, seed, gl}, gl); break;
             }
             continue;
         }
         const int cls = line_seg_class(F, axis);
         if (cls < 0) {
             const uint32_t gl = ((axis == 1 ? F.ylines[3] : F.zlines[3]) + kBlock - 1) / kBlock;
-            if (axis == 1) push_rec_e(out, kMkExtLines1, MExtLines<1>{F, dist, gl}, gl);
-            else push_rec_e(out, kMkExtLines2, MExtLines<2>{F, dist, gl}, gl);
+            if (axis == 1) push_rec_e(out, kMkExtLines1, MExtLines<1>{F, dist, seed, gl}, gl);
+            else push_rec_e(out, kMkExtLines2, MExtLines<2>{F, dist, seed, gl}, gl);
             continue;
         }
         const uint32_t gl = line_seg_grid(F, axis);
         const int32_t kind = kMkExtLinesSeg + (axis - 1) * 4 + cls;
         switch ((axis - 1) * 4 + cls) {
-            case 0: push_rec_e(out, kind, MExtLinesSeg<1, kLineSegSizes[0]>{F, dist, gl}, gl); break;
-            case 1: push_rec_e(out, kind, MExtLinesSeg<1, kLineSegSizes[1]>{F, dist, gl}, gl); break;
-            case 2: push_rec_e(out, kind, MExtLinesSeg<1, kLineSegSizes[2]>{F, dist, gl}, gl); break;
-            case 3: push_rec_e(out, kind, MExtLinesSeg<1, kLineSegSizes[3]>{F, dist, gl}, gl); break;
-            case 4: push_rec_e(out, kind, MExtLinesSeg<2, kLineSegSizes[0]>{F, dist, gl}, gl); break;
-            case 5: push_rec_e(out, kind, MExtLinesSeg<2, kLineSegSizes[1]>{F, dist, gl}, gl); break;
-            case 6: push_rec_e(out, kind, MExtLinesSeg<2, kLineSegSizes[2]>{F, dist, gl}, gl); break;
-            default: push_rec_e(out, kind, MExtLinesSeg<2, kLineSegSizes[3]>{F, dist, gl}, gl); break;
+            case 0: push_rec_e(out, kind, MExtLinesSeg<1, kLineSegSizes[0]>{F, dist, seed, gl}, gl); break;
+            case 1: push_rec_e(out, kind, MExtLinesSeg<1, kLineSegSizes[1]>{F, dist, seed, gl}, gl); break;
+            case 2: push_rec_e(out, kind, MExtLinesSeg<1, kLineSegSizes[2]>{F, dist, seed, gl}, gl); break;
+            case 3: push_rec_e(out, kind, MExtLinesSeg<1, kLineSegSizes[3]>{F, dist, seed, gl}, gl); break;
+            case 4: push_rec_e(out, kind, MExtLinesSeg<2, kLineSegSizes[0]>{F, dist, seed, gl}, gl); break;
+            case 5: push_rec_e(out, kind, MExtLinesSeg<2, kLineSegSizes[1]>{F, dist, seed, gl}, gl); break;
+            case 6: push_rec_e(out, kind, MExtLinesSeg<2, kLineSegSizes[2]>{F, dist, seed, gl}, gl); break;
+            default: push_rec_e(out, kind, MExtLinesSeg<2, kLineSegSizes[3]>{F, dist, seed, gl}, gl); break;
         }
     }
-    const uint32_t total = F.off[3];
-    const uint32_t K2 = uint32_t(K) + 2;
-    const SortBufs B = sort_bufs(counts, K);
-    *maxd = B.maxd;
-    const uint32_t nh = kCopies * K2;
-    const uint32_t gz = (nh + kBlock - 1) / kBlock;
-    push_rec_e(out, kMkExtZero, MExtZero{B.hist, nh, gz}, gz);
-    size_t G = (size_t(total) + size_t(kBlock) * kSortCpt - 1) / (size_t(kBlock) * kSortCpt);
-    G = (G + kXcds - 1) / kXcds * kXcds;
-    push_rec_e(out, kMkExtCount, MExtCount{dist, total, cap, B.hist, K2, uint32_t(G)}, uint32_t(G));
-    push_rec_e(out, kMkExtScan, MExtScan{B.hist, cap, K2, B.offs, B.poff, B.cursor, B.maxd, 1u}, 1u);
-    push_rec_e(out, kMkExtScatter,
-               MExtScatter{F, dist, total, cap, K2, B.poff, B.cursor, list, lmask, fmask, uint32_t(G)},
-               uint32_t(G));
-    if (with_layers) push_rec_e(out, kMkExtTail, MExtTail{F, list, lmask, B.offs, 1, 0, B.maxd, 1u}, 1u);
 }
 
-// Layer L of many scenes in one launch: block b of a scene takes entries
-// offs[L] + b * kBlock * kLayerCpt ... of its list (the bounds read on the
-// device), each the mean of its flagged previous-layer neighbours (as
-// k_ext_layer).  map entries: (scene << kMapShift) | block.
-constexpr int kLayerCpt = 4;
+size_t brick_arg_bytes() { return sizeof(BrickArgs); }
 
-struct MLayer {
-    Faces F;
-    const uint32_t* list;
-    const uint8_t* lmask;
-    const uint32_t* offs;
-};
-
-__global__ void __launch_bounds__(kBlock) k_multi_layer(const MLayer* __restrict__ tab,
-                                                        const uint32_t* __restrict__ map, int32_t L) {
-    const uint32_t e = map[blockIdx.x];
-    const MLayer a = tab[e >> kMapShift];
-    const uint32_t b = a.offs[L], end = a.offs[L + 1];
-    const uint32_t base = b + (e & kMapLocal) * uint32_t(kBlock * kLayerCpt) + threadIdx.x;
-    uint32_t gi[kLayerCpt], m[kLayerCpt];
-#pragma unroll
-    for (int k = 0; k < kLayerCpt; ++k) {
-        const uint32_t t = base + uint32_t(k * kBlock);
-        const uint32_t tc = t < end ? t : end - 1;
-        gi[k] = a.list[tc];
-        m[k] = t < end ? uint32_t(a.lmask[tc]) : 0u;
-    }
-    // every entry's loads, then the sums and stores
-    float fv[kLayerCpt][6];
-#pragma unroll
-    for (int k = 0; k < kLayerCpt; ++k) {
-        const int c = comp_of(a.F.off, gi[k]);
-        const uint32_t i = gi[k] - pick4(a.F.off, c);
-        const uint32_t ex = pick(a.F.ex, c), sz = ex * pick(a.F.ey, c);
-        layer_loads(pick(a.F.f, c), i, m[k], ex, sz, fv[k]);   // m = 0 past the end: nothing loaded
-    }
-#pragma unroll
-    for (int k = 0; k < kLayerCpt; ++k) loads_done(fv[k]);
-#pragma unroll
-    for (int k = 0; k < kLayerCpt; ++k) {
-        const uint32_t t = base + uint32_t(k * kBlock);
-        if (t >= end) continue;
-        const int c = comp_of(a.F.off, gi[k]);
-        pick(a.F.f, c)[gi[k] - pick4(a.F.off, c)] = layer_sum(m[k], fv[k]);
-    }
+void brick_args(unsigned char* dst, const GridDev& g, float* u, float* v, float* w, const uint16_t* dist, int32_t cap,
+                uint32_t first) {
+    const BrickArgs a{faces_of(g, u, v, w), dist, cap, first};
+    std::memcpy(dst, &a, sizeof(BrickArgs));
 }
 
-uint32_t layer_entries_per_block() { return uint32_t(kBlock * kLayerCpt); }
-
-size_t layer_arg_bytes() { return sizeof(MLayer); }
-
-void layer_args(unsigned char* dst, const GridDev& g, float* u, float* v, float* w, const uint32_t* list,
-                const uint8_t* lmask, uint32_t* counts, int32_t K) {
-    const MLayer a{faces_of(g, u, v, w), list, lmask, sort_bufs(counts, K).offs};
-    std::memcpy(dst, &a, sizeof(MLayer));
-}
-
-hipError_t launch_multi_layer(hipStream_t s, const void* tab, const uint32_t* map, uint32_t nblocks, int32_t L) {
-    if (nblocks == 0) return hipSuccess;
-    return launch_dims(k_multi_layer, "k_multi_layer", dim3(nblocks), dim3(kBlock), 0u, s,
-                       static_cast<const MLayer*>(tab), map, L);
-}
-
-// Each scene's layer offsets 0..cap+1 and its largest layer, packed for one
-// copy to the host (one block per scene).
-struct MCopyOffs {
-    static constexpr int kThreads = kBlock;
-    const uint32_t* offs;
-    const uint32_t* maxd;
-    uint32_t n;
-    uint32_t* dst;
-    __device__ void run(uint32_t) const {
-        for (uint32_t i = threadIdx.x; i < n; i += kBlock) dst[i] = offs[i];
-        if (threadIdx.x == 0) dst[n] = *maxd;
-    }
-};
-
-void rec_copy_offs(std::vector<MRec>& out, uint32_t* counts, int32_t K, int32_t cap, uint32_t* dst) {
-    const SortBufs B = sort_bufs(counts, K);
-    push_rec_e(out, kMkCopyOffs, MCopyOffs{B.offs, B.maxd, uint32_t(cap) + 2u, dst}, 1u);
-}
-
-// The sort's layers from `first` to the largest present in one work-group
-// (the layers a scene's own launches do not take).
-size_t tail_arg_bytes() { return sizeof(MExtTail); }
-
-void tail_args(unsigned char* dst, const GridDev& g, float* u, float* v, float* w, const uint32_t* list,
-               const uint8_t* lmask, uint32_t* counts, int32_t K, int32_t first, int32_t last) {
-    const SortBufs B = sort_bufs(counts, K);
-    const MExtTail a{faces_of(g, u, v, w), list, lmask, B.offs, first, last, nullptr, 1u};
-    std::memcpy(dst, &a, sizeof(MExtTail));
+hipError_t launch_multi_bricks(hipStream_t s, const void* tab, const uint16_t* scene_of, uint16_t* stamps,
+                               uint32_t total, uint32_t pass) {
+    return launch_dims(k_multi_bricks, "k_multi_bricks", dim3(std::min(total, kBrickGroups)), dim3(kBrickThreads), 0u, s,
+                       static_cast<const BrickArgs*>(tab), scene_of, stamps, total, pass);
 }
 
 template <class A>
@@ -1515,12 +1332,6 @@ hipError_t launch_multi_ext(hipStream_t s, int32_t kind, const void* tab, const 
         case kMkExtLinesSeg + 5: return launch_me<MExtLinesSeg<2, kLineSegSizes[1]>>(s, "k_multi_ext_lines_seg", tab, map, nblocks, active);
         case kMkExtLinesSeg + 6: return launch_me<MExtLinesSeg<2, kLineSegSizes[2]>>(s, "k_multi_ext_lines_seg", tab, map, nblocks, active);
         case kMkExtLinesSeg + 7: return launch_me<MExtLinesSeg<2, kLineSegSizes[3]>>(s, "k_multi_ext_lines_seg", tab, map, nblocks, active);
-        case kMkExtZero: return launch_me<MExtZero>(s, "k_multi_ext_zero", tab, map, nblocks, active);
-        case kMkExtCount: return launch_me<MExtCount>(s, "k_multi_ext_count", tab, map, nblocks, active);
-        case kMkExtScan: return launch_me<MExtScan>(s, "k_multi_ext_scan", tab, map, nblocks, active);
-        case kMkExtScatter: return launch_me<MExtScatter>(s, "k_multi_ext_scatter", tab, map, nblocks, active);
-        case kMkExtTail: return launch_me<MExtTail>(s, "k_multi_ext_tail", tab, map, nblocks, active);
-        case kMkCopyOffs: return launch_me<MCopyOffs>(s, "k_multi_copy_offs", tab, map, nblocks, active);
         default: return hipErrorInvalidValue;
     }
 }
