@@ -1357,8 +1357,8 @@ struct MRestrictTile {
 // The V-cycle on the smallest levels in one work-group, iterates in LDS.
 // Level 0 of the argument list takes its right-hand side from global memory
 // (written by the restriction of the level above) and writes its result back
-// (read by the prolongation of the level above); deeper levels keep b, x and
-// the Jacobi partner in LDS.  The arithmetic is the multi-kernel cycle's.
+// (read by the prolongation of the level above); deeper levels keep b in LDS.
+// The arithmetic is the multi-kernel cycle's.
 constexpr int kCoarseThreads = 1024;
 constexpr int kCoarseMaxLevels = 8;
 
@@ -1376,141 +1376,180 @@ struct CoarseArgs {
     CoarseLevel lv[kCoarseMaxLevels];
 };
 
-__device__ __forceinline__ void lds_sweep(const CoarseLevel& L, const uint16_t* code, const float* aw,
-                                          const float* w, const float* b, const float* xi, float* xo, bool first) {
-    const uint32_t n = uint32_t(L.nx) * uint32_t(L.ny) * uint32_t(L.nz);
-    const Flat F{n, uint32_t(L.nx), uint32_t(L.nx) * uint32_t(L.ny)};
-    for (uint32_t c = threadIdx.x; c < n; c += kCoarseThreads) {
-        const uint16_t cd = code[c];
-        const float wd = wdiag(cd, w);
-        const float bc = b[c];
-        float out;
-        if (first) {
-            out = wd * bc;
-        } else {
-            uint32_t j[6];
-            nbrs(c, F, j);
-            float v[6];
+// One work-item's cells of a level, kCoarseThreads apart: what a sweep needs
+// of them stays in registers, so a sweep reads six values from LDS and writes
+// one.  A neighbour that is not coupled is read at the cell itself, where its
+// difference is +0, as the masked one is in arow.
+constexpr int kCoarseCpt = 8;   // levels of at most 8192 cells
+struct CoarseCells {
+    uint32_t nb[kCoarseCpt][6];   // LDS byte offsets of the neighbours' iterates
+    float b[kCoarseCpt], x[kCoarseCpt], wd[kCoarseCpt], aw[kCoarseCpt];
+};
+
+// f(k, c) for this work-item's cells c.
+template <class F>
+__device__ __forceinline__ void coarse_cells(uint32_t n, F&& f) {
 #pragma unroll
-            for (int m = 0; m < 6; ++m) v[m] = xi[j[m]];
-            const float vc = xi[c];
-            out = (cd & kCodeFluid) ? vc + wd * (bc - arow(cd, vc, v, L.sx, L.sy, L.sz, aw)) : 0.0f;
-        }
-        xo[c] = out;
+    for (int k = 0; k < kCoarseCpt; ++k) {
+        if (uint32_t(k) * kCoarseThreads >= n) break;   // the same for every work-item
+        const uint32_t c = uint32_t(k) * kCoarseThreads + threadIdx.x;
+        if (c < n) f(k, c);
     }
-    __syncthreads();
+}
+
+// x, y, z of cell c < 8192 (from the quotient at the cell's centre: exact).
+__device__ __forceinline__ void coarse_xyz(uint32_t c, const CoarseLevel& L, uint32_t& x, uint32_t& y, uint32_t& z) {
+    const uint32_t row = uint32_t((float(c) + 0.5f) * (1.0f / float(L.nx)));
+    x = c - row * uint32_t(L.nx);
+    z = uint32_t((float(row) + 0.5f) * (1.0f / float(L.ny)));
+    y = row - z * uint32_t(L.ny);
+}
+
+// A x of a cell (arow's operations in its order).
+__device__ __forceinline__ float coarse_row(const CoarseLevel& L, const CoarseCells& R, int k, const char* lds) {
+    float v[6];
+#pragma unroll
+    for (int m = 0; m < 6; ++m) v[m] = *reinterpret_cast<const float*>(lds + R.nb[k][m]);
+    const float vc = R.x[k];
+    const float ex = (vc - v[0]) + (vc - v[1]);
+    const float ey = (vc - v[2]) + (vc - v[3]);
+    const float ez = (vc - v[4]) + (vc - v[5]);
+    return R.aw[k] * vc + L.sx * ex + L.sy * ey + L.sz * ez;
 }
 
 // LDS layout (floats): per level the tables aw[64], w[64]; then per level the
-// codes (uint16, each level padded to an even count); then level 0: x, t;
-// deeper levels: b, x, t.
+// codes (uint16, each level padded to an even count); then level 0: iterate,
+// residual; deeper levels: right-hand side, iterate, residual.
+//
+// Bound by the length of its chain of sweeps (22 at 17^3): a sweep is a few
+// LDS reads, the row and two barriers.  17^3: 28 us when every sweep looked
+// its cells' codes, tables and clamped neighbours up again and a coarse cell
+// formed its eight children's residuals one after another; 20 us now.
 __device__ __forceinline__ void coarse_run(const CoarseArgs& A, const CgScalars* __restrict__ sc) {
     if (sc->done) return;
     extern __shared__ float lds[];
     // Offsets (floats from lds) of each level's codes, right-hand side,
-    // iterate and scratch iterate, in LDS rather than in per-work-item arrays
-    // (which a runtime level index would put in scratch memory); par bit l
-    // swaps level l's iterate and scratch iterate.
-    __shared__ uint32_t s_code[kCoarseMaxLevels], s_b[kCoarseMaxLevels], s_x[kCoarseMaxLevels],
-        s_t[kCoarseMaxLevels], s_n[kCoarseMaxLevels];
-    float* tab = lds;
+    // iterate and residual, in LDS rather than in per-work-item arrays (which
+    // a runtime level index would put in scratch memory).
+    __shared__ uint32_t s_code[kCoarseMaxLevels], s_b[kCoarseMaxLevels], s_x[kCoarseMaxLevels], s_r[kCoarseMaxLevels];
+    char* const bytes = reinterpret_cast<char*>(lds);
+    auto cells_of = [&](int l) { return uint32_t(A.lv[l].nx) * uint32_t(A.lv[l].ny) * uint32_t(A.lv[l].nz); };
     if (threadIdx.x == 0) {
         uint32_t q = 128u * uint32_t(A.nlev);
         for (int l = 0; l < A.nlev; ++l) {
-            s_n[l] = uint32_t(A.lv[l].nx) * uint32_t(A.lv[l].ny) * uint32_t(A.lv[l].nz);
             s_code[l] = q;
-            q += (s_n[l] + 1) / 2;
+            q += (cells_of(l) + 1) / 2;
         }
         for (int l = 0; l < A.nlev; ++l) {
+            const uint32_t n = cells_of(l);
             s_b[l] = q;
-            if (l > 0) q += s_n[l];
-            s_x[l] = q; q += s_n[l];
-            s_t[l] = q; q += s_n[l];
+            if (l > 0) q += n;
+            s_x[l] = q; q += n;
+            s_r[l] = q; q += n;
         }
     }
+    CoarseCells R;
+    coarse_cells(cells_of(0), [&](int k, uint32_t c) { R.b[k] = A.b0[c]; });
     __syncthreads();
-    uint32_t par = 0;
     auto codes = [&](int l) { return reinterpret_cast<uint16_t*>(lds + s_code[l]); };
-    auto bs = [&](int l) { return l == 0 ? A.b0 : static_cast<const float*>(lds + s_b[l]); };
-    auto xs = [&](int l) { return lds + (((par >> l) & 1u) ? s_t[l] : s_x[l]); };
-    auto ts = [&](int l) { return lds + (((par >> l) & 1u) ? s_x[l] : s_t[l]); };
-    auto ns = [&](int l) { return s_n[l]; };
-    // tables and codes of every level
     for (int l = 0; l < A.nlev; ++l) {
         if (threadIdx.x < 64) {
             const float d = mask_scale_sum(threadIdx.x, A.lv[l].sx, A.lv[l].sy, A.lv[l].sz);
-            tab[128 * l + threadIdx.x] = d;
-            tab[128 * l + 64 + threadIdx.x] = d != 0.0f ? A.omega / d : 0.0f;
+            lds[128 * l + threadIdx.x] = d;
+            lds[128 * l + 64 + threadIdx.x] = d != 0.0f ? A.omega / d : 0.0f;
         }
-        for (uint32_t c = threadIdx.x; c < ns(l); c += kCoarseThreads) codes(l)[c] = A.lv[l].code[c];
+        for (uint32_t c = threadIdx.x; c < cells_of(l); c += kCoarseThreads) codes(l)[c] = A.lv[l].code[c];
     }
     __syncthreads();
+    // the cells' weights and neighbours
+    auto load = [&](int l) {
+        const CoarseLevel& L = A.lv[l];
+        const float* aw = lds + 128 * l;
+        const uint16_t* code = codes(l);
+        const uint32_t x0 = 4u * s_x[l], sy = uint32_t(L.nx), sz = uint32_t(L.nx) * uint32_t(L.ny);
+        coarse_cells(cells_of(l), [&](int k, uint32_t c) {
+            const uint16_t cd = code[c];
+            R.aw[k] = aw[air_mask(cd)];
+            R.wd[k] = wdiag(cd, aw + 64);
+            const uint32_t j[6] = {c - 1, c + 1, c - sy, c + sy, c - sz, c + sz};
+#pragma unroll
+            for (int m = 0; m < 6; ++m) R.nb[k][m] = x0 + 4u * (((cd >> (kCplShift + m)) & 1) ? j[m] : c);
+        });
+    };
+    auto store = [&](int l) {
+        float* x = lds + s_x[l];
+        coarse_cells(cells_of(l), [&](int k, uint32_t c) { x[c] = R.x[k]; });
+        __syncthreads();
+    };
+    // Non-fluid cells (weight, air weight and right-hand side 0, no neighbour)
+    // keep their 0.
+    auto sweep = [&](int l) {
+        const CoarseLevel& L = A.lv[l];
+        coarse_cells(cells_of(l), [&](int k, uint32_t) { R.x[k] = R.x[k] + R.wd[k] * (R.b[k] - coarse_row(L, R, k, bytes)); });
+        __syncthreads();
+        store(l);
+    };
     // descent
     for (int l = 0; l < A.nlev; ++l) {
         const CoarseLevel& L = A.lv[l];
-        const float* aw = tab + 128 * l;
-        const float* w = aw + 64;
+        load(l);
+        coarse_cells(cells_of(l), [&](int k, uint32_t) { R.x[k] = R.wd[k] * R.b[k]; });
+        store(l);
         const int sweeps = l == A.nlev - 1 ? A.last_sweeps : A.nu;
-        lds_sweep(L, codes(l), aw, w, bs(l), xs(l), xs(l), true);
-        for (int k = 1; k < sweeps; ++k) {
-            lds_sweep(L, codes(l), aw, w, bs(l), xs(l), ts(l), false);
-            par ^= 1u << l;
-        }
+        for (int q = 1; q < sweeps; ++q) sweep(l);
         if (l == A.nlev - 1) break;
-        // restriction of the residual into level l+1
+        // the residual (0 on non-fluid cells), then its restriction: the next
+        // level's right-hand side, in registers and kept for the ascent
+        {
+            float* r = lds + s_r[l];
+            const uint16_t* code = codes(l);
+            coarse_cells(cells_of(l), [&](int k, uint32_t c) {
+                r[c] = (code[c] & kCodeFluid) ? R.b[k] - coarse_row(L, R, k, bytes) : 0.0f;
+            });
+        }
+        __syncthreads();
         const CoarseLevel& C = A.lv[l + 1];
-        const uint32_t nc = ns(l + 1);
         const int fx = L.nx > 1 ? 2 : 1, fy = L.ny > 1 ? 2 : 1, fz = L.nz > 1 ? 2 : 1;
         const float weight = 1.0f / float(fx * fy * fz);
-        const Flat FF{ns(l), uint32_t(L.nx), uint32_t(L.nx) * uint32_t(L.ny)};
-        float* bc = const_cast<float*>(bs(l + 1));
-        const float* xf = xs(l);
-        const float* bf = bs(l);
-        for (uint32_t c = threadIdx.x; c < nc; c += kCoarseThreads) {
-            const uint32_t X = c % uint32_t(C.nx), Y = (c / uint32_t(C.nx)) % uint32_t(C.ny),
-                           Z = c / (uint32_t(C.nx) * uint32_t(C.ny));
+        const float* r = lds + s_r[l];
+        float* bc = lds + s_b[l + 1];
+        const uint16_t* code = codes(l + 1);
+        coarse_cells(cells_of(l + 1), [&](int k, uint32_t c) {
+            uint32_t X, Y, Z;
+            coarse_xyz(c, C, X, Y, Z);
             float sum = 0.0f;
             for (int dz = 0; dz < fz; ++dz)
                 for (int dy = 0; dy < fy; ++dy)
                     for (int dx = 0; dx < fx; ++dx) {
                         const uint32_t x = X * fx + dx, y = Y * fy + dy, z = Z * fz + dz;
                         if (x >= uint32_t(L.nx) || y >= uint32_t(L.ny) || z >= uint32_t(L.nz)) continue;
-                        const uint32_t f = z * FF.sz + y * FF.sy + x;
-                        const uint16_t cd = codes(l)[f];
-                        if (!(cd & kCodeFluid)) continue;
-                        uint32_t j[6];
-                        nbrs(f, FF, j);
-                        float v[6];
-#pragma unroll
-                        for (int m = 0; m < 6; ++m) v[m] = xf[j[m]];
-                        sum += bf[f] - arow(cd, xf[f], v, L.sx, L.sy, L.sz, aw);
+                        sum += r[(z * uint32_t(L.ny) + y) * uint32_t(L.nx) + x];
                     }
-            bc[c] = (codes(l + 1)[c] & kCodeFluid) ? sum * weight : 0.0f;
-        }
-        __syncthreads();
+            R.b[k] = (code[c] & kCodeFluid) ? sum * weight : 0.0f;
+            bc[c] = R.b[k];
+        });
     }
     // ascent
     for (int l = A.nlev - 2; l >= 0; --l) {
         const CoarseLevel& L = A.lv[l];
         const CoarseLevel& C = A.lv[l + 1];
-        const float* aw = tab + 128 * l;
-        const float* w = aw + 64;
         const int hx = L.nx > 1 ? 1 : 0, hy = L.ny > 1 ? 1 : 0, hz = L.nz > 1 ? 1 : 0;
-        const float* xc = xs(l + 1);
-        float* xf = xs(l);
-        for (uint32_t c = threadIdx.x; c < ns(l); c += kCoarseThreads) {
-            const uint32_t x = c % uint32_t(L.nx), y = (c / uint32_t(L.nx)) % uint32_t(L.ny),
-                           z = c / (uint32_t(L.nx) * uint32_t(L.ny));
-            if (codes(l)[c] & kCodeFluid)
-                xf[c] += xc[((z >> hz) * uint32_t(C.ny) + (y >> hy)) * uint32_t(C.nx) + (x >> hx)];
-        }
-        __syncthreads();
-        for (int k = 0; k < A.nu; ++k) {
-            lds_sweep(L, codes(l), aw, w, bs(l), xs(l), ts(l), false);
-            par ^= 1u << l;
-        }
+        coarse_cells(cells_of(l), [&](int k, uint32_t c) { R.b[k] = l == 0 ? A.b0[c] : lds[s_b[l] + c]; });
+        load(l);
+        const float* xc = lds + s_x[l + 1];
+        const float* xf = lds + s_x[l];
+        const uint16_t* code = codes(l);
+        coarse_cells(cells_of(l), [&](int k, uint32_t c) {
+            uint32_t x, y, z;
+            coarse_xyz(c, L, x, y, z);
+            R.x[k] = xf[c];
+            if (code[c] & kCodeFluid)
+                R.x[k] += xc[((z >> hz) * uint32_t(C.ny) + (y >> hy)) * uint32_t(C.nx) + (x >> hx)];
+        });
+        store(l);
+        for (int q = 0; q < A.nu; ++q) sweep(l);
     }
-    for (uint32_t c = threadIdx.x; c < ns(0); c += kCoarseThreads) A.x0[c] = xs(0)[c];
+    coarse_cells(cells_of(0), [&](int k, uint32_t c) { A.x0[c] = R.x[k]; });
 }
 
 __global__ void __launch_bounds__(kCoarseThreads) k_mg_coarse_cycle(CoarseArgs A, const CgScalars* __restrict__ sc) {
