@@ -391,14 +391,16 @@ constexpr int kMgStopExtent = 8;
 constexpr size_t kCoarseCells = 8192;    // levels this small run in one work-group
 constexpr int kCoarseLevelsMax = 8;
 constexpr size_t kCoarseLdsMax = 131072;
-// MGF_MG_AUTO fuses levels at least this large (measured at 256^3: fusing the
-// 129^3 level too is 0.8% faster per step, the 65^3 one slower)
-constexpr size_t kMarchMinCells = size_t(1) << 20;
+// MGF_MG_AUTO marches levels at least this large and takes bricks below
+// (150 x 61 x 97 interior, two steps: 4.28 ms with the line at 1M cells, which
+// leaves its 948K-cell level to bricks, 4.07 ms at 512K; at 3M cells the 130^3
+// level of a 128^3 scene goes to bricks: 4.80 -> 5.67 ms)
+constexpr size_t kMarchMinCells = size_t(1) << 19;
 
 // Whether level l (dims f; the next coarser level c) runs the fused descent
 // and ascent: three sweeps, a 3-D level above the coarse cycle, under
-// MGF_MG_AUTO at least kMarchMinCells (on smaller levels the march's serial
-// steps cost more than the launches they save); on level 0 the ascent's
+// MGF_MG_AUTO at least kMarchMinCells (smaller levels: brick_on); on level 0
+// the ascent's
 // partials of r . z must fit the scene's buffer.
 // Blocks of a fused march resident at once: two per CU.
 uint32_t march_slots(mgf_scene s) { return 2u * uint32_t(std::max(1, s->ctx->cu_count)); }
@@ -414,6 +416,19 @@ bool march_on(mgf_scene s, int l, const MgDims& f, const MgDims& c) {
     if (d.mg_kernels == MGF_MG_AUTO && n < kMarchMinCells) return false;
     const size_t part_cap = size_t(std::max<uint32_t>(kMaxBlocks, col_blocks(s->g))) * 2;
     return l > 0 || mg_march_parts(f, c) <= part_cap;
+}
+
+// Whether level l runs one brick launch each way: as march_on, on the levels
+// that do not march.
+bool brick_on(mgf_scene s, int l, const MgDims& f, const MgDims& c) {
+    const auto& d = s->desc;
+    const int nu = d.mg_sweeps > 0 ? d.mg_sweeps : 3;
+    const int L = 1 + int(s->mg.size());
+    const int l0 = s->mg_l0 < L ? s->mg_l0 : L;
+    if (d.preconditioner != MGF_PRECOND_MULTIGRID || nu != 3 || d.mg_kernels == MGF_MG_PER_SWEEP) return false;
+    if (l >= l0 || l + 1 >= L || !mg_march_ok(f) || march_on(s, l, f, c)) return false;
+    const size_t part_cap = size_t(std::max<uint32_t>(kMaxBlocks, col_blocks(s->g))) * 2;
+    return l > 0 || mg_brick_blocks(f) <= part_cap;
 }
 
 mgf_status ensure_sched(mgf_scene s);
@@ -539,11 +554,11 @@ mgf_status apply_precond(mgf_scene s, const float sa[3], const float** zout) {
     const int l0 = s->mg_l0 < L ? s->mg_l0 : L;
     // descent: pre-smoothing from zero (the first two sweeps in one pass),
     // restriction of the residual
-    // fused descent / ascent on the 3-D levels (AUTO: the large ones, where
-    // they beat one kernel per sweep; on small levels the march's serial
-    // steps cost more than the launches they save); the level-0 ascent
-    // writes one partial of r . z per block into the scene's partials buffer
+    // fused descent / ascent on the 3-D levels (AUTO: the march on the large
+    // ones, bricks on the small ones); the level-0 ascent writes its partials
+    // of r . z into the scene's partials buffer
     auto fused = [&](int l) { return l + 1 < L && march_on(s, l, lv[l].d, lv[l + 1].d); };
+    auto bricks = [&](int l) { return l + 1 < L && brick_on(s, l, lv[l].d, lv[l + 1].d); };
     for (int l = 0; l < l0; ++l) {
         Lv& v = lv[l];
         const bool coarsest = l == L - 1;
@@ -554,6 +569,12 @@ mgf_status apply_precond(mgf_scene s, const float sa[3], const float** zout) {
             probe_next_bytes(10.5 * wet + 4.5 * (nl - wet));
             MGF_HIP(launch_mg_descend(st, v.d, lv[l + 1].d, v.codes, v.b, v.x, lv[l + 1].codes,
                                       const_cast<float*>(lv[l + 1].b), omega, s->scal, v.sched, skip));
+            continue;
+        }
+        if (bricks(l)) {
+            probe_next_bytes(10.5 * double(v.d.nx) * v.d.ny * v.d.nz);
+            MGF_HIP(launch_mg_brick_descend(st, v.d, lv[l + 1].d, v.codes, v.b, v.x, lv[l + 1].codes,
+                                            const_cast<float*>(lv[l + 1].b), omega, s->scal));
             continue;
         }
         const int sweeps = coarsest ? kCoarsestSweeps : nu;
@@ -600,6 +621,13 @@ mgf_status apply_precond(mgf_scene s, const float sa[3], const float** zout) {
             probe_next_bytes(14.5 * wet + 4.0 * (ncell - wet));
             MGF_HIP(launch_mg_ascend(st, v.d, lv[l + 1].d, v.codes, v.b, v.x, lv[l + 1].x, v.t, omega, s->scal,
                                      s->red, l == 0 ? 1 : 0, v.sched, skip));
+            std::swap(v.x, v.t);
+            continue;
+        }
+        if (bricks(l)) {
+            probe_next_bytes(14.5 * ncell);
+            MGF_HIP(launch_mg_brick_ascend(st, v.d, lv[l + 1].d, v.codes, v.b, v.x, lv[l + 1].x, v.t, omega, s->scal,
+                                           s->red, l == 0 ? 1 : 0));
             std::swap(v.x, v.t);
             continue;
         }
@@ -954,6 +982,7 @@ mgf_status vcycle_records(mgf_scene s, const float sa[3], std::vector<KRec>& out
     const int skip = s->skip_dry ? 1 : 0;
     const int l0 = s->mg_l0 < L ? s->mg_l0 : L;
     auto fused = [&](int l) { return l + 1 < L && march_on(s, l, lv[l].d, lv[l + 1].d); };
+    auto bricks = [&](int l) { return l + 1 < L && brick_on(s, l, lv[l].d, lv[l + 1].d); };
     std::vector<MRec> r;
     for (int l = 0; l < l0; ++l) {
         Lv& v = lv[l];
@@ -962,6 +991,13 @@ mgf_status vcycle_records(mgf_scene s, const float sa[3], std::vector<KRec>& out
             r.clear();
             rec_mg_descend(r, v.d, lv[l + 1].d, v.codes, v.b, v.x, lv[l + 1].codes, const_cast<float*>(lv[l + 1].b),
                            omega, s->scal, v.sched, skip);
+            keyed(out, r, 0, l, 0);
+            continue;
+        }
+        if (bricks(l)) {
+            r.clear();
+            rec_mg_brick_descend(r, v.d, lv[l + 1].d, v.codes, v.b, v.x, lv[l + 1].codes,
+                                 const_cast<float*>(lv[l + 1].b), omega, s->scal);
             keyed(out, r, 0, l, 0);
             continue;
         }
@@ -1009,6 +1045,14 @@ mgf_status vcycle_records(mgf_scene s, const float sa[3], std::vector<KRec>& out
         if (fused(l)) {
             rec_mg_ascend(r, v.d, lv[l + 1].d, v.codes, v.b, v.x, lv[l + 1].x, v.t, omega, s->scal, s->red,
                           l == 0 ? 1 : 0, v.sched, skip);
+            keyed(out, r, 2, -l, 0);
+            std::swap(v.x, v.t);
+            continue;
+        }
+        if (bricks(l)) {
+            r.clear();
+            rec_mg_brick_ascend(r, v.d, lv[l + 1].d, v.codes, v.b, v.x, lv[l + 1].x, v.t, omega, s->scal, s->red,
+                                l == 0 ? 1 : 0);
             keyed(out, r, 2, -l, 0);
             std::swap(v.x, v.t);
             continue;

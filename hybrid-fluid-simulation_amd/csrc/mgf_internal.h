@@ -426,6 +426,15 @@ hipError_t launch_mg_descend(hipStream_t s, const MgDims& f, const MgDims& c, co
 hipError_t launch_mg_ascend(hipStream_t s, const MgDims& f, const MgDims& c, const uint16_t* code, const float* b,
                             const float* xi, const float* xc, float* xo, float omega, CgScalars* sc, ReduceBuf red,
                             int with_rz, const uint32_t* sched, int skip);
+// The same of a small level, brick by brick (mg_brick_blocks work-groups, one
+// partial of r . z each); no schedule.
+uint32_t mg_brick_blocks(const MgDims& f);
+hipError_t launch_mg_brick_descend(hipStream_t s, const MgDims& f, const MgDims& c, const uint16_t* code,
+                                   const float* b, float* x, const uint16_t* codec, float* bc, float omega,
+                                   const CgScalars* sc);
+hipError_t launch_mg_brick_ascend(hipStream_t s, const MgDims& f, const MgDims& c, const uint16_t* code,
+                                  const float* b, const float* xi, const float* xc, float* xo, float omega,
+                                  CgScalars* sc, ReduceBuf red, int with_rz);
 size_t mg_coarse_lds_bytes(const MgDims* levels, int nlev);
 hipError_t launch_mg_coarse_cycle(hipStream_t s, const MgDims* levels, const uint16_t* const* codes, int nlev,
                                   const float* b0, float* x0, int nu, int last_sweeps, float omega,
@@ -442,6 +451,7 @@ enum MultiKind : int32_t {
     kMkStart, kMkFinish, kMkPap, kMkUpdate, kMkRefine1, kMkRefine2, kMkAcc64, kMkSum2,
     kMkSmoothTT, kMkSmoothTF, kMkSmoothFT, kMkSmoothFF, kMkSmooth2T, kMkSmooth2F, kMkProlongT, kMkProlongF,
     kMkRestrict, kMkRestrict2, kMkRestrictTile, kMkCoarse, kMkMarchDesc, kMkMarchAsc, kMkMarchAscRz, kMkGather,
+    kMkBrickDesc, kMkBrickAsc, kMkBrickAscRz,
     kMkRefine0, kMkCodes, kMkFlatWet, kMkCoarsen, kMkMarchWet, kMkMarchPlan,
     kMkAdvectFc, kMkAdvectCc, kMkAdvectCc4, kMkMarkers, kMkRhs, kMkProject, kMkCopyWord,
     kMkExtRows, kMkExtRowsReg4, kMkExtRowsReg8, kMkExtRowsReg16, kMkExtLines1, kMkExtLines2, kMkExtRowsReg5,
@@ -487,6 +497,11 @@ void rec_mg_descend(std::vector<MRec>& out, const MgDims& f, const MgDims& c, co
 void rec_mg_ascend(std::vector<MRec>& out, const MgDims& f, const MgDims& c, const uint16_t* code, const float* b,
                    const float* xi, const float* xc, float* xo, float omega, CgScalars* sc, ReduceBuf red,
                    int with_rz, const uint32_t* sched, int skip);
+void rec_mg_brick_descend(std::vector<MRec>& out, const MgDims& f, const MgDims& c, const uint16_t* code,
+                          const float* b, float* x, const uint16_t* codec, float* bc, float omega, const CgScalars* sc);
+void rec_mg_brick_ascend(std::vector<MRec>& out, const MgDims& f, const MgDims& c, const uint16_t* code,
+                         const float* b, const float* xi, const float* xc, float* xo, float omega, CgScalars* sc,
+                         ReduceBuf red, int with_rz);
 // The finishing record's size, and its abs_target2 set in place.
 size_t finish_arg_bytes();
 void finish_set_target(unsigned char* args, double abs_target2);

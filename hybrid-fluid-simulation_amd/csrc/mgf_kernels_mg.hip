@@ -1565,6 +1565,196 @@ struct MCoarse {
 };
 
 // ===========================================================================
+// Descent and ascent of a small level (every axis halved, three sweeps) as one
+// launch each: a work-group takes a brick of 8^3 cells and its three-cell
+// halo, forms the pointwise stage on all of it (x1 = omega D^-1 b, or x3 + the
+// prolonged correction on the ascent) and each further stage one cell less
+// into the halo, in two LDS buffers by turns.  On levels that do not fill the
+// chip a launch is a few microseconds of latency whatever it does, so one
+// launch that forms 11.7 values a cell beats three that form one each (34^3:
+// 5.3 us each way against 3 x 3.7 and the gaps between them; 76 x 32 x 50:
+// 5.3 against 3 x 3.8).  The march is better from about half a million cells
+// on, where the extra values count (152 x 63 x 99: 20 us each way here).  Every value is formed by the per-sweep
+// kernels' operations in their order.
+//
+// The region's cells are numbered by how far into the halo they lie (the
+// brick's own first), so that a stage is a prefix of them: work-item t holds
+// cells t, t + 512, ... of the numbering, with their weights in registers.
+constexpr int kBkEdge = 8, kBkHalo = 3, kBkThreads = 512;
+constexpr int kBkReg = kBkEdge + 2 * kBkHalo;                 // 14
+constexpr int kBkCells = kBkReg * kBkReg * kBkReg;            // 2744
+constexpr int kBkCpt = (kBkCells + kBkThreads - 1) / kBkThreads;
+// cells of the numbering with stage 1, 2, 3 (halo 2, 1, 0)
+constexpr int kBkStage[4] = {kBkCells, 12 * 12 * 12, 10 * 10 * 10, 8 * 8 * 8};
+
+// Place (z, y, x fastest in the region) of each cell of the numbering.
+struct BrickOrder {
+    uint16_t at[kBkCpt * kBkThreads];
+};
+constexpr BrickOrder brick_order() {
+    BrickOrder o{};
+    int n = 0;
+    for (int ring = 0; ring <= kBkHalo; ++ring)
+        for (int z = 0; z < kBkReg; ++z)
+            for (int y = 0; y < kBkReg; ++y)
+                for (int x = 0; x < kBkReg; ++x) {
+                    int d = 0;
+                    for (int c : {x, y, z}) {
+                        const int a = c < kBkHalo ? kBkHalo - c : (c >= kBkHalo + kBkEdge ? c - kBkHalo - kBkEdge + 1 : 0);
+                        d = a > d ? a : d;
+                    }
+                    if (d == ring) o.at[n++] = uint16_t((z * kBkReg + y) * kBkReg + x);
+                }
+    return o;
+}
+__device__ const BrickOrder kBrickOrder = brick_order();
+
+struct Bricks {
+    int nx, ny, nz;
+    uint32_t sy, sz;
+    int cnx, cny, cnz;
+    uint32_t csy, csz;
+    uint32_t tx, ty, tz;
+};
+
+template <bool POST, bool RZ>
+__device__ __forceinline__ void brick_run(const Bricks& T, const MgLevel& L, const uint16_t* __restrict__ code,
+                                          const float* __restrict__ b, const float* __restrict__ xi,
+                                          const float* __restrict__ xc, float* __restrict__ xo,
+                                          const uint16_t* __restrict__ codec, float* __restrict__ bco, float omega,
+                                          const CgScalars* __restrict__ sc, double* __restrict__ part, uint32_t blk,
+                                          uint32_t slot) {
+    __shared__ float aw[64], w[64];
+    __shared__ float xa[kBkCells], xb[kBkCells];
+    __shared__ double sum[kBkThreads / 64];
+    if (sc->done) return;
+    const int t = threadIdx.x;
+    const uint32_t bx = blk % T.tx, br = blk / T.tx, by = br % T.ty, bz = br / T.ty;
+    const int x0 = int(bx) * kBkEdge - kBkHalo, y0 = int(by) * kBkEdge - kBkHalo, z0 = int(bz) * kBkEdge - kBkHalo;
+    int at[kBkCpt];
+    uint32_t gi[kBkCpt];
+    uint16_t cd[kBkCpt];
+    float bv[kBkCpt], x[kBkCpt], cv[kBkCpt];
+#pragma unroll
+    for (int k = 0; k < kBkCpt; ++k) at[k] = kBrickOrder.at[k * kBkThreads + t];
+#pragma unroll
+    for (int k = 0; k < kBkCpt; ++k) {
+        const int lz = at[k] / (kBkReg * kBkReg), lr = at[k] - lz * (kBkReg * kBkReg), ly = lr / kBkReg,
+                  lx = lr - ly * kBkReg;
+        const int gx = x0 + lx, gy = y0 + ly, gz = z0 + lz;
+        const bool in = unsigned(gx) < unsigned(T.nx) && unsigned(gy) < unsigned(T.ny) && unsigned(gz) < unsigned(T.nz);
+        gi[k] = in ? uint32_t(gz) * T.sz + uint32_t(gy) * T.sy + uint32_t(gx) : 0u;
+        cd[k] = code[gi[k]];
+        bv[k] = b[gi[k]];
+        if (POST) {
+            x[k] = xi[gi[k]];
+            cv[k] = xc[in ? uint32_t(gz >> 1) * T.csz + uint32_t(gy >> 1) * T.csy + uint32_t(gx >> 1) : 0u];
+        }
+        if (!in) {
+            gi[k] = ~0u;
+            cd[k] = 0;
+            bv[k] = 0.0f;
+        }
+    }
+    build_tables<true>(aw, w, L.sx, L.sy, L.sz, omega);   // a barrier
+    float wd[kBkCpt], av[kBkCpt];
+#pragma unroll
+    for (int k = 0; k < kBkCpt; ++k) {
+        wd[k] = wdiag(cd[k], w);
+        av[k] = aw[air_mask(cd[k])];
+        x[k] = POST ? x[k] + cv[k] : wd[k] * bv[k];
+        if (k * kBkThreads + t < kBkCells) xa[at[k]] = x[k];
+    }
+    __syncthreads();
+    // (A x) of cell k from the buffer `from` (arow with the air weight at hand)
+    auto row = [&](const float* from, int k) {
+        const float* c = from + at[k];
+        const float v[6] = {c[-1], c[1], c[-kBkReg], c[kBkReg], c[-kBkReg * kBkReg], c[kBkReg * kBkReg]};
+        const float ex = keep_if(x[k] - v[0], cd[k], kCplShift + 0) + keep_if(x[k] - v[1], cd[k], kCplShift + 1);
+        const float ey = keep_if(x[k] - v[2], cd[k], kCplShift + 2) + keep_if(x[k] - v[3], cd[k], kCplShift + 3);
+        const float ez = keep_if(x[k] - v[4], cd[k], kCplShift + 4) + keep_if(x[k] - v[5], cd[k], kCplShift + 5);
+        return av[k] * x[k] + L.sx * ex + L.sy * ey + L.sz * ez;
+    };
+    auto stage = [&](const float* from, float* to, int cells) {
+        // x[k] is the cell's own value in `from`
+#pragma unroll
+        for (int k = 0; k < kBkCpt; ++k) {
+            if (k * kBkThreads >= cells) break;
+            if (k * kBkThreads + t < cells) {
+                const float ax = row(from, k);
+                x[k] = (cd[k] & kCodeFluid) ? x[k] + wd[k] * (bv[k] - ax) : 0.0f;
+                if (to) to[at[k]] = x[k];
+            }
+        }
+    };
+    stage(xa, xb, kBkStage[1]);
+    __syncthreads();
+    stage(xb, xa, kBkStage[2]);
+    // this work-item's own cell of the brick: k = 0
+    if (POST) {
+        __syncthreads();
+        stage(xa, nullptr, kBkStage[3]);
+        if (gi[0] != ~0u) xo[gi[0]] = x[0];
+        if (RZ) {
+            double s = wave_sum(double(bv[0]) * double(x[0]));
+            if ((t & 63) == 0) sum[t >> 6] = s;
+            __syncthreads();
+            if (t == 0) {
+                for (int q = 1; q < kBkThreads / 64; ++q) s += sum[q];
+                part[slot] = s;
+            }
+        }
+    } else {
+        if (gi[0] != ~0u) xo[gi[0]] = x[0];
+        __syncthreads();
+        // the residual, then the coarse cells of the brick: 4^3
+        const float ax = row(xa, 0);
+        const float r = (cd[0] & kCodeFluid) ? bv[0] - ax : 0.0f;
+        float* res = xb;   // by (z, y, x) of the brick: the numbering's first 512 are in that order
+        res[t] = r;
+        __syncthreads();
+        if (t < 64) {
+            const int cx = t & 3, cy = (t >> 2) & 3, cz = t >> 4;
+            const int X = int(bx) * 4 + cx, Y = int(by) * 4 + cy, Z = int(bz) * 4 + cz;
+            if (X < T.cnx && Y < T.cny && Z < T.cnz) {
+                const float* f = res + (2 * cz * 8 + 2 * cy) * 8 + 2 * cx;
+                const float s = ((f[0] + f[1]) + (f[8] + f[9])) + ((f[64] + f[65]) + (f[72] + f[73]));
+                const uint32_t c = uint32_t(Z) * T.csz + uint32_t(Y) * T.csy + uint32_t(X);
+                bco[c] = (codec[c] & kCodeFluid) ? s * 0.125f : 0.0f;
+            }
+        }
+    }
+}
+
+template <bool POST, bool RZ>
+__global__ void __launch_bounds__(kBkThreads) k_mg_brick(Bricks T, MgLevel L, const uint16_t* __restrict__ code,
+                                                         const float* __restrict__ b, const float* __restrict__ xi,
+                                                         const float* __restrict__ xc, float* __restrict__ xo,
+                                                         const uint16_t* __restrict__ codec, float* __restrict__ bco,
+                                                         float omega, const CgScalars* __restrict__ sc,
+                                                         double* __restrict__ part) {
+    brick_run<POST, RZ>(T, L, code, b, xi, xc, xo, codec, bco, omega, sc, part, blockIdx.x, blockIdx.x);
+}
+
+template <bool POST, bool RZ>
+struct MBrick {
+    static constexpr int kThreads = kBkThreads;
+    Bricks T;
+    MgLevel L;
+    const uint16_t* code;
+    const float *b, *xi, *xc;
+    float* xo;
+    const uint16_t* codec;
+    float* bco;
+    float omega;
+    const CgScalars* sc;
+    double* part;
+    __device__ void run(uint32_t blk) const {
+        brick_run<POST, RZ>(T, L, code, b, xi, xc, xo, codec, bco, omega, sc, part, blk, blk);
+    }
+};
+
+// ===========================================================================
 // Fused descent and ascent of one level (every axis halved, three sweeps),
 // marching along z.
 //
@@ -2531,6 +2721,43 @@ hipError_t launch_mg_ascend(hipStream_t s, const MgDims& f, const MgDims& c, con
     return finish(s, red.partials, M.parts, sc, kFinishRz);
 }
 
+static Bricks make_bricks(const MgDims& f, const MgDims& c) {
+    auto tiles = [](int n) { return uint32_t((n + kBkEdge - 1) / kBkEdge); };
+    return Bricks{f.nx, f.ny, f.nz, uint32_t(f.nx), uint32_t(f.nx) * uint32_t(f.ny),
+                  c.nx, c.ny, c.nz, uint32_t(c.nx), uint32_t(c.nx) * uint32_t(c.ny),
+                  tiles(f.nx), tiles(f.ny), tiles(f.nz)};
+}
+
+uint32_t mg_brick_blocks(const MgDims& f) {
+    const Bricks T = make_bricks(f, f);
+    return T.tx * T.ty * T.tz;
+}
+
+hipError_t launch_mg_brick_descend(hipStream_t s, const MgDims& f, const MgDims& c, const uint16_t* code,
+                                   const float* b, float* x, const uint16_t* codec, float* bc, float omega,
+                                   const CgScalars* sc) {
+    return launch_dims(k_mg_brick<false, false>, "k_mg_brick", dim3(mg_brick_blocks(f)), dim3(kBkThreads), 0u, s,
+                       make_bricks(f, c), f, code, b, static_cast<const float*>(nullptr),
+                       static_cast<const float*>(nullptr), x, codec, bc, omega, sc, static_cast<double*>(nullptr));
+}
+
+hipError_t launch_mg_brick_ascend(hipStream_t s, const MgDims& f, const MgDims& c, const uint16_t* code,
+                                  const float* b, const float* xi, const float* xc, float* xo, float omega,
+                                  CgScalars* sc, ReduceBuf red, int with_rz) {
+    const uint32_t G = mg_brick_blocks(f);
+    const CgScalars* csc = sc;
+    const uint16_t* nc = nullptr;
+    float* nb = nullptr;
+    if (!with_rz)
+        return launch_dims(k_mg_brick<true, false>, "k_mg_brick", dim3(G), dim3(kBkThreads), 0u, s, make_bricks(f, c),
+                           f, code, b, xi, xc, xo, nc, nb, omega, csc, static_cast<double*>(nullptr));
+    const hipError_t e = launch_dims(k_mg_brick<true, true>, "k_mg_brick", dim3(G), dim3(kBkThreads), 0u, s,
+                                     make_bricks(f, c), f, code, b, xi, xc, xo, nc, nb, omega, csc,
+                                     red.partials);
+    if (e != hipSuccess) return e;
+    return finish(s, red.partials, G, sc, kFinishRz);
+}
+
 size_t mg_coarse_lds_bytes(const MgDims* levels, int nlev) {
     size_t floats = 128 * size_t(nlev);
     for (int l = 0; l < nlev; ++l) {
@@ -2751,6 +2978,28 @@ void rec_mg_restrict(std::vector<MRec>& out, const MgDims& f, const MgDims& c, c
              G);
 }
 
+void rec_mg_brick_descend(std::vector<MRec>& out, const MgDims& f, const MgDims& c, const uint16_t* code,
+                          const float* b, float* x, const uint16_t* codec, float* bc, float omega,
+                          const CgScalars* sc) {
+    push_rec(out, kMkBrickDesc,
+             MBrick<false, false>{make_bricks(f, c), f, code, b, nullptr, nullptr, x, codec, bc, omega, sc, nullptr},
+             mg_brick_blocks(f));
+}
+
+void rec_mg_brick_ascend(std::vector<MRec>& out, const MgDims& f, const MgDims& c, const uint16_t* code,
+                         const float* b, const float* xi, const float* xc, float* xo, float omega, CgScalars* sc,
+                         ReduceBuf red, int with_rz) {
+    const uint32_t G = mg_brick_blocks(f);
+    if (with_rz) {
+        push_rec(out, kMkBrickAscRz,
+                 MBrick<true, true>{make_bricks(f, c), f, code, b, xi, xc, xo, nullptr, nullptr, omega, sc, red.partials}, G);
+        rec_finish(out, red.partials, G, sc, kFinishRz);
+    } else {
+        push_rec(out, kMkBrickAsc,
+                 MBrick<true, false>{make_bricks(f, c), f, code, b, xi, xc, xo, nullptr, nullptr, omega, sc, nullptr}, G);
+    }
+}
+
 bool rec_mg_coarse_cycle(std::vector<MRec>& out, const MgDims* levels, const uint16_t* const* codes, int nlev,
                          const float* b0, float* x0, int nu, int last_sweeps, float omega, const CgScalars* sc) {
     if (nlev < 1 || nlev > kCoarseMaxLevels) return false;
@@ -2857,6 +3106,9 @@ hipError_t launch_multi(hipStream_t s, int32_t kind, const void* tab, const uint
         case kMkMarchDesc: return launch_m_march<MMarch<false, false>>(s, tab, map, nblocks, active);
         case kMkMarchAsc: return launch_m_march<MMarch<true, false>>(s, tab, map, nblocks, active);
         case kMkMarchAscRz: return launch_m_march<MMarch<true, true>>(s, tab, map, nblocks, active);
+        case kMkBrickDesc: return launch_m<MBrick<false, false>>(s, "k_multi_mg_brick", tab, map, nblocks, 0, active);
+        case kMkBrickAsc: return launch_m<MBrick<true, false>>(s, "k_multi_mg_brick", tab, map, nblocks, 0, active);
+        case kMkBrickAscRz: return launch_m<MBrick<true, true>>(s, "k_multi_mg_brick", tab, map, nblocks, 0, active);
         case kMkGather: return launch_m<MGather>(s, "k_multi_gather", tab, map, nblocks, 0, active);
         case kMkRefine0: return launch_m<MRefine<0>>(s, "k_multi_refine", tab, map, nblocks, 0, active);
         case kMkCodes: return launch_m<MCodes>(s, "k_multi_codes", tab, map, nblocks, 0, active);

@@ -160,10 +160,12 @@ typedef struct mgf_scene_desc {
 
 /* Kernels of the multigrid V-cycle (mgf_scene_desc.mg_kernels).  With three
  * sweeps, a 3-D level's descent (three sweeps and the restriction) and ascent
- * (prolongation and three sweeps) can each run as one fused kernel. */
-#define MGF_MG_AUTO      0  /* fused on levels of at least 1M cells (default) */
+ * (prolongation and three sweeps) can each run as one fused kernel: a march
+ * along z (large levels) or brick by brick (small ones). */
+#define MGF_MG_AUTO      0  /* the march on levels of at least 512K cells,
+                               bricks on smaller 3-D levels (default)         */
 #define MGF_MG_PER_SWEEP 1  /* one kernel per sweep on every level            */
-#define MGF_MG_FUSED     2  /* fused on every 3-D level                       */
+#define MGF_MG_FUSED     2  /* the march on every 3-D level                   */
 
 /* Per-call statistics (summed over the steps of one mgf_step call). */
 typedef struct mgf_step_stats {
@@ -359,10 +361,10 @@ MGF_API mgf_status mgf_batch_set_lockstep(mgf_context ctx, int32_t enabled);
 /* Autotuner of the lockstep batch (no counterpart in the reference).  Times
  * the V-cycle kernel choices on these scenes, each over one lockstep batch
  * call of trial_steps (>= 2) steps, and keeps the faster on every scene that
- * runs in lockstep (their mg_kernels field): MGF_MG_AUTO (fused descent and
- * ascent on levels of at least 1M cells, one kernel per sweep below) and
- * MGF_MG_FUSED (fused on every 3-D level above the coarse cycle; small
- * levels of many scenes fill the device together).  Every scene advances by
+ * runs in lockstep (their mg_kernels field): MGF_MG_AUTO (the march on
+ * levels of at least 512K cells, bricks below) and MGF_MG_FUSED (the march on
+ * every 3-D level above the coarse cycle; small levels of many scenes fill
+ * the device together).  Every scene advances by
  * 2 * trial_steps steps.  The choice changes only the summation order of
  * r.z (z = M^-1 r is bitwise the same), so the iterates differ within FP64
  * rounding; a scene then computes bitwise what it computes alone with the

@@ -71,6 +71,24 @@ def test_fused_vcycle_bitwise_per_sweep(ctx, res):
     f.close(); p.close()
 
 
+@pytest.mark.parametrize("res", [(9, 9, 9), (21, 17, 30), (24, 16, 32), (59, 12, 35), (64, 11, 40), (117, 21, 66),
+                                 (2, 2, 2100), (25, 33, 2)])
+def test_brick_vcycle_bitwise_per_sweep(ctx, res):
+    """MGF_MG_AUTO's brick kernels (levels of fewer than 512K cells above the
+    coarse cycle's 8192) against one kernel per sweep: extents that are
+    multiples of the 8-cell brick, one more, one less, and thinner than it."""
+    a = random_scene(ctx, res, 11 + sum(res), mgf.MG_AUTO)
+    p = random_scene(ctx, res, 11 + sum(res), mgf.MG_PER_SWEEP)
+    a.set_kernel_probes(True)
+    a.kernel_probes(reset=True)
+    r = np.random.default_rng(sum(res)).standard_normal(int(np.prod(res))).astype(np.float32)
+    z = check_same(a, p, r, "res %s" % (res,))
+    assert np.any(z != 0.0)
+    # level 0 always lies above the coarse cycle
+    assert a.kernel_probes(reset=True)["k_mg_brick"]["launches"] >= 2
+    a.close(); p.close()
+
+
 @pytest.mark.parametrize("res", [(1, 40, 33), (37, 1, 20), (33, 25, 1)])
 def test_fused_vcycle_2d_grids(ctx, res):
     """A grid with an axis of one cell: no level is fused (every axis must

@@ -181,6 +181,40 @@ def test_extrapolate_bitexact_long_lines(ctx, orc, res):
         ctx.free(p)
 
 
+@pytest.mark.parametrize("known", ["corner", "planes", "sparse"])
+@pytest.mark.parametrize("res,layers", [((32, 16, 16), 1000), ((31, 15, 15), 1000), ((33, 17, 17), 9),
+                                        ((63, 31, 34), 1000), ((97, 40, 2), 60), ((1, 33, 49), 1000)])
+def test_extrapolate_bitexact_bricks(ctx, orc, res, layers, known):
+    """Layers that cross the 32 x 16 x 16 bricks: extents at, below and above
+    the brick's, from one known face in a corner (every brick waits for its
+    neighbours), from known planes inside a brick and at its edge (both sides
+    wait for the middle) and from 0.5% of the faces; all layers, and caps that
+    end inside a brick."""
+    rng = np.random.default_rng(sum(res) + layers)
+    vel = rand_vel(rng, res, 1.0)
+    for k, a in enumerate(vel):
+        ext = [res[d] + (d == k) for d in range(3)]
+        keep = np.zeros(tuple(ext[::-1]), bool)               # [z][y][x]
+        if known == "corner":
+            keep[-1 if k else 0, 0, -1] = True
+        elif known == "planes":
+            keep[:, :, ext[0] // 3] = True
+            keep[min(15, ext[2] - 1), :, :] = True
+        else:
+            keep[:] = rng.random(keep.shape) < 0.005
+        a[~keep.ravel()] = FLT_MAX
+    *want, used = orc.extrapolate_fc(res, *vel, layers)
+    D = [ctx.to_device(a) for a in vel]
+    got_used = mgf.C.c_int32()
+    mgf.check(mgf.lib().mgf_op_extrapolate_fc(ctx.h, mgf.grid(res), D[0], D[1], D[2], layers,
+                                              mgf.C.byref(got_used)), "extrapolate")
+    for k, e in enumerate(want):
+        assert_bitexact(ctx.to_host(D[k], e.size), e, "extrapolate c%d" % k)
+    assert got_used.value == used
+    for p in D:
+        ctx.free(p)
+
+
 def test_extrapolate_bitexact_16bit_distances(ctx, orc):
     """Face distances are stored in 16 bits: a row of 65001 u faces with one
     known face at its start has distances up to 65000 (the sorted layers stop
