@@ -21,7 +21,9 @@ __global__ void __launch_bounds__(kBlock) k_backtrace(GridDev g, Vel V, RkCoef k
     const int64_t i = int64_t(xcd_block()) * kBlock + threadIdx.x;
     if (i >= n) return;
     float x = px[i], y = py[i], z = pz[i];
-    backtrace(V, g, order, k, x, y, z);
+    if (g.path == kPathPow2) backtrace<kPathPow2>(V, g, order, k, x, y, z);
+    else if (g.path == kPathRecip) backtrace<kPathRecip>(V, g, order, k, x, y, z);
+    else backtrace<kPathAny>(V, g, order, k, x, y, z);
     px[i] = x; py[i] = y; pz[i] = z;
 }
 
@@ -44,10 +46,10 @@ struct Inc {
     int add_a, add_b;
 };
 
-__device__ __forceinline__ void k_advect_fc_run(GridDev g, Vel in, Vel V, RkCoef k, int order,
-                                                      float* __restrict__ ou, float* __restrict__ ov,
-                                                      float* __restrict__ ow, uint32_t nfx,
-                                                      uint32_t nfy, uint32_t nfz, Inc inc, uint32_t blk) {
+template <int kPath>
+__device__ __forceinline__ void advect_fc_t(GridDev g, Vel in, Vel V, RkCoef k, int order,
+                                            float* __restrict__ ou, float* __restrict__ ov, float* __restrict__ ow,
+                                            uint32_t nfx, uint32_t nfy, uint32_t nfz, Inc inc, uint32_t blk) {
     uint32_t i = blk * kBlock + threadIdx.x;
     int c;
     if (i < nfx) c = 0;
@@ -60,9 +62,15 @@ __device__ __forceinline__ void k_advect_fc_run(GridDev g, Vel in, Vel V, RkCoef
     float px = c == 0 ? fpos(x, g.hx, g.ox) : cpos(x, g.hx, g.ox);
     float py = c == 1 ? fpos(y, g.hy, g.oy) : cpos(y, g.hy, g.oy);
     float pz = c == 2 ? fpos(z, g.hz, g.oz) : cpos(z, g.hz, g.oz);
-    backtrace(V, g, order, k, px, py, pz);
+    backtrace<kPath>(V, g, order, k, px, py, pz);
     const float* src = c == 0 ? in.u : (c == 1 ? in.v : in.w);
-    float val = sample_comp(src, c, g, px, py, pz);
+    float val;
+    if (kPath == kPathAny) {
+        val = sample_comp(src, c, g, px, py, pz);
+    } else {
+        const Point P = point_t<kPath>(g, c, px, py, pz);
+        val = gather_t(src, P.ex, P.ey, P.ez, P.x, P.y, P.z);
+    }
     // the component's increments by selection (an index at run time would
     // copy the struct to scratch memory)
     const float ia = c == 0 ? inc.a[0] : (c == 1 ? inc.a[1] : inc.a[2]);
@@ -71,6 +79,15 @@ __device__ __forceinline__ void k_advect_fc_run(GridDev g, Vel in, Vel V, RkCoef
     if (inc.add_b) val = val + ib;
     float* dst = c == 0 ? ou : (c == 1 ? ov : ow);
     dst[i] = val;
+}
+
+__device__ __forceinline__ void k_advect_fc_run(GridDev g, Vel in, Vel V, RkCoef k,
+                                                int order, float* __restrict__ ou, float* __restrict__ ov,
+                                                float* __restrict__ ow, uint32_t nfx, uint32_t nfy, uint32_t nfz,
+                                                Inc inc, uint32_t blk) {
+    if (g.path == kPathPow2) advect_fc_t<kPathPow2>(g, in, V, k, order, ou, ov, ow, nfx, nfy, nfz, inc, blk);
+    else if (g.path == kPathRecip) advect_fc_t<kPathRecip>(g, in, V, k, order, ou, ov, ow, nfx, nfy, nfz, inc, blk);
+    else advect_fc_t<kPathAny>(g, in, V, k, order, ou, ov, ow, nfx, nfy, nfz, inc, blk);
 }
 
 __global__ void __launch_bounds__(kBlock) k_advect_fc(GridDev g, Vel in, Vel V, RkCoef k, int order,
@@ -99,17 +116,42 @@ struct MAdvectFc {
 };
 
 // CSemiLagrangian::advect(CCS) (MPhysics/SemiLagrangian.cpp:135-150).
-__device__ __forceinline__ void k_advect_cc_run(GridDev g, const float* __restrict__ in, Vel V,
-                                                      RkCoef k, int order, float* __restrict__ out,
-                                                      uint32_t n, uint32_t blk) {
+// kFields fields of one step share the back-trace of their cell centres.
+template <int kPath, int kFields, class In, class Out>
+__device__ __forceinline__ void advect_cc_t(const GridDev& g, const In& in, const Vel& V, const RkCoef& k, int order,
+                                            const Out& out, uint32_t n, uint32_t blk) {
     const uint32_t i = blk * kBlock + threadIdx.x;
     if (i >= n) return;
     const uint32_t nx = uint32_t(g.nx), ny = uint32_t(g.ny);
     int x, y, z;
     decode3(i, nx, ny, g.r_nx, g.r_nxy, x, y, z);
     float px = cpos(x, g.hx, g.ox), py = cpos(y, g.hy, g.oy), pz = cpos(z, g.hz, g.oz);
-    backtrace(V, g, order, k, px, py, pz);
-    out[i] = trilerp(in, g.nx, g.ny, g.nz, g.ox, g.oy, g.oz, g, px, py, pz);
+    backtrace<kPath>(V, g, order, k, px, py, pz);
+    if (kPath == kPathAny) {
+#pragma unroll
+        for (int q = 0; q < kFields; ++q)
+            out[q][i] = trilerp(in[q], g.nx, g.ny, g.nz, g.ox, g.oy, g.oz, g, px, py, pz);
+    } else {
+        const Point P = point_t<kPath>(g, 3, px, py, pz);
+#pragma unroll
+        for (int q = 0; q < kFields; ++q) out[q][i] = gather_t(in[q], g.nx, g.ny, g.nz, P.x, P.y, P.z);
+    }
+}
+
+template <int kFields, class In, class Out>
+__device__ __forceinline__ void advect_cc_any(const GridDev& g, const In& in, const Vel& V, const RkCoef& k, int order,
+                                              const Out& out, uint32_t n, uint32_t blk) {
+    if (g.path == kPathPow2) advect_cc_t<kPathPow2, kFields>(g, in, V, k, order, out, n, blk);
+    else if (g.path == kPathRecip) advect_cc_t<kPathRecip, kFields>(g, in, V, k, order, out, n, blk);
+    else advect_cc_t<kPathAny, kFields>(g, in, V, k, order, out, n, blk);
+}
+
+__device__ __forceinline__ void k_advect_cc_run(const GridDev& g, const float* __restrict__ in, const Vel& V,
+                                                const RkCoef& k, int order, float* __restrict__ out, uint32_t n,
+                                                uint32_t blk) {
+    const float* const fi[1] = {in};
+    float* const fo[1] = {out};
+    advect_cc_any<1>(g, fi, V, k, order, fo, n, blk);
 }
 
 __global__ void __launch_bounds__(kBlock) k_advect_cc(GridDev g, const float* __restrict__ in, Vel V,
@@ -140,17 +182,9 @@ struct Cc4 {
     const float* in[4];
     float* out[4];
 };
-__device__ __forceinline__ void k_advect_cc4_run(GridDev g, Cc4 F, Vel V, RkCoef k, int order, uint32_t n, uint32_t blk) {
-    const uint32_t i = blk * kBlock + threadIdx.x;
-    if (i >= n) return;
-    const uint32_t nx = uint32_t(g.nx), ny = uint32_t(g.ny);
-    int x, y, z;
-    decode3(i, nx, ny, g.r_nx, g.r_nxy, x, y, z);
-    float px = cpos(x, g.hx, g.ox), py = cpos(y, g.hy, g.oy), pz = cpos(z, g.hz, g.oz);
-    backtrace(V, g, order, k, px, py, pz);
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-        F.out[q][i] = trilerp(F.in[q], g.nx, g.ny, g.nz, g.ox, g.oy, g.oz, g, px, py, pz);
+__device__ __forceinline__ void k_advect_cc4_run(const GridDev& g, const Cc4& F, const Vel& V, const RkCoef& k,
+                                                 int order, uint32_t n, uint32_t blk) {
+    advect_cc_any<4>(g, F.in, V, k, order, F.out, n, blk);
 }
 
 __global__ void __launch_bounds__(kBlock) k_advect_cc4(GridDev g, Cc4 F, Vel V, RkCoef k, int order, uint32_t n) {

@@ -539,14 +539,14 @@ __global__ void __launch_bounds__(kBlock) k_rk_substep(GridDev g, Vel V, int64_t
             x = __builtin_fmaf(step, ax, x0); y = __builtin_fmaf(step, ay, y0); z = __builtin_fmaf(step, az, z0);
         } else if (order == 2) {
             float bx, by, bz;
-            sample_vel(V, g, __builtin_fmaf(half, ax, x0), __builtin_fmaf(half, ay, y0), __builtin_fmaf(half, az, z0),
+            sample_vel_any(V, g, __builtin_fmaf(half, ax, x0), __builtin_fmaf(half, ay, y0), __builtin_fmaf(half, az, z0),
                        bx, by, bz);
             x = __builtin_fmaf(step, bx, x0); y = __builtin_fmaf(step, by, y0); z = __builtin_fmaf(step, bz, z0);
         } else if (order == 3) {
             float bx, by, bz, cx, cy, cz;
-            sample_vel(V, g, __builtin_fmaf(half, ax, x0), __builtin_fmaf(half, ay, y0), __builtin_fmaf(half, az, z0),
+            sample_vel_any(V, g, __builtin_fmaf(half, ax, x0), __builtin_fmaf(half, ay, y0), __builtin_fmaf(half, az, z0),
                        bx, by, bz);
-            sample_vel(V, g, __builtin_fmaf(three_q, bx, x0), __builtin_fmaf(three_q, by, y0),
+            sample_vel_any(V, g, __builtin_fmaf(three_q, bx, x0), __builtin_fmaf(three_q, by, y0),
                        __builtin_fmaf(three_q, bz, z0), cx, cy, cz);
             x = __builtin_fmaf(c3, cx, __builtin_fmaf(c2, bx, __builtin_fmaf(c1, ax, x0)));
             y = __builtin_fmaf(c3, cy, __builtin_fmaf(c2, by, __builtin_fmaf(c1, ay, y0)));
@@ -557,7 +557,7 @@ __global__ void __launch_bounds__(kBlock) k_rk_substep(GridDev g, Vel V, int64_t
         pos[3 * p] = x; pos[3 * p + 1] = y; pos[3 * p + 2] = z;
         if (resample) {
             float a, b, c;
-            sample_vel(V, g, x, y, z, a, b, c);
+            sample_vel_any(V, g, x, y, z, a, b, c);
             v1[3 * p] = a; v1[3 * p + 1] = b; v1[3 * p + 2] = c;
             m = max(m, max(__float_as_uint(fabsf(a)), max(__float_as_uint(fabsf(b)), __float_as_uint(fabsf(c)))));
         }
@@ -573,7 +573,7 @@ __global__ void __launch_bounds__(kBlock) k_sample_absmax(GridDev g, Vel V, int6
     const int64_t stride = int64_t(gridDim.x) * kBlock;
     for (int64_t p = int64_t(xcd_block()) * kBlock + threadIdx.x; p < np; p += stride) {
         float a, b, c;
-        sample_vel(V, g, pos[3 * p], pos[3 * p + 1], pos[3 * p + 2], a, b, c);
+        sample_vel_any(V, g, pos[3 * p], pos[3 * p + 1], pos[3 * p + 2], a, b, c);
         out[3 * p] = a; out[3 * p + 1] = b; out[3 * p + 2] = c;
         m = max(m, max(__float_as_uint(fabsf(a)), max(__float_as_uint(fabsf(b)), __float_as_uint(fabsf(c)))));
     }

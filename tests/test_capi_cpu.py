@@ -99,3 +99,29 @@ def test_init_without_gpu_reports_device_error():
     rc = mgf.lib().mgf_init(0, C.byref(h))
     assert rc == mgf.ERR_DEVICE
     assert b"device" in mgf.lib().mgf_last_error().lower()
+
+
+def test_reciprocal_quotient_rounds_like_the_division():
+    """The samplers' quotient x / h from the rounded reciprocal (two corrections
+    by fused multiply-adds), against the division, over the range it is used
+    in: h in 2^-20 .. 2^20, |x| from 2^-46 to 2^22 h; hard spacings (mantissas
+    at the ends and near them) and random ones."""
+    import ctypes
+    import numpy as np
+    fmaf = ctypes.CDLL("libm.so.6").fmaf
+    fmaf.restype, fmaf.argtypes = ctypes.c_float, [ctypes.c_float] * 3
+    f32 = np.float32
+    rng = np.random.default_rng(20)
+    mant = np.concatenate([1.0 + 2.0 ** -23 * np.arange(4), 2.0 - 2.0 ** -23 * np.arange(1, 5), 1.0 + rng.random(40)])
+    for m in mant:
+        h = f32(m * 2.0 ** rng.integers(-20, 20))
+        rh = f32(1.0) / h
+        q = (1.0 + rng.random(300)) * 2.0 ** rng.integers(-24, 22, 300)
+        q[:100] = np.round(q[:100] * 2.0 ** 8) / 2.0 ** 8              # quotients at and around short values
+        for x in (q * float(h) * rng.choice([-1.0, 1.0], 300)).astype(np.float32):
+            if not (2.0 ** -46 <= abs(x) < 4194304.0 * float(h)):
+                continue
+            q0 = f32(x * rh)
+            q1 = fmaf(fmaf(-q0, h, x), rh, q0)
+            q2 = fmaf(fmaf(-q1, h, x), rh, q1)
+            assert f32(q2).tobytes() == f32(x / h).tobytes(), (x, h)

@@ -80,6 +80,39 @@ def test_backtrace_bitexact(ctx, orc, order):
         ctx.free(p)
 
 
+@pytest.mark.parametrize("res", [(9, 7, 5), (2, 1, 3), (1, 6, 4), (33, 2, 1)])
+@pytest.mark.parametrize("h", [(0.1, 0.2, 0.3), (1 / 50, 1 / 3, 7.7), (1 - 2.0 ** -24, 1 + 2.0 ** -23, 2.0 ** 20),
+                               (0.5, 0.25, 2.0), (1.1 * 2.0 ** -20,) * 3, (0.9 * 2.0 ** -20, 0.1, 0.1),
+                               (0.1, 0.1, 1.5 * 2.0 ** 20)])
+def test_backtrace_sampler_paths(ctx, orc, res, h):
+    """The samplers' instances (sample_path): spacings that are powers of two,
+    others within and beyond 2^-20 .. 2^20, rows of one value; points in, on
+    the cells' and faces' planes of, around and millions of spacings outside
+    the grid."""
+    h = tuple(float(np.float32(v)) for v in h)
+    rng = np.random.default_rng(sum(res))
+    o = (0.25 * h[0], -3.7 * h[1], 11 * h[2])
+    u, v, w = rand_vel(rng, res, 1.0)
+    n = 3000
+    P = []
+    for k in range(3):
+        t = rng.uniform(-2.0, res[k] + 2.0, n)
+        t[: n // 4] = np.round(2 * t[: n // 4]) / 2                    # on planes of faces and of cell centres
+        t[n // 4: n // 2] = np.round(2 * t[n // 4: n // 2]) / 2 + rng.uniform(-1e-6, 1e-6, n // 4)
+        t[-60:] *= 10.0 ** rng.uniform(2.0, 7.0, 60)
+        P.append((o[k] + h[k] * t).astype(np.float32))
+    rng.shuffle(P[1]); rng.shuffle(P[2])
+    dt = 0.37 * min(h)
+    e = orc.backtrace(res, o, h, u, v, w, dt, 3, *P)
+    dev = [ctx.to_device(a) for a in (u, v, w)] + [ctx.to_device(a) for a in P]
+    mgf.check(mgf.lib().mgf_op_backtrace(ctx.h, mgf.grid(res, o, h), dev[0], dev[1], dev[2], np.float32(dt), 3,
+                                         dev[3], dev[4], dev[5], n), "backtrace")
+    for k in range(3):
+        assert_bitexact(ctx.to_host(dev[3 + k], n), e[k], "backtrace p%d" % k)
+    for p in dev:
+        ctx.free(p)
+
+
 def test_sample_cc_bitexact(ctx, orc):
     rng = np.random.default_rng(7)
     res, o, h = (11, 6, 4), (-1.0, 0.5, 0.25), (0.3, 0.7, 1.1)
