@@ -673,7 +673,7 @@ mgf_status cg_mixed(mgf_scene s, const float sa[3], int64_t max_it, mgf_step_sta
     // MIXED by mgf_scene_set_params gets it here
     if (!s->wet_flat) TRY(dalloc(s, &s->wet_flat, col_blocks(s->g)));
     MGF_HIP(launch_flat_wet(st, s->g, s->codes, s->wet_flat));
-    const uint8_t* wet_flat = s->skip_dry ? s->wet_flat : nullptr;
+    const uint16_t* wet_flat = s->skip_dry ? s->wet_flat : nullptr;
     if (!ident) {
         TRY(ensure_precond(s));
         TRY(mg_setup(s, sa));
@@ -681,8 +681,8 @@ mgf_status cg_mixed(mgf_scene s, const float sa[3], int64_t max_it, mgf_step_sta
     s->wet_flat_cells = s->wet0_cells = -1.0;
     if (s->probes && s->skip_dry) {
         // the bytes probed launches move: blocks without fluid move (almost) nothing
-        std::vector<uint8_t> h(col_blocks(s->g));
-        MGF_HIP(hipMemcpyAsync(h.data(), s->wet_flat, h.size(), hipMemcpyDeviceToHost, st));
+        std::vector<uint16_t> h(col_blocks(s->g));
+        MGF_HIP(hipMemcpyAsync(h.data(), s->wet_flat, h.size() * sizeof(uint16_t), hipMemcpyDeviceToHost, st));
         MGF_HIP(hipStreamSynchronize(st));
         s->wet_flat_cells = flat_wet_cells(s->g, h.data());
         // the cells each fused level's schedule marches
@@ -709,7 +709,7 @@ mgf_status cg_mixed(mgf_scene s, const float sa[3], int64_t max_it, mgf_step_sta
     const bool warm = d.warm_start && s->x64_valid;
     s->x64_valid = false;
     MGF_HIP(launch_refine_true(st, s->g, sa, s->codes, nullptr, s->x64, s->b, warm ? s->r : nullptr, warm ? 3 : 0,
-                               s->red, s->red.out2));
+                               s->red, s->red.out2, nullptr));
     MGF_HIP(hipMemcpyAsync(s->host_scratch, s->red.out2, sizeof(double) * 2, hipMemcpyDeviceToHost, st));
     MGF_HIP(hipStreamSynchronize(st));
     const double b2 = s->host_scratch[1];
@@ -762,7 +762,7 @@ mgf_status cg_mixed(mgf_scene s, const float sa[3], int64_t max_it, mgf_step_sta
         if (hs.done == 2) { rr_true = std::nan(""); break; }
         // x64 (+)= x; r = b - A x64 in FP64
         MGF_HIP(launch_refine_true(st, s->g, sa, s->codes, s->x, s->x64, s->b, s->r, (sweeps > 0 || warm) ? 2 : 1,
-                                   s->red, s->red.out2));
+                                   s->red, s->red.out2, wet_flat));
         MGF_HIP(hipMemcpyAsync(s->host_scratch, s->red.out2, sizeof(double) * 2, hipMemcpyDeviceToHost, st));
         MGF_HIP(hipStreamSynchronize(st));
         rr_true = s->host_scratch[0];
@@ -1165,7 +1165,7 @@ mgf_status phase_records(mgf_scene s, int c, std::vector<KRec>& pre, std::vector
         cf = s->mg[l].codes;
     }
     r.clear();
-    rec_refine_true(r, s->g, sa, s->codes, nullptr, s->x64, s->b, nullptr, 0, s->red, s->red.out2);
+    rec_refine_true(r, s->g, sa, s->codes, nullptr, s->x64, s->b, nullptr, 0, s->red, s->red.out2, nullptr);
     keyed(pre, r, 3, 0, 0);
     // after the solve
     r.clear();
@@ -1405,7 +1405,7 @@ mgf_status build_plan(LockPlan& P) {
             float sa[3], sg[3];
             scales(s, sa, sg);
             const double inner = s->desc.inner_tolerance > 0 ? s->desc.inner_tolerance : 1e-3;
-            const uint8_t* wet_flat = s->skip_dry ? s->wet_flat : nullptr;
+            const uint16_t* wet_flat = s->skip_dry ? s->wet_flat : nullptr;
             std::vector<MRec> r;
             start_b[i].clear(); start_r[i].clear(); cg[i].clear(); vc[i].clear();
             ref1[i].clear(); ref2[i].clear(); gat[i].clear();
@@ -1424,10 +1424,10 @@ mgf_status build_plan(LockPlan& P) {
             rec_col_update(r, s->g, s->p0, s->p1, s->x, s->r, s->scal, s->red, 0, wet_flat);
             keyed(cg[i], r, 0, 0, 1);
             r.clear();
-            rec_refine_true(r, s->g, sa, s->codes, s->x, s->x64, s->b, s->r, 1, s->red, s->red.out2);
+            rec_refine_true(r, s->g, sa, s->codes, s->x, s->x64, s->b, s->r, 1, s->red, s->red.out2, wet_flat);
             keyed(ref1[i], r, 0, 0, 0);
             r.clear();
-            rec_refine_true(r, s->g, sa, s->codes, s->x, s->x64, s->b, s->r, 2, s->red, s->red.out2);
+            rec_refine_true(r, s->g, sa, s->codes, s->x, s->x64, s->b, s->r, 2, s->red, s->red.out2, wet_flat);
             keyed(ref2[i], r, 0, 0, 0);
             r.clear();
             rec_gather(r, s->scal, s->red.out2, gsc + i, gout + 2 * i);

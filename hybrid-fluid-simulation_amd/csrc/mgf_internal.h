@@ -162,7 +162,7 @@ struct mgf_scene_s {
     float* zt = nullptr;           // Jacobi ping-pong partner of z
     uint32_t* sched0 = nullptr;    // fused-march schedule of level 0
     size_t sched0_n = 0;
-    uint8_t* wet_flat = nullptr;   // blocks of the flat CG kernels with fluid
+    uint16_t* wet_flat = nullptr;  // the flat CG kernels' segments with fluid, a mask a block
     // with probes on: cells in blocks with fluid (flat kernels, level-0
     // march) for the bytes a probed launch moved; < 0 = every cell
     double wet_flat_cells = -1.0, wet0_cells = -1.0;
@@ -184,7 +184,7 @@ struct mgf_scene_s {
     // kernel probes: every launch of the scene's entry points while enabled
     bool probes = false;
     mgf::ProbeSink sink;
-    bool skip_dry = true;          // CG / fused multigrid blocks without fluid return at once
+    bool skip_dry = true;          // CG segments and fused multigrid blocks without fluid are left out
     bool div_check = false;        // divergence check after each projection
     double* div_dev = nullptr;     // [0] largest ratio of the call, [1..2] the last sums
 
@@ -365,18 +365,18 @@ hipError_t launch_codes(hipStream_t s, int nx, int ny, int nz, const uint8_t* ma
 // Blocks of the column kernels on grid g (the partial-sum buffer must hold
 // four doubles per block).
 uint32_t col_blocks(const GridDev& g);
-// wet: per block of the flat kernels, whether it holds a fluid cell
-// (launch_flat_wet, once per set of codes); null: no block skips.
-hipError_t launch_flat_wet(hipStream_t s, const GridDev& g, const uint16_t* codes, uint8_t* wet);
-// Cells in the blocks a host copy of the wet bytes marks (measurement).
-double flat_wet_cells(const GridDev& g, const uint8_t* wet_host);
+// wet: per block of the flat kernels, which of its 64-cell segments hold fluid
+// (launch_flat_wet, once per set of codes); null: no segment is left out.
+hipError_t launch_flat_wet(hipStream_t s, const GridDev& g, const uint16_t* codes, uint16_t* wet);
+// Cells in the segments a host copy of the masks marks (measurement).
+double flat_wet_cells(const GridDev& g, const uint16_t* wet_host);
 // K_I: p = z + beta p, Ap = A z + beta Ap in place (p = z, Ap = A z on the
 // first iteration), p . Ap, alpha.
 hipError_t launch_col_p_ap(hipStream_t s, const GridDev& g, const float scale[3], const uint16_t* codes,
-                           const float* zv, float* p, float* ap, CgScalars* sc, ReduceBuf red, const uint8_t* wet);
+                           const float* zv, float* p, float* ap, CgScalars* sc, ReduceBuf red, const uint16_t* wet);
 // K_II: x += alpha p, r -= alpha Ap, r . r; identity != 0: beta = rr / rz, rz = rr.
 hipError_t launch_col_update(hipStream_t s, const GridDev& g, const float* p, const float* ap, float* x, float* r,
-                             CgScalars* sc, ReduceBuf red, int identity, const uint8_t* wet);
+                             CgScalars* sc, ReduceBuf red, int identity, const uint16_t* wet);
 // Start of an inner sweep: r = rsrc, x = 0, the scalars from r.r (target =
 // max(rel_inner^2 r.r, abs_target2)).
 hipError_t launch_cg_start(hipStream_t s, const GridDev& g, const float* rsrc, float* r, float* x, CgScalars* sc,
@@ -384,10 +384,11 @@ hipError_t launch_cg_start(hipStream_t s, const GridDev& g, const float* rsrc, f
 // Refinement: mode 0: x64 = 0; mode 1: x64 = xcorr; mode 2: x64 += xcorr;
 // mode 3: x64 kept on fluid cells, zeroed elsewhere (a warm start); then
 // (modes 1-3) r = b - A x64 in FP64, stored FP32 when r != null.  out2 (device)
-// receives ||b - A x64||^2 (0 in mode 0) and ||b||^2.
+// receives ||b - A x64||^2 (0 in mode 0) and ||b||^2.  Modes 1 and 2 leave dry
+// segments out (wet), where an earlier mode 0 or 3 has cleared x64.
 hipError_t launch_refine_true(hipStream_t s, const GridDev& g, const float scale[3], const uint16_t* codes,
                               const float* xcorr, double* x64, const float* b, float* r, int mode, ReduceBuf red,
-                              double* out2);
+                              double* out2, const uint16_t* wet);
 hipError_t launch_mg_coarsen(hipStream_t s, const MgDims& f, const MgDims& c, const uint8_t* mf, uint8_t* mc,
                              int fluid_first);
 hipError_t launch_mg_smooth(hipStream_t s, const MgDims& l, const uint16_t* code, const float* b, const float* xi,
@@ -474,12 +475,12 @@ struct MRec {
 void rec_cg_start(std::vector<MRec>& out, const GridDev& g, const float* rsrc, float* r, float* x, CgScalars* sc,
                   ReduceBuf red, double rel_inner, double abs_target2);
 void rec_col_p_ap(std::vector<MRec>& out, const GridDev& g, const float scale[3], const uint16_t* codes,
-                  const float* zv, float* p, float* ap, CgScalars* sc, ReduceBuf red, const uint8_t* wet);
+                  const float* zv, float* p, float* ap, CgScalars* sc, ReduceBuf red, const uint16_t* wet);
 void rec_col_update(std::vector<MRec>& out, const GridDev& g, const float* p, const float* ap, float* x, float* r,
-                    CgScalars* sc, ReduceBuf red, int identity, const uint8_t* wet);
+                    CgScalars* sc, ReduceBuf red, int identity, const uint16_t* wet);
 void rec_refine_true(std::vector<MRec>& out, const GridDev& g, const float scale[3], const uint16_t* codes,
                      const float* xcorr, double* x64, const float* b, float* r, int mode, ReduceBuf red,
-                     double* out2);
+                     double* out2, const uint16_t* wet);
 void rec_mg_smooth(std::vector<MRec>& out, const MgDims& l, const uint16_t* code, const float* b, const float* xi,
                    float* xo, float omega, CgScalars* sc, ReduceBuf red, int first, int with_rz);
 void rec_mg_smooth2_first(std::vector<MRec>& out, const MgDims& l, const uint16_t* code, const float* b, float* xo,
@@ -507,7 +508,7 @@ size_t finish_arg_bytes();
 void finish_set_target(unsigned char* args, double abs_target2);
 void rec_gather(std::vector<MRec>& out, const CgScalars* sc, const double* out2, CgScalars* dst_sc, double* dst2);
 void rec_codes(std::vector<MRec>& out, int nx, int ny, int nz, const uint8_t* markers, uint16_t* codes);
-void rec_flat_wet(std::vector<MRec>& out, const GridDev& g, const uint16_t* codes, uint8_t* wet);
+void rec_flat_wet(std::vector<MRec>& out, const GridDev& g, const uint16_t* codes, uint16_t* wet);
 void rec_mg_coarsen(std::vector<MRec>& out, const MgDims& f, const MgDims& c, const uint8_t* mf, uint8_t* mc,
                     int fluid_first);
 void rec_mg_march_wet(std::vector<MRec>& out, const MgDims& f, const MgDims& c, const uint16_t* code,

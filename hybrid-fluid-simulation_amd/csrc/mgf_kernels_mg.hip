@@ -157,6 +157,51 @@ __device__ __forceinline__ void nbrs(uint32_t c, const Flat& F, uint32_t (&j)[6]
     j[5] = c + F.sz <= last ? c + F.sz : last;
 }
 
+// p[c] by a 32-bit byte offset from the (uniform) pointer: no 64-bit address
+// per work-item.  flat_inner's blocks only.
+template <class T>
+__device__ __forceinline__ T ld32(const T* p, uint32_t c) {
+    return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(p) + c * uint32_t(sizeof(T)));
+}
+template <class T>
+__device__ __forceinline__ void st32(T* p, uint32_t c, T v) {
+    *reinterpret_cast<T*>(reinterpret_cast<char*>(p) + c * uint32_t(sizeof(T))) = v;
+}
+
+// Whether all cells b0 .. b0 + count - 1 and their six neighbours are in the
+// grid and have byte offsets (of doubles) within 32 bits: then nothing is
+// clamped and a neighbour is the same offset from a shifted pointer.
+__device__ __forceinline__ bool flat_inner(const Flat& F, uint32_t b0, uint32_t count) {
+    return F.n <= (1u << 29) && b0 >= F.sz && uint64_t(b0) + count + F.sz <= F.n;
+}
+
+// The cell's value and its neighbours'.
+template <bool CHECK, class T>
+__device__ __forceinline__ void ld_star(const Flat& F, const T* __restrict__ v, uint32_t c, T& vc, T (&vn)[6]) {
+    if (CHECK) {
+        uint32_t j[6];
+        nbrs(c, F, j);
+        vc = v[c];
+#pragma unroll
+        for (int m = 0; m < 6; ++m) vn[m] = v[j[m]];
+    } else {
+        vc = ld32(v, c);
+        vn[0] = ld32(v - 1, c);
+        vn[1] = ld32(v + 1, c);
+        vn[2] = ld32(v - F.sy, c);
+        vn[3] = ld32(v + F.sy, c);
+        vn[4] = ld32(v - F.sz, c);
+        vn[5] = ld32(v + F.sz, c);
+    }
+}
+template <bool CHECK, class T>
+__device__ __forceinline__ T ld_cell(const T* p, uint32_t c) { return CHECK ? p[c] : ld32(p, c); }
+template <bool CHECK, class T>
+__device__ __forceinline__ void st_cell(T* p, uint32_t c, T v) {
+    if (CHECK) p[c] = v;
+    else st32(p, c, v);
+}
+
 // Block sum of one double, stored to part[slot] by thread 0.
 __device__ __forceinline__ void block_partial(double v, double* part, uint32_t slot) {
     double a[1] = {v};
@@ -180,78 +225,100 @@ constexpr int kCpt = 4;
 
 // ---------------------------------------------------------------------------
 // Fused CG.  Each work-item handles kCpt cells 256 apart: first all loads of
-// its cells, then the arithmetic and the stores.  Only the last block can
-// hold cells past the end; the others run the body without the range test
-// (a block-uniform branch), so nothing stands between the loads.
-#define MGF_CELLS(CHECK, F, base)                                                  \
+// its cells, then the arithmetic and the stores.  The blocks of the first and
+// last planes can hold cells or neighbours past an end; the others run the body
+// without range tests and clamps (flat_inner, a block-uniform branch), so
+// nothing stands between the loads.
+#define MGF_CELLS(CHECK, F, base, rounds)                                          \
     uint32_t cidx[kCpt];                                                           \
     _Pragma("unroll") for (int k = 0; k < kCpt; ++k) {                             \
-        const uint32_t c_ = (base) + uint32_t(k) * kBlock;                         \
+        const uint32_t c_ = (base) + seg_from(rounds, k) * kBlock;                 \
         cidx[k] = (CHECK && c_ >= (F).n) ? (F).n - 1 : c_;                         \
     }
+
+// The 64-cell segments of the flat CG kernels' blocks (kBlock * kCpt
+// consecutive cells each) that hold fluid: bit k of wet[block] is cells
+// [64 k, 64 (k + 1)) of the block, wave k % 4's cells of round k / 4.  On
+// non-fluid cells b = 0, so r and x stay +0, z = M^-1 r is 0, and from the
+// first K_I of a sweep on p and Ap are +0 too: a dry segment would store the
+// values its cells hold and add +0 to the dot products, so K_I (after the
+// first iteration), K_II and the refinement (after the sweep start has cleared
+// x64) leave it out.  Segments and not whole blocks, since 1024 cells are
+// several rows of a grid whose fluid takes part of each row: 512^3 scene, K_II
+// 485 -> 360 us, K_I 538 -> 441 us, the refinement's residual 778 -> 601 us.
+constexpr uint32_t kSegAll = 0xffffu, kSegWave = 0x1111u;
+static_assert(kBlock == 256 && kCpt == 4, "a block's segments are a 16-bit mask");
+
+__device__ __forceinline__ void k_flat_wet_run(Flat F, const uint16_t* __restrict__ code,
+                                                     uint16_t* __restrict__ wet, uint32_t blk) {
+    __shared__ uint32_t m;
+    if (threadIdx.x == 0) m = 0;
+    __syncthreads();
+    const uint32_t b0 = blk * (kBlock * kCpt);
+    uint32_t bits = 0;
+#pragma unroll
+    for (int k = 0; k < kCpt; ++k) {
+        const uint32_t c = b0 + threadIdx.x + uint32_t(k) * kBlock;
+        if (__ballot(c < F.n && (code[c] & kCodeFluid))) bits |= 1u << (4 * k + int(threadIdx.x >> 6));
+    }
+    if ((threadIdx.x & 63) == 0) atomicOr(&m, bits);
+    __syncthreads();
+    if (threadIdx.x == 0) wet[blk] = uint16_t(m);
+}
+
+// The calling wave's rounds of a block's mask: bit 4 k is its segment of
+// round k (the same for the whole wave).  A round left out loads the cells of
+// the wave's first round again, which costs no traffic, rather than branch:
+// the loads of all rounds stay in flight together (with branches K_I waited
+// for each round's codes, 538 -> 493 us at 512^3 instead of 441).
+__device__ __forceinline__ uint32_t seg_rounds(uint32_t mask) {
+    return uint32_t(__builtin_amdgcn_readfirstlane(int(mask >> (threadIdx.x >> 6))));
+}
+#define MGF_SEG_ON(rounds, k) (((rounds) >> (4 * (k))) & 1u)
+__device__ __forceinline__ uint32_t seg_from(uint32_t rounds, int k) {
+    return MGF_SEG_ON(rounds, k) ? uint32_t(k) : uint32_t(__ffs(int(rounds & kSegWave)) - 1) >> 2;
+}
 
 // K_I: Az = A z (the stencil), then in place p = z + beta p and
 // Ap = Az + beta Ap (p = z, Ap = Az on the first iteration); block partials
 // of p . Ap.  Only z is read at the neighbours, so p and Ap are updated in
 // place without a race.
-template <bool CHECK>
+template <bool CHECK, bool FIRST>
 __device__ __forceinline__ double cg_pap_body(const Flat& F, uint32_t base, const uint16_t* __restrict__ code,
                                               float sx, float sy, float sz, const float* __restrict__ zv,
                                               float* __restrict__ p, float* __restrict__ ap, float beta,
-                                              bool first, const float* aw) {
-    MGF_CELLS(CHECK, F, base)
+                                              const float* aw, uint32_t rounds) {
+    MGF_CELLS(CHECK, F, base, rounds)
     uint16_t cd[kCpt];
     float zc[kCpt], zn[kCpt][6], pc[kCpt], apc[kCpt];
 #pragma unroll
     for (int k = 0; k < kCpt; ++k) {
-        uint32_t j[6];
-        nbrs(cidx[k], F, j);
-        cd[k] = code[cidx[k]];
-        zc[k] = zv[cidx[k]];
-#pragma unroll
-        for (int m = 0; m < 6; ++m) zn[k][m] = zv[j[m]];
-        if (!first) {
-            pc[k] = p[cidx[k]];
-            apc[k] = ap[cidx[k]];
+        cd[k] = ld_cell<CHECK>(code, cidx[k]);
+        ld_star<CHECK>(F, zv, cidx[k], zc[k], zn[k]);
+        if (!FIRST) {
+            pc[k] = ld_cell<CHECK>(p, cidx[k]);
+            apc[k] = ld_cell<CHECK>(ap, cidx[k]);
         }
     }
     double acc = 0.0;
 #pragma unroll
     for (int k = 0; k < kCpt; ++k) {
+        if (!MGF_SEG_ON(rounds, k)) continue;
         const float az = arow(cd[k], zc[k], zn[k], sx, sy, sz, aw);
-        const float pn = first ? zc[k] : __builtin_fmaf(beta, pc[k], zc[k]);
-        const float an = first ? az : __builtin_fmaf(beta, apc[k], az);
+        const float pn = FIRST ? zc[k] : __builtin_fmaf(beta, pc[k], zc[k]);
+        const float an = FIRST ? az : __builtin_fmaf(beta, apc[k], az);
         const uint32_t c = base + uint32_t(k) * kBlock;
         if (!CHECK || c < F.n) {
-            p[c] = pn;
-            ap[c] = an;
+            st_cell<CHECK>(p, c, pn);
+            st_cell<CHECK>(ap, c, an);
             acc += double(pn) * double(an);
         }
     }
     return acc;
 }
 
-// Blocks of the flat CG kernels (kBlock * kCpt consecutive cells each) that
-// hold no fluid cell (wet[block] == 0).  On non-fluid cells b = 0, so r and
-// x stay +0, z = M^-1 r is 0, and from the first K_I of a sweep on p and Ap
-// are +0 too: such a block would store the values its cells hold and add +0
-// to the dot products, so K_I (after the first iteration) and K_II return at
-// once with a zero partial.
-__device__ __forceinline__ void k_flat_wet_run(Flat F, const uint16_t* __restrict__ code,
-                                                     uint8_t* __restrict__ wet, uint32_t blk) {
-        const uint32_t b0 = blk * (kBlock * kCpt);
-    int any = 0;
-#pragma unroll
-    for (int k = 0; k < kCpt; ++k) {
-        const uint32_t c = b0 + threadIdx.x + uint32_t(k) * kBlock;
-        if (c < F.n) any |= code[c] & kCodeFluid;
-    }
-    any = __syncthreads_or(any);
-    if (threadIdx.x == 0) wet[blk] = uint8_t(any != 0);
-}
-
 __global__ void __launch_bounds__(kBlock) k_flat_wet(Flat F, const uint16_t* __restrict__ code,
-                                                     uint8_t* __restrict__ wet) {
+                                                     uint16_t* __restrict__ wet) {
     k_flat_wet_run(F, code, wet, xcd_block());
 }
 
@@ -259,7 +326,7 @@ struct MFlatWet {
     static constexpr int kThreads = kBlock;
     Flat F;
     const uint16_t* code;
-    uint8_t* wet;
+    uint16_t* wet;
     uint32_t G;
     __device__ void run(uint32_t vb) const { k_flat_wet_run(F, code, wet, xcd_of(vb, G)); }
 };
@@ -269,29 +336,40 @@ struct MFlatWet {
 __device__ __forceinline__ void cg_pap_run(Flat F, const uint16_t* __restrict__ code, float sx, float sy, float sz,
                                            const float* __restrict__ zv, float* __restrict__ p,
                                            float* __restrict__ ap, const CgScalars* __restrict__ sc,
-                                           double* __restrict__ part, const uint8_t* __restrict__ wet, uint32_t blk,
+                                           double* __restrict__ part, const uint16_t* __restrict__ wet, uint32_t blk,
                                            uint32_t slot) {
     __shared__ float aw[64];
     if (sc->done) return;
     const bool first = sc->iters == 0;
-    if (!first && wet && !wet[blk]) {
+    const uint32_t mask = (!first && wet) ? wet[blk] : kSegAll;
+    if (!mask) {
         if (threadIdx.x == 0) part[slot] = 0.0;
         return;
     }
+    const uint32_t rounds = seg_rounds(mask);
     build_tables<false>(aw, nullptr, sx, sy, sz, 0.0f);
     const float beta = float(sc->beta);
     const uint32_t b0 = blk * (kBlock * kCpt);
     const uint32_t base = b0 + threadIdx.x;
-    const double acc = (b0 + kBlock * kCpt <= F.n)
-                           ? cg_pap_body<false>(F, base, code, sx, sy, sz, zv, p, ap, beta, first, aw)
-                           : cg_pap_body<true>(F, base, code, sx, sy, sz, zv, p, ap, beta, first, aw);
+    // first is a template parameter: a branch on it between the loads makes
+    // them wait for one another
+    const bool inner = flat_inner(F, b0, kBlock * kCpt);
+    double acc = 0.0;
+    if (!(rounds & kSegWave)) {
+    } else if (first) {
+        acc = inner ? cg_pap_body<false, true>(F, base, code, sx, sy, sz, zv, p, ap, beta, aw, rounds)
+                    : cg_pap_body<true, true>(F, base, code, sx, sy, sz, zv, p, ap, beta, aw, rounds);
+    } else {
+        acc = inner ? cg_pap_body<false, false>(F, base, code, sx, sy, sz, zv, p, ap, beta, aw, rounds)
+                    : cg_pap_body<true, false>(F, base, code, sx, sy, sz, zv, p, ap, beta, aw, rounds);
+    }
     block_partial(acc, part, slot);
 }
 
 __global__ void __launch_bounds__(kBlock) k_cg_pap(Flat F, const uint16_t* __restrict__ code, float sx, float sy,
                                                    float sz, const float* __restrict__ zv, float* __restrict__ p,
                                                    float* __restrict__ ap, const CgScalars* __restrict__ sc,
-                                                   double* __restrict__ part, const uint8_t* __restrict__ wet) {
+                                                   double* __restrict__ part, const uint16_t* __restrict__ wet) {
     cg_pap_run(F, code, sx, sy, sz, zv, p, ap, sc, part, wet, xcd_block(), blockIdx.x);
 }
 
@@ -304,7 +382,7 @@ struct MPap {
     float *p, *ap;
     const CgScalars* sc;
     double* part;
-    const uint8_t* wet;
+    const uint16_t* wet;
     uint32_t G;
     __device__ void run(uint32_t b) const { cg_pap_run(F, code, sx, sy, sz, zv, p, ap, sc, part, wet, xcd_of(b, G), b); }
 };
@@ -314,25 +392,26 @@ struct MPap {
 template <bool CHECK>
 __device__ __forceinline__ double cg_update_body(const Flat& F, uint32_t base, const float* __restrict__ p,
                                                  const float* __restrict__ ap, float* __restrict__ x,
-                                                 float* __restrict__ r, double alpha) {
-    MGF_CELLS(CHECK, F, base)
+                                                 float* __restrict__ r, double alpha, uint32_t rounds) {
+    MGF_CELLS(CHECK, F, base, rounds)
     float pc[kCpt], ac[kCpt], x0[kCpt], r0[kCpt];
 #pragma unroll
     for (int k = 0; k < kCpt; ++k) {
-        pc[k] = p[cidx[k]];
-        ac[k] = ap[cidx[k]];
-        x0[k] = x[cidx[k]];
-        r0[k] = r[cidx[k]];
+        pc[k] = ld_cell<CHECK>(p, cidx[k]);
+        ac[k] = ld_cell<CHECK>(ap, cidx[k]);
+        x0[k] = ld_cell<CHECK>(x, cidx[k]);
+        r0[k] = ld_cell<CHECK>(r, cidx[k]);
     }
     double acc = 0.0;
 #pragma unroll
     for (int k = 0; k < kCpt; ++k) {
+        if (!MGF_SEG_ON(rounds, k)) continue;
         const float xn = float(__builtin_fma(alpha, double(pc[k]), double(x0[k])));
         const float rn = float(__builtin_fma(-alpha, double(ac[k]), double(r0[k])));
         const uint32_t c = base + uint32_t(k) * kBlock;
         if (!CHECK || c < F.n) {
-            x[c] = xn;
-            r[c] = rn;
+            st_cell<CHECK>(x, c, xn);
+            st_cell<CHECK>(r, c, rn);
             acc += double(rn) * double(rn);
         }
     }
@@ -342,24 +421,28 @@ __device__ __forceinline__ double cg_update_body(const Flat& F, uint32_t base, c
 __device__ __forceinline__ void cg_update_run(Flat F, const float* __restrict__ p, const float* __restrict__ ap,
                                               float* __restrict__ x, float* __restrict__ r,
                                               const CgScalars* __restrict__ sc, double* __restrict__ part,
-                                              const uint8_t* __restrict__ wet, uint32_t blk, uint32_t slot) {
+                                              const uint16_t* __restrict__ wet, uint32_t blk, uint32_t slot) {
     if (sc->done) return;
-    if (wet && !wet[blk]) {
+    const uint32_t mask = wet ? wet[blk] : kSegAll;
+    if (!mask) {
         if (threadIdx.x == 0) part[slot] = 0.0;
         return;
     }
+    const uint32_t rounds = seg_rounds(mask);
     const double alpha = sc->alpha;
     const uint32_t b0 = blk * (kBlock * kCpt);
     const uint32_t base = b0 + threadIdx.x;
-    const double acc = (b0 + kBlock * kCpt <= F.n) ? cg_update_body<false>(F, base, p, ap, x, r, alpha)
-                                                   : cg_update_body<true>(F, base, p, ap, x, r, alpha);
+    double acc = 0.0;
+    if (rounds & kSegWave)
+        acc = flat_inner(F, b0, kBlock * kCpt) ? cg_update_body<false>(F, base, p, ap, x, r, alpha, rounds)
+                                               : cg_update_body<true>(F, base, p, ap, x, r, alpha, rounds);
     block_partial(acc, part, slot);
 }
 
 __global__ void __launch_bounds__(kBlock) k_cg_update(Flat F, const float* __restrict__ p,
                                                       const float* __restrict__ ap, float* __restrict__ x,
                                                       float* __restrict__ r, const CgScalars* __restrict__ sc,
-                                                      double* __restrict__ part, const uint8_t* __restrict__ wet) {
+                                                      double* __restrict__ part, const uint16_t* __restrict__ wet) {
     cg_update_run(F, p, ap, x, r, sc, part, wet, xcd_block(), blockIdx.x);
 }
 
@@ -370,7 +453,7 @@ struct MUpdate {
     float *x, *r;
     const CgScalars* sc;
     double* part;
-    const uint8_t* wet;
+    const uint16_t* wet;
     uint32_t G;
     __device__ void run(uint32_t b) const { cg_update_run(F, p, ap, x, r, sc, part, wet, xcd_of(b, G), b); }
 };
@@ -396,37 +479,29 @@ template <int MODE, bool CHECK>
 __device__ __forceinline__ void refine_body(const Flat& F, uint32_t base, const uint16_t* __restrict__ code,
                                             float sx, float sy, float sz, const float* __restrict__ xc,
                                             double* __restrict__ x64, const float* __restrict__ b,
-                                            float* __restrict__ r, const float* aw, double& rr, double& bb) {
-    MGF_CELLS(CHECK, F, base)
+                                            float* __restrict__ r, const float* aw, uint32_t rounds, double& rr,
+                                            double& bb) {
+    MGF_CELLS(CHECK, F, base, rounds)
     constexpr int K = kCpt;
     uint16_t cd[K];
     float bc[K], xcc[K], xcn[K][6];
     double xo[K], xon[K][6];
 #pragma unroll
     for (int k = 0; k < K; ++k) {
-        bc[k] = b[cidx[k]];
+        bc[k] = ld_cell<CHECK>(b, cidx[k]);
         if (MODE != 0) {
-            uint32_t j[6];
-            nbrs(cidx[k], F, j);
-            cd[k] = code[cidx[k]];
-            if (MODE == 1) {
-                xcc[k] = xc[cidx[k]];
-#pragma unroll
-                for (int m = 0; m < 6; ++m) xcn[k][m] = xc[j[m]];
-            } else {
-                xo[k] = x64[cidx[k]];
-#pragma unroll
-                for (int m = 0; m < 6; ++m) xon[k][m] = x64[j[m]];
-            }
+            cd[k] = ld_cell<CHECK>(code, cidx[k]);
+            if (MODE == 1) ld_star<CHECK>(F, xc, cidx[k], xcc[k], xcn[k]);
+            else ld_star<CHECK, double>(F, x64, cidx[k], xo[k], xon[k]);
         }
     }
 #pragma unroll
     for (int k = 0; k < K; ++k) {
         const uint32_t c = base + uint32_t(k) * kBlock;
-        if (CHECK && c >= F.n) continue;
+        if (!MGF_SEG_ON(rounds, k) || (CHECK && c >= F.n)) continue;
         bb += double(bc[k]) * double(bc[k]);
         if (MODE == 0) {
-            x64[c] = 0.0;
+            st_cell<CHECK>(x64, c, 0.0);
             continue;
         }
         double vc, v[6];
@@ -434,7 +509,7 @@ __device__ __forceinline__ void refine_body(const Flat& F, uint32_t base, const 
             vc = double(xcc[k]);
 #pragma unroll
             for (int m = 0; m < 6; ++m) v[m] = double(xcn[k][m]);
-            x64[c] = vc;
+            st_cell<CHECK>(x64, c, vc);
         } else {
             vc = xo[k];
 #pragma unroll
@@ -447,7 +522,7 @@ __device__ __forceinline__ void refine_body(const Flat& F, uint32_t base, const 
             }
         }
         const double res = double(bc[k]) - arow64(cd[k], vc, v, sx, sy, sz, aw);
-        if (r) r[c] = float(res);
+        if (r) st_cell<CHECK>(r, c, float(res));
         rr += res * res;
     }
 }
@@ -456,16 +531,24 @@ template <int MODE>
 __device__ __forceinline__ void refine_run(Flat F, const uint16_t* __restrict__ code, float sx, float sy, float sz,
                                            const float* __restrict__ xc, double* __restrict__ x64,
                                            const float* __restrict__ b, float* __restrict__ r,
-                                           double* __restrict__ part, uint32_t blk, uint32_t slot) {
+                                           double* __restrict__ part, const uint16_t* __restrict__ wet, uint32_t blk,
+                                           uint32_t slot) {
     __shared__ float aw[64];
+    const uint32_t mask = ((MODE == 1 || MODE == 2) && wet) ? wet[blk] : kSegAll;
+    if (!mask) {
+        if (threadIdx.x == 0) part[2 * size_t(slot)] = part[2 * size_t(slot) + 1] = 0.0;
+        return;
+    }
+    const uint32_t rounds = seg_rounds(mask);
     build_tables<false>(aw, nullptr, sx, sy, sz, 0.0f);
     const uint32_t b0 = blk * (kBlock * kCpt);
     const uint32_t base = b0 + threadIdx.x;
     double v[2] = {0.0, 0.0};
-    if (b0 + kBlock * kCpt <= F.n)
-        refine_body<MODE, false>(F, base, code, sx, sy, sz, xc, x64, b, r, aw, v[0], v[1]);
+    if (!(rounds & kSegWave)) {
+    } else if (flat_inner(F, b0, kBlock * kCpt))
+        refine_body<MODE, false>(F, base, code, sx, sy, sz, xc, x64, b, r, aw, rounds, v[0], v[1]);
     else
-        refine_body<MODE, true>(F, base, code, sx, sy, sz, xc, x64, b, r, aw, v[0], v[1]);
+        refine_body<MODE, true>(F, base, code, sx, sy, sz, xc, x64, b, r, aw, rounds, v[0], v[1]);
     block_sum<2>(v);
     if (threadIdx.x == 0) {
         part[2 * size_t(slot)] = v[0];
@@ -477,8 +560,8 @@ template <int MODE>
 __global__ void __launch_bounds__(kBlock) k_refine(Flat F, const uint16_t* __restrict__ code, float sx, float sy,
                                                    float sz, const float* __restrict__ xc, double* __restrict__ x64,
                                                    const float* __restrict__ b, float* __restrict__ r,
-                                                   double* __restrict__ part) {
-    refine_run<MODE>(F, code, sx, sy, sz, xc, x64, b, r, part, xcd_block(), blockIdx.x);
+                                                   double* __restrict__ part, const uint16_t* __restrict__ wet) {
+    refine_run<MODE>(F, code, sx, sy, sz, xc, x64, b, r, part, wet, xcd_block(), blockIdx.x);
 }
 
 template <int MODE>
@@ -492,37 +575,64 @@ struct MRefine {
     const float* b;
     float* r;
     double* part;
+    const uint16_t* wet;
     uint32_t G;
     __device__ void run(uint32_t blk) const {
-        refine_run<MODE>(F, code, sx, sy, sz, xc, x64, b, r, part, xcd_of(blk, G), blk);
+        refine_run<MODE>(F, code, sx, sy, sz, xc, x64, b, r, part, wet, xcd_of(blk, G), blk);
     }
 };
 
-// x64 += xc, pointwise.
-__device__ __forceinline__ void acc64_run(uint32_t n, const float* __restrict__ xc, double* __restrict__ x64,
-                                          uint32_t blk) {
-    const uint32_t i = blk * kBlock + threadIdx.x;
-    if (i < n) x64[i] = x64[i] + double(xc[i]);
+// x64 += xc, pointwise, on the segments with fluid (x64 and xc are 0 elsewhere).
+template <bool CHECK>
+__device__ __forceinline__ void acc64_body(const Flat& F, uint32_t base, const float* __restrict__ xc,
+                                           double* __restrict__ x64, uint32_t rounds) {
+    MGF_CELLS(CHECK, F, base, rounds)
+    float xv[kCpt];
+    double xo[kCpt];
+#pragma unroll
+    for (int k = 0; k < kCpt; ++k) {
+        xv[k] = ld_cell<CHECK>(xc, cidx[k]);
+        xo[k] = ld_cell<CHECK, double>(x64, cidx[k]);
+    }
+#pragma unroll
+    for (int k = 0; k < kCpt; ++k) {
+        const uint32_t c = base + uint32_t(k) * kBlock;
+        if (!MGF_SEG_ON(rounds, k) || (CHECK && c >= F.n)) continue;
+        st_cell<CHECK>(x64, c, xo[k] + double(xv[k]));
+    }
 }
 
-__global__ void __launch_bounds__(kBlock) k_acc64(uint32_t n, const float* __restrict__ xc, double* __restrict__ x64) {
-    acc64_run(n, xc, x64, xcd_block());
+__device__ __forceinline__ void acc64_run(Flat F, const float* __restrict__ xc, double* __restrict__ x64,
+                                          const uint16_t* __restrict__ wet, uint32_t blk) {
+    const uint32_t mask = wet ? wet[blk] : kSegAll;
+    if (!mask) return;
+    const uint32_t rounds = seg_rounds(mask);
+    if (!(rounds & kSegWave)) return;
+    const uint32_t b0 = blk * (kBlock * kCpt);
+    if (flat_inner(F, b0, kBlock * kCpt)) acc64_body<false>(F, b0 + threadIdx.x, xc, x64, rounds);
+    else acc64_body<true>(F, b0 + threadIdx.x, xc, x64, rounds);
+}
+
+__global__ void __launch_bounds__(kBlock) k_acc64(Flat F, const float* __restrict__ xc, double* __restrict__ x64,
+                                                  const uint16_t* __restrict__ wet) {
+    acc64_run(F, xc, x64, wet, xcd_block());
 }
 
 struct MAcc64 {
     static constexpr int kThreads = kBlock;
-    uint32_t n;
+    Flat F;
     const float* xc;
     double* x64;
+    const uint16_t* wet;
     uint32_t G;
-    __device__ void run(uint32_t b) const { acc64_run(n, xc, x64, xcd_of(b, G)); }
+    __device__ void run(uint32_t b) const { acc64_run(F, xc, x64, wet, xcd_of(b, G)); }
 };
 
 // Start of an inner sweep: r = rsrc (when distinct), x = 0; partials of r.r.
 template <bool CHECK>
 __device__ __forceinline__ double start_body(const Flat& F, uint32_t base, const float* __restrict__ rsrc,
                                              float* __restrict__ r, float* __restrict__ x) {
-    MGF_CELLS(CHECK, F, base)
+    MGF_CELLS(CHECK, F, base, kSegAll)
     float v[kCpt];
 #pragma unroll
     for (int k = 0; k < kCpt; ++k) v[k] = rsrc[cidx[k]];
@@ -788,7 +898,7 @@ __device__ __forceinline__ double smooth_body(const Flat& F, const MgLevel& L, u
                                               const uint16_t* __restrict__ code, const float* __restrict__ b,
                                               const float* __restrict__ xi, float* __restrict__ xo,
                                               const float* aw, const float* w) {
-    MGF_CELLS(CHECK, F, base)
+    MGF_CELLS(CHECK, F, base, kSegAll)
     uint16_t cd[kCpt];
     float bc[kCpt], vc[kCpt], vn[kCpt][6];
 #pragma unroll
@@ -871,7 +981,7 @@ template <bool CHECK>
 __device__ __forceinline__ double smooth2_body(const Flat& F, const MgLevel& L, uint32_t base,
                                                const uint16_t* __restrict__ code, const float* __restrict__ b,
                                                float* __restrict__ xo, const float* aw, const float* w) {
-    MGF_CELLS(CHECK, F, base)
+    MGF_CELLS(CHECK, F, base, kSegAll)
     uint16_t cd[kCpt], cn[kCpt][6];
     float bc[kCpt], bn[kCpt][6];
 #pragma unroll
@@ -961,7 +1071,7 @@ __device__ __forceinline__ double smooth_prolong_body(const Flat& F, const MgLev
                                                       const float* __restrict__ b, const float* __restrict__ xi,
                                                       const float* __restrict__ xc, float* __restrict__ xo,
                                                       const float* aw, const float* w) {
-    MGF_CELLS(CHECK, F, base)
+    MGF_CELLS(CHECK, F, base, kSegAll)
     uint16_t cd[kCpt];
     float bc[kCpt], vc[kCpt], vn[kCpt][6];
     const uint32_t nx = uint32_t(L.nx), ny = uint32_t(L.ny), nz = uint32_t(L.nz);
@@ -2481,20 +2591,20 @@ hipError_t launch_cg_start(hipStream_t s, const GridDev& g, const float* rsrc, f
 
 hipError_t launch_refine_true(hipStream_t s, const GridDev& g, const float scale[3], const uint16_t* codes,
                               const float* xcorr, double* x64, const float* b, float* r, int mode, ReduceBuf red,
-                              double* out2) {
+                              double* out2, const uint16_t* wet) {
     const Flat F = make_flat(g.nx, g.ny, g.nz);
     const uint32_t G = flat_grid(F.n);
     hipError_t e;
     if (mode == 0)
-        e = LAUNCH(k_refine<0>, G, F, codes, scale[0], scale[1], scale[2], xcorr, x64, b, r, red.partials);
+        e = LAUNCH(k_refine<0>, G, F, codes, scale[0], scale[1], scale[2], xcorr, x64, b, r, red.partials, wet);
     else if (mode == 3)
-        e = LAUNCH(k_refine<3>, G, F, codes, scale[0], scale[1], scale[2], xcorr, x64, b, r, red.partials);
+        e = LAUNCH(k_refine<3>, G, F, codes, scale[0], scale[1], scale[2], xcorr, x64, b, r, red.partials, wet);
     else if (mode == 1)
-        e = LAUNCH(k_refine<1>, G, F, codes, scale[0], scale[1], scale[2], xcorr, x64, b, r, red.partials);
+        e = LAUNCH(k_refine<1>, G, F, codes, scale[0], scale[1], scale[2], xcorr, x64, b, r, red.partials, wet);
     else {
-        e = LAUNCH(k_acc64, grid_for(F.n), F.n, xcorr, x64);
+        e = LAUNCH(k_acc64, G, F, xcorr, x64, wet);
         if (e != hipSuccess) return e;
-        e = LAUNCH(k_refine<2>, G, F, codes, scale[0], scale[1], scale[2], xcorr, x64, b, r, red.partials);
+        e = LAUNCH(k_refine<2>, G, F, codes, scale[0], scale[1], scale[2], xcorr, x64, b, r, red.partials, wet);
     }
     if (e != hipSuccess) return e;
     (void)launch_dims(k_sum2, "k_sum2", dim3(1), dim3(1024), 0, s, red.partials, G, out2);
@@ -2513,23 +2623,24 @@ hipError_t launch_div_check(hipStream_t s, const GridDev& g, const uint8_t* mark
     return launch_dims(k_div_fold, "k_div_fold", dim3(1), dim3(64), 0u, s, (const double*)(out + 1), out);
 }
 
-double flat_wet_cells(const GridDev& g, const uint8_t* wet_host) {
+double flat_wet_cells(const GridDev& g, const uint16_t* wet_host) {
     const Flat F = make_flat(g.nx, g.ny, g.nz);
     const uint32_t per = uint32_t(kBlock * kCpt), nb = (F.n + per - 1) / per;
     double cells = 0.0;
     for (uint32_t b = 0; b < nb; ++b)
-        if (wet_host[b]) cells += double(std::min(per, F.n - b * per));
+        for (uint32_t k = 0; k < per / 64; ++k)
+            if ((wet_host[b] >> k) & 1) cells += double(std::min(64u, F.n - b * per - 64u * k));
     return cells;
 }
 
-hipError_t launch_flat_wet(hipStream_t s, const GridDev& g, const uint16_t* codes, uint8_t* wet) {
+hipError_t launch_flat_wet(hipStream_t s, const GridDev& g, const uint16_t* codes, uint16_t* wet) {
     if (!wet || !codes) return hipErrorInvalidValue;
     const Flat F = make_flat(g.nx, g.ny, g.nz);
     return LAUNCH(k_flat_wet, flat_grid(F.n), F, codes, wet);
 }
 
 hipError_t launch_col_p_ap(hipStream_t s, const GridDev& g, const float scale[3], const uint16_t* codes,
-                           const float* zv, float* p, float* ap, CgScalars* sc, ReduceBuf red, const uint8_t* wet) {
+                           const float* zv, float* p, float* ap, CgScalars* sc, ReduceBuf red, const uint16_t* wet) {
     const Flat F = make_flat(g.nx, g.ny, g.nz);
     const uint32_t G = flat_grid(F.n);
     hipError_t e = LAUNCH(k_cg_pap, G, F, codes, scale[0], scale[1], scale[2], zv, p, ap, sc, red.partials, wet);
@@ -2538,7 +2649,7 @@ hipError_t launch_col_p_ap(hipStream_t s, const GridDev& g, const float scale[3]
 }
 
 hipError_t launch_col_update(hipStream_t s, const GridDev& g, const float* p, const float* ap, float* x, float* r,
-                             CgScalars* sc, ReduceBuf red, int identity, const uint8_t* wet) {
+                             CgScalars* sc, ReduceBuf red, int identity, const uint16_t* wet) {
     const Flat F = make_flat(g.nx, g.ny, g.nz);
     const uint32_t G = flat_grid(F.n);
     hipError_t e = LAUNCH(k_cg_update, G, F, p, ap, x, r, sc, red.partials, wet);
@@ -2846,7 +2957,7 @@ void rec_cg_start(std::vector<MRec>& out, const GridDev& g, const float* rsrc, f
 }
 
 void rec_col_p_ap(std::vector<MRec>& out, const GridDev& g, const float scale[3], const uint16_t* codes,
-                  const float* zv, float* p, float* ap, CgScalars* sc, ReduceBuf red, const uint8_t* wet) {
+                  const float* zv, float* p, float* ap, CgScalars* sc, ReduceBuf red, const uint16_t* wet) {
     const Flat F = make_flat(g.nx, g.ny, g.nz);
     const uint32_t G = flat_grid(F.n);
     push_rec(out, kMkPap, MPap{F, codes, scale[0], scale[1], scale[2], zv, p, ap, sc, red.partials, wet, G}, G);
@@ -2854,7 +2965,7 @@ void rec_col_p_ap(std::vector<MRec>& out, const GridDev& g, const float scale[3]
 }
 
 void rec_col_update(std::vector<MRec>& out, const GridDev& g, const float* p, const float* ap, float* x, float* r,
-                    CgScalars* sc, ReduceBuf red, int identity, const uint8_t* wet) {
+                    CgScalars* sc, ReduceBuf red, int identity, const uint16_t* wet) {
     const Flat F = make_flat(g.nx, g.ny, g.nz);
     const uint32_t G = flat_grid(F.n);
     push_rec(out, kMkUpdate, MUpdate{F, p, ap, x, r, sc, red.partials, wet, G}, G);
@@ -2863,20 +2974,19 @@ void rec_col_update(std::vector<MRec>& out, const GridDev& g, const float* p, co
 
 void rec_refine_true(std::vector<MRec>& out, const GridDev& g, const float scale[3], const uint16_t* codes,
                      const float* xcorr, double* x64, const float* b, float* r, int mode, ReduceBuf red,
-                     double* out2) {
+                     double* out2, const uint16_t* wet) {
     const Flat F = make_flat(g.nx, g.ny, g.nz);
     const uint32_t G = flat_grid(F.n);
     if (mode == 0) {
-        push_rec(out, kMkRefine0, MRefine<0>{F, codes, scale[0], scale[1], scale[2], xcorr, x64, b, r, red.partials, G},
-                 G);
+        push_rec(out, kMkRefine0,
+                 MRefine<0>{F, codes, scale[0], scale[1], scale[2], xcorr, x64, b, r, red.partials, wet, G}, G);
     } else if (mode == 1) {
-        push_rec(out, kMkRefine1, MRefine<1>{F, codes, scale[0], scale[1], scale[2], xcorr, x64, b, r, red.partials, G},
-                 G);
+        push_rec(out, kMkRefine1,
+                 MRefine<1>{F, codes, scale[0], scale[1], scale[2], xcorr, x64, b, r, red.partials, wet, G}, G);
     } else {
-        const uint32_t ga = grid_for(F.n);
-        push_rec(out, kMkAcc64, MAcc64{F.n, xcorr, x64, ga}, ga);
-        push_rec(out, kMkRefine2, MRefine<2>{F, codes, scale[0], scale[1], scale[2], xcorr, x64, b, r, red.partials, G},
-                 G);
+        push_rec(out, kMkAcc64, MAcc64{F, xcorr, x64, wet, G}, G);
+        push_rec(out, kMkRefine2,
+                 MRefine<2>{F, codes, scale[0], scale[1], scale[2], xcorr, x64, b, r, red.partials, wet, G}, G);
     }
     push_rec(out, kMkSum2, MSum2{red.partials, G, out2}, 1u);
 }
@@ -2887,7 +2997,7 @@ void rec_codes(std::vector<MRec>& out, int nx, int ny, int nz, const uint8_t* ma
     push_rec(out, kMkCodes, MCodes{nx, ny, nz, markers, codes, n, G}, G);
 }
 
-void rec_flat_wet(std::vector<MRec>& out, const GridDev& g, const uint16_t* codes, uint8_t* wet) {
+void rec_flat_wet(std::vector<MRec>& out, const GridDev& g, const uint16_t* codes, uint16_t* wet) {
     const Flat F = make_flat(g.nx, g.ny, g.nz);
     const uint32_t G = flat_grid(F.n);
     push_rec(out, kMkFlatWet, MFlatWet{F, codes, wet, G}, G);

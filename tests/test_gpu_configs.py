@@ -164,6 +164,34 @@ def test_block_skip_changes_no_bit(ctx):
     a.close(); b.close()
 
 
+@pytest.mark.parametrize("res,fill", [((31, 9, 7), 0.02), ((64, 16, 5), 0.3), ((70, 33, 19), 0.004), ((128, 24, 20), 0.5),
+                                      ((15, 8, 8), 0.9)])
+@pytest.mark.parametrize("warm", [False, True])
+def test_segment_skip_changes_no_bit(ctx, res, fill, warm):
+    """The CG's 64-cell segments: fluid in a part of each row and scattered
+    single cells, a last block and a last segment that are not full, blocks of
+    the first and last planes (clamped neighbours) and between; cold and warm."""
+    rng = np.random.default_rng(sum(res))
+    x = np.arange(res[0])[None, None, :]
+    phi = np.where((x < fill * res[0]) | (rng.random(res[::-1]) < 0.001), -1.0, 1.0).astype(np.float32)
+    vel = [rng.standard_normal(int(np.prod([res[d] + (d == k) for d in range(3)]))).astype(np.float32)
+           for k in range(3)]
+    out = []
+    for skip in (True, False):
+        d = mgf.make_desc(res, (0, 0, 0), (0.1, 0.1, 0.1), 0.003, tol_mode=mgf.TOL_RELATIVE, tol=1e-6,
+                          precision=mgf.PRECISION_MIXED, precond=mgf.PRECOND_MULTIGRID, warm_start=warm)
+        s = mgf.Scene(ctx, d)
+        s.set_block_skip(skip)
+        s.upload(mgf.FIELD["fluid_domain"], phi.ravel())
+        for k in range(3):
+            s.upload(k, vel[k])
+        st = [s.step(1) for _ in range(2)]
+        out.append((snapshot(s), [(q["cg_iterations"], q["refinement_sweeps"], q["converged"]) for q in st]))
+        s.close()
+    assert out[0][1] == out[1][1] and out[0][1][0][0] > 0
+    assert_same(out[0][0], out[1][0], "res %s" % (res,))
+
+
 def test_extrapolation_16bit_limit(ctx):
     """A grid with nx + ny + nz + 3 >= 65535 is created and steps without
     extrapolation (one layer); extrapolating over more layers is refused."""
