@@ -414,7 +414,7 @@ bool march_on(mgf_scene s, int l, const MgDims& f, const MgDims& c) {
     if (l >= l0 || l + 1 >= L || !mg_march_ok(f)) return false;
     const size_t n = size_t(f.nx) * f.ny * f.nz;
     if (d.mg_kernels == MGF_MG_AUTO && n < kMarchMinCells) return false;
-    const size_t part_cap = size_t(std::max<uint32_t>(kMaxBlocks, col_blocks(s->g))) * 2;
+    const size_t part_cap = red_capacity(col_blocks(s->g));
     return l > 0 || mg_march_parts(f, c) <= part_cap;
 }
 
@@ -427,7 +427,7 @@ bool brick_on(mgf_scene s, int l, const MgDims& f, const MgDims& c) {
     const int l0 = s->mg_l0 < L ? s->mg_l0 : L;
     if (d.preconditioner != MGF_PRECOND_MULTIGRID || nu != 3 || d.mg_kernels == MGF_MG_PER_SWEEP) return false;
     if (l >= l0 || l + 1 >= L || !mg_march_ok(f) || march_on(s, l, f, c)) return false;
-    const size_t part_cap = size_t(std::max<uint32_t>(kMaxBlocks, col_blocks(s->g))) * 2;
+    const size_t part_cap = red_capacity(col_blocks(s->g));
     return l > 0 || mg_brick_blocks(f) <= part_cap;
 }
 
@@ -528,7 +528,9 @@ mgf_status mg_setup(mgf_scene s, const float sa[3]) {
 
 // z = M^-1 r; *zout receives the buffer that holds z.  The last level-0
 // kernel also reduces r . z and sets beta (see k_mg_smooth).
-mgf_status apply_precond(mgf_scene s, const float sa[3], const float** zout) {
+// fold (its rz and rr) leaves r . z to K_I and takes r . r from K_II; fold.rr
+// needs a level 0 that descends by bricks.
+mgf_status apply_precond(mgf_scene s, const float sa[3], const float** zout, const CgFold& fold = {}) {
     hipStream_t st = s->stream;
     const auto& d = s->desc;
     const MgDims d0{s->g.nx, s->g.ny, s->g.nz, sa[0], sa[1], sa[2]};
@@ -559,6 +561,7 @@ mgf_status apply_precond(mgf_scene s, const float sa[3], const float** zout) {
     // of r . z into the scene's partials buffer
     auto fused = [&](int l) { return l + 1 < L && march_on(s, l, lv[l].d, lv[l + 1].d); };
     auto bricks = [&](int l) { return l + 1 < L && brick_on(s, l, lv[l].d, lv[l + 1].d); };
+    const int rz_how = fold.rz ? kRzLeft : 1;
     for (int l = 0; l < l0; ++l) {
         Lv& v = lv[l];
         const bool coarsest = l == L - 1;
@@ -574,7 +577,8 @@ mgf_status apply_precond(mgf_scene s, const float sa[3], const float** zout) {
         if (bricks(l)) {
             probe_next_bytes(10.5 * double(v.d.nx) * v.d.ny * v.d.nz);
             MGF_HIP(launch_mg_brick_descend(st, v.d, lv[l + 1].d, v.codes, v.b, v.x, lv[l + 1].codes,
-                                            const_cast<float*>(lv[l + 1].b), omega, s->scal));
+                                            const_cast<float*>(lv[l + 1].b), omega, s->scal, s->red,
+                                            l == 0 && fold.rr ? col_blocks(s->g) : 0u));
             continue;
         }
         const int sweeps = coarsest ? kCoarsestSweeps : nu;
@@ -620,14 +624,14 @@ mgf_status apply_precond(mgf_scene s, const float sa[3], const float** zout) {
             const double wet = (skip && v.cells >= 0.0) ? v.cells : ncell;
             probe_next_bytes(14.5 * wet + 4.0 * (ncell - wet));
             MGF_HIP(launch_mg_ascend(st, v.d, lv[l + 1].d, v.codes, v.b, v.x, lv[l + 1].x, v.t, omega, s->scal,
-                                     s->red, l == 0 ? 1 : 0, v.sched, skip));
+                                     s->red, l == 0 ? rz_how : 0, v.sched, skip));
             std::swap(v.x, v.t);
             continue;
         }
         if (bricks(l)) {
             probe_next_bytes(14.5 * ncell);
             MGF_HIP(launch_mg_brick_ascend(st, v.d, lv[l + 1].d, v.codes, v.b, v.x, lv[l + 1].x, v.t, omega, s->scal,
-                                           s->red, l == 0 ? 1 : 0));
+                                           s->red, l == 0 ? rz_how : 0));
             std::swap(v.x, v.t);
             continue;
         }
@@ -701,6 +705,18 @@ mgf_status cg_mixed(mgf_scene s, const float sa[3], int64_t max_it, mgf_step_sta
             f = c;
         }
     }
+    // which dot products the kernels that need them finish
+    CgFold fold, start_fold;
+    const uint32_t G = col_blocks(s->g);
+    fold.alpha = G <= kFoldMax;
+    if (!ident && !s->mg.empty()) {
+        const MgDims f{s->g.nx, s->g.ny, s->g.nz, sa[0], sa[1], sa[2]};
+        const bool bricks = brick_on(s, 0, f, s->mg[0].d), march = march_on(s, 0, f, s->mg[0].d);
+        const uint32_t parts = bricks ? mg_brick_blocks(f) : (march ? uint32_t(mg_march_parts(f, s->mg[0].d)) : 0u);
+        if (parts <= kFoldMax) fold.rz = parts;
+        fold.rr = bricks && G <= kFoldMax;
+    }
+    start_fold.rz = fold.rz;
     const double ncell_all = double(s->ncell);
     const double flat_cells = s->wet_flat_cells >= 0.0 ? s->wet_flat_cells : ncell_all;
     bool first_pap = true;
@@ -731,7 +747,7 @@ mgf_status cg_mixed(mgf_scene s, const float sa[3], int64_t max_it, mgf_step_sta
         MGF_HIP(launch_cg_start(st, s->g, rsrc, s->r, s->x, s->scal, s->red, inner, target2));
         first_pap = true;
         const float* zv = s->r;
-        if (!ident) TRY(apply_precond(s, sa, &zv));
+        if (!ident) TRY(apply_precond(s, sa, &zv, start_fold));
         // r.r at the sweep start and the sweep's target, as the device sets them
         const double rr0 = rr_true;
         const double sweep_target = std::max(inner * inner * rr0, target2);
@@ -743,12 +759,13 @@ mgf_status cg_mixed(mgf_scene s, const float sa[3], int64_t max_it, mgf_step_sta
             const int k = int(std::min<int64_t>(predict(rr_now, sweep_target), std::max<int64_t>(left, 1)));
             for (int q = 0; q < k; ++q) {
                 probe_next_bytes(22.0 * (first_pap ? ncell_all : flat_cells));
-                MGF_HIP(launch_col_p_ap(st, s->g, sa, s->codes, zv, s->p0, s->p1, s->scal, s->red, wet_flat));
+                MGF_HIP(launch_col_p_ap(st, s->g, sa, s->codes, zv, s->p0, s->p1, s->scal, s->red, wet_flat,
+                                        fold));
                 first_pap = false;
                 probe_next_bytes(24.0 * flat_cells);
                 MGF_HIP(launch_col_update(st, s->g, s->p0, s->p1, s->x, s->r, s->scal, s->red, ident ? 1 : 0,
-                                          wet_flat));
-                if (!ident) TRY(apply_precond(s, sa, &zv));
+                                          wet_flat, fold));
+                if (!ident) TRY(apply_precond(s, sa, &zv, fold));
             }
             MGF_HIP(hipMemcpyAsync(&hs, s->scal, sizeof(CgScalars), hipMemcpyDeviceToHost, st));
             MGF_HIP(hipStreamSynchronize(st));
@@ -757,6 +774,11 @@ mgf_status cg_mixed(mgf_scene s, const float sa[3], int64_t max_it, mgf_step_sta
             rr_now = hs.rr;
             done_before = hs.iters;
             if (hs.done || it_total + hs.iters >= max_it) break;
+        }
+        if (!hs.done && fold.rz) {   // the last r . z, which no K_I follows, is looked at too
+            MGF_HIP(launch_finish_rz(st, s->scal, s->red, fold.rz));
+            MGF_HIP(hipMemcpyAsync(&hs, s->scal, sizeof(CgScalars), hipMemcpyDeviceToHost, st));
+            MGF_HIP(hipStreamSynchronize(st));
         }
         it_total += hs.iters;
         if (hs.done == 2) { rr_true = std::nan(""); break; }
@@ -844,7 +866,7 @@ mgf_status alloc_scene(mgf_scene s) {
     A(&s->codes, s->ncell);
     if (s->desc.precision == MGF_PRECISION_MIXED) A(&s->wet_flat, col_blocks(s->g));
     A(&s->scal, 1);
-    A(&s->red.partials, size_t(std::max<uint32_t>(kMaxBlocks, col_blocks(s->g))) * 2);
+    A(&s->red.partials, red_capacity(col_blocks(s->g)));
     A(&s->red.out2, 2);
     A(&s->div_dev, 3);
     if (st == MGF_OK) st = alloc_extrapolation(s, s->nfx + s->nfy + s->nfz);
@@ -2540,7 +2562,7 @@ mgf_status mgf_scene_apply_preconditioner(mgf_scene s, const float* r, float* z,
     MGF_HIP(hipMemcpyAsync(z, zv, sizeof(float) * s->ncell, hipMemcpyDeviceToDevice, st));
     MGF_HIP(hipMemcpyAsync(&hs, s->scal, sizeof(CgScalars), hipMemcpyDeviceToHost, st));
     TRY(sync(s));
-    if (rz) *rz = hs.rz;
+    if (rz) *rz = hs.rz_new;
     return MGF_OK;
 }
 

@@ -17,8 +17,8 @@ namespace mgf {
 
 // Device scalars of the fused CG (one struct per scene, in device memory).
 struct CgScalars {
-    double rz;        // r . z of the current iteration
-    double rz_new;
+    double rz;        // r . z of the iteration before (beta's divisor)
+    double rz_new;    // r . z of the current z
     double pap;       // p . A p
     double alpha;
     double beta;
@@ -370,13 +370,30 @@ uint32_t col_blocks(const GridDev& g);
 hipError_t launch_flat_wet(hipStream_t s, const GridDev& g, const uint16_t* codes, uint16_t* wet);
 // Cells in the segments a host copy of the masks marks (measurement).
 double flat_wet_cells(const GridDev& g, const uint16_t* wet_host);
+// Dot products left to the kernel that needs them (Fold, mgf_kernels_mg.hip)
+// instead of a finishing launch: r . z of the level-0 ascent (its partials,
+// with_rz = kRzLeft) to K_I, p . Ap to K_II, r . r to the level-0 brick descent.
+constexpr uint32_t kFoldMax = 512;
+struct CgFold {
+    uint32_t rz = 0;      // partials of r . z K_I finishes
+    bool alpha = false;   // K_II finishes p . Ap
+    bool rr = false;      // r . r is left
+};
+constexpr int kRzLeft = 2;
+// Finishes r . z after all (beta, rz_new).
+hipError_t launch_finish_rz(hipStream_t s, CgScalars* sc, ReduceBuf red, uint32_t count);
+// Doubles in a scene's partials buffer, from the blocks of its flat kernels.
+inline size_t red_capacity(uint32_t flat_blocks) {
+    return size_t(flat_blocks > uint32_t(kMaxBlocks) ? flat_blocks : uint32_t(kMaxBlocks)) * 2;
+}
 // K_I: p = z + beta p, Ap = A z + beta Ap in place (p = z, Ap = A z on the
 // first iteration), p . Ap, alpha.
 hipError_t launch_col_p_ap(hipStream_t s, const GridDev& g, const float scale[3], const uint16_t* codes,
-                           const float* zv, float* p, float* ap, CgScalars* sc, ReduceBuf red, const uint16_t* wet);
+                           const float* zv, float* p, float* ap, CgScalars* sc, ReduceBuf red, const uint16_t* wet,
+                           const CgFold& fold);
 // K_II: x += alpha p, r -= alpha Ap, r . r; identity != 0: beta = rr / rz, rz = rr.
 hipError_t launch_col_update(hipStream_t s, const GridDev& g, const float* p, const float* ap, float* x, float* r,
-                             CgScalars* sc, ReduceBuf red, int identity, const uint16_t* wet);
+                             CgScalars* sc, ReduceBuf red, int identity, const uint16_t* wet, const CgFold& fold);
 // Start of an inner sweep: r = rsrc, x = 0, the scalars from r.r (target =
 // max(rel_inner^2 r.r, abs_target2)).
 hipError_t launch_cg_start(hipStream_t s, const GridDev& g, const float* rsrc, float* r, float* x, CgScalars* sc,
@@ -428,11 +445,12 @@ hipError_t launch_mg_ascend(hipStream_t s, const MgDims& f, const MgDims& c, con
                             const float* xi, const float* xc, float* xo, float omega, CgScalars* sc, ReduceBuf red,
                             int with_rz, const uint32_t* sched, int skip);
 // The same of a small level, brick by brick (mg_brick_blocks work-groups, one
-// partial of r . z each); no schedule.
+// partial of r . z each); no schedule.  rr: the partials of r . r the descent
+// finishes first (0: none).
 uint32_t mg_brick_blocks(const MgDims& f);
 hipError_t launch_mg_brick_descend(hipStream_t s, const MgDims& f, const MgDims& c, const uint16_t* code,
                                    const float* b, float* x, const uint16_t* codec, float* bc, float omega,
-                                   const CgScalars* sc);
+                                   CgScalars* sc, ReduceBuf red, uint32_t rr);
 hipError_t launch_mg_brick_ascend(hipStream_t s, const MgDims& f, const MgDims& c, const uint16_t* code,
                                   const float* b, const float* xi, const float* xc, float* xo, float omega,
                                   CgScalars* sc, ReduceBuf red, int with_rz);

@@ -219,6 +219,112 @@ __device__ __forceinline__ uint32_t udiv(uint32_t a, uint32_t d, double rd) {
     return q;
 }
 
+// ---------------------------------------------------------------------------
+// Finishing a dot product: the sum of its `count` block partials in a fixed
+// order (that of kFinishBlock work-items, whoever forms it) and the scalars it
+// decides.  rz_new is r . z of the current z; rz that of the iteration before,
+// which beta divides by.
+enum FinishKind : int {
+    kFinishInit = 4,      // r.r -> rz, rr, sweep_r0, target2, done; iters, alpha, beta = 0
+    kFinishAlpha = 0,     // pap -> alpha
+    kFinishRrIdent = 1,   // rr -> iters, done; beta = rr / rz, rz = rr (identity)
+    kFinishRr = 2,        // rr -> iters, done (preconditioned: beta comes later)
+    kFinishRz = 3,        // r . z -> beta = rz_new / rz (0 before the first iteration), rz_new
+};
+constexpr int kFinishBlock = 1024, kFinishWaves = kFinishBlock / 64;
+
+// What work-item i of kFinishBlock adds up: four independent chains, so its
+// loads are in flight together.
+__device__ __forceinline__ double finish_chain(const double* __restrict__ part, uint32_t count, uint32_t i) {
+    double s4[4] = {0.0, 0.0, 0.0, 0.0};
+    for (; i + 3 * kFinishBlock < count; i += 4 * kFinishBlock) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) s4[q] += part[i + uint32_t(q) * kFinishBlock];
+    }
+    for (; i < count; i += kFinishBlock) s4[0] += part[i];
+    return (s4[0] + s4[1]) + (s4[2] + s4[3]);
+}
+
+__device__ __forceinline__ double finish_total(const double (&sh)[kFinishWaves]) {
+    double t = 0.0;
+#pragma unroll
+    for (int q = 0; q < kFinishWaves; ++q) t += sh[q];
+    return t;
+}
+
+// The scalars after sum t (one work-item).
+__device__ __forceinline__ void finish_scalars(CgScalars* sc, int kind, double t, double rel_inner,
+                                               double abs_target2) {
+    switch (kind) {
+        case kFinishInit: {
+            sc->rz = t;
+            sc->rz_new = t;
+            sc->rr = t;
+            sc->sweep_r0 = t;
+            const double rel2 = rel_inner * rel_inner * t;
+            sc->target2 = rel2 > abs_target2 ? rel2 : abs_target2;
+            sc->done = (t <= sc->target2 || t == 0.0) ? 1 : 0;
+            sc->iters = 0;
+            sc->beta = 0.0;
+            sc->alpha = 0.0;
+            break;
+        }
+        case kFinishAlpha:
+            sc->pap = t;
+            if (!isfinite(t)) { sc->done = 2; sc->alpha = 0.0; }
+            else if (t == 0.0) { sc->done = 1; sc->alpha = 0.0; }
+            else sc->alpha = sc->rz_new / t;
+            break;
+        case kFinishRrIdent:
+        case kFinishRr:
+            sc->rr = t;
+            sc->iters = sc->iters + 1;
+            if (kind == kFinishRrIdent) {
+                sc->beta = t / sc->rz_new;
+                sc->rz_new = t;
+            }
+            sc->rz = sc->rz_new;
+            if (t <= sc->target2) sc->done = 1;
+            else if (!isfinite(t)) sc->done = 2;
+            break;
+        default:  // kFinishRz
+            sc->beta = sc->iters == 0 ? 0.0 : t / sc->rz;
+            sc->rz_new = t;
+            if (!isfinite(t)) sc->done = 2;
+            break;
+    }
+}
+
+// A dot product finished by the kernel that needs it instead of a launch of
+// one work-group in between: every work-group forms the same sum (in
+// finish_chain's order, so bit for bit k_finish's) and decides alike, and the
+// first one stores the scalars.  What is stored is not read by the others,
+// except done, which tells a work-group what it would find itself.  The
+// partials lie where the kernel does not write its own (fold_slots).  Worth it
+// while the partials are few (kFoldMax): a launch between two kernels costs about
+// 3.5 us, the sum in each work-group about 1 us with 40 partials (34^3, four
+// steps: 3.79 -> 3.45 ms) and as much as the launch with a thousand (152 x 63 x
+// 99, 926 partials: no change; 130^3, 2152: 4.75 -> 4.84 ms).  count 0: the
+// scalars are finished.
+struct Fold {
+    const double* part;
+    uint32_t count;
+    CgScalars* sc;
+};
+
+// The sum, in every work-item (called by all work-items of the block).
+__device__ __forceinline__ double fold_sum(const Fold& f) {
+    __shared__ double sh[kFinishWaves];
+    const uint32_t lane = threadIdx.x & 63u, waves = blockDim.x >> 6;
+    for (uint32_t v = threadIdx.x >> 6; v < uint32_t(kFinishWaves); v += waves) {
+        double s = 0.0;
+        if (v * 64u < f.count) s = wave_sum(finish_chain(f.part, f.count, v * 64u + lane));
+        if (lane == 0) sh[v] = s;
+    }
+    __syncthreads();
+    return finish_total(sh);
+}
+
 // Cells per work-item of the fine-grid kernels (256 apart): fewer block
 // partials to finish, the LDS tables amortised, more loads in flight.
 constexpr int kCpt = 4;
@@ -336,11 +442,20 @@ struct MFlatWet {
 __device__ __forceinline__ void cg_pap_run(Flat F, const uint16_t* __restrict__ code, float sx, float sy, float sz,
                                            const float* __restrict__ zv, float* __restrict__ p,
                                            float* __restrict__ ap, const CgScalars* __restrict__ sc,
-                                           double* __restrict__ part, const uint16_t* __restrict__ wet, uint32_t blk,
-                                           uint32_t slot) {
+                                           double* __restrict__ part, const uint16_t* __restrict__ wet,
+                                           const Fold& rz, uint32_t blk, uint32_t slot) {
     __shared__ float aw[64];
     if (sc->done) return;
     const bool first = sc->iters == 0;
+    float beta;
+    if (rz.count) {
+        const double t = fold_sum(rz);
+        beta = float(first ? 0.0 : t / sc->rz);
+        if (slot == 0 && threadIdx.x == 0) finish_scalars(rz.sc, kFinishRz, t, 0.0, 0.0);
+        if (!isfinite(t)) return;
+    } else {
+        beta = float(sc->beta);
+    }
     const uint32_t mask = (!first && wet) ? wet[blk] : kSegAll;
     if (!mask) {
         if (threadIdx.x == 0) part[slot] = 0.0;
@@ -348,7 +463,6 @@ __device__ __forceinline__ void cg_pap_run(Flat F, const uint16_t* __restrict__ 
     }
     const uint32_t rounds = seg_rounds(mask);
     build_tables<false>(aw, nullptr, sx, sy, sz, 0.0f);
-    const float beta = float(sc->beta);
     const uint32_t b0 = blk * (kBlock * kCpt);
     const uint32_t base = b0 + threadIdx.x;
     // first is a template parameter: a branch on it between the loads makes
@@ -369,8 +483,9 @@ __device__ __forceinline__ void cg_pap_run(Flat F, const uint16_t* __restrict__ 
 __global__ void __launch_bounds__(kBlock) k_cg_pap(Flat F, const uint16_t* __restrict__ code, float sx, float sy,
                                                    float sz, const float* __restrict__ zv, float* __restrict__ p,
                                                    float* __restrict__ ap, const CgScalars* __restrict__ sc,
-                                                   double* __restrict__ part, const uint16_t* __restrict__ wet) {
-    cg_pap_run(F, code, sx, sy, sz, zv, p, ap, sc, part, wet, xcd_block(), blockIdx.x);
+                                                   double* __restrict__ part, const uint16_t* __restrict__ wet,
+                                                   Fold rz) {
+    cg_pap_run(F, code, sx, sy, sz, zv, p, ap, sc, part, wet, rz, xcd_block(), blockIdx.x);
 }
 
 struct MPap {
@@ -384,7 +499,7 @@ struct MPap {
     double* part;
     const uint16_t* wet;
     uint32_t G;
-    __device__ void run(uint32_t b) const { cg_pap_run(F, code, sx, sy, sz, zv, p, ap, sc, part, wet, xcd_of(b, G), b); }
+    __device__ void run(uint32_t b) const { cg_pap_run(F, code, sx, sy, sz, zv, p, ap, sc, part, wet, Fold{}, xcd_of(b, G), b); }
 };
 
 // K_II (pointwise): x += alpha p; r -= alpha Ap (each formed in FP64, stored
@@ -421,15 +536,24 @@ __device__ __forceinline__ double cg_update_body(const Flat& F, uint32_t base, c
 __device__ __forceinline__ void cg_update_run(Flat F, const float* __restrict__ p, const float* __restrict__ ap,
                                               float* __restrict__ x, float* __restrict__ r,
                                               const CgScalars* __restrict__ sc, double* __restrict__ part,
-                                              const uint16_t* __restrict__ wet, uint32_t blk, uint32_t slot) {
+                                              const uint16_t* __restrict__ wet, const Fold& pap, uint32_t blk,
+                                              uint32_t slot) {
     if (sc->done) return;
+    double alpha;
+    if (pap.count) {
+        const double t = fold_sum(pap);
+        alpha = sc->rz_new / t;
+        if (slot == 0 && threadIdx.x == 0) finish_scalars(pap.sc, kFinishAlpha, t, 0.0, 0.0);
+        if (!isfinite(t) || t == 0.0) return;
+    } else {
+        alpha = sc->alpha;
+    }
     const uint32_t mask = wet ? wet[blk] : kSegAll;
     if (!mask) {
         if (threadIdx.x == 0) part[slot] = 0.0;
         return;
     }
     const uint32_t rounds = seg_rounds(mask);
-    const double alpha = sc->alpha;
     const uint32_t b0 = blk * (kBlock * kCpt);
     const uint32_t base = b0 + threadIdx.x;
     double acc = 0.0;
@@ -442,8 +566,9 @@ __device__ __forceinline__ void cg_update_run(Flat F, const float* __restrict__ 
 __global__ void __launch_bounds__(kBlock) k_cg_update(Flat F, const float* __restrict__ p,
                                                       const float* __restrict__ ap, float* __restrict__ x,
                                                       float* __restrict__ r, const CgScalars* __restrict__ sc,
-                                                      double* __restrict__ part, const uint16_t* __restrict__ wet) {
-    cg_update_run(F, p, ap, x, r, sc, part, wet, xcd_block(), blockIdx.x);
+                                                      double* __restrict__ part, const uint16_t* __restrict__ wet,
+                                                      Fold pap) {
+    cg_update_run(F, p, ap, x, r, sc, part, wet, pap, xcd_block(), blockIdx.x);
 }
 
 struct MUpdate {
@@ -455,7 +580,7 @@ struct MUpdate {
     double* part;
     const uint16_t* wet;
     uint32_t G;
-    __device__ void run(uint32_t b) const { cg_update_run(F, p, ap, x, r, sc, part, wet, xcd_of(b, G), b); }
+    __device__ void run(uint32_t b) const { cg_update_run(F, p, ap, x, r, sc, part, wet, Fold{}, xcd_of(b, G), b); }
 };
 
 // Refinement (outer sweeps of the mixed solver).
@@ -709,73 +834,15 @@ struct MSum2 {
     __device__ void run(uint32_t) const { sum2_run(part, count, out); }
 };
 
-// The one-block finishing kernel: sums `count` partials in a fixed order and
-// updates the scalars.
-enum FinishKind : int {
-    kFinishInit = 4,      // r.r -> rz, rr, sweep_r0, target2, done; iters, alpha, beta = 0
-    kFinishAlpha = 0,     // pap -> alpha
-    kFinishRrIdent = 1,   // rr -> iters, done; beta = rr / rz, rz = rr (identity)
-    kFinishRr = 2,        // rr -> iters, done (preconditioned: beta comes later)
-    kFinishRz = 3,        // r . z -> beta = rz / rz_old (0 before the first iteration), rz
-};
-constexpr int kFinishBlock = 1024;
-
+// A finishing launch of its own, one work-group.
 __device__ __forceinline__ void finish_run(const double* __restrict__ part, uint32_t count, CgScalars* sc, int kind,
                                            double rel_inner, double abs_target2) {
     if (kind != kFinishInit && sc->done) return;
-    // four independent chains: the loads of a thread are in flight together
-    double s4[4] = {0.0, 0.0, 0.0, 0.0};
-    uint32_t i = threadIdx.x;
-    for (; i + 3 * kFinishBlock < count; i += 4 * kFinishBlock) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) s4[q] += part[i + uint32_t(q) * kFinishBlock];
-    }
-    for (; i < count; i += kFinishBlock) s4[0] += part[i];
-    double s = (s4[0] + s4[1]) + (s4[2] + s4[3]);
-    __shared__ double sh[kFinishBlock / 64];
-    s = wave_sum(s);
+    __shared__ double sh[kFinishWaves];
+    const double s = wave_sum(finish_chain(part, count, threadIdx.x));
     if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
     __syncthreads();
-    if (threadIdx.x != 0) return;
-    double t = 0.0;
-#pragma unroll
-    for (int q = 0; q < kFinishBlock / 64; ++q) t += sh[q];
-    switch (kind) {
-        case kFinishInit: {
-            sc->rz = t;
-            sc->rr = t;
-            sc->sweep_r0 = t;
-            const double rel2 = rel_inner * rel_inner * t;
-            sc->target2 = rel2 > abs_target2 ? rel2 : abs_target2;
-            sc->done = (t <= sc->target2 || t == 0.0) ? 1 : 0;
-            sc->iters = 0;
-            sc->beta = 0.0;
-            sc->alpha = 0.0;
-            break;
-        }
-        case kFinishAlpha:
-            sc->pap = t;
-            if (!isfinite(t)) { sc->done = 2; sc->alpha = 0.0; }
-            else if (t == 0.0) { sc->done = 1; sc->alpha = 0.0; }
-            else sc->alpha = sc->rz / t;
-            break;
-        case kFinishRrIdent:
-        case kFinishRr:
-            sc->rr = t;
-            sc->iters = sc->iters + 1;
-            if (kind == kFinishRrIdent) {
-                sc->beta = t / sc->rz;
-                sc->rz = t;
-            }
-            if (t <= sc->target2) sc->done = 1;
-            else if (!isfinite(t)) sc->done = 2;
-            break;
-        default:  // kFinishRz
-            sc->beta = sc->iters == 0 ? 0.0 : t / sc->rz;
-            sc->rz = t;
-            if (!isfinite(t)) sc->done = 2;
-            break;
-    }
+    if (threadIdx.x == 0) finish_scalars(sc, kind, finish_total(sh), rel_inner, abs_target2);
 }
 
 __global__ void __launch_bounds__(kFinishBlock) k_finish(const double* __restrict__ part, uint32_t count,
@@ -1732,12 +1799,17 @@ __device__ __forceinline__ void brick_run(const Bricks& T, const MgLevel& L, con
                                           const float* __restrict__ b, const float* __restrict__ xi,
                                           const float* __restrict__ xc, float* __restrict__ xo,
                                           const uint16_t* __restrict__ codec, float* __restrict__ bco, float omega,
-                                          const CgScalars* __restrict__ sc, double* __restrict__ part, uint32_t blk,
-                                          uint32_t slot) {
+                                          const CgScalars* __restrict__ sc, double* __restrict__ part, const Fold& rr,
+                                          uint32_t blk, uint32_t slot) {
     __shared__ float aw[64], w[64];
     __shared__ float xa[kBkCells], xb[kBkCells];
     __shared__ double sum[kBkThreads / 64];
     if (sc->done) return;
+    if (!POST && rr.count) {
+        const double t = fold_sum(rr);
+        if (slot == 0 && threadIdx.x == 0) finish_scalars(rr.sc, kFinishRr, t, 0.0, 0.0);
+        if (t <= sc->target2 || !isfinite(t)) return;
+    }
     const int t = threadIdx.x;
     const uint32_t bx = blk % T.tx, br = blk / T.tx, by = br % T.ty, bz = br / T.ty;
     const int x0 = int(bx) * kBkEdge - kBkHalo, y0 = int(by) * kBkEdge - kBkHalo, z0 = int(bz) * kBkEdge - kBkHalo;
@@ -1842,8 +1914,8 @@ __global__ void __launch_bounds__(kBkThreads) k_mg_brick(Bricks T, MgLevel L, co
                                                          const float* __restrict__ xc, float* __restrict__ xo,
                                                          const uint16_t* __restrict__ codec, float* __restrict__ bco,
                                                          float omega, const CgScalars* __restrict__ sc,
-                                                         double* __restrict__ part) {
-    brick_run<POST, RZ>(T, L, code, b, xi, xc, xo, codec, bco, omega, sc, part, blockIdx.x, blockIdx.x);
+                                                         double* __restrict__ part, Fold rr) {
+    brick_run<POST, RZ>(T, L, code, b, xi, xc, xo, codec, bco, omega, sc, part, rr, blockIdx.x, blockIdx.x);
 }
 
 template <bool POST, bool RZ>
@@ -1860,7 +1932,7 @@ struct MBrick {
     const CgScalars* sc;
     double* part;
     __device__ void run(uint32_t blk) const {
-        brick_run<POST, RZ>(T, L, code, b, xi, xc, xo, codec, bco, omega, sc, part, blk, blk);
+        brick_run<POST, RZ>(T, L, code, b, xi, xc, xo, codec, bco, omega, sc, part, Fold{}, blk, blk);
     }
 };
 
@@ -2639,21 +2711,34 @@ hipError_t launch_flat_wet(hipStream_t s, const GridDev& g, const uint16_t* code
     return LAUNCH(k_flat_wet, flat_grid(F.n), F, codes, wet);
 }
 
+hipError_t launch_finish_rz(hipStream_t s, CgScalars* sc, ReduceBuf red, uint32_t count) {
+    return finish(s, red.partials, count, sc, kFinishRz);
+}
+
+// K_I's partials when K_II finishes them: the end of the buffer, so that K_II
+// (whose own partials start it) and K_I (which reads r . z's there) do not
+// write what they read.  red_capacity() is at least 16 kFoldMax doubles.
+static double* fold_slots(ReduceBuf red, uint32_t G) { return red.partials + (red_capacity(G) - G); }
+
 hipError_t launch_col_p_ap(hipStream_t s, const GridDev& g, const float scale[3], const uint16_t* codes,
-                           const float* zv, float* p, float* ap, CgScalars* sc, ReduceBuf red, const uint16_t* wet) {
+                           const float* zv, float* p, float* ap, CgScalars* sc, ReduceBuf red, const uint16_t* wet,
+                           const CgFold& fold) {
     const Flat F = make_flat(g.nx, g.ny, g.nz);
     const uint32_t G = flat_grid(F.n);
-    hipError_t e = LAUNCH(k_cg_pap, G, F, codes, scale[0], scale[1], scale[2], zv, p, ap, sc, red.partials, wet);
-    if (e != hipSuccess) return e;
+    double* part = fold.alpha ? fold_slots(red, G) : red.partials;
+    hipError_t e = LAUNCH(k_cg_pap, G, F, codes, scale[0], scale[1], scale[2], zv, p, ap, sc, part, wet,
+                          (Fold{red.partials, fold.rz, sc}));
+    if (e != hipSuccess || fold.alpha) return e;
     return finish(s, red.partials, G, sc, kFinishAlpha);
 }
 
 hipError_t launch_col_update(hipStream_t s, const GridDev& g, const float* p, const float* ap, float* x, float* r,
-                             CgScalars* sc, ReduceBuf red, int identity, const uint16_t* wet) {
+                             CgScalars* sc, ReduceBuf red, int identity, const uint16_t* wet, const CgFold& fold) {
     const Flat F = make_flat(g.nx, g.ny, g.nz);
     const uint32_t G = flat_grid(F.n);
-    hipError_t e = LAUNCH(k_cg_update, G, F, p, ap, x, r, sc, red.partials, wet);
-    if (e != hipSuccess) return e;
+    hipError_t e = LAUNCH(k_cg_update, G, F, p, ap, x, r, sc, red.partials, wet,
+                          (Fold{fold_slots(red, G), fold.alpha ? G : 0u, sc}));
+    if (e != hipSuccess || fold.rr) return e;
     return finish(s, red.partials, G, sc, identity ? kFinishRrIdent : kFinishRr);
 }
 
@@ -2828,7 +2913,7 @@ hipError_t launch_mg_ascend(hipStream_t s, const MgDims& f, const MgDims& c, con
         e = launch_dims(k_mg_march<true, false>, "k_mg_march", dim3(G), dim3(kMThreads), 0u, s, M, f, code, b, xi, xc, xo,
                         static_cast<const uint16_t*>(nullptr), static_cast<float*>(nullptr), omega, csc,
                         static_cast<double*>(nullptr), sched);
-    if (e != hipSuccess || !with_rz) return e;
+    if (e != hipSuccess || !with_rz || with_rz == kRzLeft) return e;
     return finish(s, red.partials, M.parts, sc, kFinishRz);
 }
 
@@ -2846,10 +2931,12 @@ uint32_t mg_brick_blocks(const MgDims& f) {
 
 hipError_t launch_mg_brick_descend(hipStream_t s, const MgDims& f, const MgDims& c, const uint16_t* code,
                                    const float* b, float* x, const uint16_t* codec, float* bc, float omega,
-                                   const CgScalars* sc) {
+                                   CgScalars* sc, ReduceBuf red, uint32_t rr) {
+    const CgScalars* csc = sc;
     return launch_dims(k_mg_brick<false, false>, "k_mg_brick", dim3(mg_brick_blocks(f)), dim3(kBkThreads), 0u, s,
                        make_bricks(f, c), f, code, b, static_cast<const float*>(nullptr),
-                       static_cast<const float*>(nullptr), x, codec, bc, omega, sc, static_cast<double*>(nullptr));
+                       static_cast<const float*>(nullptr), x, codec, bc, omega, csc, static_cast<double*>(nullptr),
+                       Fold{red.partials, rr, sc});
 }
 
 hipError_t launch_mg_brick_ascend(hipStream_t s, const MgDims& f, const MgDims& c, const uint16_t* code,
@@ -2861,11 +2948,11 @@ hipError_t launch_mg_brick_ascend(hipStream_t s, const MgDims& f, const MgDims& 
     float* nb = nullptr;
     if (!with_rz)
         return launch_dims(k_mg_brick<true, false>, "k_mg_brick", dim3(G), dim3(kBkThreads), 0u, s, make_bricks(f, c),
-                           f, code, b, xi, xc, xo, nc, nb, omega, csc, static_cast<double*>(nullptr));
+                           f, code, b, xi, xc, xo, nc, nb, omega, csc, static_cast<double*>(nullptr), Fold{});
     const hipError_t e = launch_dims(k_mg_brick<true, true>, "k_mg_brick", dim3(G), dim3(kBkThreads), 0u, s,
                                      make_bricks(f, c), f, code, b, xi, xc, xo, nc, nb, omega, csc,
-                                     red.partials);
-    if (e != hipSuccess) return e;
+                                     red.partials, Fold{});
+    if (e != hipSuccess || with_rz == kRzLeft) return e;
     return finish(s, red.partials, G, sc, kFinishRz);
 }
 

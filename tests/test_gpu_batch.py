@@ -65,6 +65,42 @@ def test_batch_matches_scenes_stepped_alone(ctx, precision, precond):
         s.close()
 
 
+@pytest.mark.parametrize("precond", [mgf.PRECOND_MULTIGRID, mgf.PRECOND_JACOBI, mgf.PRECOND_IDENTITY])
+@pytest.mark.parametrize("res", [(2, 2, 2), (9, 9, 9), (40, 25, 30), (64, 64, 64), (80, 80, 81), (82, 80, 80),
+                                 (84, 80, 78)])
+def test_dot_products_finished_by_their_consumers(ctx, res, precond):
+    """A scene alone lets the kernels that need a dot product finish it (up to
+    512 partials, 512K cells: one less, that many and one more); in a batch each
+    is a launch of its own.  The same bits and counts, also when the iterations
+    end before the tolerance and when there is nothing to solve."""
+    rng = np.random.default_rng(sum(res))
+    phi = np.where(rng.random(int(np.prod(res))) < 0.6, -1.0, 1.0).astype(np.float32)
+    phi[0] = 1.0
+    vel = [rng.standard_normal(int(np.prod([res[d] + (d == k) for d in range(3)]))).astype(np.float32)
+           for k in range(3)]
+    for max_it, still in ((0, False), (3, False), (0, True)):
+        pair = []
+        for _ in range(3):
+            d = mgf.make_desc(res, (0, 0, 0), (0.1, 0.1, 0.1), 0.003, rk=mgf.RK1, tol_mode=mgf.TOL_RELATIVE, tol=1e-6,
+                              max_it=max_it, precision=mgf.PRECISION_MIXED, precond=precond,
+                              gravity=(0, 0, 0) if still else (0, -9.8, 0))
+            s = mgf.Scene(ctx, d)
+            s.upload(mgf.FIELD["fluid_domain"], phi)
+            for k in range(3):
+                s.upload(k, 0 * vel[k] if still else vel[k])
+            pair.append(s)
+        _, stats, _ = mgf.batch_step(ctx, pair[:2], 1, workers=1)
+        st = mgf.StepStats()
+        rc = mgf.lib().mgf_step(pair[2].h, 1, mgf.C.byref(st))
+        assert rc in (mgf.OK, 4)
+        for key in ("cg_iterations", "converged", "refinement_sweeps"):
+            assert getattr(stats[0], key) == getattr(st, key), key
+        assert np.float64(stats[0].residual_rel).tobytes() == np.float64(st.residual_rel).tobytes()
+        assert_same(snapshot(pair[0]), snapshot(pair[2]), "res %s" % (res,))
+        for s in pair:
+            s.close()
+
+
 def test_batch_without_latency_and_repeat(ctx):
     """Two batched calls (no per-step latency) equal one solo call of the summed
     steps; the worker count does not change the results."""
