@@ -397,14 +397,13 @@ constexpr size_t kCoarseLdsMax = 131072;
 // level of a 128^3 scene goes to bricks: 4.80 -> 5.67 ms)
 constexpr size_t kMarchMinCells = size_t(1) << 19;
 
-// Whether level l (dims f; the next coarser level c) runs the fused descent
-// and ascent: three sweeps, a 3-D level above the coarse cycle, under
-// MGF_MG_AUTO at least kMarchMinCells (smaller levels: brick_on); on level 0
-// the ascent's
-// partials of r . z must fit the scene's buffer.
 // Blocks of a fused march resident at once: two per CU.
 uint32_t march_slots(mgf_scene s) { return 2u * uint32_t(std::max(1, s->ctx->cu_count)); }
 
+// Whether level l (dims f; the next coarser level c) marches its descent and
+// ascent: three sweeps, a 3-D level above the coarse cycle, under MGF_MG_AUTO
+// at least kMarchMinCells (smaller levels: brick_on); on level 0 the ascent's
+// partials of r . z must fit the scene's buffer.
 bool march_on(mgf_scene s, int l, const MgDims& f, const MgDims& c) {
     const auto& d = s->desc;
     const int nu = d.mg_sweeps > 0 ? d.mg_sweeps : 3;
