@@ -89,6 +89,41 @@ def test_brick_vcycle_bitwise_per_sweep(ctx, res):
     a.close(); p.close()
 
 
+@pytest.mark.parametrize("res", [(1, 1, 1), (3, 1, 2), (1, 5, 7), (2, 3, 5), (4, 4, 4), (5, 3, 1), (7, 6, 5), (33, 9, 4),
+                                 (64, 3, 3), (130, 2, 9)])
+def test_stencil_codes_give_the_markers_diagonal(ctx, res):
+    """The codes' four-cell words and their edges (rows shorter than a word, the
+    first and last plane, a last word that is not full): one damped Jacobi sweep
+    from zero is r / d with d from the markers, neighbour by neighbour."""
+    rng = np.random.default_rng(sum(res))
+    n = int(np.prod(res))
+    sdf = np.where(rng.random(n) < 0.25, -1.0, 1.0).astype(np.float32)
+    phi = np.where(rng.random(n) < 0.6, -1.0, 1.0).astype(np.float32)
+    h, dt = (0.1, 0.2, 0.3), 0.01
+    s = mgf.Scene(ctx, mgf.make_desc(res, (0, 0, 0), h, dt, tol_mode=mgf.TOL_RELATIVE, tol=1e-6,
+                                     precision=mgf.PRECISION_MIXED, precond=mgf.PRECOND_JACOBI))
+    s.add_solid(sdf)
+    s.update_boundaries()                       # the solid marker, which a step would refresh
+    s.upload(3, phi)
+    r = rng.standard_normal(n).astype(np.float32)
+    z, _ = s.apply_preconditioner(r)
+    s.close()
+    shape = res[::-1]
+    solid, wet = (sdf < 0).reshape(shape), ((phi < 0) & ~(sdf < 0)).reshape(shape)
+    d = np.zeros(shape)
+    for axis in range(3):                       # z, y, x
+        scale = dt / h[2 - axis] ** 2           # density 1
+        free = ~solid
+        up = np.zeros(shape); dn = np.zeros(shape)
+        sl = lambda a, b: tuple(slice(a, b) if k == axis else slice(None) for k in range(3))
+        up[sl(0, -1)] = free[sl(1, None)]
+        dn[sl(1, None)] = free[sl(0, -1)]
+        d += scale * (up + dn)
+    want = np.where(wet & (d > 0), r.reshape(shape) / np.where(d > 0, d, 1.0), 0.0).ravel()
+    # d sums at most six rounded scales, one reciprocal and one product: 9 roundings
+    assert np.all(np.abs(z - want) <= 9 * 2.0 ** -23 * np.abs(want))
+
+
 @pytest.mark.parametrize("res", [(1, 40, 33), (37, 1, 20), (33, 25, 1)])
 def test_fused_vcycle_2d_grids(ctx, res):
     """A grid with an axis of one cell: no level is fused (every axis must
