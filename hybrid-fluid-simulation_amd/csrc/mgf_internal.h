@@ -373,6 +373,9 @@ double flat_wet_cells(const GridDev& g, const uint16_t* wet_host);
 // Dot products left to the kernel that needs them (Fold, mgf_kernels_mg.hip)
 // instead of a finishing launch: r . z of the level-0 ascent (its partials,
 // with_rz = kRzLeft) to K_I, p . Ap to K_II, r . r to the level-0 brick descent.
+// Each is folded or not by its own count of partials (a marched level of 96 x 96
+// x 64 cells has 512 of r . z, its flat kernels 576 of p . Ap), so none may rest
+// on another one being folded too.
 constexpr uint32_t kFoldMax = 512;
 struct CgFold {
     uint32_t rz = 0;      // partials of r . z K_I finishes

@@ -355,7 +355,7 @@ __device__ __forceinline__ void finish_scalars(CgScalars* sc, int kind, double t
 // finish_chain's order, so bit for bit k_finish's) and decides alike, and the
 // first one stores the scalars.  What is stored is not read by the others,
 // except done, which tells a work-group what it would find itself.  The
-// partials lie where the kernel does not write its own (fold_slots).  Worth it
+// partials lie where the kernel does not write its own (pap_slots).  Worth it
 // while the partials are few (kFoldMax): a launch between two kernels costs about
 // 3.5 us, the sum in each work-group about 1 us with 40 partials (34^3, four
 // steps: 3.79 -> 3.45 ms) and as much as the launch with a thousand (152 x 63 x
@@ -2771,21 +2771,26 @@ hipError_t launch_finish_rz(hipStream_t s, CgScalars* sc, ReduceBuf red, uint32_
     return finish(s, red.partials, count, sc, kFinishRz);
 }
 
-// K_I's partials when K_II finishes them: the end of the buffer, so that K_II
-// (whose own partials start it) and K_I (which reads r . z's there) do not
-// write what they read.  red_capacity() is at least 16 kFoldMax doubles.
-static double* fold_slots(ReduceBuf red, uint32_t G) { return red.partials + (red_capacity(G) - G); }
+// K_I's partials: the G words at the end of the buffer.  Where fold.rz is set,
+// every work-group of K_I reads r . z's partials at the buffer's start while
+// others store theirs, and K_II's own start it while it reads K_I's; so the
+// two places may not meet, whichever of the sums is folded.  They do not: the
+// buffer holds at least 2 G doubles and 2 kMaxBlocks, a folded sum has at most
+// kFoldMax (launch_col_p_ap refuses more).
+static_assert(kFoldMax <= uint32_t(kMaxBlocks), "r . z's folded partials end before K_I's begin");
+static double* pap_slots(ReduceBuf red, uint32_t G) { return red.partials + (red_capacity(G) - G); }
 
 hipError_t launch_col_p_ap(hipStream_t s, const GridDev& g, const float scale[3], const uint16_t* codes,
                            const float* zv, float* p, float* ap, CgScalars* sc, ReduceBuf red, const uint16_t* wet,
                            const CgFold& fold) {
     const Flat F = make_flat(g.nx, g.ny, g.nz);
     const uint32_t G = flat_grid(F.n);
-    double* part = fold.alpha ? fold_slots(red, G) : red.partials;
+    if (fold.rz > kFoldMax) return hipErrorInvalidValue;
+    double* part = pap_slots(red, G);
     hipError_t e = LAUNCH(k_cg_pap, G, F, codes, scale[0], scale[1], scale[2], zv, p, ap, sc, part, wet,
                           (Fold{red.partials, fold.rz, sc}));
     if (e != hipSuccess || fold.alpha) return e;
-    return finish(s, red.partials, G, sc, kFinishAlpha);
+    return finish(s, part, G, sc, kFinishAlpha);
 }
 
 hipError_t launch_col_update(hipStream_t s, const GridDev& g, const float* p, const float* ap, float* x, float* r,
@@ -2793,7 +2798,7 @@ hipError_t launch_col_update(hipStream_t s, const GridDev& g, const float* p, co
     const Flat F = make_flat(g.nx, g.ny, g.nz);
     const uint32_t G = flat_grid(F.n);
     hipError_t e = LAUNCH(k_cg_update, G, F, p, ap, x, r, sc, red.partials, wet,
-                          (Fold{fold_slots(red, G), fold.alpha ? G : 0u, sc}));
+                          (Fold{pap_slots(red, G), fold.alpha ? G : 0u, sc}));
     if (e != hipSuccess || fold.rr) return e;
     return finish(s, red.partials, G, sc, identity ? kFinishRrIdent : kFinishRr);
 }

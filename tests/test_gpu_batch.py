@@ -65,14 +65,9 @@ def test_batch_matches_scenes_stepped_alone(ctx, precision, precond):
         s.close()
 
 
-@pytest.mark.parametrize("precond", [mgf.PRECOND_MULTIGRID, mgf.PRECOND_JACOBI, mgf.PRECOND_IDENTITY])
-@pytest.mark.parametrize("res", [(2, 2, 2), (9, 9, 9), (40, 25, 30), (64, 64, 64), (80, 80, 81), (82, 80, 80),
-                                 (84, 80, 78)])
-def test_dot_products_finished_by_their_consumers(ctx, res, precond):
-    """A scene alone lets the kernels that need a dot product finish it (up to
-    512 partials, 512K cells: one less, that many and one more); in a batch each
-    is a launch of its own.  The same bits and counts, also when the iterations
-    end before the tolerance and when there is nothing to solve."""
+def compare_alone_with_batch(ctx, res, precond=mgf.PRECOND_MULTIGRID, mg_kernels=mgf.MG_AUTO):
+    """One step of a scene alone (which folds dot products) and in a batch
+    (which does not): the same bits and counts."""
     rng = np.random.default_rng(sum(res))
     phi = np.where(rng.random(int(np.prod(res))) < 0.6, -1.0, 1.0).astype(np.float32)
     phi[0] = 1.0
@@ -82,7 +77,7 @@ def test_dot_products_finished_by_their_consumers(ctx, res, precond):
         pair = []
         for _ in range(3):
             d = mgf.make_desc(res, (0, 0, 0), (0.1, 0.1, 0.1), 0.003, rk=mgf.RK1, tol_mode=mgf.TOL_RELATIVE, tol=1e-6,
-                              max_it=max_it, precision=mgf.PRECISION_MIXED, precond=precond,
+                              max_it=max_it, precision=mgf.PRECISION_MIXED, precond=precond, mg_kernels=mg_kernels,
                               gravity=(0, 0, 0) if still else (0, -9.8, 0))
             s = mgf.Scene(ctx, d)
             s.upload(mgf.FIELD["fluid_domain"], phi)
@@ -99,6 +94,39 @@ def test_dot_products_finished_by_their_consumers(ctx, res, precond):
         assert_same(snapshot(pair[0]), snapshot(pair[2]), "res %s" % (res,))
         for s in pair:
             s.close()
+
+
+@pytest.mark.parametrize("precond", [mgf.PRECOND_MULTIGRID, mgf.PRECOND_JACOBI, mgf.PRECOND_IDENTITY])
+@pytest.mark.parametrize("res", [(2, 2, 2), (9, 9, 9), (40, 25, 30), (64, 64, 64), (80, 80, 81), (82, 80, 80),
+                                 (84, 80, 78)])
+def test_dot_products_finished_by_their_consumers(ctx, res, precond):
+    """A scene alone lets the kernels that need a dot product finish it (up to
+    512 partials, 512K cells: one less, that many and one more); in a batch each
+    is a launch of its own.  The same bits and counts, also when the iterations
+    end before the tolerance and when there is nothing to solve."""
+    compare_alone_with_batch(ctx, res, precond=precond)
+
+
+def fold_counts(res):
+    """Partials of p . Ap and r . r (blocks of 1024 cells), and of r . z where
+    level 0 takes bricks (8^3 cells) or marches (26 x 26 x 2)."""
+    up = lambda a, b: -(-a // b)
+    return (up(res[0] * res[1] * res[2], 1024), up(res[0], 8) * up(res[1], 8) * up(res[2], 8),
+            up(res[0], 26) * up(res[1], 26) * up(res[2], 2))
+
+
+@pytest.mark.parametrize("res,kernels,rz_folded,pap_folded", [
+    ((96, 96, 64), mgf.MG_AUTO, True, False), ((100, 100, 64), mgf.MG_AUTO, True, False),
+    ((104, 104, 60), mgf.MG_AUTO, True, False), ((78, 78, 98), mgf.MG_AUTO, True, False),
+    ((64, 64, 64), mgf.MG_FUSED, True, True), ((104, 104, 40), mgf.MG_FUSED, True, True),
+    ((78, 80, 82), mgf.MG_FUSED, True, True), ((80, 80, 80), mgf.MG_FUSED, False, True)])
+def test_dot_products_folded_on_a_marched_level(ctx, res, kernels, rz_folded, pap_folded):
+    """Level 0 marches: K_I finishes r . z (up to 512 partials) whether or not
+    K_II finishes p . Ap, and K_I's own partials stay clear of those it reads."""
+    flat, _, march = fold_counts(res)
+    assert kernels == mgf.MG_FUSED or res[0] * res[1] * res[2] >= 1 << 19      # it marches
+    assert (march <= 512, flat <= 512) == (rz_folded, pap_folded)
+    compare_alone_with_batch(ctx, res, mg_kernels=kernels)
 
 
 def test_batch_without_latency_and_repeat(ctx):
