@@ -355,7 +355,10 @@ __device__ __forceinline__ void finish_scalars(CgScalars* sc, int kind, double t
 // finish_chain's order, so bit for bit k_finish's) and decides alike, and the
 // first one stores the scalars.  What is stored is not read by the others,
 // except done, which tells a work-group what it would find itself.  The
-// partials lie where the kernel does not write its own (pap_slots).  Worth it
+// partials lie where the kernel does not write its own (pap_slots).  The waves
+// of a work-group may load done on either side of the first one's store, so
+// they agree on it before any of them leaves: one that left alone would take
+// its part of the sum with it.  Worth it
 // while the partials are few (kFoldMax): a launch between two kernels costs about
 // 3.5 us, the sum in each work-group about 1 us with 40 partials (34^3, four
 // steps: 3.79 -> 3.45 ms) and as much as the launch with a thousand (152 x 63 x
@@ -367,17 +370,25 @@ struct Fold {
     CgScalars* sc;
 };
 
-// The sum, in every work-item (called by all work-items of the block).
-__device__ __forceinline__ double fold_sum(const Fold& f) {
+// The sum t, in every work-item (called by all work-items of the block); false,
+// for all of them, if a wave found done.
+__device__ __forceinline__ bool fold_sum(const Fold& f, double& t) {
     __shared__ double sh[kFinishWaves];
-    const uint32_t lane = threadIdx.x & 63u, waves = blockDim.x >> 6;
-    for (uint32_t v = threadIdx.x >> 6; v < uint32_t(kFinishWaves); v += waves) {
+    __shared__ int over[kFinishWaves];
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
+    const int done = __builtin_amdgcn_readfirstlane(f.sc->done);
+    if (lane == 0) over[wave] = done;
+    for (uint32_t v = wave; v < uint32_t(kFinishWaves) && !done; v += waves) {
         double s = 0.0;
         if (v * 64u < f.count) s = wave_sum(finish_chain(f.part, f.count, v * 64u + lane));
         if (lane == 0) sh[v] = s;
     }
     __syncthreads();
-    return finish_total(sh);
+    int any = 0;
+    for (uint32_t q = 0; q < waves; ++q) any |= over[q];
+    if (any) return false;
+    t = finish_total(sh);
+    return true;
 }
 
 // Cells per work-item of the fine-grid kernels (256 apart): fewer block
@@ -500,15 +511,16 @@ __device__ __forceinline__ void cg_pap_run(Flat F, const uint16_t* __restrict__ 
                                            double* __restrict__ part, const uint16_t* __restrict__ wet,
                                            const Fold& rz, uint32_t blk, uint32_t slot) {
     __shared__ float aw[64];
-    if (sc->done) return;
     const bool first = sc->iters == 0;
     float beta;
     if (rz.count) {
-        const double t = fold_sum(rz);
+        double t;
+        if (!fold_sum(rz, t)) return;
         beta = float(first ? 0.0 : t / sc->rz);
         if (slot == 0 && threadIdx.x == 0) finish_scalars(rz.sc, kFinishRz, t, 0.0, 0.0);
         if (!isfinite(t)) return;
     } else {
+        if (sc->done) return;
         beta = float(sc->beta);
     }
     const uint32_t mask = (!first && wet) ? wet[blk] : kSegAll;
@@ -593,14 +605,15 @@ __device__ __forceinline__ void cg_update_run(Flat F, const float* __restrict__ 
                                               const CgScalars* __restrict__ sc, double* __restrict__ part,
                                               const uint16_t* __restrict__ wet, const Fold& pap, uint32_t blk,
                                               uint32_t slot) {
-    if (sc->done) return;
     double alpha;
     if (pap.count) {
-        const double t = fold_sum(pap);
+        double t;
+        if (!fold_sum(pap, t)) return;
         alpha = sc->rz_new / t;
         if (slot == 0 && threadIdx.x == 0) finish_scalars(pap.sc, kFinishAlpha, t, 0.0, 0.0);
         if (!isfinite(t) || t == 0.0) return;
     } else {
+        if (sc->done) return;
         alpha = sc->alpha;
     }
     const uint32_t mask = wet ? wet[blk] : kSegAll;
@@ -1859,11 +1872,13 @@ __device__ __forceinline__ void brick_run(const Bricks& T, const MgLevel& L, con
     __shared__ float aw[64], w[64];
     __shared__ float xa[kBkCells], xb[kBkCells];
     __shared__ double sum[kBkThreads / 64];
-    if (sc->done) return;
     if (!POST && rr.count) {
-        const double t = fold_sum(rr);
+        double t;
+        if (!fold_sum(rr, t)) return;
         if (slot == 0 && threadIdx.x == 0) finish_scalars(rr.sc, kFinishRr, t, 0.0, 0.0);
         if (t <= sc->target2 || !isfinite(t)) return;
+    } else if (sc->done) {
+        return;
     }
     const int t = threadIdx.x;
     const uint32_t bx = blk % T.tx, br = blk / T.tx, by = br % T.ty, bz = br / T.ty;

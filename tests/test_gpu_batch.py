@@ -129,6 +129,25 @@ def test_dot_products_folded_on_a_marched_level(ctx, res, kernels, rz_folded, pa
     compare_alone_with_batch(ctx, res, mg_kernels=kernels)
 
 
+@pytest.mark.parametrize("res", [(16, 16, 16), (64, 64, 128), (88, 88, 80)])
+def test_solve_that_ends_at_a_zero_curvature(ctx, res):
+    """A closed box of fluid with a uniform divergence: r is constant, A r is
+    exactly zero and the first iteration ends the solve inside K_II (which
+    finishes p . Ap itself up to 512 blocks: 4, 512 and, for the finishing
+    launch, 605).  The pressure stays exactly zero."""
+    d = mgf.make_desc(res, (0, 0, 0), (1.0, 1.0, 1.0), 1.0, tol_mode=mgf.TOL_RELATIVE, tol=1e-6, max_it=5,
+                      precision=mgf.PRECISION_MIXED, precond=mgf.PRECOND_IDENTITY)
+    s = mgf.Scene(ctx, d)
+    s.upload(mgf.FIELD["fluid_domain"], np.full(int(np.prod(res)), -1.0, np.float32))
+    s.upload(0, np.tile(np.arange(res[0] + 1, dtype=np.float32), res[1] * res[2]))
+    st = s.pressure_solve(allow_unconverged=True)
+    assert st["cg_iterations"] == 0 and st["converged"] == 0
+    rhs = s.download(mgf.FIELD["rhs"])
+    assert np.all(rhs == rhs[0]) and rhs[0] != 0
+    assert np.all(s.download(mgf.FIELD["pressure"]) == 0.0)
+    s.close()
+
+
 def test_batch_without_latency_and_repeat(ctx):
     """Two batched calls (no per-step latency) equal one solo call of the summed
     steps; the worker count does not change the results."""
