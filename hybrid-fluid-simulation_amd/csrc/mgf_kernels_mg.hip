@@ -364,6 +364,8 @@ __device__ __forceinline__ void finish_scalars(CgScalars* sc, int kind, double t
 // steps: 3.79 -> 3.45 ms) and as much as the launch with a thousand (152 x 63 x
 // 99, 926 partials: no change; 130^3, 2152: 4.75 -> 4.84 ms).  count 0: the
 // scalars are finished.
+// The kernels' own pointer to the scalars may not be __restrict__: sc here is
+// the same struct, and is written.
 struct Fold {
     const double* part;
     uint32_t count;
@@ -507,7 +509,7 @@ struct MFlatWet {
 // writes its partial sums to slot `slot` (the launch's own block index).
 __device__ __forceinline__ void cg_pap_run(Flat F, const uint16_t* __restrict__ code, float sx, float sy, float sz,
                                            const float* __restrict__ zv, float* __restrict__ p,
-                                           float* __restrict__ ap, const CgScalars* __restrict__ sc,
+                                           float* __restrict__ ap, const CgScalars* sc,
                                            double* __restrict__ part, const uint16_t* __restrict__ wet,
                                            const Fold& rz, uint32_t blk, uint32_t slot) {
     __shared__ float aw[64];
@@ -549,7 +551,7 @@ __device__ __forceinline__ void cg_pap_run(Flat F, const uint16_t* __restrict__ 
 
 __global__ void __launch_bounds__(kBlock) k_cg_pap(Flat F, const uint16_t* __restrict__ code, float sx, float sy,
                                                    float sz, const float* __restrict__ zv, float* __restrict__ p,
-                                                   float* __restrict__ ap, const CgScalars* __restrict__ sc,
+                                                   float* __restrict__ ap, const CgScalars* sc,
                                                    double* __restrict__ part, const uint16_t* __restrict__ wet,
                                                    Fold rz) {
     cg_pap_run(F, code, sx, sy, sz, zv, p, ap, sc, part, wet, rz, xcd_block(), blockIdx.x);
@@ -602,7 +604,7 @@ __device__ __forceinline__ double cg_update_body(const Flat& F, uint32_t base, c
 
 __device__ __forceinline__ void cg_update_run(Flat F, const float* __restrict__ p, const float* __restrict__ ap,
                                               float* __restrict__ x, float* __restrict__ r,
-                                              const CgScalars* __restrict__ sc, double* __restrict__ part,
+                                              const CgScalars* sc, double* __restrict__ part,
                                               const uint16_t* __restrict__ wet, const Fold& pap, uint32_t blk,
                                               uint32_t slot) {
     double alpha;
@@ -633,7 +635,7 @@ __device__ __forceinline__ void cg_update_run(Flat F, const float* __restrict__ 
 
 __global__ void __launch_bounds__(kBlock) k_cg_update(Flat F, const float* __restrict__ p,
                                                       const float* __restrict__ ap, float* __restrict__ x,
-                                                      float* __restrict__ r, const CgScalars* __restrict__ sc,
+                                                      float* __restrict__ r, const CgScalars* sc,
                                                       double* __restrict__ part, const uint16_t* __restrict__ wet,
                                                       Fold pap) {
     cg_update_run(F, p, ap, x, r, sc, part, wet, pap, xcd_block(), blockIdx.x);
@@ -1867,7 +1869,7 @@ __device__ __forceinline__ void brick_run(const Bricks& T, const MgLevel& L, con
                                           const float* __restrict__ b, const float* __restrict__ xi,
                                           const float* __restrict__ xc, float* __restrict__ xo,
                                           const uint16_t* __restrict__ codec, float* __restrict__ bco, float omega,
-                                          const CgScalars* __restrict__ sc, double* __restrict__ part, const Fold& rr,
+                                          const CgScalars* sc, double* __restrict__ part, const Fold& rr,
                                           uint32_t blk, uint32_t slot) {
     __shared__ float aw[64], w[64];
     __shared__ float xa[kBkCells], xb[kBkCells];
@@ -1983,7 +1985,7 @@ __global__ void __launch_bounds__(kBkThreads) k_mg_brick(Bricks T, MgLevel L, co
                                                          const float* __restrict__ b, const float* __restrict__ xi,
                                                          const float* __restrict__ xc, float* __restrict__ xo,
                                                          const uint16_t* __restrict__ codec, float* __restrict__ bco,
-                                                         float omega, const CgScalars* __restrict__ sc,
+                                                         float omega, const CgScalars* sc,
                                                          double* __restrict__ part, Fold rr) {
     brick_run<POST, RZ>(T, L, code, b, xi, xc, xo, codec, bco, omega, sc, part, rr, blockIdx.x, blockIdx.x);
 }
