@@ -1884,6 +1884,7 @@ void pool_release(mgf_context ctx) {
 }
 
 OpScratch::OpScratch(mgf_context ctx, size_t bytes) : buf(ctx->op) {
+    if (bytes == 0) return;
     kept = bytes <= kOpScratchKeep && buf.mu.try_lock();
     if (kept && buf.bytes < bytes) {
         if (buf.p) (void)hipFree(buf.p);
@@ -2848,8 +2849,8 @@ mgf_status mgf_op_particles_to_grid(mgf_context ctx, const mgf_grid* grid, int32
         return fail(MGF_ERR_INVALID, "particle-to-grid algorithm must be P2GSUM, LINEAR, QUADRATIC or CUBIC");
     MGF_HIP(hipSetDevice(ctx->device));
     const GridDev g = make_grid(grid);
-    OpScratch work(ctx, sizeof(uint32_t) * p2g_work_words(g, n));
-    if (!work.p) return fail(MGF_ERR_NOMEM, "particle splat scratch");
+    // without scratch (none needed, or none to be had) the splat does not sort
+    OpScratch work(ctx, sizeof(uint32_t) * p2g_work_words(g, n, alg));
     const hipError_t e = launch_p2g(ctx->stream, g, field_kind, n, pos, values, span, offset, alg, field, weight,
                                     normalize, static_cast<uint32_t*>(work.p));
     const hipError_t w = hipStreamSynchronize(ctx->stream);   // also after a failed launch: the scratch is returned

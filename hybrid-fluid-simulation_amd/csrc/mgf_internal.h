@@ -594,8 +594,8 @@ hipError_t launch_fluid_sdf(hipStream_t s, const GridDev& g, const float* phi, i
                             float* out);
 // ---- particles (mgf_kernels_particles.hip); kind 0 cells, 1..3 face grids ----
 size_t pg_field_count(const GridDev& g, int kind);
-// work: p2g_work_words(g, np) words of scratch.
-size_t p2g_work_words(const GridDev& g, int64_t np);
+// work: p2g_work_words words of scratch, or null (the splat then does not sort).
+size_t p2g_work_words(const GridDev& g, int64_t np, int alg);
 hipError_t launch_p2g(hipStream_t s, const GridDev& g, int kind, int64_t np, const float* pos, const float* val,
                       int span, int off, int alg, float* field, float* weight, int normalize, uint32_t* work);
 hipError_t launch_g2p(hipStream_t s, const GridDev& g, int kind, int64_t np, const float* pos, const float* field,

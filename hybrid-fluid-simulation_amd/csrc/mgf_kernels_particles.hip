@@ -125,11 +125,16 @@ constexpr int kTileEdge = 8;
 constexpr int kSplatBlock = kTileEdge * kTileEdge * kTileEdge;   // a work-item a cell
 constexpr uint32_t kSplatRounds = 4;
 constexpr uint32_t kSplatChunk = kSplatRounds * kSplatBlock;
+// Particles of a cell summed by its own work-item; what a denser cell holds
+// beyond is summed by all work-items, kSplatRounds each.
+constexpr uint32_t kSplatCell = 64;
 // Particles sorted at a time: bounds the scratch; the sums just continue.
 constexpr int64_t kSplatSegment = int64_t(1) << 24;
-// The tile counts of a work-group's particles go through LDS up to this many
-// tiles (32 KB); beyond, straight to the global counters (a loosely sorted
-// set then has few particles of many tiles, and no counter is crowded).
+// A work-group of the sort counts its particles through LDS in a window of this
+// many tiles (32 KB) around the tile of one of them: all tiles of a grid of up
+// to 160^3 cells; beyond, the tiles of the particles' neighbourhood, since sets
+// are generated cell by cell and move little against their order.  Particles
+// outside the window take global atomics, one a tile and wave.
 constexpr uint32_t kSplatLdsTiles = 8192;
 constexpr uint32_t kSplatItems = 16;                             // particles a work-item of those passes
 
@@ -195,103 +200,159 @@ __global__ void __launch_bounds__(kBlock) k_splat_clear(size_t n, float* __restr
     if (i < nt) counts[i] = 0u;
 }
 
-// counts[t] += this work-group's particles of tile t.  lds_tiles (dynamic LDS
-// words): the number of tiles, or 0 for global atomics.
+// First tile of a work-group's window of min(nt, kSplatLdsTiles): around the
+// tile of a particle in its middle.
+template <int ALG>
+__device__ __forceinline__ uint32_t splat_window(const PGrid& g, uint32_t np, const float* __restrict__ pos, uint32_t base,
+                                                 uint32_t nt) {
+    if (nt <= kSplatLdsTiles) return 0;
+    const uint32_t p = base + kBlock * kSplatItems / 2;
+    const uint32_t t = splat_at<ALG>(g, pos, p < np ? p : np - 1).tile;
+    return t < kSplatLdsTiles / 2 ? 0 : min(t - kSplatLdsTiles / 2, nt - kSplatLdsTiles);
+}
+
+// The lanes of the wave with `on` and this lane's tile (0 where not on).
+__device__ __forceinline__ uint64_t same_tile(bool on, uint32_t tile) {
+    uint64_t mine = 0;
+    for (uint64_t todo = __ballot(on); todo;) {
+        const uint32_t t = uint32_t(__builtin_amdgcn_readlane(int(tile), __ffsll((unsigned long long)todo) - 1));
+        const uint64_t same = __ballot(on && tile == t);
+        if (on && tile == t) mine = same;
+        todo &= ~same;
+    }
+    return mine;
+}
+__device__ __forceinline__ uint32_t rank_in(uint64_t lanes) {
+    return __builtin_amdgcn_mbcnt_hi(uint32_t(lanes >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(lanes), 0u));
+}
+
+// counts[t] += this work-group's particles of tile t.  Dynamic LDS: the window.
 template <int ALG>
 __global__ void __launch_bounds__(kBlock) k_splat_count(PGrid g, uint32_t np, const float* __restrict__ pos,
-                                                        uint32_t* counts, uint32_t lds_tiles) {
+                                                        uint32_t* counts, uint32_t nt) {
     extern __shared__ uint32_t hist[];
     const uint32_t base = blockIdx.x * (kBlock * kSplatItems);
-    for (uint32_t i = threadIdx.x; i < lds_tiles; i += kBlock) hist[i] = 0u;
+    const uint32_t win = min(nt, kSplatLdsTiles), lo = splat_window<ALG>(g, np, pos, base, nt);
+    for (uint32_t i = threadIdx.x; i < win; i += kBlock) hist[i] = 0u;
     __syncthreads();
 #pragma unroll 4
     for (uint32_t j = 0; j < kSplatItems; ++j) {
+        if (base + j * kBlock >= np) break;   // the same for every work-item
         const uint32_t p = base + j * kBlock + threadIdx.x;
-        if (p < np) {
-            const uint32_t t = splat_at<ALG>(g, pos, p).tile;
-            if (lds_tiles) atomicAdd(&hist[t], 1u);
-            else atomicAdd(&counts[t], 1u);
+        const uint32_t t = splat_at<ALG>(g, pos, p < np ? p : np - 1).tile;
+        if (p < np && t - lo < win) atomicAdd(&hist[t - lo], 1u);
+        if (win < nt) {
+            const uint64_t mine = same_tile(p < np && t - lo >= win, t);
+            if (mine && rank_in(mine) == 0) atomicAdd(&counts[t], uint32_t(__popcll(mine)));
         }
     }
     __syncthreads();
-    for (uint32_t i = threadIdx.x; i < lds_tiles; i += kBlock)
-        if (hist[i]) atomicAdd(&counts[i], hist[i]);
+    for (uint32_t i = threadIdx.x; i < win; i += kBlock)
+        if (hist[i]) atomicAdd(&counts[lo + i], hist[i]);
 }
 
 // One work-group: counts -> start (exclusive prefix, start[nt] = the total)
 // and cursor, and the chunks in tile order: work[2 j] = tile, work[2 j + 1] =
-// its first sorted particle; *nwork = their number.
+// its first sorted particle; *nwork = their number.  counts is 16-byte aligned
+// and readable up to the next multiple of four words.
 __global__ void __launch_bounds__(1024) k_splat_scan(uint32_t nt, const uint32_t* __restrict__ counts,
                                                      uint32_t* __restrict__ start, uint32_t* __restrict__ cursor,
                                                      uint32_t* __restrict__ work, uint32_t* __restrict__ nwork) {
-    __shared__ uint32_t pp[1024], pc[1024];
-    const uint32_t t = threadIdx.x, per = (nt + 1023) / 1024;
-    const uint32_t b = min(nt, t * per), e = min(nt, b + per);
-    uint32_t sp = 0, sc = 0;
-    for (uint32_t i = b; i < e; ++i) {
-        const uint32_t c = counts[i];
-        sp += c;
-        sc += (c + kSplatChunk - 1) / kSplatChunk;
-    }
-    pp[t] = sp;
-    pc[t] = sc;
-    __syncthreads();
-    for (uint32_t o = 1; o < 1024; o <<= 1) {
-        const uint32_t vp = t >= o ? pp[t - o] : 0u, vc = t >= o ? pc[t - o] : 0u;
-        __syncthreads();
-        pp[t] += vp;
-        pc[t] += vc;
-        __syncthreads();
-    }
-    uint32_t run = t ? pp[t - 1] : 0u, w = t ? pc[t - 1] : 0u;
-    for (uint32_t i = b; i < e; ++i) {
-        const uint32_t c = counts[i];
-        start[i] = run;
-        cursor[i] = run;
-        for (uint32_t q = 0; q < c; q += kSplatChunk, ++w) {
-            work[2 * size_t(w)] = i;
-            work[2 * size_t(w) + 1] = run + q;
+    __shared__ uint32_t sp[16], sc[16];
+    const uint32_t t = threadIdx.x, lane = t & 63u, wave = t >> 6;
+    uint32_t run = 0, w = 0;   // particles and chunks of the tiles before
+    for (uint32_t b = 0; b < nt; b += 4096) {
+        const uint32_t i = b + 4 * t;
+        uint4 c4 = make_uint4(0u, 0u, 0u, 0u);
+        if (i < nt) c4 = *reinterpret_cast<const uint4*>(counts + i);
+        const uint32_t c[4] = {c4.x, i + 1 < nt ? c4.y : 0u, i + 2 < nt ? c4.z : 0u, i + 3 < nt ? c4.w : 0u};
+        uint32_t ip = 0, ic = 0;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            ip += c[k];
+            ic += (c[k] + kSplatChunk - 1) / kSplatChunk;
         }
-        run += c;
+        const uint32_t mp = ip, mc = ic;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t up = uint32_t(__shfl_up(int(ip), o, 64)), uc = uint32_t(__shfl_up(int(ic), o, 64));
+            if (lane >= uint32_t(o)) {
+                ip += up;
+                ic += uc;
+            }
+        }
+        if (lane == 63) {
+            sp[wave] = ip;
+            sc[wave] = ic;
+        }
+        __syncthreads();
+        uint32_t q = run + ip - mp, j = w + ic - mc;
+#pragma unroll
+        for (uint32_t v = 0; v < 16; ++v) {
+            const uint32_t vp = sp[v], vc = sc[v];
+            if (v < wave) {
+                q += vp;
+                j += vc;
+            }
+            run += vp;
+            w += vc;
+        }
+        __syncthreads();
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k) {
+            if (i + k >= nt) break;
+            start[i + k] = q;
+            cursor[i + k] = q;
+            for (uint32_t e = 0; e < c[k]; e += kSplatChunk, ++j) {
+                work[2 * size_t(j)] = i + k;
+                work[2 * size_t(j) + 1] = q + e;
+            }
+            q += c[k];
+        }
     }
-    if (t == 1023) {
-        start[nt] = pp[1023];
-        *nwork = pc[1023];
+    if (t == 0) {
+        start[nt] = run;
+        *nwork = w;
     }
 }
 
-// order = the particles by tile.  With lds_tiles a work-group ranks its
-// particles of a tile in LDS and reserves their slots with one atomic.
+// order = the particles by tile.  A work-group ranks its particles of a tile
+// in LDS and reserves their slots with one atomic a tile (outside the window a
+// wave does).
 template <int ALG>
 __global__ void __launch_bounds__(kBlock) k_splat_order(PGrid g, uint32_t np, const float* __restrict__ pos,
-                                                        uint32_t* cursor, uint32_t* __restrict__ order,
-                                                        uint32_t lds_tiles) {
+                                                        uint32_t* cursor, uint32_t* __restrict__ order, uint32_t nt) {
     extern __shared__ uint32_t hist[];
     const uint32_t base = blockIdx.x * (kBlock * kSplatItems);
-    if (!lds_tiles) {
-        for (uint32_t j = 0; j < kSplatItems; ++j) {
-            const uint32_t p = base + j * kBlock + threadIdx.x;
-            if (p < np) order[atomicAdd(&cursor[splat_at<ALG>(g, pos, p).tile], 1u)] = p;
+    const uint32_t win = min(nt, kSplatLdsTiles), lo = splat_window<ALG>(g, np, pos, base, nt);
+    for (uint32_t i = threadIdx.x; i < win; i += kBlock) hist[i] = 0u;
+    __syncthreads();
+    uint32_t tile[kSplatItems], rank[kSplatItems];   // tile: in the window
+#pragma unroll
+    for (uint32_t j = 0; j < kSplatItems; ++j) {
+        tile[j] = ~0u;
+        if (base + j * kBlock >= np) continue;   // the same for every work-item
+        const uint32_t p = base + j * kBlock + threadIdx.x;
+        const uint32_t t = splat_at<ALG>(g, pos, p < np ? p : np - 1).tile;
+        if (p < np) tile[j] = t - lo;
+        rank[j] = tile[j] < win ? atomicAdd(&hist[tile[j]], 1u) : 0u;
+        if (win < nt) {
+            const uint64_t mine = same_tile(p < np && tile[j] >= win, t);
+            const uint32_t r = rank_in(mine);
+            uint32_t at = 0;
+            if (mine && r == 0) at = atomicAdd(&cursor[t], uint32_t(__popcll(mine)));
+            at = uint32_t(__shfl(int(at), mine ? __ffsll((unsigned long long)mine) - 1 : 0, 64));
+            if (mine) order[at + r] = p;
         }
-        return;
-    }
-    for (uint32_t i = threadIdx.x; i < lds_tiles; i += kBlock) hist[i] = 0u;
-    __syncthreads();
-    uint32_t tile[kSplatItems], rank[kSplatItems];
-#pragma unroll
-    for (uint32_t j = 0; j < kSplatItems; ++j) {
-        const uint32_t p = base + j * kBlock + threadIdx.x;
-        tile[j] = p < np ? splat_at<ALG>(g, pos, p).tile : 0u;
-        rank[j] = p < np ? atomicAdd(&hist[tile[j]], 1u) : 0u;
     }
     __syncthreads();
-    for (uint32_t i = threadIdx.x; i < lds_tiles; i += kBlock)
-        if (hist[i]) hist[i] = atomicAdd(&cursor[i], hist[i]);
+    for (uint32_t i = threadIdx.x; i < win; i += kBlock)
+        if (hist[i]) hist[i] = atomicAdd(&cursor[lo + i], hist[i]);
     __syncthreads();
 #pragma unroll
     for (uint32_t j = 0; j < kSplatItems; ++j) {
         const uint32_t p = base + j * kBlock + threadIdx.x;
-        if (p < np) order[hist[tile[j]] + rank[j]] = p;
+        if (tile[j] < win) order[hist[tile[j]] + rank[j]] = p;
     }
 }
 
@@ -340,8 +401,8 @@ __global__ void __launch_bounds__(kSplatBlock) k_splat_tiles(PGrid g, const floa
     __syncthreads();
     uint32_t q = incl - mine;
     for (int w = 0; w < (t >> 6); ++w) q += wsum[w];
-    first[t] = q;
-    __syncthreads();
+    first[t] = q;   // as it stays
+    const bool dense = __syncthreads_or(mine > kSplatCell);
 #pragma unroll
     for (uint32_t j = 0; j < kSplatRounds; ++j)
         if (j * kSplatBlock + t < n) part[first[cell[j]] + rank[j]] = v[j];
@@ -350,8 +411,7 @@ __global__ void __launch_bounds__(kSplatBlock) k_splat_tiles(PGrid g, const floa
     float av[N * N * N], aw[N * N * N];
 #pragma unroll
     for (int k = 0; k < N * N * N; ++k) av[k] = aw[k] = 0.0f;
-    for (const uint32_t q1 = q + mine; q < q1; ++q) {
-        const float4 s = part[q];
+    auto add = [&](const float4& s) {
         if constexpr (ALG == MGF_PG_P2GSUM) {
             av[0] += s.w;
         } else {
@@ -371,7 +431,7 @@ __global__ void __launch_bounds__(kSplatBlock) k_splat_tiles(PGrid g, const floa
                     atomicAdd(&field[node], wt * s.w);
                     atomicAdd(&weight[node], wt);
                 });
-                continue;
+                return;
             }
 #pragma unroll
             for (int z = 0; z < N; ++z)
@@ -384,15 +444,50 @@ __global__ void __launch_bounds__(kSplatBlock) k_splat_tiles(PGrid g, const floa
                         aw[(z * N + y) * N + x] += wt;
                     }
         }
-    }
-    const int at = ((t / (kTileEdge * kTileEdge)) * E + (t / kTileEdge) % kTileEdge) * E + t % kTileEdge;
+    };
+    // LDS place of corner k of the cell with lowest node `at`
+    auto corner = [](int at, int k) { return at + ((k / (N * N)) * E + (k / N) % N) * E + k % N; };
+    auto node_of = [](uint32_t c) {
+        return ((int(c) / (kTileEdge * kTileEdge)) * E + (int(c) / kTileEdge) % kTileEdge) * E + int(c) % kTileEdge;
+    };
+    for (const uint32_t q1 = q + min(mine, kSplatCell); q < q1; ++q) add(part[q]);
+    const int at = node_of(uint32_t(t));
 #pragma unroll
     for (int k = 0; k < N * N * N; ++k) {
-        const int o = at + ((k / (N * N)) * E + (k / N) % N) * E + k % N;
         if (mine) {
-            sv[o] += av[k];
-            if (ALG != MGF_PG_P2GSUM) sw[o] += aw[k];
+            sv[corner(at, k)] += av[k];
+            if (ALG != MGF_PG_P2GSUM) sw[corner(at, k)] += aw[k];
         }
+        __syncthreads();
+    }
+    // Cells of more than kSplatCell particles: a work-item sums the rest of
+    // kSplatRounds consecutive ones and adds them to the tile by atomics, once
+    // a cell.
+    if (dense) {
+        uint32_t cur = ~0u;
+        auto flush = [&]() {
+            if (cur == ~0u) return;
+            const int o = node_of(cur);
+#pragma unroll
+            for (int k = 0; k < N * N * N; ++k) {
+                atomicAdd(&sv[corner(o, k)], av[k]);
+                if (ALG != MGF_PG_P2GSUM) atomicAdd(&sw[corner(o, k)], aw[k]);
+            }
+        };
+        const uint32_t b = uint32_t(t) * kSplatRounds, e = min(n, b + kSplatRounds);
+        for (uint32_t i = b; i < e; ++i) {
+            const float4 s = part[i];
+            const uint32_t c = splat_at<ALG>(g, s.x, s.y, s.z).cell;
+            if (i - first[c] < kSplatCell) continue;
+            if (c != cur) {
+                flush();
+                cur = c;
+#pragma unroll
+                for (int k = 0; k < N * N * N; ++k) av[k] = aw[k] = 0.0f;
+            }
+            add(s);
+        }
+        flush();
         __syncthreads();
     }
     const uint32_t ntx = splat_tiles(g.nx, N), nty = splat_tiles(g.ny, N);
@@ -404,6 +499,78 @@ __global__ void __launch_bounds__(kSplatBlock) k_splat_tiles(PGrid g, const floa
         const uint32_t node = pg_index(g, bx + i % E, by + (i / E) % E, bz + i / (E * E));
         atomicAdd(&field[node], a);
         if (ALG != MGF_PG_P2GSUM) atomicAdd(&weight[node], w);
+    }
+}
+
+// The same sums without a sort: a work-group's particles are merged in an LDS
+// hash table by node (those of a set in cell order are neighbours and share
+// the nodes of their supports), and the flush issues one global atomic a
+// distinct node.  A contribution that finds no slot within kProbe probes goes
+// straight to global memory.
+constexpr uint32_t kEmptyKey = 0xFFFFFFFFu;
+constexpr int kProbe = 32;
+
+template <int HB>
+__device__ __forceinline__ void lds_accumulate(uint32_t* keys, float* sv, float* sw, uint32_t key, float a, float b,
+                                               bool with_w, float* gf, float* gw) {
+    constexpr uint32_t T = 1u << HB;
+    uint32_t h = (key * 2654435761u) >> (32 - HB);
+    for (int probe = 0; probe < kProbe; ++probe) {
+        // a slot once claimed keeps its key: read first, claim empty slots only
+        uint32_t k = __atomic_load_n(&keys[h], __ATOMIC_RELAXED);
+        if (k == kEmptyKey) k = atomicCAS(&keys[h], kEmptyKey, key);
+        if (k == kEmptyKey || k == key) {
+            atomicAdd(&sv[h], a);
+            if (with_w) atomicAdd(&sw[h], b);
+            return;
+        }
+        h = (h + 1) & (T - 1);
+    }
+    atomicAdd(gf, a);
+    if (with_w) atomicAdd(gw, b);
+}
+
+// Tables of 1024 slots for P2GSUM and LINEAR (8 nodes a particle), 2048 for
+// the 64-node supports.
+template <int ALG>
+__global__ void __launch_bounds__(kBlock) k_p2g_hash(PGrid g, int64_t np, const float* __restrict__ pos,
+                                                     const float* __restrict__ val, int span, int off,
+                                                     float* __restrict__ field, float* __restrict__ weight) {
+    constexpr int HB = ALG == MGF_PG_P2GSUM || ALG == MGF_PG_LINEAR ? 10 : 11;
+    constexpr uint32_t T = 1u << HB;
+    __shared__ uint32_t keys[T];
+    __shared__ float sv[T], sw[T];
+    for (uint32_t i = threadIdx.x; i < T; i += kBlock) {
+        keys[i] = kEmptyKey;
+        sv[i] = 0.0f;
+        sw[i] = 0.0f;
+    }
+    __syncthreads();
+    const int64_t p = int64_t(xcd_block()) * kBlock + threadIdx.x;
+    if (p < np) {
+        const float px = pos[3 * p], py = pos[3 * p + 1], pz = pos[3 * p + 2], v = val[int64_t(span) * p + off];
+        if constexpr (ALG == MGF_PG_P2GSUM) {
+            const uint32_t node = pos_cell(g, px, py, pz);
+            lds_accumulate<HB>(keys, sv, sw, node, v, 0.0f, false, &field[node], nullptr);
+        } else {
+            PStencil st;
+            pg_stencil(g, px, py, pz, ALG, st);
+            constexpr int N = ALG == MGF_PG_LINEAR ? 2 : 4, lo = N == 2 ? 0 : -1;
+#pragma unroll 1
+            for (int k = 0; k < N * N * N; ++k) {
+                const int x = k % N, y = (k / N) % N, z = k / (N * N);
+                const uint32_t node = pg_index(g, st.i0[0] + x + lo, st.i0[1] + y + lo, st.i0[2] + z + lo);
+                const float wt = st.w[0][x] * st.w[1][y] * st.w[2][z];
+                lds_accumulate<HB>(keys, sv, sw, node, wt * v, wt, true, &field[node], &weight[node]);
+            }
+        }
+    }
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < T; i += kBlock) {
+        const uint32_t k = keys[i];
+        if (k == kEmptyKey) continue;
+        atomicAdd(&field[k], sv[i]);
+        if (ALG != MGF_PG_P2GSUM) atomicAdd(&weight[k], sw[i]);
     }
 }
 
@@ -1000,7 +1167,40 @@ static size_t splat_tile_cap(const GridDev& g) {
     return size_t(splat_tiles(g.nx + 1, 4)) * splat_tiles(g.ny + 1, 4) * splat_tiles(g.nz + 1, 4);
 }
 static size_t splat_work_cap(size_t nt, size_t seg) { return std::min(nt, seg) + seg / kSplatChunk + 1; }
-size_t p2g_work_words(const GridDev& g, int64_t np) {
+
+// Whether the splat sorts (else k_p2g_hash), by what either costs: the sort a
+// little for every tile (the scan) and more for each that holds particles (an
+// LDS tile to clear and flush), the hash table a constant (its chain of probes)
+// and more for each particle.  The constants are in ns, from particles spread
+// over whole grids, hash / sort in us:
+//   64^3 cells    100: LINEAR 39 / 34, QUADRATIC 214 / 36, CUBIC 215 / 41
+//   256^3 (36K tiles)
+//     LINEAR      100 50 / 99, 100K 125 / 270, 300K 285 / 295, 1M 824 / 439
+//     QUADRATIC   100 228 / 106, 10K 260 / 287, 100K 668 / 592, 1M 6230 / 773
+//     CUBIC       100 230 / 106, 10K 260 / 506, 100K 669 / 1500, 300K 1950 / 1760
+//   512^3 (275K)  LINEAR 1M 1010 / 1940, 3M 2500 / 2170; QUADRATIC 300K 2130 / 3210,
+//                 1M 6430 / 4620; CUBIC 1M 6420 / 12100, 3M 18600 / 13800
+// Sets that fill a part of the grid have fewer tiles with particles than is
+// assumed, so grids whose tiles fit the window sort the wide kernels at any
+// count (10K CUBIC in 0.3 of 160 x 160 x 117, three fields each way: 815 / 524; the
+// same spread over 160^3 would be some 0.1 ms a field slower than the table).
+// P2GSUM adds one value a particle and little is left to save: 300K over 64^3
+// cells 36 / 51, 1M 72 / 72, 1M over 32^3 131 / 66; 5.0M moved by up to 4 cells
+// against their order 333 / 135, but in order 76 / 106; beyond the window 40M
+// moved 1940 / 1130, in order 454 / 840, 8M in random order 442 / 1196.
+static bool splat_sorts(const GridDev& g, int64_t np, int alg) {
+    if (np <= 0) return false;
+    const double nt = double(splat_tile_cap(g)), n = double(np), held = std::min(n, nt);
+    switch (alg) {
+        case MGF_PG_P2GSUM: return n >= 786432.0 && nt <= double(kSplatLdsTiles);
+        case MGF_PG_LINEAR: return 1.4 * nt + 6.0 * held <= 12.0e3 + 0.74 * n;
+        case MGF_PG_QUADRATIC: return nt <= double(kSplatLdsTiles) || 1.4 * nt + 18.0 * held <= 170.0e3 + 6.0 * n;
+        default: return nt <= double(kSplatLdsTiles) || 1.4 * nt + 41.0 * held <= 170.0e3 + 6.0 * n;
+    }
+}
+
+size_t p2g_work_words(const GridDev& g, int64_t np, int alg) {
+    if (!splat_sorts(g, np, alg)) return 0;
     const size_t nt = splat_tile_cap(g), seg = size_t(std::min<int64_t>(std::max<int64_t>(np, 1), kSplatSegment));
     return 3 * nt + 2 + 2 * splat_work_cap(nt, seg) + seg;
 }
@@ -1013,47 +1213,53 @@ static hipError_t splat_segment(hipStream_t s, const PGrid& p, uint32_t np, cons
     const size_t nw = splat_work_cap(nt, np);
     uint32_t *counts = work, *start = counts + cap, *cursor = start + cap + 1, *nwork = cursor + cap,
              *list = nwork + 1, *order = list + 2 * splat_work_cap(cap, np);
-    const uint32_t lds = nt <= kSplatLdsTiles ? uint32_t(nt) : 0u;
+    const uint32_t lds = uint32_t(std::min<size_t>(nt, kSplatLdsTiles));
     const dim3 sg((np + kBlock * kSplatItems - 1) / (kBlock * kSplatItems));
     hipError_t e = launch_dims(k_splat_count<ALG>, "k_splat_count", sg, dim3(kBlock), lds * 4u, s, p, np, pos, counts,
-                               lds);
+                               uint32_t(nt));
     if (e != hipSuccess) return e;
     e = launch_dims(k_splat_scan, "k_splat_scan", dim3(1), dim3(1024), 0, s, uint32_t(nt), counts, start, cursor, list,
                     nwork);
     if (e == hipSuccess)
         e = launch_dims(k_splat_order<ALG>, "k_splat_order", sg, dim3(kBlock), lds * 4u, s, p, np, pos, cursor, order,
-                        lds);
+                        uint32_t(nt));
     if (e == hipSuccess)
         e = launch_dims(k_splat_tiles<ALG>, "k_splat_tiles", dim3(uint32_t(nw)), dim3(kSplatBlock), 0, s, p, pos, val,
                         span, off, start, order, list, nwork, field, weight);
     return e;
 }
 
+template <int ALG>
+static hipError_t splat_hash(hipStream_t s, const PGrid& p, int64_t np, const float* pos, const float* val, int span,
+                             int off, float* field, float* weight) {
+    return LAUNCH(k_p2g_hash<ALG>, grid_for(size_t(np)), p, np, pos, val, span, off, field, weight);
+}
+
 hipError_t launch_p2g(hipStream_t s, const GridDev& g, int kind, int64_t np, const float* pos, const float* val,
                       int span, int off, int alg, float* field, float* weight, int normalize, uint32_t* work) {
     const PGrid p = pgrid_of(g, kind);
     const size_t n = size_t(p.nx) * p.ny * p.nz, cap = splat_tile_cap(g);
+    const bool sorted = work && splat_sorts(g, np, alg);
     hipError_t e = hipSuccess;
     int64_t first = 0;
     do {
         // counts of a segment; the field and the weight once
-        e = LAUNCH(k_splat_clear, grid_for(std::max(first ? size_t(0) : n, cap)), first ? size_t(0) : n, field, weight,
-                   cap, work);
-        const int64_t m = std::min<int64_t>(np - first, kSplatSegment);
+        const size_t nf = first ? 0 : n, nc = sorted ? cap : 0;
+        e = LAUNCH(k_splat_clear, grid_for(std::max(nf, nc)), nf, field, weight, nc, work);
+        const int64_t m = sorted ? std::min<int64_t>(np - first, kSplatSegment) : np;
         if (e != hipSuccess || m <= 0) break;
         const float* ps = pos + 3 * first;
         const float* vs = val + int64_t(span) * first;
+        auto run = [&](auto a) {
+            constexpr int ALG = decltype(a)::value;
+            return sorted ? splat_segment<ALG>(s, p, uint32_t(m), ps, vs, span, off, work, cap, field, weight)
+                          : splat_hash<ALG>(s, p, m, ps, vs, span, off, field, weight);
+        };
         switch (alg) {
-            case MGF_PG_P2GSUM:
-                e = splat_segment<MGF_PG_P2GSUM>(s, p, uint32_t(m), ps, vs, span, off, work, cap, field, weight);
-                break;
-            case MGF_PG_LINEAR:
-                e = splat_segment<MGF_PG_LINEAR>(s, p, uint32_t(m), ps, vs, span, off, work, cap, field, weight);
-                break;
-            case MGF_PG_QUADRATIC:
-                e = splat_segment<MGF_PG_QUADRATIC>(s, p, uint32_t(m), ps, vs, span, off, work, cap, field, weight);
-                break;
-            default: e = splat_segment<MGF_PG_CUBIC>(s, p, uint32_t(m), ps, vs, span, off, work, cap, field, weight); break;
+            case MGF_PG_P2GSUM: e = run(std::integral_constant<int, MGF_PG_P2GSUM>()); break;
+            case MGF_PG_LINEAR: e = run(std::integral_constant<int, MGF_PG_LINEAR>()); break;
+            case MGF_PG_QUADRATIC: e = run(std::integral_constant<int, MGF_PG_QUADRATIC>()); break;
+            default: e = run(std::integral_constant<int, MGF_PG_CUBIC>()); break;
         }
         first += m;
     } while (e == hipSuccess && first < np);

@@ -385,8 +385,8 @@ mgf_status mgf_psolver_create(mgf_context ctx, const mgf_grid* grid, int32_t kin
             TRY(owned_alloc(s->allocations, &s->acc, p2g_acc_floats(g)));
             TRY(owned_alloc(s->allocations, &s->pos_s, 3 * size_t(particles->n)));
             TRY(owned_alloc(s->allocations, &s->vel_s, 3 * size_t(particles->n)));
-        } else {
-            TRY(owned_alloc(s->allocations, &s->splat_work, p2g_work_words(g, particles->n)));
+        } else if (const size_t words = p2g_work_words(g, particles->n, alg)) {
+            TRY(owned_alloc(s->allocations, &s->splat_work, words));
         }
         MGF_HIP(hipStreamSynchronize(ctx->stream));
         return MGF_OK;

@@ -155,6 +155,93 @@ def test_p2g_tiles(ctx, orc, alg, n, edge):
 
 
 @pytest.mark.parametrize("alg", ALGS_P2G)
+def test_p2g_dense_cells(ctx, orc, alg):
+    """Cells of 64 particles (what a cell's own work-item sums), one more, and
+    many more, over chunk ends (2048).  Bound as above."""
+    res, origin, spacing = (18, 9, 25), (0.0, 0.0, 0.0), (0.25, 0.25, 0.25)
+    rng = np.random.default_rng(7)
+    cells = np.repeat([(3, 3, 3), (4, 3, 3), (3, 4, 3), (12, 5, 20), (17, 8, 24)], (64, 65, 700, 3000, 129), axis=0)
+    pos = ((cells + rng.uniform(0.0, 1.0, cells.shape)) * 0.25).astype(np.float32)
+    val = rng.standard_normal(len(pos)).astype(np.float32)
+    for order in (np.arange(len(pos)), rng.permutation(len(pos))):
+        for kind in (0, 2):
+            p, v = pos[order], val[order]
+            f, w = mgf.particles_to_grid(ctx, res, origin, spacing, kind, p, v, alg, normalize=False)
+            ef, ew = orc.p2g(res, origin, spacing, kind, p, v, alg, normalize=False)
+            sf, sw = orc.p2g(res, origin, spacing, kind, p, np.abs(v), alg, normalize=False)
+            bound = 2.0 * (len(pos) + 4) * 2.0 ** -24
+            assert np.all(np.abs(f - ef.ravel()) <= bound * sf.ravel() + 1e-37), (alg, kind)
+            assert np.all(np.abs(w - ew.ravel()) <= bound * sw.ravel() + 1e-37), (alg, kind)
+
+
+MANY_TILES = (200, 168, 176)   # 26 x 22 x 23 = 13156 tiles (of the extents + 1), 8192 of them in a sort's window
+
+
+@pytest.mark.parametrize("alg", ALGS_P2G)
+@pytest.mark.parametrize("order", ["cells", "layers", "random"])
+def test_p2g_more_tiles_than_the_window(ctx, orc, alg, order):
+    """Grids whose tiles do not fit the sort's LDS window: particles cell by
+    cell, every other one of a far layer (outside the window, waves of one
+    tile), and in random order (a wave of many tiles); one particle fewer
+    than the sort takes and that many (P2GSUM never sorts here).  Bound: the
+    terms of a node are the particles of the 4^3 cells around it."""
+    res, origin, spacing = MANY_TILES, (0.0, 0.0, 0.0), (0.5, 0.5, 0.5)
+    tiles = 13156
+    first = {"p2gsum": 70000, "linear": int(np.ceil((7.4 * tiles - 12.0e3) / 0.74)),
+             "quadratic": int(np.ceil((19.4 * tiles - 170.0e3) / 6.0)),
+             "cubic": int(np.ceil((42.4 * tiles - 170.0e3) / 6.0))}[alg]
+    rng = np.random.default_rng(11)
+    i = np.arange(first) // 8
+    cell = np.stack([i % res[0], (i // res[0]) % res[1], 3 + i // (res[0] * res[1])], 1)
+    if order == "layers":
+        cell[1::2, 2] = 171
+    elif order == "random":
+        cell = np.stack([rng.integers(0, r, first) for r in res], 1)
+    pos = ((cell + rng.uniform(0.0, 1.0, cell.shape)) * 0.5).astype(np.float32)
+    val = rng.standard_normal(first).astype(np.float32)
+    most = np.bincount((cell[:, 2] * res[1] + cell[:, 1]) * res[0] + cell[:, 0]).max()
+    bound = 2.0 * (64 * most + 4) * 2.0 ** -24
+    for n in (first - 1, first):
+        p, v = pos[:n], val[:n]
+        f, w = mgf.particles_to_grid(ctx, res, origin, spacing, 3, p, v, alg, normalize=False)
+        ef, ew = orc.p2g(res, origin, spacing, 3, p, v, alg, normalize=False)
+        sf, sw = orc.p2g(res, origin, spacing, 3, p, np.abs(v), alg, normalize=False)
+        assert np.all(np.abs(f - ef.ravel()) <= bound * sf.ravel() + 1e-37), (alg, n)
+        assert np.all(np.abs(w - ew.ravel()) <= bound * sw.ravel() + 1e-37), (alg, n)
+
+
+@pytest.mark.parametrize("alg, n", [("p2gsum", 786431), ("p2gsum", 786432), ("p2gsum", (1 << 24) + 4099),
+                                    ("linear", (1 << 24) + 4099), ("quadratic", (1 << 24) + 4099)])
+def test_p2g_segments(ctx, alg, n):
+    """More particles than are sorted at a time (2^24), and P2GSUM either side
+    of the count from which it sorts.  Particles on nodes with small whole
+    values: every weight is a multiple of 1/512 and every sum exact."""
+    res, spacing = (40, 24, 16), (0.25, 0.25, 0.25)
+    rng = np.random.default_rng(n)
+    cells = res[0] * res[1] * res[2]
+    at = rng.integers(0, cells, n)
+    pos = np.empty((n, 3), np.float32)
+    for k, c in enumerate((at % res[0], (at // res[0]) % res[1], at // (res[0] * res[1]))):
+        pos[:, k] = (c + 0.5) * 0.25
+    val = rng.integers(-2, 3, n).astype(np.float32)
+    f, w = mgf.particles_to_grid(ctx, res, (0.0, 0.0, 0.0), spacing, 0, pos, val, alg, normalize=False)
+    for got, x in ((f, val), (w, np.ones(n) if alg != "p2gsum" else np.zeros(n))):
+        exp = np.bincount(at, weights=x, minlength=cells).reshape(res[2], res[1], res[0])
+        if alg == "quadratic":
+            for axis in range(3):
+                out = 0.75 * exp
+                e = np.moveaxis(exp, axis, 0)
+                o = np.moveaxis(out, axis, 0)
+                o[1:] += 0.125 * e[:-1]
+                o[:-1] += 0.125 * e[1:]
+                o[0] += 0.125 * e[0]        # corners clamp to the grid
+                o[-1] += 0.125 * e[-1]
+                exp = out
+        assert np.abs(exp).max() * 512 < 2 ** 24
+        assert np.array_equal(got.astype(np.float64), exp.ravel())
+
+
+@pytest.mark.parametrize("alg", ALGS_P2G)
 def test_p2g_values_not_finite(ctx, orc, alg):
     """Infinities and NaN reach the same nodes as in the oracle (a zero
     corner weight times an infinity is a NaN), and no others."""
