@@ -982,10 +982,36 @@ void keyed(std::vector<KRec>& out, const std::vector<MRec>& recs, int a, int b, 
     for (size_t k = 0; k < recs.size(); ++k) out.push_back(KRec{a, b, c, int(k), recs[k]});
 }
 
+// Cells of each level that take bricks when their scene is alone, over the
+// scenes of a batch.
+std::vector<double> brick_cells(const std::vector<mgf_scene>& sc) {
+    std::vector<double> n(17, 0.0);
+    for (mgf_scene s : sc) {
+        MgDims f{s->g.nx, s->g.ny, s->g.nz, 1.0f, 1.0f, 1.0f};
+        for (size_t l = 0; l < s->mg.size(); ++l) {
+            const MgDims& c = s->mg[l].d;
+            if (brick_on(s, int(l), f, c)) n[l] += double(f.nx) * f.ny * f.nz;
+            f = c;
+        }
+    }
+    return n;
+}
+
+// A batch runs these levels by bricks while they are fewer cells than this in
+// all.  With more, whose launches fill the chip, the 11.7 values that a brick
+// forms a cell cost more than the launches they save, and a launch a sweep it
+// is: z is the same bit for bit, and rec_mg_smooth_bricks sums r . z in the
+// bricks' order.  Three steps, every level by bricks / a launch a sweep from 1M
+// cells / from 2M / always: 64 scenes of 64^3 50.9 / 42.8 / 43.0 / 43.2 ms, 256
+// uneven ones 229.8 / 196.3 / 198.6 / 199.7, 16 of 48^3 9.28 / 8.78 / 8.91 / 9.34,
+// 8 of 64^3 9.57 / 9.01 / 9.16 / 9.42; 4 of 64^3 6.71 / 6.76 / 6.85 / 7.30.
+constexpr double kBrickBatchCells = 1048576.0;
+
 // apply_precond's launches for scene s as keyed records; *zout = the buffer
-// that ends up holding z.  Keys: (0, level, step) on the way down, (1, 0, 0)
+// that ends up holding z.  cells: brick_cells of the batch.  Keys: (0, level, step) on the way down, (1, 0, 0)
 // the coarse cycle, (2, -level, step) on the way up.
-mgf_status vcycle_records(mgf_scene s, const float sa[3], std::vector<KRec>& out, const float** zout) {
+mgf_status vcycle_records(mgf_scene s, const float sa[3], const std::vector<double>& cells, std::vector<KRec>& out,
+                          const float** zout) {
     const auto& d = s->desc;
     const MgDims d0{s->g.nx, s->g.ny, s->g.nz, sa[0], sa[1], sa[2]};
     const int nu = d.mg_sweeps > 0 ? d.mg_sweeps : 3;
@@ -1003,7 +1029,8 @@ mgf_status vcycle_records(mgf_scene s, const float sa[3], std::vector<KRec>& out
     const int skip = s->skip_dry ? 1 : 0;
     const int l0 = s->mg_l0 < L ? s->mg_l0 : L;
     auto fused = [&](int l) { return l + 1 < L && march_on(s, l, lv[l].d, lv[l + 1].d); };
-    auto bricks = [&](int l) { return l + 1 < L && brick_on(s, l, lv[l].d, lv[l + 1].d); };
+    auto bricked = [&](int l) { return l + 1 < L && brick_on(s, l, lv[l].d, lv[l + 1].d); };
+    auto bricks = [&](int l) { return bricked(l) && cells[size_t(l)] < kBrickBatchCells; };
     std::vector<MRec> r;
     for (int l = 0; l < l0; ++l) {
         Lv& v = lv[l];
@@ -1084,7 +1111,8 @@ mgf_status vcycle_records(mgf_scene s, const float sa[3], std::vector<KRec>& out
         std::swap(v.x, v.t);
         for (int k = 1; k < nu; ++k) {
             r.clear();
-            rec_mg_smooth(r, v.d, v.codes, v.b, v.x, v.t, omega, s->scal, s->red, 0, rz_at(k));
+            if (rz_at(k) && bricked(l)) rec_mg_smooth_bricks(r, v.d, v.codes, v.b, v.x, v.t, omega, s->scal, s->red);
+            else rec_mg_smooth(r, v.d, v.codes, v.b, v.x, v.t, omega, s->scal, s->red, 0, rz_at(k));
             keyed(out, r, 2, -l, k);
             std::swap(v.x, v.t);
         }
@@ -1408,6 +1436,7 @@ mgf_status build_plan(LockPlan& P) {
     const size_t n = P.sc.size();
     if (n >= (size_t(1) << (32 - kMapShift))) return fail(MGF_ERR_INVALID, "too many scenes for one lockstep batch");
     std::vector<std::vector<KRec>> start_b(n), start_r(n), cg(n), vc(n), ref1(n), ref2(n), gat(n);
+    const std::vector<double> bricks = brick_cells(P.sc);
     P.zv.assign(n, nullptr);
     // the gather outputs live in the plan's buffer: their offsets are known
     // before the device buffer exists, so records hold device addresses
@@ -1437,7 +1466,7 @@ mgf_status build_plan(LockPlan& P) {
             r.clear();
             rec_cg_start(r, s->g, s->r, s->r, s->x, s->scal, s->red, inner, 0.0);
             keyed(start_r[i], r, 0, 0, 0);
-            TRY(vcycle_records(s, sa, vc[i], &P.zv[i]));
+            TRY(vcycle_records(s, sa, bricks, vc[i], &P.zv[i]));
             r.clear();
             rec_col_p_ap(r, s->g, sa, s->codes, P.zv[i], s->p0, s->p1, s->scal, s->red, wet_flat);
             keyed(cg[i], r, 0, 0, 0);

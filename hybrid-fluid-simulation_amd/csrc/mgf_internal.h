@@ -473,7 +473,7 @@ enum MultiKind : int32_t {
     kMkStart, kMkFinish, kMkPap, kMkUpdate, kMkRefine1, kMkRefine2, kMkAcc64, kMkSum2,
     kMkSmoothTT, kMkSmoothTF, kMkSmoothFT, kMkSmoothFF, kMkSmooth2T, kMkSmooth2F, kMkProlongT, kMkProlongF,
     kMkRestrict, kMkRestrict2, kMkRestrictTile, kMkCoarse, kMkMarchDesc, kMkMarchAsc, kMkMarchAscRz, kMkGather,
-    kMkBrickDesc, kMkBrickAsc, kMkBrickAscRz,
+    kMkBrickDesc, kMkBrickAsc, kMkBrickAscRz, kMkSmoothBrick,
     kMkRefine0, kMkCodes, kMkFlatWet, kMkCoarsen, kMkMarchWet, kMkMarchPlan,
     kMkAdvectFc, kMkAdvectCc, kMkAdvectCc4, kMkMarkers, kMkRhs, kMkProject, kMkCopyWord,
     kMkExtRows, kMkExtRowsReg4, kMkExtRowsReg8, kMkExtRowsReg16, kMkExtLines1, kMkExtLines2, kMkExtRowsReg5,
@@ -524,6 +524,9 @@ void rec_mg_brick_descend(std::vector<MRec>& out, const MgDims& f, const MgDims&
 void rec_mg_brick_ascend(std::vector<MRec>& out, const MgDims& f, const MgDims& c, const uint16_t* code,
                          const float* b, const float* xi, const float* xc, float* xo, float omega, CgScalars* sc,
                          ReduceBuf red, int with_rz);
+// A sweep of level 0 with r . z summed brick by brick, as rec_mg_brick_ascend does.
+void rec_mg_smooth_bricks(std::vector<MRec>& out, const MgDims& l, const uint16_t* code, const float* b,
+                          const float* xi, float* xo, float omega, CgScalars* sc, ReduceBuf red);
 // The finishing record's size, and its abs_target2 set in place.
 size_t finish_arg_bytes();
 void finish_set_target(unsigned char* args, double abs_target2);

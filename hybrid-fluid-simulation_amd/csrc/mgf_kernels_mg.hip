@@ -2008,6 +2008,76 @@ struct MBrick {
     }
 };
 
+// The last sweep of a level-0 ascent in a batch whose launches fill the chip:
+// k_mg_smooth's arithmetic with kSbRow bricks along x a work-group, so that the
+// partials of r . z are brick_run's and the sum is bit for bit that of the
+// scene alone.  A work-item has the same cell of each brick: rows of 8 cells
+// that together are 128 bytes, with all loads in flight at once.
+constexpr int kSbRow = 4;
+__device__ __forceinline__ void smooth_brick_run(const Bricks& T, const MgLevel& L, const uint16_t* __restrict__ code,
+                                                 const float* __restrict__ b, const float* __restrict__ xi,
+                                                 float* __restrict__ xo, float omega,
+                                                 const CgScalars* __restrict__ sc, double* __restrict__ part,
+                                                 uint32_t blk) {
+    __shared__ float aw[64], w[64];
+    __shared__ double sum[kSbRow][kBkThreads / 64];
+    if (sc->done) return;
+    const int t = threadIdx.x;
+    const uint32_t rx = (T.tx + kSbRow - 1) / kSbRow;
+    const uint32_t bx = blk % rx * kSbRow, br = blk / rx, by = br % T.ty, bz = br / T.ty;
+    const int x = int(bx) * kBkEdge + (t & 7), y = int(by) * kBkEdge + ((t >> 3) & 7), z = int(bz) * kBkEdge + (t >> 6);
+    const bool row = y < T.ny && z < T.nz;
+    const Flat F{T.sz * uint32_t(T.nz), T.sy, T.sz};
+    uint32_t i[kSbRow];
+    uint16_t cd[kSbRow];
+    float bc[kSbRow], vc[kSbRow], v[kSbRow][6];
+#pragma unroll
+    for (int q = 0; q < kSbRow; ++q) {
+        i[q] = row && x + 8 * q < T.nx ? uint32_t(z) * T.sz + uint32_t(y) * T.sy + uint32_t(x + 8 * q) : 0u;
+        uint32_t j[6];
+        nbrs(i[q], F, j);
+        cd[q] = code[i[q]];
+        bc[q] = b[i[q]];
+        vc[q] = xi[i[q]];
+#pragma unroll
+        for (int m = 0; m < 6; ++m) v[q][m] = xi[j[m]];
+    }
+    build_tables<true>(aw, w, L.sx, L.sy, L.sz, omega);
+#pragma unroll
+    for (int q = 0; q < kSbRow; ++q) {
+        const bool in = row && x + 8 * q < T.nx;
+        const float ax = arow(cd[q], vc[q], v[q], L.sx, L.sy, L.sz, aw);
+        const float out = (cd[q] & kCodeFluid) ? vc[q] + wdiag(cd[q], w) * (bc[q] - ax) : 0.0f;
+        if (in) xo[i[q]] = out;
+        const double s = wave_sum(in ? double(bc[q]) * double(out) : 0.0);
+        if ((t & 63) == 0) sum[q][t >> 6] = s;
+    }
+    __syncthreads();
+    if (t < kSbRow && bx + uint32_t(t) < T.tx) {
+        double s = sum[t][0];
+        for (int q = 1; q < kBkThreads / 64; ++q) s += sum[t][q];
+        part[br * T.tx + bx + uint32_t(t)] = s;
+    }
+}
+
+struct MSmoothBrick {
+    static constexpr int kThreads = kBkThreads;
+    Bricks T;
+    MgLevel L;
+    const uint16_t* code;
+    const float *b, *xi;
+    float* xo;
+    float omega;
+    const CgScalars* sc;
+    double* part;
+    uint32_t G;
+    __device__ void run(uint32_t vb) const {
+        const uint32_t blk = xcd_of(vb, G);
+        if (blk < (T.tx + kSbRow - 1) / kSbRow * T.ty * T.tz)
+            smooth_brick_run(T, L, code, b, xi, xo, omega, sc, part, blk);
+    }
+};
+
 // ===========================================================================
 // Fused descent and ascent of one level (every axis halved, three sweeps),
 // marching along z.
@@ -3275,6 +3345,14 @@ void rec_mg_brick_ascend(std::vector<MRec>& out, const MgDims& f, const MgDims& 
     }
 }
 
+void rec_mg_smooth_bricks(std::vector<MRec>& out, const MgDims& l, const uint16_t* code, const float* b,
+                          const float* xi, float* xo, float omega, CgScalars* sc, ReduceBuf red) {
+    const Bricks T = make_bricks(l, l);
+    const uint32_t rows = (T.tx + kSbRow - 1) / kSbRow * T.ty * T.tz, G = (rows + kXcds - 1) / kXcds * kXcds;
+    push_rec(out, kMkSmoothBrick, MSmoothBrick{T, l, code, b, xi, xo, omega, sc, red.partials, G}, G);
+    rec_finish(out, red.partials, mg_brick_blocks(l), sc, kFinishRz);
+}
+
 bool rec_mg_coarse_cycle(std::vector<MRec>& out, const MgDims* levels, const uint16_t* const* codes, int nlev,
                          const float* b0, float* x0, int nu, int last_sweeps, float omega, const CgScalars* sc) {
     if (nlev < 1 || nlev > kCoarseMaxLevels) return false;
@@ -3383,6 +3461,7 @@ hipError_t launch_multi(hipStream_t s, int32_t kind, const void* tab, const uint
         case kMkMarchAscRz: return launch_m_march<MMarch<true, true>>(s, tab, map, nblocks, active);
         case kMkBrickDesc: return launch_m<MBrick<false, false>>(s, "k_multi_mg_brick", tab, map, nblocks, 0, active);
         case kMkBrickAsc: return launch_m<MBrick<true, false>>(s, "k_multi_mg_brick", tab, map, nblocks, 0, active);
+        case kMkSmoothBrick: return launch_m<MSmoothBrick>(s, "k_multi_mg_smooth", tab, map, nblocks, 0, active);
         case kMkBrickAscRz: return launch_m<MBrick<true, true>>(s, "k_multi_mg_brick", tab, map, nblocks, 0, active);
         case kMkGather: return launch_m<MGather>(s, "k_multi_gather", tab, map, nblocks, 0, active);
         case kMkRefine0: return launch_m<MRefine<0>>(s, "k_multi_refine", tab, map, nblocks, 0, active);

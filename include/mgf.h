@@ -163,7 +163,9 @@ typedef struct mgf_scene_desc {
  * (prolongation and three sweeps) can each run as one fused kernel: a march
  * along z (large levels) or brick by brick (small ones). */
 #define MGF_MG_AUTO      0  /* the march on levels of at least 512K cells,
-                               bricks on smaller 3-D levels (default)         */
+                               bricks on smaller 3-D levels, in a lockstep
+                               batch a kernel per sweep on those that fill
+                               the device together (default)                  */
 #define MGF_MG_PER_SWEEP 1  /* one kernel per sweep on every level            */
 #define MGF_MG_FUSED     2  /* the march on every 3-D level                   */
 
@@ -362,7 +364,8 @@ MGF_API mgf_status mgf_batch_set_lockstep(mgf_context ctx, int32_t enabled);
  * the V-cycle kernel choices on these scenes, each over one lockstep batch
  * call of trial_steps (>= 2) steps, and keeps the faster on every scene that
  * runs in lockstep (their mg_kernels field): MGF_MG_AUTO (the march on
- * levels of at least 512K cells, bricks below) and MGF_MG_FUSED (the march on
+ * levels of at least 512K cells, below bricks or, from 1M cells of a level in
+ * the batch, a kernel per sweep) and MGF_MG_FUSED (the march on
  * every 3-D level above the coarse cycle; small levels of many scenes fill
  * the device together).  Every scene advances by
  * 2 * trial_steps steps.  The choice changes only the summation order of

@@ -129,6 +129,38 @@ def test_dot_products_folded_on_a_marched_level(ctx, res, kernels, rz_folded, pa
     compare_alone_with_batch(ctx, res, mg_kernels=kernels)
 
 
+def test_small_levels_of_a_full_batch(ctx):
+    """Scenes whose level 0 takes bricks alone, more than 1M cells of it in the
+    batch: there it takes a launch a sweep, the last one with r . z in the
+    bricks' order (8^3 cells, four bricks a work-group), and the lower levels,
+    fewer cells, take bricks.  The same bits and counts."""
+    sizes = [(66, 66, 66), (65, 70, 61), (40, 25, 30), (98, 33, 67), (72, 64, 80), (97, 50, 50)]
+    assert sum(int(np.prod(r)) for r in sizes) >= 1 << 20
+    pairs = []
+    for res in sizes:
+        rng = np.random.default_rng(sum(res))
+        phi = np.where(rng.random(int(np.prod(res))) < 0.6, -1.0, 1.0).astype(np.float32)
+        vel = [rng.standard_normal(int(np.prod([res[d] + (d == k) for d in range(3)]))).astype(np.float32)
+               for k in range(3)]
+        pair = []
+        for _ in range(2):
+            s = mgf.Scene(ctx, mgf.make_desc(res, (0, 0, 0), (0.1, 0.1, 0.1), 0.003, rk=mgf.RK1,
+                                             tol_mode=mgf.TOL_RELATIVE, tol=1e-6, precision=mgf.PRECISION_MIXED,
+                                             precond=mgf.PRECOND_MULTIGRID))
+            s.upload(mgf.FIELD["fluid_domain"], phi)
+            for k in range(3):
+                s.upload(k, vel[k])
+            pair.append(s)
+        pairs.append(pair)
+    status, stats, _ = mgf.batch_step(ctx, [p[0] for p in pairs], 2, workers=1)
+    assert status == [mgf.OK] * len(sizes)
+    for i, (a, b) in enumerate(pairs):
+        assert stats[i].cg_iterations == b.step(2)["cg_iterations"], sizes[i]
+        assert_same(snapshot(a), snapshot(b), "res %s" % (sizes[i],))
+        a.close()
+        b.close()
+
+
 @pytest.mark.parametrize("res", [(16, 16, 16), (64, 64, 128), (88, 88, 80)])
 def test_solve_that_ends_at_a_zero_curvature(ctx, res):
     """A closed box of fluid with a uniform divergence: r is constant, A r is
