@@ -1768,9 +1768,13 @@ mgf_status div_end(mgf_scene s, mgf_step_stats* acc) {
 // largest distance and the brick stamps uint32[kNaWorkWords].
 constexpr size_t kNaFaces = size_t(1) << 22;   // faces of all three components
 constexpr int32_t kNaMaxK = 4093;              // nx + ny + nz + 3 with more than one layer
-// A brick of a grid within those limits holds at least 128 faces on average
-// (16 x 16 x 1 in a grid one cell thick, an axis rounded up at worst by half).
+// Bricks of a component of extents e: at most (ex + 31)(ey + 15)(ez + 15) / 8192,
+// and each product of two extents is at most that of all three, so over the
+// three components at most the number below (12741 was the most that a search
+// found, at 1 x 2177 x 481).  A word a brick, rounded up to 8, and the far words.
+constexpr size_t kNaBricks = (62 * kNaFaces + 3 * 465 * size_t(kNaMaxK) + 3 * 6975) / 8192;
 constexpr size_t kNaWorkWords = size_t(1) << 17;
+static_assert(kExtFarWords + kNaBricks + 8 <= kNaWorkWords, "every grid within the limits has its stamps");
 constexpr size_t na_align(size_t b) { return (b + 255) / 256 * 256; }
 constexpr size_t kNaDistOff = 0;
 constexpr size_t kNaWorkOff = kNaDistOff + na_align(2 * kNaFaces);
@@ -2991,7 +2995,7 @@ mgf_status mgf_op_extrapolate_fc_noalloc(mgf_context ctx, const mgf_grid* grid, 
                                          " faces exceed its scratch (" + std::to_string(kNaFaces) + " faces)");
     const GridDev g = make_grid(grid);
     const int32_t K = ext_max_distance(g);
-    if (layers > 1 && (K > kNaMaxK || ext_work_words(g) > kNaWorkWords))
+    if (layers > 1 && K > kNaMaxK)
         return fail(MGF_ERR_INVALID, "mgf_op_extrapolate_fc_noalloc: nx + ny + nz + 3 = " + std::to_string(K) +
                                          " exceeds its scratch (" + std::to_string(kNaMaxK) + ")");
     std::string err;

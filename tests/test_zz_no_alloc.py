@@ -67,3 +67,19 @@ def test_noalloc_refuses_grids_beyond_its_scratch(ctx):
     st = mgf.lib().mgf_op_extrapolate_fc_noalloc(ctx.h, mgf.grid(thin), mgf.C.c_void_p(16), mgf.C.c_void_p(16),
                                                  mgf.C.c_void_p(16), 1000, mgf.C.byref(used))
     assert st == mgf.ERR_INVALID
+
+
+def test_noalloc_with_the_most_bricks(ctx):
+    """The grid within both limits (4194304 faces, extents of 4090 in all) with
+    the most bricks of 32 x 16 x 16 faces that a search found: its stamps fit
+    the scratch."""
+    res = (1, 2177, 481)
+    arrs = faces(np.random.default_rng(12), res, 0.002)
+    assert sum(a.size for a in arrs) <= 4194304 and sum(res) + 3 <= 4093
+    st_a, ref, used_a = run(ctx, "mgf_op_extrapolate_fc", res, arrs, 1000)
+    mgf.check(st_a, "mgf_op_extrapolate_fc")
+    st_b, got, used_b = run(ctx, "mgf_op_extrapolate_fc_noalloc", res, arrs, 1000)
+    mgf.check(st_b, "mgf_op_extrapolate_fc_noalloc")
+    assert used_a == used_b and used_a > 1
+    for k in range(3):
+        assert np.array_equal(got[k].view(np.uint32), ref[k].view(np.uint32)), k
