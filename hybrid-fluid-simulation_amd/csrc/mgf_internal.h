@@ -420,14 +420,11 @@ hipError_t launch_mg_smooth2_first(hipStream_t s, const MgDims& l, const uint16_
 hipError_t launch_mg_smooth_prolong(hipStream_t s, const MgDims& f, const MgDims& c, const uint16_t* code,
                                     const float* b, const float* xi, const float* xc, float* xo, float omega,
                                     CgScalars* sc, ReduceBuf red, int with_rz);
-// The V-cycle of levels[0..nlev) in one work-group with the iterates in LDS:
-// b0 = right-hand side of levels[0] (global), x0 = its result (global).
 // Fused descent (the first three sweeps from zero and the restriction of the
 // residual) and ascent (prolongation and three sweeps; with_rz: r . z) of a
-// level whose every axis is halved (mg_march_ok).  mg_march_grid = blocks of
-// one launch; mg_march_parts = the partials of r . z the ascent writes.
+// level whose every axis is halved (mg_march_ok).  mg_march_parts = the
+// partials of r . z the ascent writes.
 bool mg_march_ok(const MgDims& f);
-uint32_t mg_march_grid(const MgDims& f, const MgDims& c);
 uint32_t mg_march_parts(const MgDims& f, const MgDims& c);
 // The schedule of a fused level (32-bit words, mg_march_sched_words): made by
 // launch_mg_march_wet and then launch_mg_march_plan once per set of codes,
@@ -457,6 +454,8 @@ hipError_t launch_mg_brick_descend(hipStream_t s, const MgDims& f, const MgDims&
 hipError_t launch_mg_brick_ascend(hipStream_t s, const MgDims& f, const MgDims& c, const uint16_t* code,
                                   const float* b, const float* xi, const float* xc, float* xo, float omega,
                                   CgScalars* sc, ReduceBuf red, int with_rz);
+// The V-cycle of levels[0..nlev) in one work-group with the iterates in LDS:
+// b0 = right-hand side of levels[0] (global), x0 = its result (global).
 size_t mg_coarse_lds_bytes(const MgDims* levels, int nlev);
 hipError_t launch_mg_coarse_cycle(hipStream_t s, const MgDims* levels, const uint16_t* const* codes, int nlev,
                                   const float* b0, float* x0, int nu, int last_sweeps, float omega,
@@ -475,7 +474,7 @@ enum MultiKind : int32_t {
     kMkRestrict, kMkRestrict2, kMkRestrictTile, kMkCoarse, kMkMarchDesc, kMkMarchAsc, kMkMarchAscRz, kMkGather,
     kMkBrickDesc, kMkBrickAsc, kMkBrickAscRz, kMkSmoothBrick,
     kMkRefine0, kMkCodes, kMkFlatWet, kMkCoarsen, kMkMarchWet, kMkMarchPlan,
-    kMkAdvectFc, kMkAdvectCc, kMkAdvectCc4, kMkMarkers, kMkRhs, kMkProject, kMkCopyWord,
+    kMkAdvectFc, kMkAdvectCc, kMkAdvectCc4, kMkMarkers, kMkRhs, kMkProject,
     kMkExtRows, kMkExtRowsReg4, kMkExtRowsReg8, kMkExtRowsReg16, kMkExtLines1, kMkExtLines2, kMkExtRowsReg5,
     kMkExtLinesSeg,                          // 8 kinds: (axis - 1) * 4 + segment size class
     kMkExtLinesSegLast = kMkExtLinesSeg + 7,
@@ -548,7 +547,6 @@ void rec_markers(std::vector<MRec>& out, const GridDev& g, const uint8_t* solid_
 void rec_rhs(std::vector<MRec>& out, const GridDev& g, Vel U, Vel S, const uint8_t* markers, float* b);
 void rec_project(std::vector<MRec>& out, const GridDev& g, const float sg[3], const uint8_t* markers, const float* p32,
                  const double* p64, float* u, float* v, float* w, const float* us, const float* vs, const float* ws);
-void rec_copy_word(std::vector<MRec>& out, const uint32_t* src, uint32_t* dst);
 // The extrapolation's distance transform; mark = the scene's bricks in the
 // stamp buffer of pass 1, far = its kExtFarWords words.
 void rec_ext_distance(std::vector<MRec>& out, const GridDev& g, float* u, float* v, float* w, uint16_t* dist,

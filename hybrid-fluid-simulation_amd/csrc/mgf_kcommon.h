@@ -123,7 +123,5 @@ inline hipError_t launch_k(K kern, const char* name, uint32_t grid, hipStream_t 
     return launch_dims(kern, name, dim3(grid), dim3(kBlock), 0u, s, args...);
 }
 #define LAUNCH(kern, grid, ...) launch_k(kern, #kern, uint32_t(grid), s, __VA_ARGS__)
-// with an explicit kernel name (templates: one name for every instantiation)
-#define LAUNCHN(kern, name, grid, ...) launch_k(kern, name, uint32_t(grid), s, __VA_ARGS__)
 
 }  // namespace mgf

@@ -885,20 +885,6 @@ void rec_project(std::vector<MRec>& out, const GridDev& g, const float sg[3], co
     push_rec_k(out, kMkProject, MProject{g, markers, sg[0], sg[1], sg[2], p32, p64, u, v, w, us, vs, ws, n, G}, G);
 }
 
-// Copies one 32-bit word per scene into a packed array (one work-item).
-struct MCopyWord {
-    static constexpr int kThreads = 64;
-    const uint32_t* src;
-    uint32_t* dst;
-    __device__ void run(uint32_t) const {
-        if (threadIdx.x == 0) *dst = *src;
-    }
-};
-
-void rec_copy_word(std::vector<MRec>& out, const uint32_t* src, uint32_t* dst) {
-    push_rec_k(out, kMkCopyWord, MCopyWord{src, dst}, 1u);
-}
-
 template <class A>
 static hipError_t launch_mk(hipStream_t s, const char* name, const void* tab, const uint32_t* map, uint32_t nblocks,
                             const uint8_t* active) {
@@ -915,7 +901,6 @@ hipError_t launch_multi_k(hipStream_t s, int32_t kind, const void* tab, const ui
         case kMkMarkers: return launch_mk<MMarkers>(s, "k_multi_markers", tab, map, nblocks, active);
         case kMkRhs: return launch_mk<MRhs>(s, "k_multi_rhs", tab, map, nblocks, active);
         case kMkProject: return launch_mk<MProject>(s, "k_multi_project", tab, map, nblocks, active);
-        case kMkCopyWord: return launch_mk<MCopyWord>(s, "k_multi_copy_word", tab, map, nblocks, active);
         default: return launch_multi_ext(s, kind, tab, map, nblocks, shmem, active);
     }
 }

@@ -2991,8 +2991,6 @@ static March make_march(const MgDims& f, const MgDims& c, int skip = 1) {
     return M;
 }
 
-uint32_t mg_march_grid(const MgDims& f, const MgDims& c) { return make_march(f, c).gmax; }
-
 uint32_t mg_march_parts(const MgDims& f, const MgDims& c) { return make_march(f, c).parts; }
 
 size_t mg_march_sched_words(const MgDims& f, const MgDims& c) {
