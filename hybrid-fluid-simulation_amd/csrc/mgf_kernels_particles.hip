@@ -235,13 +235,18 @@ __global__ void __launch_bounds__(kBlock) k_splat_count(PGrid g, uint32_t np, co
     const uint32_t win = min(nt, kSplatLdsTiles), lo = splat_window<ALG>(g, np, pos, base, nt);
     for (uint32_t i = threadIdx.x; i < win; i += kBlock) hist[i] = 0u;
     __syncthreads();
+    if (win == nt) {
 #pragma unroll 4
-    for (uint32_t j = 0; j < kSplatItems; ++j) {
-        if (base + j * kBlock >= np) break;   // the same for every work-item
-        const uint32_t p = base + j * kBlock + threadIdx.x;
-        const uint32_t t = splat_at<ALG>(g, pos, p < np ? p : np - 1).tile;
-        if (p < np && t - lo < win) atomicAdd(&hist[t - lo], 1u);
-        if (win < nt) {
+        for (uint32_t j = 0; j < kSplatItems; ++j) {
+            const uint32_t p = base + j * kBlock + threadIdx.x;
+            if (p < np) atomicAdd(&hist[splat_at<ALG>(g, pos, p).tile], 1u);
+        }
+    } else {
+        for (uint32_t j = 0; j < kSplatItems; ++j) {
+            if (base + j * kBlock >= np) break;   // the same for every work-item
+            const uint32_t p = base + j * kBlock + threadIdx.x;
+            const uint32_t t = splat_at<ALG>(g, pos, p < np ? p : np - 1).tile;
+            if (p < np && t - lo < win) atomicAdd(&hist[t - lo], 1u);
             const uint64_t mine = same_tile(p < np && t - lo >= win, t);
             if (mine && rank_in(mine) == 0) atomicAdd(&counts[t], uint32_t(__popcll(mine)));
         }
@@ -397,12 +402,19 @@ __global__ void __launch_bounds__(kSplatBlock) k_splat_tiles(PGrid g, const floa
         const uint32_t u = uint32_t(__shfl_up(int(incl), o, 64));
         if ((t & 63) >= o) incl += u;
     }
-    if ((t & 63) == 63) wsum[t >> 6] = incl;
+    // with bit 31: a cell of the wave holds more than kSplatCell
+    const bool crowded = __any(mine > kSplatCell);
+    if ((t & 63) == 63) wsum[t >> 6] = incl | (crowded ? 1u << 31 : 0u);
     __syncthreads();
-    uint32_t q = incl - mine;
-    for (int w = 0; w < (t >> 6); ++w) q += wsum[w];
+    uint32_t q = incl - mine, dense = 0;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) {
+        const uint32_t u = wsum[w];
+        q += w < (t >> 6) ? u & 0x7fffffffu : 0u;
+        dense |= u >> 31;
+    }
     first[t] = q;   // as it stays
-    const bool dense = __syncthreads_or(mine > kSplatCell);
+    __syncthreads();
 #pragma unroll
     for (uint32_t j = 0; j < kSplatRounds; ++j)
         if (j * kSplatBlock + t < n) part[first[cell[j]] + rank[j]] = v[j];
