@@ -362,8 +362,9 @@ __device__ __forceinline__ void finish_scalars(CgScalars* sc, int kind, double t
 // while the partials are few (kFoldMax): a launch between two kernels costs about
 // 3.5 us, the sum in each work-group about 1 us with 40 partials (34^3, four
 // steps: 3.79 -> 3.45 ms) and as much as the launch with a thousand (152 x 63 x
-// 99, 926 partials: no change; 130^3, 2152: 4.75 -> 4.84 ms).  count 0: the
-// scalars are finished.
+// 99, 926 partials: no change; 130^3, 2152: 4.75 -> 4.84 ms).  Instances of
+// their own: where a store to the scalars may come first, the others' loads of
+// them could not be scalar loads (514^3 step 0.7% slower).
 // The kernels' own pointer to the scalars may not be __restrict__: sc here is
 // the same struct, and is written.
 struct Fold {
@@ -507,6 +508,7 @@ struct MFlatWet {
 
 // A kernel body runs block `blk` of its launch (after the XCD remapping) and
 // writes its partial sums to slot `slot` (the launch's own block index).
+template <bool FOLD>
 __device__ __forceinline__ void cg_pap_run(Flat F, const uint16_t* __restrict__ code, float sx, float sy, float sz,
                                            const float* __restrict__ zv, float* __restrict__ p,
                                            float* __restrict__ ap, const CgScalars* sc,
@@ -515,7 +517,7 @@ __device__ __forceinline__ void cg_pap_run(Flat F, const uint16_t* __restrict__ 
     __shared__ float aw[64];
     const bool first = sc->iters == 0;
     float beta;
-    if (rz.count) {
+    if constexpr (FOLD) {
         double t;
         if (!fold_sum(rz, t)) return;
         beta = float(first ? 0.0 : t / sc->rz);
@@ -549,12 +551,13 @@ __device__ __forceinline__ void cg_pap_run(Flat F, const uint16_t* __restrict__ 
     block_partial(acc, part, slot);
 }
 
+template <bool FOLD>
 __global__ void __launch_bounds__(kBlock) k_cg_pap(Flat F, const uint16_t* __restrict__ code, float sx, float sy,
                                                    float sz, const float* __restrict__ zv, float* __restrict__ p,
                                                    float* __restrict__ ap, const CgScalars* sc,
                                                    double* __restrict__ part, const uint16_t* __restrict__ wet,
                                                    Fold rz) {
-    cg_pap_run(F, code, sx, sy, sz, zv, p, ap, sc, part, wet, rz, xcd_block(), blockIdx.x);
+    cg_pap_run<FOLD>(F, code, sx, sy, sz, zv, p, ap, sc, part, wet, rz, xcd_block(), blockIdx.x);
 }
 
 struct MPap {
@@ -568,7 +571,9 @@ struct MPap {
     double* part;
     const uint16_t* wet;
     uint32_t G;
-    __device__ void run(uint32_t b) const { cg_pap_run(F, code, sx, sy, sz, zv, p, ap, sc, part, wet, Fold{}, xcd_of(b, G), b); }
+    __device__ void run(uint32_t b) const {
+        cg_pap_run<false>(F, code, sx, sy, sz, zv, p, ap, sc, part, wet, Fold{}, xcd_of(b, G), b);
+    }
 };
 
 // K_II (pointwise): x += alpha p; r -= alpha Ap (each formed in FP64, stored
@@ -602,13 +607,14 @@ __device__ __forceinline__ double cg_update_body(const Flat& F, uint32_t base, c
     return acc;
 }
 
+template <bool FOLD>
 __device__ __forceinline__ void cg_update_run(Flat F, const float* __restrict__ p, const float* __restrict__ ap,
                                               float* __restrict__ x, float* __restrict__ r,
                                               const CgScalars* sc, double* __restrict__ part,
                                               const uint16_t* __restrict__ wet, const Fold& pap, uint32_t blk,
                                               uint32_t slot) {
     double alpha;
-    if (pap.count) {
+    if constexpr (FOLD) {
         double t;
         if (!fold_sum(pap, t)) return;
         alpha = sc->rz_new / t;
@@ -633,12 +639,13 @@ __device__ __forceinline__ void cg_update_run(Flat F, const float* __restrict__ 
     block_partial(acc, part, slot);
 }
 
+template <bool FOLD>
 __global__ void __launch_bounds__(kBlock) k_cg_update(Flat F, const float* __restrict__ p,
                                                       const float* __restrict__ ap, float* __restrict__ x,
                                                       float* __restrict__ r, const CgScalars* sc,
                                                       double* __restrict__ part, const uint16_t* __restrict__ wet,
                                                       Fold pap) {
-    cg_update_run(F, p, ap, x, r, sc, part, wet, pap, xcd_block(), blockIdx.x);
+    cg_update_run<FOLD>(F, p, ap, x, r, sc, part, wet, pap, xcd_block(), blockIdx.x);
 }
 
 struct MUpdate {
@@ -650,7 +657,9 @@ struct MUpdate {
     double* part;
     const uint16_t* wet;
     uint32_t G;
-    __device__ void run(uint32_t b) const { cg_update_run(F, p, ap, x, r, sc, part, wet, Fold{}, xcd_of(b, G), b); }
+    __device__ void run(uint32_t b) const {
+        cg_update_run<false>(F, p, ap, x, r, sc, part, wet, Fold{}, xcd_of(b, G), b);
+    }
 };
 
 // Refinement (outer sweeps of the mixed solver).
@@ -1864,7 +1873,7 @@ struct Bricks {
     uint32_t tx, ty, tz;
 };
 
-template <bool POST, bool RZ>
+template <bool POST, bool RZ, bool FOLD>
 __device__ __forceinline__ void brick_run(const Bricks& T, const MgLevel& L, const uint16_t* __restrict__ code,
                                           const float* __restrict__ b, const float* __restrict__ xi,
                                           const float* __restrict__ xc, float* __restrict__ xo,
@@ -1874,7 +1883,7 @@ __device__ __forceinline__ void brick_run(const Bricks& T, const MgLevel& L, con
     __shared__ float aw[64], w[64];
     __shared__ float xa[kBkCells], xb[kBkCells];
     __shared__ double sum[kBkThreads / 64];
-    if (!POST && rr.count) {
+    if constexpr (FOLD) {
         double t;
         if (!fold_sum(rr, t)) return;
         if (slot == 0 && threadIdx.x == 0) finish_scalars(rr.sc, kFinishRr, t, 0.0, 0.0);
@@ -1980,14 +1989,14 @@ __device__ __forceinline__ void brick_run(const Bricks& T, const MgLevel& L, con
     }
 }
 
-template <bool POST, bool RZ>
+template <bool POST, bool RZ, bool FOLD>
 __global__ void __launch_bounds__(kBkThreads) k_mg_brick(Bricks T, MgLevel L, const uint16_t* __restrict__ code,
                                                          const float* __restrict__ b, const float* __restrict__ xi,
                                                          const float* __restrict__ xc, float* __restrict__ xo,
                                                          const uint16_t* __restrict__ codec, float* __restrict__ bco,
                                                          float omega, const CgScalars* sc,
                                                          double* __restrict__ part, Fold rr) {
-    brick_run<POST, RZ>(T, L, code, b, xi, xc, xo, codec, bco, omega, sc, part, rr, blockIdx.x, blockIdx.x);
+    brick_run<POST, RZ, FOLD>(T, L, code, b, xi, xc, xo, codec, bco, omega, sc, part, rr, blockIdx.x, blockIdx.x);
 }
 
 template <bool POST, bool RZ>
@@ -2004,7 +2013,7 @@ struct MBrick {
     const CgScalars* sc;
     double* part;
     __device__ void run(uint32_t blk) const {
-        brick_run<POST, RZ>(T, L, code, b, xi, xc, xo, codec, bco, omega, sc, part, Fold{}, blk, blk);
+        brick_run<POST, RZ, false>(T, L, code, b, xi, xc, xo, codec, bco, omega, sc, part, Fold{}, blk, blk);
     }
 };
 
@@ -2874,8 +2883,8 @@ hipError_t launch_col_p_ap(hipStream_t s, const GridDev& g, const float scale[3]
     const uint32_t G = flat_grid(F.n);
     if (fold.rz > kFoldMax) return hipErrorInvalidValue;
     double* part = pap_slots(red, G);
-    hipError_t e = LAUNCH(k_cg_pap, G, F, codes, scale[0], scale[1], scale[2], zv, p, ap, sc, part, wet,
-                          (Fold{red.partials, fold.rz, sc}));
+    hipError_t e = launch_k(fold.rz ? k_cg_pap<true> : k_cg_pap<false>, "k_cg_pap", G, s, F, codes, scale[0], scale[1],
+                            scale[2], zv, p, ap, sc, part, wet, Fold{red.partials, fold.rz, sc});
     if (e != hipSuccess || fold.alpha) return e;
     return finish(s, part, G, sc, kFinishAlpha);
 }
@@ -2884,8 +2893,8 @@ hipError_t launch_col_update(hipStream_t s, const GridDev& g, const float* p, co
                              CgScalars* sc, ReduceBuf red, int identity, const uint16_t* wet, const CgFold& fold) {
     const Flat F = make_flat(g.nx, g.ny, g.nz);
     const uint32_t G = flat_grid(F.n);
-    hipError_t e = LAUNCH(k_cg_update, G, F, p, ap, x, r, sc, red.partials, wet,
-                          (Fold{pap_slots(red, G), fold.alpha ? G : 0u, sc}));
+    hipError_t e = launch_k(fold.alpha ? k_cg_update<true> : k_cg_update<false>, "k_cg_update", G, s, F, p, ap, x, r, sc,
+                            red.partials, wet, Fold{pap_slots(red, G), G, sc});
     if (e != hipSuccess || fold.rr) return e;
     return finish(s, red.partials, G, sc, identity ? kFinishRrIdent : kFinishRr);
 }
@@ -3079,7 +3088,7 @@ hipError_t launch_mg_brick_descend(hipStream_t s, const MgDims& f, const MgDims&
                                    const float* b, float* x, const uint16_t* codec, float* bc, float omega,
                                    CgScalars* sc, ReduceBuf red, uint32_t rr) {
     const CgScalars* csc = sc;
-    return launch_dims(k_mg_brick<false, false>, "k_mg_brick", dim3(mg_brick_blocks(f)), dim3(kBkThreads), 0u, s,
+    return launch_dims(rr ? k_mg_brick<false, false, true> : k_mg_brick<false, false, false>, "k_mg_brick", dim3(mg_brick_blocks(f)), dim3(kBkThreads), 0u, s,
                        make_bricks(f, c), f, code, b, static_cast<const float*>(nullptr),
                        static_cast<const float*>(nullptr), x, codec, bc, omega, csc, static_cast<double*>(nullptr),
                        Fold{red.partials, rr, sc});
@@ -3093,9 +3102,9 @@ hipError_t launch_mg_brick_ascend(hipStream_t s, const MgDims& f, const MgDims& 
     const uint16_t* nc = nullptr;
     float* nb = nullptr;
     if (!with_rz)
-        return launch_dims(k_mg_brick<true, false>, "k_mg_brick", dim3(G), dim3(kBkThreads), 0u, s, make_bricks(f, c),
+        return launch_dims(k_mg_brick<true, false, false>, "k_mg_brick", dim3(G), dim3(kBkThreads), 0u, s, make_bricks(f, c),
                            f, code, b, xi, xc, xo, nc, nb, omega, csc, static_cast<double*>(nullptr), Fold{});
-    const hipError_t e = launch_dims(k_mg_brick<true, true>, "k_mg_brick", dim3(G), dim3(kBkThreads), 0u, s,
+    const hipError_t e = launch_dims(k_mg_brick<true, true, false>, "k_mg_brick", dim3(G), dim3(kBkThreads), 0u, s,
                                      make_bricks(f, c), f, code, b, xi, xc, xo, nc, nb, omega, csc,
                                      red.partials, Fold{});
     if (e != hipSuccess || with_rz == kRzLeft) return e;
