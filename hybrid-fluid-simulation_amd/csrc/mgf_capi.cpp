@@ -279,13 +279,14 @@ mgf_status advect(mgf_scene s, bool with_forces) {
     probe_next_bytes(12.0 * double(s->nfx + s->nfy + s->nfz));
     MGF_HIP(launch_advect_fc(st, s->g, V, V, dt, s->desc.rk_order, s->u[n], s->v[n], s->w[n], addg,
                              g, addf, f));
+    const double vel_bytes = 4.0 * double(s->nfx + s->nfy + s->nfz);   // the back-trace's
     if (s->color[0][0]) {
         const float* ic[3] = {s->color[c][0], s->color[c][1], s->color[c][2]};
         float* oc[3] = {s->color[n][0], s->color[n][1], s->color[n][2]};
-        probe_next_bytes(32.0 * double(s->ncell));
+        probe_next_bytes(32.0 * double(s->ncell) + vel_bytes);
         MGF_HIP(launch_advect_cc4(st, s->g, s->phi[c], ic, V, dt, s->desc.rk_order, s->phi[n], oc));
     } else {
-        probe_next_bytes(8.0 * double(s->ncell));
+        probe_next_bytes(8.0 * double(s->ncell) + vel_bytes);
         MGF_HIP(launch_advect_cc(st, s->g, s->phi[c], V, dt, s->desc.rk_order, s->phi[n]));
     }
     s->cur = n;

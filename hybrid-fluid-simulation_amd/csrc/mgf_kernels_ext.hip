@@ -560,9 +560,14 @@ struct MExtRowsReg {
 // One launch per layer is bound by launches and latency: a layer is a thin
 // shell, 222 of them at 256^3, 8 us each for gathers that move 11x the bytes
 // they need, after a counting sort of the faces by distance (0.32 ms); 1.96 ms
-// in all.  A brick in LDS takes all the layers that cross it in one visit:
-// 18 passes of 74 us (1.34 ms; 512^3: 10.2 -> 4.7 ms).  What bounds a pass is
-// a visit's latency, about 20 us (load 5, masks 3, sort 4, a layer 0.3).
+// in all (a 256^3 scene whose fluid fills a third of the box).  A brick in LDS
+// takes all the layers that cross it in one visit: 18 passes of 74 us there
+// (1.34 ms; 512^3: 10.2 -> 4.7 ms).  What bounds a pass is
+// a visit's latency, about 20 us (load 5, masks 3, sort 4, a layer 0.3).  Long
+// thin grids are chains of passes with one brick or a few each: 65000 x 1 x 1
+// faces from one end 55 ms in 2000 passes (by layers 274 ms), 30 x 30 x 2000 6.4
+// (6.1), and flat ones fill a sixteenth of a brick: 1000 x 1000 x 1 with a
+// thousandth known 1.04 (0.97), from a corner 3.4 (6.2).
 //
 // Which faces a visit can set: a face at distance L needs its neighbours at
 // distance L - 1 (a path down to a known face is a shortest one, so it is

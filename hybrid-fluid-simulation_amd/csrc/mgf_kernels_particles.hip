@@ -5,11 +5,14 @@
 // MixPICAndFLIP.cpp).
 //
 // Particle positions and per-particle vectors are interleaved x, y, z
-// (3 * i + k), as the reference stores them.  One work-item per particle.
-// Particle-to-grid sums use FP32 atomics as the reference does (in LDS, then
-// one per node and work-group), so their rounding depends on the order the
-// atomics land in; grid-to-particle sums,
-// counts and the advection are order-free and bitwise the oracle's.
+// (3 * i + k), as the reference stores them.  One work-item per particle,
+// where nothing else is said.  Particle-to-grid sums have no fixed order, as the
+// reference's FP32 atomics have none: the tile-sorted splat sums a cell's
+// particles in the order in which they were ranked in LDS, and adds every node
+// that a tile's particles touch to the fields by atomics (two a node, one for
+// P2GSUM, which has no weight); the unsorted one adds to LDS by atomics too.
+// Grid-to-particle sums, counts and the advection are order-free and bitwise
+// the oracle's.
 #include "mgf_internal.h"
 #include "mgf_kcommon.h"
 
@@ -117,7 +120,7 @@ __device__ __forceinline__ void for_corners(const PGrid& g, const PStencil& st, 
 // sums each cell's particles in the registers of one work-item (a slot per
 // corner) and adds the slots to a dense LDS tile of nodes one corner at a
 // time: for a fixed corner the cells' nodes are distinct, so plain adds do.
-// The tile is flushed with one global atomic per node touched.
+// The tile is flushed with global atomics, one a field and node touched.
 // 1.23M QUADRATIC particles on 101 x 83 x 61 cells, one field: 10.0 ms with an
 // LDS hash table of a work-group's nodes, 0.54 ms (after the same sort) with
 // LDS float atomics per corner, 0.081 ms this way (and 0.035 ms for the sort).

@@ -210,7 +210,11 @@ typedef struct mgf_scene_s*   mgf_scene;
 
 /* ---- context ------------------------------------------------------------ */
 /* Replaces CCudaContextManager::initCudaContext / freeCudaContext
- * (MPhysics/CudaContextManager.cpp:3-40). */
+ * (MPhysics/CudaContextManager.cpp:3-40).  A context keeps the scratch of
+ * mgf_op_extrapolate_fc and mgf_op_particles_to_grid from call to call: one
+ * device buffer of the largest call's size, at most 256 MB (a call that needs
+ * more, or finds it in use by another thread's call, allocates and frees its
+ * own).  mgf_shutdown frees it. */
 MGF_API mgf_status mgf_init(int32_t device, mgf_context* out);
 MGF_API mgf_status mgf_shutdown(mgf_context ctx);
 MGF_API const char* mgf_status_string(mgf_status s);
@@ -495,8 +499,11 @@ MGF_API mgf_status mgf_op_apply_forces(mgf_context ctx, const mgf_grid* grid,
  * field and weight (same extents) are zeroed, every particle adds
  * weight*values[span*i + offset] to the clamped corners of its kernel support
  * and the weight to `weight` (P2GSUM: the value to its own cell), then, with
- * normalize, field /= weight where weight > 0.  The sums are FP32 atomics, as
- * in the reference, so their rounding depends on the order they land in. */
+ * normalize, field /= weight where weight > 0.  The sums are FP32 and, as the
+ * reference's, in no fixed order: particles are first summed per work-group (in
+ * registers and LDS), then added to the fields by atomics.  Sets that are worth
+ * it are sorted by tile first, in scratch of 4 B a particle (at most 2^24 at a
+ * time) and 12 B a tile of 8^3 nodes; a call that cannot get it does not sort. */
 MGF_API mgf_status mgf_op_particles_to_grid(mgf_context ctx, const mgf_grid* grid, int32_t field_kind,
         int64_t n, const float* pos, const float* values, int32_t span, int32_t offset, int32_t alg,
         float* field, float* weight, int32_t normalize);
@@ -569,7 +576,9 @@ MGF_API mgf_status mgf_particles_advect(mgf_particles p, const mgf_grid* grid, c
  * (MixPICAndFLIP.cpp:64-134), on a particle set they borrow (it must outlive
  * the solver).  The solver holds the grid-shaped state of the reference class:
  * the previous output velocity (FLIP, MIX), the weight fields, and the flags
- * that make the first scalar / vector call seed the particles' values. */
+ * that make the first scalar / vector call seed the particles' values; also,
+ * LINEAR: the particles in bin order (28 B a particle) and a slot per bin and
+ * corner; QUADRATIC, CUBIC: the splat's scratch (mgf_op_particles_to_grid). */
 typedef struct mgf_psolver_s* mgf_psolver;
 #define MGF_PSOLVER_PIC  0
 #define MGF_PSOLVER_FLIP 1

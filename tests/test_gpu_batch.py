@@ -100,10 +100,12 @@ def compare_alone_with_batch(ctx, res, precond=mgf.PRECOND_MULTIGRID, mg_kernels
 @pytest.mark.parametrize("res", [(2, 2, 2), (9, 9, 9), (40, 25, 30), (64, 64, 64), (80, 80, 81), (82, 80, 80),
                                  (84, 80, 78)])
 def test_dot_products_finished_by_their_consumers(ctx, res, precond):
-    """A scene alone lets the kernels that need a dot product finish it (up to
-    512 partials, 512K cells: one less, that many and one more); in a batch each
-    is a launch of its own.  The same bits and counts, also when the iterations
-    end before the tolerance and when there is nothing to solve."""
+    """A scene alone lets the kernels that need a dot product finish it up to 512
+    partials; in a batch each is a launch of its own.  p . Ap and r . r (a partial
+    per 1024 cells) with counts up to the limit, at it and one above; r . z by
+    bricks on the small sizes (the next test has it on a march).  The same
+    bits and counts, also when the iterations end before the tolerance and when
+    there is nothing to solve."""
     compare_alone_with_batch(ctx, res, precond=precond)
 
 
