@@ -395,7 +395,8 @@ constexpr size_t kCoarseLdsMax = 131072;
 // MGF_MG_AUTO marches levels at least this large and takes bricks below
 // (150 x 61 x 97 interior, two steps: 4.28 ms with the line at 1M cells, which
 // leaves its 948K-cell level to bricks, 4.07 ms at 512K; at 3M cells the 130^3
-// level of a 128^3 scene goes to bricks: 4.80 -> 5.67 ms)
+// level of a 128^3 scene goes to bricks: 4.80 -> 5.67 ms; no line below 512K
+// was tried)
 constexpr size_t kMarchMinCells = size_t(1) << 19;
 
 // Blocks of a fused march resident at once: two per CU.
