@@ -231,7 +231,7 @@ struct mgf_psolver_s {
 
 namespace mgf {
 
-// Device scratch for one operator call on ctx (null: the allocation failed).
+// Device scratch for one operator call on ctx (null: none asked for, or the allocation failed).
 struct OpScratch {
     OpScratch(mgf_context ctx, size_t bytes);
     ~OpScratch();   // the context's stream must have finished with it

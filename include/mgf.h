@@ -503,7 +503,7 @@ MGF_API mgf_status mgf_op_apply_forces(mgf_context ctx, const mgf_grid* grid,
  * reference's, in no fixed order: particles are first summed per work-group (in
  * registers and LDS), then added to the fields by atomics.  Sets that are worth
  * it are sorted by tile first, in scratch of 4 B a particle (at most 2^24 at a
- * time) and 12 B a tile of 8^3 nodes; a call that cannot get it does not sort. */
+ * time) and 20 B a tile of 8^3 nodes; a call that cannot get it does not sort. */
 MGF_API mgf_status mgf_op_particles_to_grid(mgf_context ctx, const mgf_grid* grid, int32_t field_kind,
         int64_t n, const float* pos, const float* values, int32_t span, int32_t offset, int32_t alg,
         float* field, float* weight, int32_t normalize);
